@@ -4,7 +4,7 @@
 //   k_syrk_f64     Pi_w = R^T diag(c_w) R on v_mfma_f64_16x16x4_f64, one R tile in
 //                  LDS shared by 4 waves = 4 frequencies  (dgemm of rpa_core_MO.f90:402)
 //   k_set_diag     diag_w (tr Pi, rpa_CC.f90:444-447); Pi_w[P][P] += 1 (448-450)
-//   k_potrf_diag   Cholesky + inverse of a 64x64 diagonal block (one wave)
+//   k_potrf_diag   Cholesky + inverse of a 64x64 diagonal block (four waves)
 //   k_trsm         L21 = A21 L11^{-T} on MFMA
 //   k_chol_update  trailing update A22 -= L21 L21^T on MFMA
 //   k_energy       E = sum_w w/(2 pi) (2 sum log L_kk - tr Pi_w)  (rpa_CC.f90:451-453)
@@ -219,7 +219,7 @@ int launch_set_diag(brpa_ctx *ctx, const FragDev *fr, const int64_t *pre, int nf
 // ---------------------------------------------------------------------------
 // Blocked right-looking Cholesky of A_w = 1 + Pi_w (lower triangle, row-major),
 // three launches per 64-column step j (j0 = 64 j):
-//   k_potrf_diag   one wave per matrix: factors the diagonal block in LDS,
+//   k_potrf_diag   one work-group per matrix: factors the diagonal block in LDS,
 //                  writes its log-det partial and L11^{-1} (own buffer; A11
 //                  itself is never written back, so no work-group of the same
 //                  step can read a half-factored block)
@@ -345,123 +345,229 @@ __device__ __forceinline__ double wave_bcast(double v, int l) {
     return __hiloint2double(hi, lo);
 }
 
-// Diagonal block of step `step` of matrix w with one wave, left-looking: lane
-// r keeps row r of the 64 x 64 block in registers.  At column c every lane
-// subtracts the dot product of its row with row c (rows of L are complete up
-// to column c - 1 and are read from LDS as broadcast ds_read_b128, four
-// partial sums), the pivot comes from lane c by readlane, and the finished
-// column goes to LDS.  No barrier inside the factorisation (one wave).  Then
-// column `lane` of L11^{-1} by forward substitution over the rows of L in LDS
-// (reciprocal diagonal precomputed; uniform loops, x_k = 0 above the lane's
-// column).  Outputs: linv, log-det partial, status, optional L11 write-back.
-__global__ __launch_bounds__(64) void k_potrf_diag(const FragDev *__restrict__ fr,
-                                                  const int64_t *__restrict__ pre, int nfrag,
-                                                  int step) {
-    // row pitch 66 doubles: 16-byte aligned rows; broadcast reads are conflict-free
+// 1 / p for p within 2^-1000 .. 2^1000: the hardware estimate and two Newton
+// steps (5 dependent instructions instead of the ~12 of a division)
+__device__ __forceinline__ double rcp_newton(double p) {
+    double x = __builtin_amdgcn_rcp(p);
+    x = fma(fma(-p, x, 1.0), x, x);
+    return fma(fma(-p, x, 1.0), x, x);
+}
+
+// Diagonal block of step `step` of matrix w, one work-group of four waves per
+// matrix.  The 64 x 64 block sits in LDS as 4 x 4 blocks of 16:
+//   panel p     wave 0: lane r holds row r of the 16 panel columns in registers
+//               and eliminates column by column.  The multiplier is a(r, c) /
+//               pivot, and the row of the pivot comes from lanes c+1 .. by
+//               readlane (the block is symmetric), so no LDS access and no
+//               square root lies between two pivots; the columns are scaled by
+//               1 / sqrt(pivot) at the end, all 16 at once.
+//   column p+1  waves 1-3: A(i, p+1) -= L(i, p) L(p+1, p)^T on MFMA
+//   the other blocks right of it by waves 1-3 while wave 0 runs panel p+1
+//   L11^{-1}    wave j: L(j, j)^{-1} by substitution (lane n: column n), then block
+//               column j on MFMA, X(i, j) = -X(i, i) sum_k L(i, k)
+//               X(k, j).  The accumulator layout of X(k, j) is the operand layout
+//               of the next product, so the column stays in registers.
+// Outputs: linv, log-det partial, status, optional L11 write-back.
+//
+// Bound by latency: 64 pivots in a chain of readlane, reciprocal, multiply and
+// fma.  Measured per launch on MI355X: 17.7 us for 16 matrices, 20.7 us for 512
+// (61.3 and 65.4 us for one left-looking wave per matrix with rows of L from LDS,
+// the square root and division in the chain and the whole inverse by substitution).
+__global__ __launch_bounds__(256) void k_potrf_diag(const FragDev *__restrict__ fr,
+                                                   const int64_t *__restrict__ pre, int nfrag,
+                                                   int step) {
+    // row pitch 66 doubles: 16-byte aligned rows, 16 rows on 16 distinct 4-bank groups
     constexpr int LP = CHOL_NB + 2;
-    __shared__ __attribute__((aligned(16))) double L[CHOL_NB][LP];
+    constexpr int XP = 18;
+    __shared__ __attribute__((aligned(16))) double S[CHOL_NB][LP];
+    __shared__ __attribute__((aligned(16))) double Xd[4][16][XP];   // L(p, p)^{-1}
     __shared__ double rdiag[CHOL_NB];
     __shared__ int64_t s_pre[FIND_LDS_MAX + 1];
     const int64_t b = blockIdx.x;
     const int f = find_frag_lds(pre, nfrag, b, s_pre);
     const int w = (int)(b - (nfrag <= FIND_LDS_MAX ? s_pre[f] : pre[f]));
     const FragDev &F = fr[f];
-    const int lane = threadIdx.x;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     const int N = F.N;
     const int j0 = step * CHOL_NB;
     const int nbj = min(CHOL_NB, N - j0);
     double *A = F.Pi + (int64_t)w * N * N;
-    // row `lane` of the block straight into registers, lower triangle only (the
-    // other triangle is never read); rows/cols past nbj padded with the identity
-    double a[CHOL_NB];
-    const gdouble_t *Arow = (const gdouble_t *)(A + (int64_t)(j0 + min(lane, nbj - 1)) * N + j0);
+    const gdouble_t *G = (const gdouble_t *)A;
+    // lower triangle only (the other one is never read); rows and columns past
+    // nbj are those of the identity
+    {
+        double v[16];
 #pragma unroll
-    for (int c = 0; c < CHOL_NB; ++c) {
-        const bool in = lane < nbj && c < nbj;
-        const double v = (in && c <= lane) ? Arow[min(c, nbj - 1)] : 0.0;
-        a[c] = in ? v : (lane == c ? 1.0 : 0.0);
-    }
-    int bad = 0;
-#pragma unroll
-    for (int c = 0; c < CHOL_NB; ++c) {
-        if (c > 0) {
-            // a[c] -= sum_{k<c} L[lane][k] L[c][k]; row c of L from LDS
-            double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
-#pragma unroll
-            for (int k = 0; k < c; k += 4) {
-                const d2v_t u = *reinterpret_cast<const d2v_t *>(&L[c][k]);
-                s0 = fma(a[k], u.x, s0);
-                if (k + 1 < c) s1 = fma(a[k + 1], u.y, s1);
-                if (k + 2 < c) {
-                    const d2v_t u2 = *reinterpret_cast<const d2v_t *>(&L[c][k + 2]);
-                    s2 = fma(a[k + 2], u2.x, s2);
-                    if (k + 3 < c) s3 = fma(a[k + 3], u2.y, s3);
-                }
-            }
-            a[c] -= (s0 + s1) + (s2 + s3);
+        for (int u = 0; u < 16; ++u) {
+            const int r = wave + 4 * u;
+            const bool in = r < nbj && lane <= r;
+            v[u] = G[in ? (int64_t)(j0 + r) * N + j0 + lane : 0];
+            v[u] = in ? v[u] : ((r >= nbj && lane == r) ? 1.0 : 0.0);
         }
-        double piv = wave_bcast(a[c], c);
-        if (!(piv > 0.0) || !isfinite(piv)) {
-            bad = 1;
-            piv = 1.0;
-        }
-        const double d = sqrt(piv);
-        const double rd = 1.0 / d;
-        // lanes above row c hold values of the upper triangle, never read
-        a[c] = (lane == c) ? d : a[c] * rd;
-        L[lane][c] = a[c];
-        if (lane == c) rdiag[c] = rd;
-        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int u = 0; u < 16; ++u) S[wave + 4 * u][lane] = v[u];
     }
     __syncthreads();
-    // column `lane` of X = L11^{-1}: x_i = (delta_i,lane - sum_{k<i} L_ik x_k) / L_ii,
-    // x_i = 0 for i < lane; a[] now holds x
+    const int l16 = lane & 15, g4 = lane >> 4;
+    // S(i, j) -= L(i, p) L(j, p)^T for 16 x 16 blocks
+    auto update = [&](int i, int j, int p) {
+        d4_t acc;
 #pragma unroll
-    for (int i = 0; i < CHOL_NB; ++i) {
-        double s0 = (i == lane) ? 1.0 : 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
+        for (int r = 0; r < 4; ++r) acc[r] = S[16 * i + g4 + 4 * r][16 * j + l16];
 #pragma unroll
-        for (int k = 0; k < i; k += 4) {
-            const d2v_t u = *reinterpret_cast<const d2v_t *>(&L[i][k]);
-            s0 = fma(-u.x, a[k], s0);
-            if (k + 1 < i) s1 = fma(-u.y, a[k + 1], s1);
-            if (k + 2 < i) {
-                const d2v_t u2 = *reinterpret_cast<const d2v_t *>(&L[i][k + 2]);
-                s2 = fma(-u2.x, a[k + 2], s2);
-                if (k + 3 < i) s3 = fma(-u2.y, a[k + 3], s3);
+        for (int s = 0; s < 4; ++s)
+            acc = __builtin_amdgcn_mfma_f64_16x16x4f64(-S[16 * i + l16][16 * p + 4 * s + g4],
+                                                       S[16 * j + l16][16 * p + 4 * s + g4], acc, 0,
+                                                       0, 0);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) S[16 * i + g4 + 4 * r][16 * j + l16] = acc[r];
+    };
+    // column l16 of L(p, p)^{-1}: x_i = (delta_in - sum_{k<i} L_ik x_k) / L_ii
+    auto invert = [&](int p) {
+        double x[16];
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            double s0 = i == l16 ? 1.0 : 0.0, s1 = 0.0;
+#pragma unroll
+            for (int k = 0; k < i; k += 2) {
+                const d2v_t u = *reinterpret_cast<const d2v_t *>(&S[16 * p + i][16 * p + k]);
+                s0 = fma(-u.x, x[k], s0);
+                if (k + 1 < i) s1 = fma(-u.y, x[k + 1], s1);
             }
+            x[i] = (s0 + s1) * rdiag[16 * p + i];
         }
-        a[i] = ((s0 + s1) + (s2 + s3)) * rdiag[i];
-        __builtin_amdgcn_sched_barrier(0);
+        if (lane < 16)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) Xd[p][i][l16] = x[i];
+    };
+    int bad = 0;
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+        if (wave == 0) {
+            double a[16];
+            d2v_t *row = reinterpret_cast<d2v_t *>(&S[lane][16 * p]);
+#pragma unroll
+            for (int t = 0; t < 8; ++t) {
+                const d2v_t u = row[t];
+                a[2 * t] = u.x;
+                a[2 * t + 1] = u.y;
+            }
+            double mypiv = 1.0;
+            bool inrange = true;
+#pragma unroll
+            for (int c = 0; c < 16; ++c) {
+                const double piv = wave_bcast(a[c], 16 * p + c);
+                inrange = inrange && piv >= 0x1p-1000 && piv <= 0x1p+1000;
+                const double m = a[c] * rcp_newton(piv);
+                mypiv = lane == 16 * p + c ? piv : mypiv;
+                // lanes above row j update entries of the upper triangle, never read
+#pragma unroll
+                for (int j = c + 1; j < 16; ++j)
+                    a[j] = fma(-m, wave_bcast(a[c], 16 * p + j), a[j]);
+            }
+            if (!inrange) {
+                // a pivot that is not positive, or outside the range of rcp_newton: the
+                // panel again, on its columns in LDS, with divisions
+#pragma unroll 1
+                for (int c = 0; c < 16; ++c) {
+                    const int pc = 16 * p + c;
+                    double piv = S[pc][pc];
+                    if (!(piv > 0.0) || !isfinite(piv)) {
+                        bad = 1;
+                        piv = 1.0;
+                    }
+                    mypiv = lane == pc ? piv : mypiv;
+                    const double m = S[lane][pc] / piv;
+#pragma unroll 1
+                    for (int j = c + 1; j < 16; ++j)
+                        if (lane >= 16 * p + j)
+                            S[lane][16 * p + j] = fma(-m, S[16 * p + j][pc], S[lane][16 * p + j]);
+                }
+#pragma unroll
+                for (int t = 0; t < 8; ++t) {
+                    const d2v_t u = row[t];
+                    a[2 * t] = u.x;
+                    a[2 * t + 1] = u.y;
+                }
+            }
+            const double d = sqrt(mypiv), rd = 1.0 / d;
+#pragma unroll
+            for (int c = 0; c < 16; ++c)
+                a[c] = lane == 16 * p + c ? d : a[c] * wave_bcast(rd, 16 * p + c);
+            if (lane >= 16 * p) {
+#pragma unroll
+                for (int t = 0; t < 8; ++t) row[t] = (d2v_t){a[2 * t], a[2 * t + 1]};
+                if (lane < 16 * p + 16) rdiag[lane] = rd;
+            }
+        } else {
+            // panel p - 1: the blocks right of column p
+            if (p == 1) update(wave == 1 ? 2 : 3, wave == 3 ? 3 : 2, 0);
+            if (p == 2 && wave == 1) update(3, 3, 1);
+        }
+        __syncthreads();
+        if (p < 3) {
+            if (wave > p) update(wave, p + 1, p);
+            __syncthreads();
+        }
     }
     double *linv = F.linv + (int64_t)w * CHOL_NB * CHOL_NB;
+    invert(wave);
+    if (wave == 3) {
+        // log-det partial: one log per lane, then a fixed butterfly in double-double
+        dd_t sl = {lane < nbj ? log(S[lane][lane]) : 0.0, 0.0};
 #pragma unroll
-    for (int i = 0; i < CHOL_NB; ++i) linv[i * CHOL_NB + lane] = a[i];
+        for (int off = 32; off > 0; off >>= 1) {
+            const dd_t o = {__shfl_xor(sl.hi, off), __shfl_xor(sl.lo, off)};
+            sl = dd_add(sl, o);
+        }
+        if (lane == 0) {
+            double *part = F.ldpart + ((int64_t)w * F.nsteps + step) * 2;
+            part[0] = sl.hi;
+            part[1] = sl.lo;
+        }
+    }
     if (F.keep_l11) {
-        // the factored block back into Pi (lower triangle and diagonal), one
-        // row per pass with the lanes along the columns; no other work item
-        // reads this diagonal block
-        for (int r = 0; r < nbj; ++r)
-            if (lane <= r) A[(int64_t)(j0 + r) * N + j0 + lane] = L[r][lane];
+        // the factored block back into Pi (lower triangle and diagonal); no
+        // other work item reads this diagonal block
+        for (int r = wave; r < nbj; r += 4)
+            if (lane <= r) A[(int64_t)(j0 + r) * N + j0 + lane] = S[r][lane];
     }
-    // log-det partial: one log per lane, then a fixed butterfly in double-double
-    dd_t sl = {lane < nbj ? log(L[lane][lane]) : 0.0, 0.0};
+    __syncthreads();
+    // block column `wave` of L11^{-1}; x[k] holds X(k, wave) as l16 = column,
+    // g4 + 4 r = row, which is also the B operand of step r
+    d4_t x[4];
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-        const dd_t o = {__shfl_xor(sl.hi, off), __shfl_xor(sl.lo, off)};
-        sl = dd_add(sl, o);
+    for (int i = 0; i < 4; ++i) {
+        x[i] = (d4_t){0.0, 0.0, 0.0, 0.0};
+        if (i == wave) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) x[i][r] = Xd[i][g4 + 4 * r][l16];
+        } else if (i > wave) {
+            d4_t t = (d4_t){0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+            for (int k = 0; k < i; ++k)
+                if (k >= wave)
+#pragma unroll
+                    for (int s = 0; s < 4; ++s)
+                        t = __builtin_amdgcn_mfma_f64_16x16x4f64(S[16 * i + l16][16 * k + 4 * s + g4],
+                                                                 x[k][s], t, 0, 0, 0);
+#pragma unroll
+            for (int s = 0; s < 4; ++s)
+                x[i] = __builtin_amdgcn_mfma_f64_16x16x4f64(-Xd[i][l16][4 * s + g4], t[s], x[i], 0,
+                                                            0, 0);
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            linv[(16 * i + g4 + 4 * r) * CHOL_NB + 16 * wave + l16] = x[i][r];
     }
-    if (lane == 0) {
-        double *part = F.ldpart + ((int64_t)w * F.nsteps + step) * 2;
-        part[0] = sl.hi;
-        part[1] = sl.lo;
-    }
-    if (lane == 0 && bad) F.status[w] = 1;
+    if (threadIdx.x == 0 && bad) F.status[w] = 1;
 }
 
 int launch_potrf_diag(brpa_ctx *ctx, const FragDev *fr, const int64_t *pre, int nfrag,
                       int64_t total, int step) {
     if (total <= 0) return BRPA_OK;
-    hipLaunchKernelGGL(k_potrf_diag, dim3(grid1(total)), dim3(64), 0, ctx->stream, fr, pre, nfrag,
+    hipLaunchKernelGGL(k_potrf_diag, dim3(grid1(total)), dim3(256), 0, ctx->stream, fr, pre, nfrag,
                        step);
     LAUNCH_CHECK(ctx);
     return BRPA_OK;
