@@ -97,7 +97,7 @@ Counts counts_of(const HostFrag &f, int nsteps_max, int precision, int i8_varian
     const int64_t nt16 = cdiv(N, 128);
     c.syrk16 = (precision == BRPA_SPLIT_BF16) ? F * (nt16 * (nt16 + 1) / 2) : 0;
     const bool i8 = precision == BRPA_SPLIT_I8;
-    c.colscale8 = i8 ? cdiv(N, 64) : 0;
+    c.colscale8 = i8 ? cdiv(K, CS_ROWS) * cdiv(N, 64) : 0;
     c.split8 = i8 ? cdiv(K, I8_KB) * cdiv(N, 64) : 0;
     for (int v = 0; v < I8V_COUNT; ++v) {
         const int64_t t = cdiv(N, syrk_i8_tile(v));
@@ -125,7 +125,7 @@ size_t frag_bytes(const HostFrag &h, int precision) {
     }
     if (precision == BRPA_SPLIT_I8) {
         size_t kpad = cdiv(K, I8_KB) * I8_KB;
-        b += F * NSLICE * N * kpad + 8 * F * N + 8 * F * K;
+        b += F * NSLICE * N * kpad + 8 * F * N + 8 * F * K + 24 * cdiv(K, CS_ROWS) * F * N;
     }
     return b;
 }
@@ -237,6 +237,7 @@ int run_chunk(brpa_ctx *ctx, int precision, const std::vector<HostFrag> &fr, dou
                 d.sdtab = ar.take<double>((size_t)F * K);
                 d.sl8 = ar.take<int8_t>((size_t)F * NSLICE * N * d.Kpad8);
                 d.scale8 = ar.take<double>((size_t)F * N);
+                d.dpart = ar.take<double>((size_t)cdiv(K, CS_ROWS) * F * N * 3);
             }
             if (ar.base) hd[f] = d;
         }
@@ -285,7 +286,7 @@ int run_chunk(brpa_ctx *ctx, int precision, const std::vector<HostFrag> &fr, dou
             BRPA_TRY(se(BRPA_STAGE_PI));
         } else if (precision == BRPA_SPLIT_I8) {
             BRPA_TRY(sb(BRPA_STAGE_SPLIT));
-            BRPA_TRY(launch_colscale_i8(ctx, d_fr, DP(5), nfrag, TOT(5)));
+            BRPA_TRY(launch_colscale_i8(ctx, d_fr, DP(5), nfrag, TOT(5), DP(2), TOT(2)));
             BRPA_TRY(launch_split_i8(ctx, d_fr, DP(6), nfrag, TOT(6)));
             BRPA_TRY(se(BRPA_STAGE_SPLIT));
             BRPA_TRY(sb(BRPA_STAGE_PI));

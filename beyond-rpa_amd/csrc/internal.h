@@ -180,7 +180,8 @@ struct FragDev {
     double *energy;          // 1 (device)
     int *status;             // F Cholesky status (0 ok)
     double *linv;            // F x 64 x 64 inverse of the current diagonal block
-    double *dpart;           // split-BF16: F x nblk x N x 2 double-double diagonal partials
+    double *dpart;           // split-BF16: F x nblk x N x 2 double-double diagonal partials;
+                             // split-int8: ceil(K/CS_ROWS) x F x N x {column max, diagonal hi, lo}
     int K, N, F, nsteps;
     int nocc, nvir;
     const double *eocc, *evir, *freqs;   // device copies
@@ -206,6 +207,7 @@ constexpr int SYRK_T = 64;    // FP64 SYRK tile
 constexpr int SPLIT_KB = 128; // split-BF16 exactness block (rows per scale)
 constexpr int NSLICE = 4;     // bf16 (or int8) slices per FP64 value in the split forms
 constexpr int I8_KB = 128;    // split-int8: rows per split work-group (Kpad8 is a multiple)
+constexpr int CS_ROWS = 512;   // split-int8: rows per work-group of the column pass
 constexpr int I8_KMAX = 65536;// split-int8: largest K with exact int32 level sums
 
 // Launch wrappers (defined in the kernel files).  `pre` arrays are device
@@ -226,7 +228,9 @@ int launch_energy(brpa_ctx *, const FragDev *, int nfrag);
 int launch_fill_int(brpa_ctx *, int *p, int64_t n, int v);
 int launch_split(brpa_ctx *, const FragDev *, const int64_t *pre, int nfrag, int64_t total);
 int launch_syrk_bf16(brpa_ctx *, const FragDev *, const int64_t *pre, int nfrag, int64_t total);
-int launch_colscale_i8(brpa_ctx *, const FragDev *, const int64_t *pre, int nfrag, int64_t total);
+// pre_fin / total_fin: work-groups of ceil(F*N/256) (the pass over the row chunks' partials)
+int launch_colscale_i8(brpa_ctx *, const FragDev *, const int64_t *pre, int nfrag, int64_t total,
+                       const int64_t *pre_fin, int64_t total_fin);
 int launch_split_i8(brpa_ctx *, const FragDev *, const int64_t *pre, int nfrag, int64_t total);
 // split-int8 product kernel variants (chosen per fragment-size bucket by the
 // autotuner): 128x128 tiles in launch order, the same with one contiguous tile

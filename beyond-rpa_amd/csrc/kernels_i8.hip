@@ -34,108 +34,138 @@ typedef __attribute__((address_space(1))) const double gdbl_t;
 typedef int v4i_t __attribute__((ext_vector_type(4)));
 
 // ---------------------------------------------------------------------------
-// Column pass.  Work-groups per fragment: ceil(N/64).  Thread tid handles
-// column P0 + tid%64 and rows tid/64 + 4 i; frequencies in groups of 16.
-// For each (w, P): scale8 = max_k |sqrt(c_w(k)) R[k][P]| / 127 and
+// Column pass.  For each (w, P): scale8 = max_k |sqrt(c_w(k)) R[k][P]| / 127 and
 // diag = sum_k c_w(k) R[k][P]^2 in double-double (rpa_CC.f90:444-447 sums the
-// trace in REAL(F128)).
-constexpr int CS_WG = 16;   // frequencies per register group
+// trace in REAL(F128)).  Work-groups per fragment: ceil(K/512) row chunks x
+// ceil(N/64) column groups; a lane holds one column, each wave walks a quarter
+// of the chunk's rows eight at a time, and the two tables come as scalar loads
+// (the row is the same for the whole wave).  Frequencies in groups of 8: their
+// maxima and sums stay in 48 registers.  The four waves are combined in LDS in
+// wave order, and k_colscale_fin_i8 adds the chunks in order.
+//
+// Bound by FP64 VALU work (about 13 operations per element and frequency).
+// At K = 10800, N = 1800, 24 frequencies the two kernels take 350 us; one
+// work-group per 64 columns over all of K kept 29 of 256 CUs busy there (4809 us).
+// Over 32 fragments of the batch shapes: 1361 us, before 3359.
+constexpr int CS_WG = 16;       // frequencies per group of the split pass
+constexpr int CSF = 8;          // frequencies per register group of the column pass
+constexpr int CSR = 8;          // rows per step of a wave
+typedef __attribute__((address_space(4))) const double cdbl_t;
 
 __global__ __launch_bounds__(256) void k_colscale_i8(const FragDev *__restrict__ fr,
                                                     const int64_t *__restrict__ pre, int nfrag) {
-    constexpr int CH = 64;   // rows per table chunk staged in LDS
     __shared__ int64_t s_pre[FIND_LDS_MAX + 1];
-    __shared__ double sSD[CS_WG][CH], sCD[CS_WG][CH];
-    __shared__ double sM[4][64], sH[4][64], sL[4][64];
+    __shared__ double sM[4][4][64], sH[4][4][64], sL[4][4][64];
     const int64_t b = blockIdx.x;
-    const int f = find_frag_lds(pre, nfrag, b, s_pre);
+    const int f = __builtin_amdgcn_readfirstlane(find_frag_lds(pre, nfrag, b, s_pre));
     const FragDev &F = fr[f];
-    const int N = F.N, K = F.K;
-    const int P0 = (int)(b - (nfrag <= FIND_LDS_MAX ? s_pre[f] : pre[f])) * 64;
-    const int tid = threadIdx.x, c = tid & 63, g = tid >> 6;
+    const int N = F.N, K = F.K, nF = F.F;
+    const int ncg = (N + 63) / 64;
+    const int lb = __builtin_amdgcn_readfirstlane(
+        (int)(b - (nfrag <= FIND_LDS_MAX ? s_pre[f] : pre[f])));
+    const int ck = lb / ncg, P0 = (lb - ck * ncg) * 64;
+    const int c = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     const int P = P0 + c;
     const bool colok = P < N;
-    const gdbl_t *R = (const gdbl_t *)F.R;
-    const gdbl_t *SD = (const gdbl_t *)F.sdtab;
-    const gdbl_t *CD = (const gdbl_t *)F.dtab;
-    for (int w0 = 0; w0 < F.F; w0 += CS_WG) {
-        const int nw = min(CS_WG, F.F - w0);
-        double m[CS_WG];
-        dd_t ds[CS_WG];
+    const gdbl_t *R = (const gdbl_t *)F.R + (colok ? P : 0);
+    const int kb = ck * CS_ROWS + wave * (CS_ROWS / 4), ke = min(K, kb + CS_ROWS / 4);
+    for (int w0 = 0; w0 < nF; w0 += CSF) {
+        const int nw = min(CSF, nF - w0);
+        const cdbl_t *SD = (const cdbl_t *)(uintptr_t)F.sdtab + (int64_t)w0 * K;
+        const cdbl_t *CD = (const cdbl_t *)(uintptr_t)F.dtab + (int64_t)w0 * K;
+        double m[CSF], hi[CSF], lo[CSF];
 #pragma unroll
-        for (int i = 0; i < CS_WG; ++i) {
-            m[i] = 0.0;
-            ds[i] = (dd_t){0.0, 0.0};
-        }
-        for (int k0 = 0; k0 < K; k0 += CH) {
-            // this chunk's rows of the two tables (zeros past K or past nw)
-            __syncthreads();
-            for (int e = tid; e < CS_WG * CH; e += 256) {
-                const int i = e / CH, r = e - i * CH;
-                const bool ok = i < nw && k0 + r < K;
-                const int64_t idx = ok ? (int64_t)(w0 + i) * K + k0 + r : 0;
-                const double sd = SD[idx], cd = CD[idx];
-                sSD[i][r] = ok ? sd : 0.0;
-                sCD[i][r] = ok ? cd : 0.0;
+        for (int i = 0; i < CSF; ++i) m[i] = hi[i] = lo[i] = 0.0;
+        auto step = [&](double x, double r2, double r2e, double sd, double cw, int i) {
+            m[i] = fmax(m[i], fabs(x * sd));
+            const double p = cw * r2, pe = fma(cw, r2, -p) + cw * r2e;
+            // TwoSum of hi and p; the errors collect in lo
+            const double s = hi[i] + p, bb = s - hi[i];
+            lo[i] += ((hi[i] - (s - bb)) + (p - bb)) + pe;
+            hi[i] = s;
+        };
+        int k = kb;
+        for (; k + CSR <= ke; k += CSR) {
+            double x[CSR], r2[CSR], r2e[CSR];
+#pragma unroll
+            for (int r = 0; r < CSR; ++r) x[r] = R[(int64_t)(k + r) * N];
+#pragma unroll
+            for (int r = 0; r < CSR; ++r) {
+                r2[r] = x[r] * x[r];
+                r2e[r] = fma(x[r], x[r], -r2[r]);
             }
-            // this thread's 16 rows of the chunk (rows g + 4 j), loads first
-            double rv[CH / 4];
 #pragma unroll
-            for (int j = 0; j < CH / 4; ++j) {
-                const int k = k0 + g + 4 * j;
-                const bool ok = colok && k < K;
-                rv[j] = R[ok ? (int64_t)k * N + P : 0];
-                rv[j] = ok ? rv[j] : 0.0;
-            }
-            __syncthreads();
-#pragma unroll 2
-            for (int j = 0; j < CH / 4; ++j) {
-                const int r = g + 4 * j;
-                const double x = rv[j];
-                const double r2 = x * x, r2e = fma(x, x, -r2);
+            for (int i = 0; i < CSF; ++i)
+                if (i < nw) {
 #pragma unroll
-                for (int i = 0; i < CS_WG; ++i) {
-                    const double y = x * sSD[i][r];
-                    m[i] = fmax(m[i], fabs(y));
-                    const double cw = sCD[i][r];
-                    const double p = cw * r2, pe = fma(cw, r2, -p) + cw * r2e;
-                    ds[i] = dd_add(ds[i], p);
-                    ds[i].lo += pe;
+                    for (int r = 0; r < CSR; ++r)
+                        step(x[r], r2[r], r2e[r], SD[i * K + k + r], CD[i * K + k + r], i);
                 }
-            }
         }
-        // combine the 4 row groups, one frequency at a time
-        for (int i = 0; i < nw; ++i) {
-            double mi = m[0], hi = ds[0].hi, lo = ds[0].lo;
+        for (; k < ke; ++k) {
+            const double x = R[(int64_t)k * N], r2 = x * x, r2e = fma(x, x, -r2);
 #pragma unroll
-            for (int q = 1; q < CS_WG; ++q)
-                if (q == i) {
-                    mi = m[q];
-                    hi = ds[q].hi;
-                    lo = ds[q].lo;
-                }
-            sM[g][c] = mi;
-            sH[g][c] = hi;
-            sL[g][c] = lo;
+            for (int i = 0; i < CSF; ++i)
+                if (i < nw) step(x, r2, r2e, SD[i * K + k], CD[i * K + k], i);
+        }
+        // combine the four waves, four frequencies at a time
+#pragma unroll
+        for (int i0 = 0; i0 < CSF; i0 += 4) {
             __syncthreads();
-            if (tid < 64 && colok) {
-                const double mm = fmax(fmax(sM[0][c], sM[1][c]), fmax(sM[2][c], sM[3][c]));
-                dd_t t = {sH[0][c], sL[0][c]};
-                for (int q = 1; q < 4; ++q) t = dd_add(t, (dd_t){sH[q][c], sL[q][c]});
-                const int64_t o = (int64_t)(w0 + i) * N + P;
-                F.scale8[o] = mm / 127.0;
-                F.diag[o] = t.hi + t.lo;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                sM[wave][i][c] = m[i0 + i];
+                sH[wave][i][c] = hi[i0 + i];
+                sL[wave][i][c] = lo[i0 + i];
             }
             __syncthreads();
+            const int w = w0 + i0 + wave;
+            if (w < nF && colok) {
+                const double mm = fmax(fmax(sM[0][wave][c], sM[1][wave][c]),
+                                       fmax(sM[2][wave][c], sM[3][wave][c]));
+                dd_t t = {sH[0][wave][c], sL[0][wave][c]};
+#pragma unroll
+                for (int q = 1; q < 4; ++q) t = dd_add(t, (dd_t){sH[q][wave][c], sL[q][wave][c]});
+                double *o = F.dpart + (((int64_t)ck * nF + w) * N + P) * 3;
+                o[0] = mm;
+                o[1] = t.hi;
+                o[2] = t.lo;
+            }
         }
     }
 }
 
+// scale8 and diag from the row chunks' partials, in chunk order.  Work-groups
+// per fragment: ceil(F*N/256).
+__global__ __launch_bounds__(256) void k_colscale_fin_i8(const FragDev *__restrict__ fr,
+                                                        const int64_t *__restrict__ pre,
+                                                        int nfrag) {
+    const int64_t b = blockIdx.x;
+    const int f = find_frag(pre, nfrag, b);
+    const FragDev &F = fr[f];
+    const int64_t e = (b - pre[f]) * 256 + threadIdx.x, FN = (int64_t)F.F * F.N;
+    if (e >= FN) return;
+    const int nck = (F.K + CS_ROWS - 1) / CS_ROWS;
+    double m = 0.0;
+    dd_t t = {0.0, 0.0};
+    for (int q = 0; q < nck; ++q) {
+        const double *o = F.dpart + ((int64_t)q * FN + e) * 3;
+        m = fmax(m, o[0]);
+        t = dd_add(t, (dd_t){o[1], o[2]});
+    }
+    F.scale8[e] = m / 127.0;
+    F.diag[e] = t.hi + t.lo;
+}
+
 int launch_colscale_i8(brpa_ctx *ctx, const FragDev *fr, const int64_t *pre, int nfrag,
-                       int64_t total) {
+                       int64_t total, const int64_t *pre_fin, int64_t total_fin) {
     if (total <= 0) return BRPA_OK;
     hipLaunchKernelGGL(k_colscale_i8, dim3((unsigned)total), dim3(256), 0, ctx->stream, fr, pre,
                        nfrag);
+    LAUNCH_CHECK(ctx);
+    hipLaunchKernelGGL(k_colscale_fin_i8, dim3((unsigned)total_fin), dim3(256), 0, ctx->stream, fr,
+                       pre_fin, nfrag);
     LAUNCH_CHECK(ctx);
     return BRPA_OK;
 }
