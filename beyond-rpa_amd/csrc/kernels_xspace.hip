@@ -91,30 +91,35 @@ int launch_ritz_resid(brpa_ctx *ctx, const double *AZ, const double *Z, const do
 }
 
 // ---------------------------------------------------------------------------
-// Exchange contraction from an explicit Coulomb matrix G = R R^T (K x K,
-// column-major, upper triangle and diagonal valid):
-//   part[c] = sum_{r <= c} w_rc G(r, c) (gamma M(r', c') + delta [r == c]),
-//   r = i v + a, c = j v + b, r' = j v + a, c' = i v + b, w = 2 (r < c), 1 (r = c).
-// G and the symmetric T2 matrix M are both symmetric and so is the permuted
-// M, so the upper triangle with these weights is the full sum.  One work-group
-// per column c; its rows r <= c run as (i, a) with i <= j, so the reads of G
-// (column c) and of M (column c' = i v + b, rows j v + a) are contiguous in a.
-// Fixed-order reduction (per-thread sums, wave butterfly, the waves in order).
-__global__ __launch_bounds__(256) void k_sosex_contract(const double *__restrict__ G, int64_t K,
-                                                        int v, const double *__restrict__ M,
+// Exchange contraction from explicit blocks of the Coulomb matrix G = R R^T and of
+// the symmetric amplitude matrix M, for the occupied ranges I (ni indices) and J:
+//   part[c] = sum_r w_rc G(r, c) (gamma M(r', c') + delta [r == c]),
+//   r = i v + a, c = j v + b, r' = j v + a, c' = i v + b  (i, j counted in I, J).
+// G holds the rows of I and columns of J, M the rows of J and columns of I.
+// ni == 0: I = J, the rows r <= c with w = 2 (r < c), 1 (r = c).  G and M are
+// symmetric and so is the permuted M, so the upper triangle with these weights is
+// the full sum; only the upper triangle of G is read.  Otherwise all rows with
+// w = 2 (the block J, I adds the same).  One work-group per column c, so the
+// reads of G (column c) and of M (column c' = i v + b, rows j v + a) are contiguous
+// in a.  Fixed-order reduction (per-thread sums, wave butterfly, the waves in order).
+__global__ __launch_bounds__(256) void k_sosex_contract(const double *__restrict__ G, int64_t ldg,
+                                                        int v, int ni,
+                                                        const double *__restrict__ M, int64_t ldm,
                                                         double gamma, double delta,
                                                         double *__restrict__ part) {
     __shared__ double sred[4];
     const int64_t c = blockIdx.x;
     const int j = (int)(c / v), b = (int)(c - (int64_t)j * v);
-    const double *__restrict__ Gc = G + K * c;
+    const double *__restrict__ Gc = G + ldg * c;
+    const bool tri = ni == 0;
+    const int iend = tri ? j + 1 : ni;
     double s = 0.0;
-    for (int i = 0; i <= j; ++i) {
-        const int amax = i < j ? v : b + 1;   // rows r = i v + a <= c
-        const double *__restrict__ Mc = M + K * ((int64_t)i * v + b) + (int64_t)j * v;
+    for (int i = 0; i < iend; ++i) {
+        const int amax = tri && i == j ? b + 1 : v;   // rows r = i v + a <= c
+        const double *__restrict__ Mc = M + ldm * ((int64_t)i * v + b) + (int64_t)j * v;
         const double *__restrict__ Gr = Gc + (int64_t)i * v;
         for (int a = threadIdx.x; a < amax; a += 256) {
-            const bool dg = i == j && a == b;
+            const bool dg = tri && i == j && a == b;
             double t = gamma * Mc[a];
             if (dg) t += delta;
             s = fma(dg ? Gr[a] : 2.0 * Gr[a], t, s);
@@ -127,17 +132,18 @@ __global__ __launch_bounds__(256) void k_sosex_contract(const double *__restrict
     if (threadIdx.x == 0) part[c] = (sred[0] + sred[1]) + (sred[2] + sred[3]);
 }
 
-int launch_sosex_contract(brpa_ctx *ctx, const double *G, int64_t K, int64_t v, const double *M,
-                          double gamma, double delta, double *part) {
-    if (K <= 0) return BRPA_OK;
-    if (K > INT32_MAX || v <= 0 || K % v != 0)
+int launch_sosex_contract(brpa_ctx *ctx, const double *G, int64_t ldg, int64_t v, int64_t ni,
+                          int64_t nj, const double *M, int64_t ldm, double gamma, double delta,
+                          double *part) {
+    if (v <= 0 || nj <= 0) return BRPA_OK;
+    if (nj * v > INT32_MAX || ni * v > INT32_MAX)
         return brpa_fail(ctx, BRPA_ERR_ARG, "exchange contraction: bad sizes");
     size_t slot = 0;
     BRPA_TRY(kstat_begin(ctx, &slot));
-    hipLaunchKernelGGL(k_sosex_contract, dim3((unsigned)K), dim3(256), 0, ctx->stream, G, K,
-                       (int)v, M, gamma, delta, part);
+    hipLaunchKernelGGL(k_sosex_contract, dim3((unsigned)(nj * v)), dim3(256), 0, ctx->stream, G,
+                       ldg, (int)v, (int)ni, M, ldm, gamma, delta, part);
     LAUNCH_CHECK(ctx);
-    // algorithmic flop of the contraction itself (one multiply-add per G element
-    // of the upper triangle)
-    return kstat_end(ctx, slot, BRPA_KERNEL_SOSEX_DOT, (double)K * (double)(K + 1));
+    // algorithmic flop of the contraction itself (one multiply-add per G element read)
+    const double kj = (double)nj * (double)v, ki = (double)ni * (double)v;
+    return kstat_end(ctx, slot, BRPA_KERNEL_SOSEX_DOT, ni == 0 ? kj * (kj + 1.0) : 2.0 * ki * kj);
 }

@@ -22,7 +22,7 @@
 #include <mutex>
 #include <vector>
 
-#include "internal.h"
+#include "dense.h"
 
 int launch_guess(brpa_ctx *, double *O, int64_t m, int64_t n, uint64_t seed);
 int launch_normalize_columns(brpa_ctx *, double *X, int64_t m, int64_t n);
@@ -42,6 +42,12 @@ int launch_transpose(brpa_ctx *, const double *in, int64_t m, int64_t n, double 
 int launch_pair_dot(brpa_ctx *, const double *W1, const double *W2, const double *B, int64_t n_rows,
                     int64_t nt, int64_t stride, int npair, double *part);
 int sosex_nchunk(int64_t n_rows, int64_t nt);
+int launch_gemm_f64(brpa_ctx *, bool ta, bool tb, int64_t m, int64_t n, int64_t k, double alpha,
+                    const double *A, int64_t lda, const double *B, int64_t ldb, double beta,
+                    double *C, int64_t ldc, bool upper);
+int launch_sosex_contract(brpa_ctx *, const double *G, int64_t ldg, int64_t v, int64_t ni,
+                          int64_t nj, const double *M, int64_t ldm, double gamma, double delta,
+                          double *part);
 int sosex_i8_vpad(int64_t v);
 size_t sosex_i8_slice_bytes(int64_t nblk, int64_t ncols, int64_t v);
 // rs: optional row scale (X[r][c] * rs[r] is sliced)
@@ -683,6 +689,107 @@ int t2_build(brpa_ctx *ctx, int precision, const double *R, int64_t naux, const 
     return BRPA_OK;
 }
 
+namespace {
+
+// SOSEX in the explicit ov space: E = -alpha sum_{aibj} (ai|bj) T(aj, bi) with
+// G = R R^T and T = V diag(B) V^T formed block by block on the library's GEMM,
+// K^2 (N + NT2) flop for both, then contracted by k_sosex_contract.  Blocks are
+// pairs I <= J of occupied ranges of at most kSosexBlock ov rows, so a block pair
+// needs 2 x 8 kSosexBlock^2 bytes (4.3 GB); on I = J only the tiles on or above
+// the diagonal are formed.
+constexpr int64_t kSosexBlock = 16384;
+
+// Chosen when its products take less time than those of the pair forms, which
+// need 2 o (o + 1) v N NT2 flop: at o = 40, v = 360, N = 1800, NT2 = 5400 the
+// explicit form runs at 60 TFLOP/s, the split-int8 pair kernel at 105 and the FP64
+// pair products at 60 of their own flop counts.  The ratio of the flop counts is
+// about v (N + NT2) / (2 N NT2), so the pair forms remain for few amplitude
+// vectors (NT2 below ~ v / 2).
+bool sosex_prefers_explicit(int precision, int64_t o, int64_t v, int64_t N, int64_t nt) {
+    const double K = (double)o * (double)v;
+    const double ex = K * K * ((double)N + (double)nt) / 60.0;
+    const double pr = 2.0 * (double)o * (double)(o + 1) * (double)v * (double)N * (double)nt /
+                      (precision == BRPA_SPLIT_I8 ? 105.0 : 60.0);
+    return ex < pr && v <= kSosexBlock;
+}
+
+int sosex_explicit(brpa_ctx *ctx, double *ec, double alpha, const double *V,
+                   const std::vector<double> &hB, const double *R, int64_t o, int64_t v, int64_t N,
+                   int64_t nt) {
+    const int64_t K = o * v;
+    const bool rdev = is_device_ptr(R), vdev = is_device_ptr(V);
+    const int64_t ob = std::min(o, std::max<int64_t>(1, kSosexBlock / v)), bs = ob * v;
+    // split-k partial tiles (up to 8) for blocks that leave the chip idle
+    const int64_t nsplit = std::min<int64_t>(8 * bs * bs, (int64_t)1 << 27);
+    double *dR, *dV, *dB, *VB, *G, *M, *part, *splitws;
+    auto layout = [&](Arena &ar) {
+        dR = rdev ? const_cast<double *>(R) : ar.take<double>(K * N);
+        dV = vdev ? const_cast<double *>(V) : ar.take<double>(K * nt);
+        dB = ar.take<double>(nt);
+        VB = ar.take<double>(K * nt);
+        G = ar.take<double>(bs * bs);
+        M = ar.take<double>(bs * bs);
+        part = ar.take<double>(cdiv(o, ob) * K);
+        splitws = ar.take<double>(nsplit);
+    };
+    Arena count, ar;
+    layout(count);
+    BRPA_TRY(ws_reserve(ctx, count.off, &ar));
+    layout(ar);
+    if (!rdev) BRPA_TRY(to_device(ctx, dR, R, 8 * K * N));
+    if (!vdev) BRPA_TRY(to_device(ctx, dV, V, 8 * K * nt));
+    BRPA_TRY(copy_sync(ctx, dB, hB.data(), 8 * nt, hipMemcpyHostToDevice));
+    struct SplitLend {
+        brpa_ctx *c;
+        ~SplitLend() {
+            c->split_ws = nullptr;
+            c->split_ws_cap = 0;
+        }
+    } lend{ctx};
+    ctx->split_ws = splitws;
+    ctx->split_ws_cap = (size_t)nsplit;
+    kstat_drop(ctx);
+    BRPA_HIP(ctx, hipEventRecord(ctx->ev0, ctx->stream));
+    BRPA_TRY(stage_begin(ctx, BRPA_STAGE_SOSEX));
+    // R and V are column-major N x K and NT2 x K here: every product is TN, both
+    // operands contiguous in k
+    BRPA_TRY(launch_row_scale(ctx, VB, dV, dB, nt, K));
+    int64_t np = 0;
+    for (int64_t i0 = 0; i0 < o; i0 += ob) {
+        const int64_t ni = std::min(ob, o - i0), mi = ni * v;
+        for (int64_t j0 = i0; j0 < o; j0 += ob) {
+            const int64_t nj = std::min(ob, o - j0), mj = nj * v;
+            const bool same = i0 == j0;
+            const double *RI = dR + i0 * v * N, *RJ = dR + j0 * v * N;
+            const double *VJ = VB + j0 * v * nt, *VI = dV + i0 * v * nt;
+            // G (I, J) and M (J, I)
+            BRPA_TRY(launch_gemm_f64(ctx, true, false, mi, mj, N, 1.0, RI, N, RJ, N, 0.0, G, mi,
+                                     same));
+            BRPA_TRY(launch_gemm_f64(ctx, true, false, mj, mi, nt, 1.0, VJ, nt, VI, nt, 0.0, M, mj,
+                                     same));
+            if (same) BRPA_TRY(dense_symm_fill(ctx, M, mj));
+            BRPA_TRY(launch_sosex_contract(ctx, G, mi, v, same ? 0 : ni, nj, M, mj, 1.0, 0.0,
+                                           part + np));
+            np += mj;
+        }
+    }
+    BRPA_TRY(stage_end(ctx, BRPA_STAGE_SOSEX));
+    BRPA_HIP(ctx, hipEventRecord(ctx->ev1, ctx->stream));
+    std::vector<double> hp(np);
+    BRPA_TRY(copy_sync(ctx, hp.data(), part, 8 * np, hipMemcpyDeviceToHost));
+    BRPA_TRY(stage_collect(ctx, BRPA_STAGE_SOSEX));
+    BRPA_TRY(kstat_collect(ctx));
+    float ms = 0.f;
+    BRPA_HIP(ctx, hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1));
+    ctx->last_kernel_ms = ms;
+    long double s = 0.0L;
+    for (double x : hp) s += (long double)x;
+    *ec = (double)(-(long double)alpha * s);
+    return BRPA_OK;
+}
+
+}  // namespace
+
 extern "C" {
 
 int brpa_t2_compute(brpa_ctx *ctx, int precision, const double *R, int64_t naux,
@@ -908,6 +1015,8 @@ int brpa_sosex(brpa_ctx *ctx, int precision, double *ec_exchange, double alpha, 
     // B = A, or A/(1-4A^2) for the cumulant route (rpa_CC_Exchange.f90:62-68)
     std::vector<double> hB(nt);
     for (int64_t k = 0; k < nt; ++k) hB[k] = s2_operator ? hA[k] / (1.0 - 4.0 * hA[k] * hA[k]) : hA[k];
+    if (sosex_prefers_explicit(precision, o, v, N, nt))
+        return sosex_explicit(ctx, ec_exchange, alpha, V, hB, R, o, v, N, nt);
     const bool rdev = is_device_ptr(R), vdev = is_device_ptr(V);
     if (precision == BRPA_SPLIT_I8) {
         // fused split-int8 pair kernel: 5 int8 slices per value, 15 products,

@@ -44,8 +44,9 @@ int launch_scale(brpa_ctx *, double *x, double a, int64_t n);
 int launch_add_diag(brpa_ctx *, double *M, int64_t n, double a);
 int launch_ritz_resid(brpa_ctx *, const double *AZ, const double *Z, const double *theta,
                       int64_t n, int64_t m, double *out);
-int launch_sosex_contract(brpa_ctx *, const double *G, int64_t K, int64_t v, const double *M,
-                          double gamma, double delta, double *part);
+int launch_sosex_contract(brpa_ctx *, const double *G, int64_t ldg, int64_t v, int64_t ni,
+                          int64_t nj, const double *M, int64_t ldm, double gamma, double delta,
+                          double *part);
 
 namespace {
 constexpr double kPi = 3.14159265358979323846;
@@ -603,7 +604,7 @@ int exchange_xspace(brpa_ctx *ctx, const double *R, int64_t naux, const double *
     // R[ai][P] is the column-major N x K matrix R^T, contiguous in P), then the
     // contraction with the T2 matrix
     BRPA_TRY(dense_syrk(ctx, true, K, N, 1.0, dR, N, 0.0, Im, K));
-    BRPA_TRY(launch_sosex_contract(ctx, Im, K, nvir, Y, gamma, delta, part));
+    BRPA_TRY(launch_sosex_contract(ctx, Im, K, nvir, 0, nocc, Y, K, gamma, delta, part));
     BRPA_TRY(stage_end(ctx, BRPA_STAGE_SOSEX));
     BRPA_HIP(ctx, hipEventRecord(ctx->ev1, ctx->stream));
     std::vector<double> hp(nparts);

@@ -452,7 +452,8 @@ int brpa_t2_copyout_ov(brpa_ctx *ctx, double *A, double *V);
  * W_ij = R_i V_j^T.  Replaces rpa_CC_Exchange_SOSEX
  * (rpa/rpa_CC_Exchange.f90:36-97).  V: C V[ai][mu] (Fortran Vkai(NVecsT2, v, o)),
  * R: C R[ai][P] (Fortran Rkai(NVecsPiU, v, o)).  precision: BRPA_FP64 (the
- * drop-in: rocBLAS FP64 GEMMs per pair block, double-double pair sums) or
+ * drop-in: rocBLAS FP64 GEMMs per pair block, double-double pair sums in the pair
+ * form) or
  * BRPA_SPLIT_I8 (one fused gfx950 kernel: W_ij and W_ji tiles from 5 int8
  * slices per value, 15 products with exact int32 level sums, FP64
  * combination, double-double tile sums; W is never stored; nvir <= 65536). */
