@@ -448,12 +448,13 @@ int brpa_t2_copyout_ov(brpa_ctx *ctx, double *A, double *V);
 
 /* ---- exchange correction ---------------------------------------------------- */
 /* EcExchange = -alpha sum_{aibj} (aj|bi) T(ai,bj), T = V^T diag(B) V with
- * B = A (or A/(1-4A^2) when s2_operator), evaluated pair by pair
- * W_ij = R_i V_j^T.  Replaces rpa_CC_Exchange_SOSEX
+ * B = A (or A/(1-4A^2) when s2_operator).  Where it takes less time (all but few
+ * amplitude vectors) (ai|bj) and T are formed as ov x ov blocks on the library's
+ * FP64 GEMM in both precisions (up to 4.3 GB of device scratch beside a copy of V);
+ * otherwise pair by pair, W_ij = R_i V_j^T, in `precision`.  Replaces rpa_CC_Exchange_SOSEX
  * (rpa/rpa_CC_Exchange.f90:36-97).  V: C V[ai][mu] (Fortran Vkai(NVecsT2, v, o)),
  * R: C R[ai][P] (Fortran Rkai(NVecsPiU, v, o)).  precision: BRPA_FP64 (the
- * drop-in: rocBLAS FP64 GEMMs per pair block, double-double pair sums in the pair
- * form) or
+ * drop-in: rocBLAS FP64 GEMMs per pair block, double-double pair sums) or
  * BRPA_SPLIT_I8 (one fused gfx950 kernel: W_ij and W_ji tiles from 5 int8
  * slices per value, 15 products with exact int32 level sums, FP64
  * combination, double-double tile sums; W is never stored; nvir <= 65536). */
