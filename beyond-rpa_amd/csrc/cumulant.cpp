@@ -1,6 +1,7 @@
 // THC SOSEX + 2g cumulant terms (rpa_CCD_corrections_1b2g,
 // rpa/rpa_CCD_Corrections.f90:79-290): YU = Yga U_mu by rocBLAS dgemm for a
-// chunk of amplitude vectors, then the fused k_thc_1b2g contraction.
+// chunk of amplitude vectors, then the fused k_thc_1b2g contraction, or, with many
+// vectors, the products of YU and U with the integrals formed once.
 #include <rocblas/rocblas.h>
 
 #include <algorithm>
@@ -8,12 +9,41 @@
 #include <cstring>
 #include <vector>
 
-#include "internal.h"
+#include "dense.h"
 
 int rocblas_handle_of(brpa_ctx *ctx, void **h);
 int thc_1b2g_npairs(int64_t G);
 int launch_thc_1b2g(brpa_ctx *, const double *YU, const double *X, const double *Z, int64_t G,
                     int64_t o, int64_t nmu, double *part, double *diag, int64_t mu0, double *S);
+
+int launch_thc_pairs(brpa_ctx *, const double *Y, const double *X, int64_t G, int64_t v, int64_t o,
+                     double *P, int64_t ldp);
+int launch_thc_xx(brpa_ctx *, const double *X, int64_t G, int64_t o, double *XX, int64_t ldp);
+int launch_swap_occ(brpa_ctx *, const double *W, int64_t v, int64_t o, double *D, int64_t ldd);
+int64_t thc_s2_blocks(int64_t G);
+int launch_thc_s2(brpa_ctx *, const double *YU, const double *X, const double *Q, int64_t ldq,
+                  int64_t G, int64_t o, int64_t nmu, double *part, double *diag, int64_t mu0,
+                  const double *U, int64_t K, const double *DU, double *S);
+int launch_gemm_f64(brpa_ctx *, bool ta, bool tb, int64_t m, int64_t n, int64_t k, double alpha,
+                    const double *A, int64_t lda, const double *B, int64_t ldb, double beta,
+                    double *C, int64_t ldc, bool upper);
+
+namespace {
+
+// The explicit form needs 2 G^2 K + G K^2 flop for D = (aj|bi), G^2 o (o + 1) for Q and
+// 2 K^2 NT2 for D U on the GEMM (60 TFLOP/s), with about 150 us of launches on small
+// sizes; the fused kernel 2 G^2 o NT2 at 27 TFLOP/s.  At o = 36, v = 300, G = 4032 the
+// line lies near 500 vectors: 2100 of them take 31 ms explicitly, 98 ms fused.
+// Two K x K and two G x K matrices have to fit 64 GB.
+bool explicit_pays(int64_t G, int64_t o, int64_t v, int64_t nt) {
+    const double g = (double)G, K = (double)o * (double)v, n = (double)nt;
+    const double ex = (2 * g * g * K + g * K * K + g * g * o * (o + 1) + 2 * K * K * n) / 60e6 + 150;
+    const double fu = 2 * g * g * o * n / 27e6 + 20;
+    return ex < fu && o * v <= 46340 && o * (o + 1) / 2 <= 65535 &&
+           8.0 * (2 * K * K + 2 * g * K) <= 64e9;
+}
+
+}  // namespace
 
 extern "C" {
 
@@ -40,6 +70,10 @@ int brpa_thc_1b2g(brpa_ctx *ctx, const double *Zgh, const double *Xgi, const dou
     else
         std::memcpy(a.data(), Am, 8 * nt);
     const int npairs = thc_1b2g_npairs(G);
+    const bool ex = explicit_pays(G, o, v, nt);
+    const int64_t K = o * v;
+    // even leading dimensions: the GEMM then loads its panels straight into LDS
+    const int64_t gp = G + (G & 1), kp = K + (K & 1), L = o * (o + 1) / 2;
     // amplitude vectors per chunk: YU (G x o per vector) below ~1 GB, at most 65535
     const int64_t nmu = std::max<int64_t>(
         1, std::min<int64_t>({nt, (int64_t)65535, (int64_t)(128ll << 20) / (G * o)}));
@@ -47,6 +81,7 @@ int brpa_thc_1b2g(brpa_ctx *ctx, const double *Zgh, const double *Xgi, const dou
                udev = is_device_ptr(Uaim), ddev = yxu_diag && is_device_ptr(yxu_diag);
     const double *dZ = Zgh, *dX = Xgi, *dY = Yga, *dU = Uaim;
     double *YU, *part, *S, *dD = yxu_diag;
+    double *Zp = nullptr, *P, *ZP, *Q, *W, *D, *Up = nullptr, *DU;
     auto layout = [&](Arena &ar) {
         if (!zdev) dZ = ar.take<double>(G * G);
         if (!xdev) dX = ar.take<double>(G * o);
@@ -54,8 +89,17 @@ int brpa_thc_1b2g(brpa_ctx *ctx, const double *Zgh, const double *Xgi, const dou
         if (!udev) dU = ar.take<double>(v * o * nt);
         if (yxu_diag && !ddev) dD = ar.take<double>(G * nt);
         YU = ar.take<double>(G * o * nmu);
-        part = ar.take<double>((int64_t)npairs * nmu * 2);
+        part = ar.take<double>(ex ? thc_s2_blocks(G) * nmu : (int64_t)npairs * nmu * 2);
         S = ar.take<double>(2 * nt);
+        if (!ex) return;
+        if (gp != G) Zp = ar.take<double>(gp * G);
+        if (kp != K) Up = ar.take<double>(kp * nt);
+        P = ar.take<double>(gp * std::max(K, L));
+        ZP = ar.take<double>(gp * K);
+        Q = ar.take<double>(gp * L);
+        W = ar.take<double>(K * K);
+        D = ar.take<double>(kp * K);
+        DU = ar.take<double>(K * nt);
     };
     Arena count, ar;
     layout(count);
@@ -76,6 +120,27 @@ int brpa_thc_1b2g(brpa_ctx *ctx, const double *Zgh, const double *Xgi, const dou
                  : brpa_fail(ctx, BRPA_ERR_SOLVER, "rocblas_set_stream failed"));
     BRPA_HIP(ctx, hipEventRecord(ctx->ev0, ctx->stream));
     const double one = 1.0, zero = 0.0;
+    if (ex) {
+        const double *Zs = dZ;
+        if (Zp) {
+            BRPA_HIP(ctx, hipMemcpy2DAsync(Zp, 8 * gp, dZ, 8 * G, 8 * G, G, hipMemcpyDeviceToDevice,
+                                           ctx->stream));
+            Zs = Zp;
+        }
+        // Q = Z XX, D from P^T (Z P); Z is symmetric, so every product is TN
+        BRPA_TRY(launch_thc_xx(ctx, dX, G, o, P, gp));
+        BRPA_TRY(launch_gemm_f64(ctx, true, false, G, L, G, 1.0, Zs, gp, P, gp, 0.0, Q, gp, false));
+        BRPA_TRY(launch_thc_pairs(ctx, dY, dX, G, v, o, P, gp));
+        BRPA_TRY(launch_gemm_f64(ctx, true, false, G, K, G, 1.0, Zs, gp, P, gp, 0.0, ZP, gp, false));
+        BRPA_TRY(launch_gemm_f64(ctx, true, false, K, K, G, 1.0, P, gp, ZP, gp, 0.0, W, K, true));
+        BRPA_TRY(launch_swap_occ(ctx, W, v, o, D, kp));
+        // D U of every vector in one product (its grid is too small chunk by chunk)
+        if (Up)
+            BRPA_HIP(ctx, hipMemcpy2DAsync(Up, 8 * kp, dU, 8 * K, 8 * K, nt,
+                                           hipMemcpyDeviceToDevice, ctx->stream));
+        BRPA_TRY(launch_gemm_f64(ctx, true, false, K, nt, K, 1.0, D, kp, Up ? Up : dU, kp, 0.0, DU,
+                                 K, false));
+    }
     for (int64_t mu0 = 0; mu0 < nt; mu0 += nmu) {
         const int64_t m = std::min(nmu, nt - mu0);
         // YU(:, i + o mu) = Yga U(:, i, mu): column-major G x (o m), K = v
@@ -84,9 +149,15 @@ int brpa_thc_1b2g(brpa_ctx *ctx, const double *Zgh, const double *Xgi, const dou
                           dU + v * o * mu0, (rocblas_int)v, &zero, YU, (rocblas_int)G) !=
             rocblas_status_success)
             return brpa_fail(ctx, BRPA_ERR_SOLVER, "brpa_thc_1b2g: rocblas_dgemm failed");
+        if (ex) {
+            BRPA_TRY(launch_thc_s2(ctx, YU, dX, Q, gp, G, o, m, part, yxu_diag ? dD : nullptr, mu0,
+                                   dU + K * mu0, K, DU + K * mu0, S));
+            continue;
+        }
         BRPA_TRY(launch_thc_1b2g(ctx, YU, dX, dZ, G, o, m, part, yxu_diag ? dD : nullptr, mu0, S));
     }
     BRPA_HIP(ctx, hipEventRecord(ctx->ev1, ctx->stream));
+    kstat_drop(ctx);
     std::vector<double> hs(2 * nt);
     BRPA_TRY(copy_sync(ctx, hs.data(), S, 8 * 2 * nt, hipMemcpyDeviceToHost));
     if (yxu_diag && !ddev) BRPA_TRY(copy_sync(ctx, yxu_diag, dD, 8 * G * nt, hipMemcpyDeviceToHost));

@@ -13,6 +13,17 @@
 // writes two partial sums; M never reaches memory.  The partials are reduced
 // per mu in a fixed order (double-double), so the result does not depend on
 // scheduling.
+//
+// With many vectors it costs less to form what does not depend on mu once
+// (thc_1b2g_explicit in cumulant.cpp):
+//   S2g_mu = sum_g sum_{ij} YU(g, i) YU(g, j) Q(g, ij),  Q = Z (X_i o X_j),
+//   S1b_mu = U_mu^T D U_mu,  D(ai, bj) = (aj|bi) = (P^T Z P)(aj, bi),
+//            P(g, aj) = Y(g, a) X(g, j).
+// The products run on the library's GEMM; here are the kernels around them:
+//   k_thc_pairs, k_thc_xx  P and the X_i o X_j, i >= j
+//   k_swap_occ             D from the upper triangle of P^T Z P
+//   k_thc_s2               S2g partials and the diagonal M_mu(g, g)
+//   k_thc_terms            both sums of each vector
 #include "device_common.h"
 #include "internal.h"
 
@@ -160,7 +171,204 @@ __global__ __launch_bounds__(256) void k_thc_1b2g_reduce(const double *__restric
     }
 }
 
+// P(g, a + v j) = Y(g, a) X(g, j), leading dimension ldp; y: column a + v j
+__global__ __launch_bounds__(256) void k_thc_pairs(const double *__restrict__ Y,
+                                                   const double *__restrict__ X, int G, int v,
+                                                   double *__restrict__ P, int64_t ldp) {
+    const int g = blockIdx.x * 256 + threadIdx.x, c = blockIdx.y;
+    if (g >= G) return;
+    const int j = c / v, a = c - j * v;
+    P[g + ldp * c] = Y[g + (int64_t)G * a] * X[g + (int64_t)G * j];
+}
+
+// XX(g, i (i + 1) / 2 + j) = X(g, i) X(g, j), i >= j
+__global__ __launch_bounds__(256) void k_thc_xx(const double *__restrict__ X, int G,
+                                                double *__restrict__ XX, int64_t ldp) {
+    const int g = blockIdx.x * 256 + threadIdx.x;
+    int i, j;
+    pair_decode(blockIdx.y, i, j);
+    if (g < G) XX[g + ldp * blockIdx.y] = X[g + (int64_t)G * i] * X[g + (int64_t)G * j];
+}
+
+// D(a + v i, b + v j) = W(a + v j, b + v i) for the symmetric W (K x K, upper triangle
+// valid): one 32 x 32 tile of the v x v block of one pair i >= j per work-group.
+// W is read along its columns; the block (i, j) of D is written the same way, its
+// mirror (j, i) through LDS.  Bound by memory: W's triangle read and D written.
+__global__ __launch_bounds__(256) void k_swap_occ(const double *__restrict__ W, int64_t K, int v,
+                                                  int nt, double *__restrict__ D, int64_t ldd) {
+    __shared__ double t[32][33];
+    const int64_t b = blockIdx.x;
+    const int pair = (int)(b / (nt * nt)), tile = (int)(b - (int64_t)pair * nt * nt);
+    int i, j;
+    pair_decode(pair, i, j);
+    const int a0 = 32 * (tile % nt), b0 = 32 * (tile / nt);
+    const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
+    for (int y = ty; y < 32; y += 8) {
+        const int a = a0 + tx, bb = b0 + y;
+        if (a < v && bb < v) {
+            const int64_t r = a + (int64_t)v * j, c = bb + (int64_t)v * i;
+            const double x = W[min(r, c) + K * max(r, c)];
+            t[y][tx] = x;
+            D[a + (int64_t)v * i + ldd * (bb + (int64_t)v * j)] = x;
+        }
+    }
+    if (i == j) return;
+    __syncthreads();
+    for (int y = ty; y < 32; y += 8) {
+        const int a = a0 + y, bb = b0 + tx;
+        if (a < v && bb < v) D[bb + (int64_t)v * j + ldd * (a + (int64_t)v * i)] = t[tx][y];
+    }
+}
+
+// S2g partials: part[mu * ngb + gb] = sum over 64 grid points of sum_{i >= j} (2 -
+// delta_ij) Q(g, ij) YU(g, i) YU(g, j), for 8 vectors per wave (grid: x = 64
+// points, y = 32 vectors).  A lane holds one point; rows of Q in blocks of four
+// keep 32 accumulators per lane, so a column j costs 12 loads for 32 fma.  diag
+// (may be null): M_mu(g, g) = sum_i YU(g, i) X(g, i).  Bound by L2 reads of YU
+// (o / 8 passes) and Q: 3.5 ms for 2100 vectors at o = 36, G = 4032 (5.9 ms
+// without the second column in flight).
+constexpr int S2V = 8;
+__global__ __launch_bounds__(256) void k_thc_s2(const double *__restrict__ YU,
+                                                const double *__restrict__ X,
+                                                const double *__restrict__ Q, int64_t ldq, int G,
+                                                int o, int nmu, double *__restrict__ part,
+                                                double *__restrict__ diag, int64_t mu0) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int gb = blockIdx.x, m0 = blockIdx.y * (4 * S2V) + wave * S2V;
+    if (m0 >= nmu) return;
+    const int g = gb * 64 + lane;
+    const bool ok = g < G;
+    const int gc = ok ? g : G - 1;
+    const double *yu[S2V];
+#pragma unroll
+    for (int u = 0; u < S2V; ++u) yu[u] = YU + (int64_t)G * o * min(m0 + u, nmu - 1) + gc;
+    const double *__restrict__ Qg = Q + gc;
+    double s[S2V];
+#pragma unroll
+    for (int u = 0; u < S2V; ++u) s[u] = 0.0;
+    for (int i0 = 0; i0 < o; i0 += 4) {
+        double t[4][S2V];
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+            for (int u = 0; u < S2V; ++u) t[q][u] = 0.0;
+#pragma unroll 2
+        for (int j = 0; j < min(o, i0 + 4); ++j) {
+            double qv[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int i = i0 + q;
+                const bool in = i < o && j <= i;
+                const double x = Qg[ldq * (in ? (int64_t)i * (i + 1) / 2 + j : 0)];
+                qv[q] = in ? (j == i ? x : 2.0 * x) : 0.0;
+            }
+#pragma unroll
+            for (int u = 0; u < S2V; ++u) {
+                const double y = yu[u][(int64_t)G * j];
+#pragma unroll
+                for (int q = 0; q < 4; ++q) t[q][u] = fma(qv[q], y, t[q][u]);
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            if (i0 + q < o)
+#pragma unroll
+                for (int u = 0; u < S2V; ++u)
+                    s[u] = fma(t[q][u], yu[u][(int64_t)G * (i0 + q)], s[u]);
+    }
+#pragma unroll
+    for (int u = 0; u < S2V; ++u) {
+        double x = ok ? s[u] : 0.0;
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) x += __shfl_xor(x, off);
+        if (lane == 0 && m0 + u < nmu) part[(int64_t)(m0 + u) * gridDim.x + gb] = x;
+    }
+    if (!diag || !ok) return;
+#pragma unroll
+    for (int u = 0; u < S2V; ++u) s[u] = 0.0;
+    for (int i = 0; i < o; ++i) {
+        const double x = X[g + (int64_t)G * i];
+#pragma unroll
+        for (int u = 0; u < S2V; ++u) s[u] = fma(yu[u][(int64_t)G * i], x, s[u]);
+    }
+#pragma unroll
+    for (int u = 0; u < S2V; ++u)
+        if (m0 + u < nmu) diag[g + (int64_t)G * (mu0 + m0 + u)] = s[u];
+}
+
+// S[2 (mu0 + mu)] = sum of the S2g partials, S[2 (mu0 + mu) + 1] = U_mu^T (D U_mu),
+// both in double-double: thread stripes in order, then a fixed tree
+__global__ __launch_bounds__(256) void k_thc_terms(const double *__restrict__ part, int ngb,
+                                                   const double *__restrict__ U, int64_t K,
+                                                   const double *__restrict__ DU,
+                                                   double *__restrict__ S, int64_t mu0) {
+    __shared__ dd_t sh[2][256];
+    const int64_t mu = blockIdx.x;
+    const int tid = threadIdx.x;
+    dd_t a = {0.0, 0.0}, b = {0.0, 0.0};
+    for (int t = tid; t < ngb; t += 256) a = dd_add(a, part[mu * ngb + t]);
+    for (int64_t k = tid; k < K; k += 256) {
+        const double x = U[k + K * mu], y = DU[k + K * mu], p = x * y;
+        b = dd_add(b, (dd_t){p, fma(x, y, -p)});
+    }
+    sh[0][tid] = a;
+    sh[1][tid] = b;
+    __syncthreads();
+    for (int k = 128; k > 0; k >>= 1) {
+        if (tid < k) {
+            sh[0][tid] = dd_add(sh[0][tid], sh[0][tid + k]);
+            sh[1][tid] = dd_add(sh[1][tid], sh[1][tid + k]);
+        }
+        __syncthreads();
+    }
+    if (tid == 0) {
+        S[(mu0 + mu) * 2] = sh[0][0].hi + sh[0][0].lo;
+        S[(mu0 + mu) * 2 + 1] = sh[1][0].hi + sh[1][0].lo;
+    }
+}
+
 }  // namespace
+
+int launch_thc_pairs(brpa_ctx *ctx, const double *Y, const double *X, int64_t G, int64_t v,
+                     int64_t o, double *P, int64_t ldp) {
+    hipLaunchKernelGGL(k_thc_pairs, dim3((unsigned)((G + 255) / 256), (unsigned)(v * o)), dim3(256),
+                       0, ctx->stream, Y, X, (int)G, (int)v, P, ldp);
+    LAUNCH_CHECK(ctx);
+    return BRPA_OK;
+}
+
+int launch_thc_xx(brpa_ctx *ctx, const double *X, int64_t G, int64_t o, double *XX, int64_t ldp) {
+    hipLaunchKernelGGL(k_thc_xx, dim3((unsigned)((G + 255) / 256), (unsigned)(o * (o + 1) / 2)),
+                       dim3(256), 0, ctx->stream, X, (int)G, XX, ldp);
+    LAUNCH_CHECK(ctx);
+    return BRPA_OK;
+}
+
+int launch_swap_occ(brpa_ctx *ctx, const double *W, int64_t v, int64_t o, double *D, int64_t ldd) {
+    const int64_t nt = (v + 31) / 32, blocks = nt * nt * (o * (o + 1) / 2);
+    if (blocks > INT32_MAX)
+        return brpa_fail(ctx, BRPA_ERR_ARG, "THC 1b2g: sizes beyond the supported grid");
+    hipLaunchKernelGGL(k_swap_occ, dim3((unsigned)blocks), dim3(256), 0, ctx->stream, W, v * o,
+                       (int)v, (int)nt, D, ldd);
+    LAUNCH_CHECK(ctx);
+    return BRPA_OK;
+}
+
+int64_t thc_s2_blocks(int64_t G) { return (G + 63) / 64; }
+
+// part: nmu * thc_s2_blocks(G) doubles
+int launch_thc_s2(brpa_ctx *ctx, const double *YU, const double *X, const double *Q, int64_t ldq,
+                  int64_t G, int64_t o, int64_t nmu, double *part, double *diag, int64_t mu0,
+                  const double *U, int64_t K, const double *DU, double *S) {
+    const unsigned ngb = (unsigned)thc_s2_blocks(G);
+    hipLaunchKernelGGL(k_thc_s2, dim3(ngb, (unsigned)((nmu + 4 * S2V - 1) / (4 * S2V))), dim3(256),
+                       0, ctx->stream, YU, X, Q, ldq, (int)G, (int)o, (int)nmu, part, diag, mu0);
+    LAUNCH_CHECK(ctx);
+    hipLaunchKernelGGL(k_thc_terms, dim3((unsigned)nmu), dim3(256), 0, ctx->stream, part, (int)ngb,
+                       U, K, DU, S, mu0);
+    LAUNCH_CHECK(ctx);
+    return BRPA_OK;
+}
 
 int thc_1b2g_npairs(int64_t G) {
     const int64_t nb = (G + CB - 1) / CB;

@@ -360,8 +360,11 @@ int brpa_thc_piu(brpa_ctx *ctx, double *PiU, double *Rkai, const double *Xga, co
  * device.  eig_sosex / eig_2g (host, may be NULL): RPAOutput%EigSOSEX(mu) =
  * -S1b A and Eig2g(mu) = -4 S2g A^2; yxu_diag (may be NULL, host or device,
  * ngrid x NVecsT2): YXUggm(g, mu) = M_mu(g, g), the 2b/2c/2d intermediate.
- * One fused FP64 MFMA kernel per chunk of vectors: M is built and contracted
- * in registers, never stored. */
+ * Few vectors: one fused FP64 MFMA kernel per chunk of vectors, M built and
+ * contracted in registers, never stored.  Many: (aj|bi) (ov x ov) and Z (X_i o X_j)
+ * are formed once and every vector's two terms follow from products with them
+ * (device scratch 2 (ov)^2 + 2 ov ngrid + ov NVecsT2 doubles, at most 64 GB for the
+ * first two). */
 int brpa_thc_1b2g(brpa_ctx *ctx, const double *Zgh, const double *Xgi, const double *Yga,
                   const double *Uaim, const double *Am, int64_t ngrid, int64_t nocc, int64_t nvir,
                   int64_t nvecs_t2, double *ec1b, double *ec2g, double *eig_sosex, double *eig_2g,
