@@ -75,7 +75,7 @@ constexpr int GGROUP = 8;  // tile rows per group of the tile order (panel reuse
 // an operand contiguous in rows, an even row count (dma = 1), each stage goes
 // from global memory straight into LDS (global_load_lds_dwordx4, 16 bytes per
 // lane, 1 KB per wave instruction) with no register staging and no LDS store
-// instructions (layouts at dma_sources).  Rows past m (n) repeat the last row
+// instructions (layouts at dma_offsets).  Rows past m (n) repeat the last row
 // (pair): they only reach products that are not stored.  A last stage with
 // fewer than 16 k goes through registers with zeros past kend.  The k order of
 // the sum is the same as in the register-staged form.
@@ -111,41 +111,31 @@ typedef double d2_t __attribute__((ext_vector_type(2)));
 // the k rows 4 w + c, lane L the rows 2 L, 2 L + 1.  dk: the lane's k offset
 // within a stage (KC, pair start) or its k row.
 constexpr int DMA_KPR = 132;
+// off: the lane's byte offsets from the tile's base at k = 0 (dma_base); the
+// launch checks that 128 rows stay within 32 bits
 template <bool KC>
-__host__ __device__ __forceinline__ void dma_sources(const double *X, int64_t ldx, int r0,
-                                                     int rows, int wave, int lane,
-                                                     const double *(&p)[4], int (&dk)[4]) {
+__device__ __forceinline__ void dma_offsets(int64_t ldx, int r0, int rows, int wave, int lane,
+                                            uint32_t (&off)[4], int (&dk)[4]) {
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
         if (KC) {
             const int row = 32 * wave + 8 * c + (lane >> 3);
             dk[c] = 2 * ((lane & 7) ^ ((row >> 1) & 7));
-            p[c] = X + ldx * (int64_t)min(r0 + row, rows - 1) + dk[c];
+            off[c] = 8u * ((uint32_t)ldx * (uint32_t)(min(r0 + row, rows - 1) - r0) + (uint32_t)dk[c]);
         } else {
             // rows is even here: the last pair is rows - 2, rows - 1
             dk[c] = 4 * wave + c;
-            p[c] = X + min(r0 + 2 * lane, rows - 2) + ldx * (int64_t)dk[c];
+            off[c] = 8u * ((uint32_t)(min(r0 + 2 * lane, rows - 2) - r0) + (uint32_t)ldx * (uint32_t)dk[c]);
         }
     }
 }
 template <bool KC>
-__host__ __device__ __forceinline__ int dma_block(int wave, int c) {
-    return KC ? (32 * wave + 8 * c) * GKB : (4 * wave + c) * DMA_KPR;
+__device__ __forceinline__ const char *dma_base(const double *X, int64_t ldx, int r0) {
+    return reinterpret_cast<const char *>(X + (KC ? ldx * r0 : (int64_t)r0));
 }
-// the lane's 16 bytes of a last stage with k < kend, zeros past it
 template <bool KC>
-__host__ __device__ __forceinline__ d2_t dma_tail(const double *p, int64_t ldx, int k0, int dk,
-                                                  int kend) {
-    d2_t v;
-    if (KC) {
-        v.x = k0 + dk < kend ? p[k0] : 0.0;
-        v.y = k0 + dk + 1 < kend ? p[k0 + 1] : 0.0;
-    } else {
-        const bool ok = k0 + dk < kend;
-        v.x = ok ? p[ldx * k0] : 0.0;
-        v.y = ok ? p[ldx * k0 + 1] : 0.0;
-    }
-    return v;
+__device__ __forceinline__ int dma_block(int wave, int c) {
+    return KC ? (32 * wave + 8 * c) * GKB : (4 * wave + c) * DMA_KPR;
 }
 // fragment of row `row` at the k pair 2 g4 + hh of a stage
 template <bool KC>
@@ -161,25 +151,35 @@ __host__ __device__ __forceinline__ d2_t dma_frag(const double *L, int row, int 
     return v;
 }
 
-// one operand's stage at k0 into the LDS buffer L: direct loads when the stage
-// is full, else through registers with zeros past kend
+// one operand's full stage at k0 into the LDS buffer L, straight from global memory
 template <bool KC>
-__device__ __forceinline__ void dma_stage(const double *(&p)[4], int (&dk)[4],
-                                          int64_t ldx, double *L, int wave, int lane, int k0,
-                                          int kend) {
-    if (k0 + GKB <= kend) {
-        // the builtin exists for the device pass only; the host pass never runs this
+__device__ __forceinline__ void dma_stage(const char *base, const uint32_t (&off)[4], int64_t ldx,
+                                          double *L, int wave, int k0) {
+    // the builtin exists for the device pass only; the host pass never runs this
 #if defined(__HIP_DEVICE_COMPILE__)
+    const char *b = base + 8 * (KC ? (int64_t)k0 : ldx * k0);
 #pragma unroll
-        for (int c = 0; c < 4; ++c)
-            __builtin_amdgcn_global_load_lds(p[c] + (KC ? (int64_t)k0 : ldx * k0),
-                                             L + dma_block<KC>(wave, c), 16, 0, 0);
+    for (int c = 0; c < 4; ++c)
+        __builtin_amdgcn_global_load_lds(
+            reinterpret_cast<const __attribute__((address_space(1))) void *>(
+                (__attribute__((address_space(1))) const char *)b + off[c]),
+            (__attribute__((address_space(3))) void *)(L + dma_block<KC>(wave, c)), 16, 0, 0);
 #endif
-    } else {
+}
+// the last stage when it has fewer than 16 k: through registers, zeros past kend
+template <bool KC>
+__device__ __forceinline__ void dma_stage_tail(const char *base, const uint32_t (&off)[4],
+                                               const int (&dk)[4], int64_t ldx, double *L, int wave,
+                                               int lane, int k0, int kend) {
+    const char *b = base + 8 * (KC ? (int64_t)k0 : ldx * k0);
 #pragma unroll
-        for (int c = 0; c < 4; ++c)
-            *reinterpret_cast<d2_t *>(L + dma_block<KC>(wave, c) + 2 * lane) =
-                dma_tail<KC>(p[c], ldx, k0, dk[c], kend);
+    for (int c = 0; c < 4; ++c) {
+        const double *p = reinterpret_cast<const double *>(b + off[c]);
+        const bool ok0 = k0 + dk[c] < kend, ok1 = KC ? k0 + dk[c] + 1 < kend : ok0;
+        d2_t v;
+        v.x = ok0 ? p[0] : 0.0;
+        v.y = ok1 ? p[1] : 0.0;
+        *reinterpret_cast<d2_t *>(L + dma_block<KC>(wave, c) + 2 * lane) = v;
     }
 }
 
@@ -209,7 +209,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     const double *__restrict__ B = g.B + item1 * g.sB1 + item2 * g.sB2;
     const int m = g.m, n = g.n;
     const int64_t lda = g.lda, ldb = g.ldb;
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave >> 1, wn = wave & 1;
     const int m0 = ti * GT, n0 = tj * GT;
     int kbeg = 0, kend = g.k;
@@ -272,43 +273,96 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         if (kbeg < kend) {
             const int rl = lane & 15, g4 = lane >> 4;
             constexpr bool KCA = TA, KCB = !TB;   // operand contiguous in k
-            const double *pa[4], *pb[4];
+            uint32_t oa[4], ob[4];
             int ka[4], kb[4];
-            dma_sources<KCA>(A, lda, m0, m, wave, lane, pa, ka);
-            dma_sources<KCB>(B, ldb, n0, n, wave, lane, pb, kb);
-            dma_stage<KCA>(pa, ka, lda, sA[0], wave, lane, kbeg, kend);
-            dma_stage<KCB>(pb, kb, ldb, sB[0], wave, lane, kbeg, kend);
-            __syncthreads();
-            int buf = 0;
-            for (int k0 = kbeg; k0 < kend; k0 += GKB, buf ^= 1) {
-                d2_t a[4][2], b[4][2];
+            dma_offsets<KCA>(lda, m0, m, wave, lane, oa, ka);
+            dma_offsets<KCB>(ldb, n0, n, wave, lane, ob, kb);
+            const char *ba = dma_base<KCA>(A, lda, m0), *bb = dma_base<KCB>(B, ldb, n0);
+            auto stage = [&](int buf, int k0) {
+                dma_stage<KCA>(ba, oa, lda, sA[buf], wave, k0);
+                dma_stage<KCB>(bb, ob, ldb, sB[buf], wave, k0);
+            };
+            auto stage_tail = [&](int buf, int k0) {
+                dma_stage_tail<KCA>(ba, oa, ka, lda, sA[buf], wave, lane, k0, kend);
+                dma_stage_tail<KCB>(bb, ob, kb, ldb, sB[buf], wave, lane, k0, kend);
+            };
+            // one half of a stage: two k per lane
+            auto frags = [&](d2_t (&a)[4], d2_t (&b)[4], int buf, int hh) {
 #pragma unroll
-                for (int hh = 0; hh < 2; ++hh) {
+                for (int i = 0; i < 4; ++i)
+                    a[i] = dma_frag<KCA>(sA[buf], 64 * wm + 16 * i + rl, g4, hh);
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    b[j] = dma_frag<KCB>(sB[buf], 64 * wn + 16 * j + rl, g4, hh);
+            };
+            auto mma = [&](const d2_t (&a)[4], const d2_t (&b)[4]) {
+#pragma unroll
+                for (int st = 0; st < 2; ++st)
 #pragma unroll
                     for (int i = 0; i < 4; ++i)
-                        a[i][hh] = dma_frag<KCA>(sA[buf], 64 * wm + 16 * i + rl, g4, hh);
 #pragma unroll
-                    for (int j = 0; j < 4; ++j)
-                        b[j][hh] = dma_frag<KCB>(sB[buf], 64 * wn + 16 * j + rl, g4, hh);
+                        for (int j = 0; j < 4; ++j)
+                            acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(b[j][st], a[i][st],
+                                                                             acc[i][j], 0, 0, 0);
+            };
+            d2_t a0[4], b0[4], a1[4], b1[4];
+            // The fragments of either half of a stage are read while the other half
+            // is multiplied, one LDS read after each of the first MFMAs and then one
+            // load of the coming stage after each of the next.  The barrier stands
+            // between the halves: by then the next stage has landed and every wave
+            // has read the current one, whose buffer takes the loads of the stage
+            // after the next.  Bound by MFMA issue: TN 8192 x 8192 x 2048 73.0
+            // TFLOP/s, 4096^3 66.7, 3072^2 x 4096 (whose last 64 of 576 tiles run one
+            // per CU) 52 (68.5, 64.0 and 38-46 with all reads, then all loads, ahead
+            // of the stage's MFMAs).
+            const int nfull = (kend - kbeg) / GKB, ns = (kend - kbeg + GKB - 1) / GKB;
+            auto put = [&](int buf, int q) {
+                if (q < nfull)
+                    stage(buf, kbeg + GKB * q);
+                else if (q < ns)
+                    stage_tail(buf, kbeg + GKB * q);
+            };
+            put(0, 0);
+            __syncthreads();
+            put(1, 1);
+            frags(a0, b0, 0, 0);
+            int buf = 0, q = 0;
+            for (; q + 2 < nfull; ++q, buf ^= 1) {
+                frags(a1, b1, buf, 1);
+                mma(a0, b0);
+#pragma unroll
+                for (int u = 0; u < 8; ++u) {
+                    __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);     // MFMA
+                    __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);   // LDS read
                 }
-                // the other buffer was last read before the previous barrier
-                if (k0 + GKB < kend) {
-                    dma_stage<KCA>(pa, ka, lda, sA[buf ^ 1], wave, lane, k0 + GKB, kend);
-                    dma_stage<KCB>(pb, kb, ldb, sB[buf ^ 1], wave, lane, k0 + GKB, kend);
-                }
-#pragma unroll
-                for (int hh = 0; hh < 2; ++hh)
-#pragma unroll
-                    for (int st = 0; st < 2; ++st)
-#pragma unroll
-                        for (int i = 0; i < 4; ++i)
-#pragma unroll
-                            for (int j = 0; j < 4; ++j)
-                                acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(
-                                    b[j][hh][st], a[i][hh][st], acc[i][j], 0, 0, 0);
-                // keep the barrier (and its wait for the loads in flight) after the MFMAs
+                __builtin_amdgcn_sched_group_barrier(0x8, 24, 0);
                 __builtin_amdgcn_sched_barrier(0);
                 __syncthreads();
+                frags(a0, b0, buf ^ 1, 0);
+                stage(buf, kbeg + GKB * (q + 2));
+                mma(a1, b1);
+#pragma unroll
+                for (int u = 0; u < 8; ++u) {
+                    __builtin_amdgcn_sched_group_barrier(0x8, 1, 1);
+                    __builtin_amdgcn_sched_group_barrier(0x100, 1, 1);
+                }
+#pragma unroll
+                for (int u = 0; u < 8; ++u) {
+                    __builtin_amdgcn_sched_group_barrier(0x8, 1, 1);
+                    __builtin_amdgcn_sched_group_barrier(0x20, 1, 1);   // global -> LDS
+                }
+                __builtin_amdgcn_sched_group_barrier(0x8, 16, 1);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            for (; q < ns; ++q, buf ^= 1) {
+                frags(a1, b1, buf, 1);
+                mma(a0, b0);
+                if (q + 1 < ns) {
+                    __syncthreads();
+                    put(buf, q + 2);
+                    frags(a0, b0, buf ^ 1, 0);
+                }
+                mma(a1, b1);
             }
         }
     } else if (kbeg < kend) {
@@ -449,7 +503,7 @@ int launch_gemm_f64_batched(brpa_ctx *ctx, bool ta, bool tb, int64_t m, int64_t 
     // strides, aligned bases); a rows-contiguous operand also needs an even row
     // count, so that its last row pair lies inside the matrix
     g.dma = (lda % 2 == 0 && ldb % 2 == 0 && sA1 % 2 == 0 && sA2 % 2 == 0 && sB1 % 2 == 0 &&
-             sB2 % 2 == 0 && (reinterpret_cast<uintptr_t>(A) & 15) == 0 &&
+             sB2 % 2 == 0 && lda < (1 << 21) && ldb < (1 << 21) && (reinterpret_cast<uintptr_t>(A) & 15) == 0 &&
              (reinterpret_cast<uintptr_t>(B) & 15) == 0 && (ta || m % 2 == 0) &&
              (!tb || n % 2 == 0))
                 ? 1
