@@ -85,12 +85,11 @@ struct Counts {
     std::vector<int64_t> pdiag, trsm, update;   // per Cholesky step
 };
 
-Counts counts_of(const HostFrag &f, int nsteps_max, int precision, int i8_variant) {
+Counts counts_of(const HostFrag &f, int nsteps_max, int precision, int i8_variant, bool quad) {
     Counts c;
     const int64_t K = f.nocc * f.nvir, N = f.naux, F = f.nfreqs;
     c.dtab = cdiv(F * K, 256);
-    const int64_t nt = cdiv(N, SYRK_T);
-    c.syrk = (precision == BRPA_FP64) ? nt * (nt + 1) / 2 * cdiv(F, 4) : 0;
+    c.syrk = (precision == BRPA_FP64) ? syrk_items(N, F, quad) : 0;
     c.setdiag = cdiv(F * N, 256);
     const int64_t kpad = cdiv(K, SPLIT_KB) * SPLIT_KB;
     c.split = (precision == BRPA_SPLIT_BF16) ? (kpad / SPLIT_KB) * cdiv(N, 64) : 0;
@@ -146,8 +145,13 @@ int run_chunk(brpa_ctx *ctx, int precision, const std::vector<HostFrag> &fr, dou
         const int c = ctx->i8_choice[tune_bucket(fr[f].naux)];
         var[f] = ctx->tune_force >= 0 ? ctx->tune_force : (c >= 0 ? c : I8V_T128);
     }
+    int64_t syrk_n[2] = {0, 0};
+    for (int f = 0; f < nfrag; ++f)
+        for (int q = 0; q < 2; ++q) syrk_n[q] += syrk_items(fr[f].naux, fr[f].nfreqs, q == 1);
+    const bool quad = syrk_quad(ctx, syrk_n[0], syrk_n[1]);
     std::vector<Counts> cnt(nfrag);
-    for (int f = 0; f < nfrag; ++f) cnt[f] = counts_of(fr[f], nsteps_max, precision, var[f]);
+    for (int f = 0; f < nfrag; ++f)
+        cnt[f] = counts_of(fr[f], nsteps_max, precision, var[f], quad);
 
     // prefix arrays: [dtab, syrk, setdiag, split, syrk16, colscale8, split8,
     //                 syrk8 per variant, pdiag_0..S-1, trsm_0..S-1, update_0..S-1]
@@ -282,7 +286,7 @@ int run_chunk(brpa_ctx *ctx, int precision, const std::vector<HostFrag> &fr, dou
         BRPA_TRY(se(BRPA_STAGE_AUX));
         if (precision == BRPA_FP64) {
             BRPA_TRY(sb(BRPA_STAGE_PI));
-            BRPA_TRY(launch_syrk_f64(ctx, d_fr, DP(1), nfrag, TOT(1)));
+            BRPA_TRY(launch_syrk_f64(ctx, d_fr, DP(1), nfrag, TOT(1), quad, false));
             BRPA_TRY(se(BRPA_STAGE_PI));
         } else if (precision == BRPA_SPLIT_I8) {
             BRPA_TRY(sb(BRPA_STAGE_SPLIT));

@@ -80,9 +80,10 @@ extern "C" int brpa_ecrpa_grad(brpa_ctx *ctx, const double *R, int64_t naux, con
     const bool rdev = is_device_ptr(R), gdev = is_device_ptr(dR);
     FragDev fd{};
     std::vector<int64_t> pre = {0, 0, 0, 0, 0, 0};
-    const int64_t nt = cdiv(N, SYRK_T), nsteps = cdiv(N, CHOL_NB);
+    const bool quad = syrk_quad(ctx, syrk_items(N, F, false), syrk_items(N, F, true));
+    const int64_t nsteps = cdiv(N, CHOL_NB);
     pre[1] = cdiv(F * K, 256);
-    pre[3] = nt * (nt + 1) / 2 * cdiv(F, 4);
+    pre[3] = syrk_items(N, F, quad);
     pre[5] = cdiv(F * N, 256);
     FragDev *dfd;
     int64_t *dpre;
@@ -140,7 +141,7 @@ extern "C" int brpa_ecrpa_grad(brpa_ctx *ctx, const double *R, int64_t naux, con
     BRPA_HIP(ctx, hipEventRecord(ctx->ev0, s));
     // Pi_k (recomputed), 1 + Pi_k, its Cholesky factor (all k batched)
     BRPA_TRY(launch_dtab(ctx, dfd, dpre, 1, pre[1]));
-    BRPA_TRY(launch_syrk_f64(ctx, dfd, dpre + 2, 1, pre[3]));
+    BRPA_TRY(launch_syrk_f64(ctx, dfd, dpre + 2, 1, pre[3], quad, false));
     BRPA_TRY(launch_set_diag(ctx, dfd, dpre + 4, 1, pre[5], 0));
     BRPA_TRY(launch_fill(ctx, ddR, K * N, 0.0));
     BRPA_TRY(launch_fill(ctx, dd, K, 0.0));

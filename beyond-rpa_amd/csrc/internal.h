@@ -165,7 +165,7 @@ int copy_sync(brpa_ctx *ctx, void *dst, const void *src, size_t bytes, hipMemcpy
 //   R     : K x N row-major (R[ai][P]), K = nocc*nvir
 //   dtab  : F x K, dtab[w][k] = 4 d_k/(d_k^2 + u_w^2)   (prefactor included)
 //   Pi    : F x N x N row-major, lower triangle + diagonal is what the
-//           Cholesky reads; the SYRK writes both triangles
+//           Cholesky reads (the SYRK writes the other one on request)
 //   diag  : F x N exact FP64 diagonal of Pi
 //   ldpart: F x nsteps x 2 double-double partial log-det sums of the
 //           Cholesky diagonal blocks
@@ -213,7 +213,15 @@ constexpr int I8_KMAX = 65536;// split-int8: largest K with exact int32 level su
 // Launch wrappers (defined in the kernel files).  `pre` arrays are device
 // prefix sums over fragments of the number of work-groups per fragment.
 int launch_dtab(brpa_ctx *, const FragDev *, const int64_t *pre, int nfrag, int64_t total);
-int launch_syrk_f64(brpa_ctx *, const FragDev *, const int64_t *pre, int nfrag, int64_t total);
+// FP64 SYRK: quad selects its form (syrk_quad) and with it the work-groups per
+// fragment (syrk_items); both: also the upper triangle of Pi (the Cholesky reads
+// the lower one and the diagonal).
+int64_t syrk_items(int64_t N, int64_t F, bool quad);
+// whether the quad form is the faster one for a launch of these many work-groups
+// (summed over the fragments) in either form
+bool syrk_quad(const brpa_ctx *, int64_t wide_total, int64_t quad_total);
+int launch_syrk_f64(brpa_ctx *, const FragDev *, const int64_t *pre, int nfrag, int64_t total,
+                    bool quad, bool both);
 // mode: 0 = Pi's own diagonal, 1 = split-BF16 partials, 2 = diag precomputed
 int launch_set_diag(brpa_ctx *, const FragDev *, const int64_t *pre, int nfrag, int64_t total,
                     int mode);

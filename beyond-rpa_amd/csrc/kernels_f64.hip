@@ -2,7 +2,8 @@
 //
 //   k_dtab         c_w(ai) = 4 d/(d^2+u_w^2)           (rpa_core_MO.f90:379-401)
 //   k_syrk_f64     Pi_w = R^T diag(c_w) R on v_mfma_f64_16x16x4_f64, one R tile in
-//                  LDS shared by 4 waves = 4 frequencies  (dgemm of rpa_core_MO.f90:402)
+//                  LDS shared by 4 waves = 4 frequencies, or the quadrants of one
+//                  frequency's tile  (dgemm of rpa_core_MO.f90:402)
 //   k_set_diag     diag_w (tr Pi, rpa_CC.f90:444-447); Pi_w[P][P] += 1 (448-450)
 //   k_potrf_diag   Cholesky + inverse of a 64x64 diagonal block (four waves)
 //   k_trsm         L21 = A21 L11^{-T} on MFMA
@@ -25,6 +26,8 @@
 static inline unsigned grid1(int64_t total) { return (unsigned)total; }
 
 typedef double d2v_t __attribute__((ext_vector_type(2)));
+typedef __attribute__((address_space(1))) const double gdouble_t;
+typedef __attribute__((address_space(1))) double gdouble_mut_t;
 
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void k_dtab(const FragDev *__restrict__ fr,
@@ -53,107 +56,268 @@ int launch_dtab(brpa_ctx *ctx, const FragDev *fr, const int64_t *pre, int nfrag,
 }
 
 // ---------------------------------------------------------------------------
-// FP64 SYRK on MFMA.  One work-group = one 64x64 tile pair (tp >= tq) and a
-// group of 4 frequencies; wave w computes the whole tile for frequency
-// 4*g + w from the R tiles staged once in LDS.
+// FP64 SYRK on MFMA: one 64x64 tile pair (tp >= tq) per work-group, the two 64-column
+// panels of R staged in LDS 16 rows at a time.
 //
 // MFMA v_mfma_f64_16x16x4_f64 operand layout (lane l):
 //   A[m = l%16][k = l/16], B[k = l/16][n = l%16],
 //   D: 4 doubles, D[r] = C[m = l/16 + 4*r][n = l%16]  (probed on gfx950; the
 //   f32 shapes use 4*(l/16) + r instead).
-constexpr int KB = 16;        // rows of R per LDS stage
-constexpr int LDS_PAD = 16;   // +16 doubles per row: rows r and r+1 land 32 banks apart
+// Step s (of 4) of a stage takes the rows 4 s + l/16.
+//
+//   wide  (QUAD = false)  four frequencies per work-group: wave w computes the whole
+//         tile for frequency 4 g + w, so R is staged once for four products
+//   quad  (QUAD = true)   one frequency: wave (w/2, w%2) computes a 32x32 quadrant,
+//         for launches whose wide form would not fill the chip (syrk_quad)
+//
+// The stages go straight from global memory into LDS, double-buffered, rows of 64
+// doubles with the 16-double blocks of odd rows swapped in pairs, so that the four
+// lane groups of an operand read (four consecutive rows) hit both halves of the 64
+// banks.  An even N and a 16-byte aligned R take 16 bytes per lane (V = 16), others
+// 4 bytes (V = 4, four times the load instructions).  Columns past N repeat the last
+// one (pair): they only reach products that are not stored.  A last stage with fewer
+// than 16 rows goes through registers with zeros past K.  A diagonal tile needs one
+// panel and the blocks i >= j only.
+//
+// Bound by MFMA issue.  The reads of one half of a stage run while the other half is
+// multiplied, the barrier stands between the halves (as in k_gemm_f64).  Measured at
+// K = 19200, N = 2400, 16 frequencies: 64.1 TFLOP/s (56.2 with register-staged
+// stages between two barriers); K = 10800, N = 1800, 24 frequencies: 60.9 (51.1),
+// N = 1801: 59.3 (50.9).
+constexpr int KB = 16;                    // rows of R per LDS stage
+constexpr int SYRK_P = KB * SYRK_T;       // doubles per panel stage
 
-__device__ __forceinline__ void syrk_f64_tile(const double *__restrict__ R, int K, int N,
-                                              const double *__restrict__ dtab, int F, int w0,
-                                              double *__restrict__ Pi, int tp, int tq) {
-    __shared__ double sA[KB][SYRK_T + LDS_PAD];
-    __shared__ double sB[KB][SYRK_T + LDS_PAD];
-    __shared__ double sD[4][KB];
-    const int tid = threadIdx.x;
-    const int wave = tid >> 6, lane = tid & 63;
-    const int p0 = tp * SYRK_T, q0 = tq * SYRK_T;
-    const int w = w0 + wave;
+struct SyrkPanel {
+    uint32_t off[4];   // V = 16: the two loads of a wave; V = 4: [half][row parity]
+};
 
-    d4_t acc[4][4];
+// byte offsets from R + k0 N + c0 of the lane's part of a wave's loads
+template <int V>
+__device__ __forceinline__ SyrkPanel syrk_panel(int N, int c0, int wave, int lane) {
+    SyrkPanel p;
+    if (V == 16) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = (d4_t){0.0, 0.0, 0.0, 0.0};
-
-    double ra[4], rb[4], rd = 0.0;
-    auto gload = [&](int k0) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            int e = tid + 256 * i;
-            int r = e >> 6, c = e & 63;
-            int k = k0 + r;
-            bool kin = k < K;
-            ra[i] = (kin && p0 + c < N) ? R[(int64_t)k * N + p0 + c] : 0.0;
-            rb[i] = (kin && q0 + c < N) ? R[(int64_t)k * N + q0 + c] : 0.0;
+        for (int t = 0; t < 2; ++t) {
+            const int kr = 4 * wave + 2 * t + (lane >> 5);
+            const int c = 2 * ((lane & 31) ^ (8 * (kr & 1)));
+            p.off[t] = 8u * ((uint32_t)kr * (uint32_t)N + (uint32_t)(min(c0 + c, N - 2) - c0));
         }
-        if (tid < 4 * KB) {
-            int ww = w0 + (tid / KB), k = k0 + (tid % KB);
-            rd = (ww < F && k < K) ? dtab[(int64_t)ww * K + k] : 0.0;
-        }
-    };
-    auto lstore = [&]() {
+    } else {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            int e = tid + 256 * i;
-            int r = e >> 6, c = e & 63;
-            sA[r][c] = ra[i];
-            sB[r][c] = rb[i];
-        }
-        if (tid < 4 * KB) sD[tid / KB][tid % KB] = rd;
-    };
-
-    gload(0);
-    for (int k0 = 0; k0 < K; k0 += KB) {
-        __syncthreads();
-        lstore();
-        __syncthreads();
-        if (k0 + KB < K) gload(k0 + KB);
-#pragma unroll
-        for (int kk = 0; kk < KB; kk += 4) {
-            const int kr = kk + (lane >> 4);
-            const double dv = sD[wave][kr];
-            double a[4], bv[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) a[i] = sA[kr][16 * i + (lane & 15)] * dv;
-#pragma unroll
-            for (int j = 0; j < 4; ++j) bv[j] = sB[kr][16 * j + (lane & 15)];
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int j = 0; j < 4; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i], bv[j], acc[i][j], 0, 0, 0);
+        for (int q = 0; q < 4; ++q) {
+            const int c = (32 * (q >> 1) + (lane >> 1)) ^ (16 * (q & 1));
+            p.off[q] = 8u * (uint32_t)(min(c0 + c, N - 1) - c0) + 4u * (lane & 1);
         }
     }
-
-    if (w >= F) return;
-    double *C = Pi + (int64_t)w * N * N;
-    const bool diag = (tp == tq);
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                int p = p0 + 16 * i + (lane >> 4) + 4 * r;
-                int q = q0 + 16 * j + (lane & 15);
-                if (p < N && q < N) {
-                    double v = acc[i][j][r];
-                    C[(int64_t)p * N + q] = v;
-                    if (!diag) C[(int64_t)q * N + p] = v;
-                }
-            }
+    return p;
 }
 
-// Work-groups per fragment: npairs(ceil(N/64)) * ceil(F/4), pair-major within
-// a frequency group.
-__global__ __launch_bounds__(256) void k_syrk_f64(const FragDev *__restrict__ fr,
-                                                 const int64_t *__restrict__ pre, int nfrag) {
+template <int V>
+__device__ __forceinline__ void syrk_stage(const SyrkPanel &p, const char *base, int N, double *L,
+                                           int wave) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    typedef __attribute__((address_space(1))) const char gchar_t;
+    typedef __attribute__((address_space(3))) void lvoid_t;
+    if (V == 16) {
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+            __builtin_amdgcn_global_load_lds(
+                (const __attribute__((address_space(1))) void *)((gchar_t *)base + p.off[t]),
+                (lvoid_t *)(L + (4 * wave + 2 * t) * SYRK_T), 16, 0, 0);
+    } else {
+#pragma unroll
+        for (int t = 0; t < 8; ++t) {
+            const int kr = 4 * wave + (t >> 1);
+            __builtin_amdgcn_global_load_lds(
+                (const __attribute__((address_space(1))) void *)((gchar_t *)base +
+                                                                 8 * (int64_t)N * kr +
+                                                                 p.off[2 * (t & 1) + ((t >> 1) & 1)]),
+                (lvoid_t *)(L + kr * SYRK_T + 32 * (t & 1)), 4, 0, 0);
+        }
+    }
+#endif
+}
+
+// rows k0 .. K - 1 (fewer than 16) of a panel, zeros below
+__device__ __forceinline__ void syrk_stage_tail(const double *__restrict__ R, int K, int N, int k0,
+                                                int c0, double *L, int tid) {
+    const gdouble_t *G = (const gdouble_t *)R;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        const int kr = (tid >> 6) + 4 * u, c = tid & 63;
+        const bool ok = k0 + kr < K && c0 + c < N;
+        const double v = G[ok ? (int64_t)(k0 + kr) * N + c0 + c : 0];
+        L[kr * SYRK_T + (c ^ (16 * (kr & 1)))] = ok ? v : 0.0;
+    }
+}
+
+template <int V, bool QUAD, bool DIAG>
+__device__ __forceinline__ void syrk_f64_tile(const FragDev &F, int w0, int tp, int tq, int both,
+                                              double *__restrict__ sA, double *__restrict__ sB) {
+    const double *__restrict__ R = F.R;
+    const int K = F.K, N = F.N;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int p0 = tp * SYRK_T, q0 = tq * SYRK_T;
+    const int w = QUAD ? w0 : w0 + wave;
+    constexpr int NB = QUAD ? 2 : 4;            // 16-row blocks per wave and side
+    const int bi = QUAD ? 2 * (wave >> 1) : 0, bj = QUAD ? 2 * (wave & 1) : 0;
+    // waves past the last frequency, and the quadrant above the diagonal, only stage
+    const bool active = w < F.F && !(QUAD && DIAG && bj > bi);
+    const int rl = lane & 15, g4 = lane >> 4;
+    const SyrkPanel pa = syrk_panel<V>(N, p0, wave, lane);
+    const SyrkPanel pb = DIAG ? pa : syrk_panel<V>(N, q0, wave, lane);
+    const char *ba = reinterpret_cast<const char *>(R + p0);
+    const char *bb = reinterpret_cast<const char *>(R + q0);
+    const int nfull = K / KB, ns = (K + KB - 1) / KB;
+    auto stage = [&](int buf, int q) {
+        const int64_t o = 8 * (int64_t)N * (KB * q);
+        syrk_stage<V>(pa, ba + o, N, sA + buf * SYRK_P, wave);
+        if (!DIAG) syrk_stage<V>(pb, bb + o, N, sB + buf * SYRK_P, wave);
+    };
+    auto put = [&](int buf, int q) {
+        if (q < nfull) {
+            stage(buf, q);
+        } else if (q < ns) {
+            syrk_stage_tail(R, K, N, KB * q, p0, sA + buf * SYRK_P, tid);
+            if (!DIAG) syrk_stage_tail(R, K, N, KB * q, q0, sB + buf * SYRK_P, tid);
+        }
+    };
+    put(0, 0);
+    if (!active) {
+        __syncthreads();
+        put(1, 1);
+        for (int q = 0; q + 1 < ns; ++q) {
+            __syncthreads();
+            put(q & 1, q + 2);
+        }
+        return;
+    }
+    d4_t acc[NB][NB];
+#pragma unroll
+    for (int i = 0; i < NB; ++i)
+#pragma unroll
+        for (int j = 0; j < NB; ++j) acc[i][j] = (d4_t){0.0, 0.0, 0.0, 0.0};
+    // element (row 4 s + g4, column 16 b + rl) of a stage; the block index of odd rows
+    // has its low bit flipped
+    const int x0 = g4 * SYRK_T + rl + 16 * (g4 & 1), x1 = g4 * SYRK_T + rl - 16 * (g4 & 1);
+    auto frags = [&](double (&a)[2][NB], double (&b)[2][NB], int buf, int h) {
+        const double *LA = sA + buf * SYRK_P + 16 * bi;
+        const double *LB = (DIAG ? sA : sB) + buf * SYRK_P + 16 * bj;
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+#pragma unroll
+            for (int i = 0; i < NB; ++i)
+                a[s][i] = LA[(i & 1 ? x1 : x0) + 16 * i + 4 * (2 * h + s) * SYRK_T];
+#pragma unroll
+            for (int j = 0; j < NB; ++j)
+                b[s][j] = LB[(j & 1 ? x1 : x0) + 16 * j + 4 * (2 * h + s) * SYRK_T];
+        }
+    };
+    auto mma = [&](const double (&a)[2][NB], const double (&b)[2][NB], double d0, double d1) {
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+#pragma unroll
+            for (int i = 0; i < NB; ++i) {
+                const double x = a[s][i] * (s ? d1 : d0);
+#pragma unroll
+                for (int j = 0; j < NB; ++j)
+                    if (QUAD || !DIAG || i >= j)
+                        acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(x, b[s][j], acc[i][j], 0, 0, 0);
+            }
+    };
+    // c_w of the lane's four rows of stage q
+    const gdouble_t *dt = (const gdouble_t *)F.dtab + (int64_t)w * K;
+    auto coef = [&](double (&d)[4], int q) {
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            const int k = KB * q + 4 * s + g4;
+            d[s] = dt[min(k, K - 1)];   // rows past K are zero
+        }
+    };
+    double a0[2][NB], b0[2][NB], a1[2][NB], b1[2][NB], dv[4], dn[4];
+    coef(dv, 0);
+    __syncthreads();
+    put(1, 1);
+    frags(a0, b0, 0, 0);
+    int buf = 0, q = 0;
+    for (; q + 2 < nfull; ++q, buf ^= 1) {
+        coef(dn, q + 1);
+        frags(a1, b1, buf, 1);
+        mma(a0, b0, dv[0], dv[1]);
+        if (!QUAD) {
+            constexpr int NM = DIAG ? 20 : 32;
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+                __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);     // MFMA
+                __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);   // LDS read
+            }
+            __builtin_amdgcn_sched_group_barrier(0x8, NM - 8, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        __syncthreads();
+        frags(a0, b0, buf ^ 1, 0);
+        stage(buf, q + 2);
+        mma(a1, b1, dv[2], dv[3]);
+        if (!QUAD) {
+            constexpr int NM = DIAG ? 20 : 32, NL = (V == 16 ? 2 : 8) * (DIAG ? 1 : 2);
+            constexpr int NL1 = NL < NM - 8 ? NL : NM - 8;
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+                __builtin_amdgcn_sched_group_barrier(0x8, 1, 1);
+                __builtin_amdgcn_sched_group_barrier(0x100, 1, 1);
+            }
+#pragma unroll
+            for (int u = 0; u < NL1; ++u) {
+                __builtin_amdgcn_sched_group_barrier(0x8, 1, 1);
+                __builtin_amdgcn_sched_group_barrier(0x20, 1, 1);    // global -> LDS
+            }
+            __builtin_amdgcn_sched_group_barrier(0x8, NM - 8 - NL1, 1);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int s = 0; s < 4; ++s) dv[s] = dn[s];
+    }
+    for (; q < ns; ++q, buf ^= 1) {
+        coef(dn, min(q + 1, ns - 1));
+        frags(a1, b1, buf, 1);
+        mma(a0, b0, dv[0], dv[1]);
+        if (q + 1 < ns) {
+            __syncthreads();
+            put(buf, q + 2);
+            frags(a0, b0, buf ^ 1, 0);
+        }
+        mma(a1, b1, dv[2], dv[3]);
+#pragma unroll
+        for (int s = 0; s < 4; ++s) dv[s] = dn[s];
+    }
+
+    gdouble_mut_t *C = (gdouble_mut_t *)(F.Pi + (int64_t)w * N * N);
+#pragma unroll
+    for (int i = 0; i < NB; ++i)
+#pragma unroll
+        for (int j = 0; j < NB; ++j) {
+            if (DIAG && bi + i < bj + j) continue;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int p = p0 + 16 * (bi + i) + g4 + 4 * r;
+                const int c = q0 + 16 * (bj + j) + rl;
+                if (p < N && c <= p) {
+                    const double v = acc[i][j][r];
+                    C[(int64_t)p * N + c] = v;
+                    if (both) C[(int64_t)c * N + p] = v;
+                }
+            }
+        }
+}
+
+// Work-groups per fragment: syrk_items(N, F, QUAD), pair-major within a frequency
+// (group).  both: the upper triangle of Pi is written too.
+template <bool QUAD>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, QUAD ? 4 : 2))) void
+k_syrk_f64(const FragDev *__restrict__ fr, const int64_t *__restrict__ pre, int nfrag, int both) {
+    __shared__ __attribute__((aligned(16))) double sA[2 * SYRK_P];
+    __shared__ __attribute__((aligned(16))) double sB[2 * SYRK_P];
     int64_t b = blockIdx.x;
     int f = find_frag(pre, nfrag, b);
     const FragDev &F = fr[f];
@@ -163,12 +327,47 @@ __global__ __launch_bounds__(256) void k_syrk_f64(const FragDev *__restrict__ fr
     int g = (int)(lb / npairs), pair = (int)(lb - (int64_t)g * npairs);
     int tp, tq;
     tri_decode(pair, tp, tq);
-    syrk_f64_tile(F.R, F.K, F.N, F.dtab, F.F, 4 * g, F.Pi, tp, tq);
+    const int w0 = QUAD ? g : 4 * g;
+    const bool wide = F.N % 2 == 0 && (reinterpret_cast<uintptr_t>(F.R) & 15) == 0;
+    if (tp == tq) {
+        if (wide)
+            syrk_f64_tile<16, QUAD, true>(F, w0, tp, tq, both, sA, sB);
+        else
+            syrk_f64_tile<4, QUAD, true>(F, w0, tp, tq, both, sA, sB);
+    } else {
+        if (wide)
+            syrk_f64_tile<16, QUAD, false>(F, w0, tp, tq, both, sA, sB);
+        else
+            syrk_f64_tile<4, QUAD, false>(F, w0, tp, tq, both, sA, sB);
+    }
 }
 
-int launch_syrk_f64(brpa_ctx *ctx, const FragDev *fr, const int64_t *pre, int nfrag, int64_t total) {
+int64_t syrk_items(int64_t N, int64_t F, bool quad) {
+    const int64_t nt = (N + SYRK_T - 1) / SYRK_T;
+    return nt * (nt + 1) / 2 * (quad ? F : (F + 3) / 4);
+}
+
+// In units of one tile's four products on a CU: the wide form takes one per
+// work-group, the quad form a quarter, at 1.2 times the cost (twice the LDS reads and
+// four times the loads per product).  What decides is the last round of work-groups
+// over the CUs.  Measured (wide, quad, us): 112 tiles 84, 59; 220 tiles 401, 466;
+// 360 tiles of 10 frequencies 897, 688, of 12 954, 928; 612 tiles 1803, 1829; 2610
+// tiles 13794, 16927.
+bool syrk_quad(const brpa_ctx *ctx, int64_t wide_total, int64_t quad_total) {
+    const int64_t ncu = ctx->ncu > 0 ? ctx->ncu : 256;
+    const int64_t wide = (wide_total + ncu - 1) / ncu, quad = (quad_total + ncu - 1) / ncu;
+    return 0.25 * 1.2 * (double)quad < (double)wide;
+}
+
+int launch_syrk_f64(brpa_ctx *ctx, const FragDev *fr, const int64_t *pre, int nfrag, int64_t total,
+                    bool quad, bool both) {
     if (total <= 0) return BRPA_OK;
-    hipLaunchKernelGGL(k_syrk_f64, dim3(grid1(total)), dim3(256), 0, ctx->stream, fr, pre, nfrag);
+    if (quad)
+        hipLaunchKernelGGL(k_syrk_f64<true>, dim3(grid1(total)), dim3(256), 0, ctx->stream, fr, pre,
+                           nfrag, both ? 1 : 0);
+    else
+        hipLaunchKernelGGL(k_syrk_f64<false>, dim3(grid1(total)), dim3(256), 0, ctx->stream, fr,
+                           pre, nfrag, both ? 1 : 0);
     LAUNCH_CHECK(ctx);
     return BRPA_OK;
 }
@@ -255,8 +454,6 @@ __device__ __forceinline__ void mma64_xyt(const double (*sX)[CHOL_NB + 1],
     }
 }
 
-typedef __attribute__((address_space(1))) const double gdouble_t;
-typedef __attribute__((address_space(1))) double gdouble_mut_t;
 
 template <int ROWS, int THREADS, int NP>
 __device__ __forceinline__ void load_panels64(double (*const *s)[CHOL_NB + 1],

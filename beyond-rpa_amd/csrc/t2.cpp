@@ -269,9 +269,9 @@ int t2_build(brpa_ctx *ctx, int precision, const double *R, int64_t naux, const 
     int8_t *SCR = nullptr, *SRR = nullptr, *SOT = nullptr, *SY = nullptr;
     double *scCR = nullptr, *scRR = nullptr, *scOT = nullptr, *scY = nullptr, *pmx = nullptr;
     std::vector<int64_t> pre = {0, 0, 0, 0, 0, 0};
-    const int64_t ntile = cdiv(N, SYRK_T);
+    const bool quad = syrk_quad(ctx, syrk_items(N, F, false), syrk_items(N, F, true));
     pre[1] = cdiv(F * K, 256);                      // dtab
-    pre[3] = ntile * (ntile + 1) / 2 * cdiv(F, 4);  // syrk
+    pre[3] = syrk_items(N, F, quad);              // syrk
     pre[5] = cdiv(F * N, 256);                      // set_diag
     int64_t *dpre = nullptr;
     FragDev *dfd = nullptr;
@@ -363,7 +363,7 @@ int t2_build(brpa_ctx *ctx, int precision, const double *R, int64_t naux, const 
 
     // Pi_k for all k (FP64 MFMA SYRK), then 1 + l Pi_k and its Cholesky factor
     BRPA_TRY(launch_dtab(ctx, dfd, dpre, 1, pre[1]));
-    BRPA_TRY(launch_syrk_f64(ctx, dfd, dpre + 2, 1, pre[3]));
+    BRPA_TRY(launch_syrk_f64(ctx, dfd, dpre + 2, 1, pre[3], quad, false));
     if (lambda != 1.0) BRPA_TRY(launch_scale(ctx, fd.Pi, lambda, F * N * N));
     BRPA_TRY(launch_set_diag(ctx, dfd, dpre + 4, 1, pre[5], 0));
     // all F factors in one batched blocked Cholesky (the library's own kernels).

@@ -83,8 +83,8 @@ int brpa_thc_piu(brpa_ctx *ctx, double *PiU, double *Rkai, const double *Xga, co
     const bool rdev = Rkai && is_device_ptr(Rkai);
     // the SYRK writes Pi directly into a device PiU that it overwrites
     const bool direct = pdev && !accumulate;
-    const int64_t ntile = cdiv(N, SYRK_T);
-    const int64_t total = ntile * (ntile + 1) / 2 * cdiv(F, 4);
+    const bool quad = syrk_quad(ctx, syrk_items(N, F, false), syrk_items(N, F, true));
+    const int64_t total = syrk_items(N, F, quad);
     FragDev fd{};
     FragDev *dfd = nullptr;
     int64_t *dpre = nullptr;
@@ -127,7 +127,7 @@ int brpa_thc_piu(brpa_ctx *ctx, double *PiU, double *Rkai, const double *Xga, co
     BRPA_TRY(launch_thc_r(ctx, dXa, dXi, dZ, G, nocc, nvir, N, dR));
     BRPA_TRY(stage_end(ctx, BRPA_STAGE_THC_R));
     BRPA_TRY(stage_begin(ctx, BRPA_STAGE_THC_PI));
-    BRPA_TRY(launch_syrk_f64(ctx, dfd, dpre, 1, total));
+    BRPA_TRY(launch_syrk_f64(ctx, dfd, dpre, 1, total, quad, true));
     BRPA_TRY(stage_end(ctx, BRPA_STAGE_THC_PI));
     BRPA_HIP(ctx, hipEventRecord(ctx->ev1, ctx->stream));
     if (accumulate) {

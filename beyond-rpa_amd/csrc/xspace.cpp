@@ -149,9 +149,9 @@ int exchange_xspace(brpa_ctx *ctx, const double *R, int64_t naux, const double *
     int *dinfo;
     DenseChol dc;
     std::vector<int64_t> pre = {0, 0, 0, 0, 0, 0};
-    const int64_t ntile = cdiv(N, SYRK_T);
+    const bool quad = syrk_quad(ctx, syrk_items(N, F, false), syrk_items(N, F, true));
     pre[1] = cdiv(F * K, 256);                      // dtab
-    pre[3] = ntile * (ntile + 1) / 2 * cdiv(F, 4);  // syrk
+    pre[3] = syrk_items(N, F, quad);              // syrk
     pre[5] = cdiv(F * N, 256);                      // set_diag
     const int64_t nparts = K;   // one partial sum per column of the contraction
     const int64_t nsplitws = std::max<int64_t>(
@@ -240,7 +240,7 @@ int exchange_xspace(brpa_ctx *ctx, const double *R, int64_t naux, const double *
     // 1. Pi_k (FP64 MFMA SYRK), 1 + l Pi_k, Cholesky factors of all F in one batch
     BRPA_TRY(begin(BRPA_STAGE_T2_PI));
     BRPA_TRY(launch_dtab(ctx, dfd, dpre, 1, pre[1]));
-    BRPA_TRY(launch_syrk_f64(ctx, dfd, dpre + 2, 1, pre[3]));
+    BRPA_TRY(launch_syrk_f64(ctx, dfd, dpre + 2, 1, pre[3], quad, false));
     if (lambda != 1.0) BRPA_TRY(launch_scale(ctx, fd.Pi, lambda, F * N * N));
     BRPA_TRY(launch_set_diag(ctx, dfd, dpre + 4, 1, pre[5], 0));
     BRPA_TRY(chol_single(ctx, dfd, dchol, N, F));
