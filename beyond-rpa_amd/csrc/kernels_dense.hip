@@ -32,7 +32,6 @@
 namespace {
 constexpr int GT = 128;    // GEMM tile edge
 constexpr int GKB = 16;    // k per LDS stage
-constexpr int GPAD = 16;   // LDS row padding: rows k and k+1 start 128 B apart mod 256 B
 constexpr int GGROUP = 8;  // tile rows per group of the tile order (panel reuse in L2)
 }
 
@@ -40,23 +39,15 @@ constexpr int GGROUP = 8;  // tile rows per group of the tile order (panel reuse
 // Batched C = alpha op(A) op(B) diag(cs) + beta C on 128 x 128 tiles, four
 // waves of 64 x 64 per work-group, v_mfma_f64_16x16x4_f64.
 //
-// Stages of 16 k go to LDS as [row][k] for both operands (row pitch 18
-// doubles), double-buffered: the next stage is loaded into registers while
-// the current one is multiplied, and stored into the other buffer halfway
-// through it, one barrier per stage.  Every thread moves pairs of consecutive
-// k of one row (one ds_write_b128).  In a stage, lane l of a wave supplies the k values
-// 4 (l / 16) .. +3 of its row to the four MFMA steps, so its operands for the
-// whole stage are two ds_read_b128 per 16-row block; the 16 rows of such a
-// read land on distinct 4-bank groups (pitch 36 dwords).  The k order inside
-// a stage is a permutation of the sum, the same for both operands.  The MFMA
-// takes the B fragment as its first operand, so the accumulator rows run along
-// the lanes (D[r] = C(row = lane%16, col = lane/16 + 4r) of a 16 x 16 block)
-// and the stores of C are contiguous across lanes.
-//
-// Global loads by orientation: op(A) = A (TA = false) holds rows contiguous,
-// so lanes take consecutive rows at two k; TA holds k contiguous, so eight
-// lanes read one row's 16 consecutive k.  op(B) = B (TB = false) is k-
-// contiguous, TB rows-contiguous.
+// Stages of 16 k go straight from global memory into LDS (global_load_lds, no
+// register staging and no LDS store instructions), double-buffered, in the
+// layouts at dma_offsets.  In a stage, lane l of a wave supplies the k values
+// 4 (l / 16) .. +3 of its row to the four MFMA steps.  The k order inside a stage
+// is a permutation of the sum, the same for both operands.  The MFMA takes the B
+// fragment as its first operand, so the accumulator rows run along the lanes
+// (D[r] = C(row = lane%16, col = lane/16 + 4r) of a 16 x 16 block) and the stores
+// of C are contiguous across lanes.  op(A) = A (TA = false) holds rows contiguous,
+// TA holds k contiguous; op(B) = B (TB = false) is k-contiguous, TB rows-contiguous.
 //
 // Batches: work-group x = (item along dimension 1) * tiles + tile, y = item
 // along dimension 2; every operand moves by its own stride per item.  Tile
@@ -71,20 +62,17 @@ constexpr int GGROUP = 8;  // tile rows per group of the tile order (panel reuse
 // Split k (nsplit > 1, one item only): work-group z takes the z-th chunk of k
 // and writes its partial tile to P + z m n (ld m); k_gemm_reduce then adds the
 // partials in order and applies alpha, cs and beta.
-// With even leading dimensions and strides, 16-byte aligned operands and, for
-// an operand contiguous in rows, an even row count (dma = 1), each stage goes
-// from global memory straight into LDS (global_load_lds_dwordx4, 16 bytes per
-// lane, 1 KB per wave instruction) with no register staging and no LDS store
-// instructions (layouts at dma_offsets).  Rows past m (n) repeat the last row
-// (pair): they only reach products that are not stored.  A last stage with
-// fewer than 16 k goes through registers with zeros past kend.  The k order of
-// the sum is the same as in the register-staged form.
+// V: bytes per lane of the loads.  16 (1 KB per wave instruction) with even leading
+// dimensions and strides, 16-byte aligned operands and, for an operand contiguous in
+// rows, an even row count; 4 (256 bytes) otherwise.  Rows past m (n) repeat the last
+// row (pair): they only reach products that are not stored.  A last stage with fewer
+// than 16 k goes through registers with zeros past kend.
 struct GemmArgs {
     int m, n, k;
     int mt, nt, ntiles;
     int upper, tri, nb1;
     int nsplit, kchunk;
-    int dma;   // operands staged by direct global -> LDS loads
+    int far;   // a leading dimension too large for 32-bit offsets: every stage through registers
     double alpha, beta;
     const double *A;
     int64_t lda, sA1, sA2;
@@ -98,44 +86,56 @@ struct GemmArgs {
 };
 
 namespace {
-constexpr int KP = GKB + 2;   // LDS row pitch (doubles)
 typedef double d2_t __attribute__((ext_vector_type(2)));
 }
 
-// Direct-to-LDS staging of one operand of a 128-row tile and 16-k stage.
-// k-contiguous (KC): [row][k] with unpadded 16-double rows; wave w loads the
-// 8-row blocks 32 w + 8 c (c < 4), lane L the k pair (L % 8) ^ ((row >> 1) & 7)
-// of row 8 c + L / 8 of its block.  Rows-contiguous: [k][row] with rows of
-// DMA_KPR doubles (a pitch of 4 rows moves by half of the 64 LDS banks, so
-// the four lane groups of a fragment read hit disjoint halves); wave w loads
-// the k rows 4 w + c, lane L the rows 2 L, 2 L + 1.  dk: the lane's k offset
-// within a stage (KC, pair start) or its k row.
+// LDS layout of one operand's 128-row tile and 16-k stage.  k-contiguous (KC): [row][k]
+// with unpadded 16-double rows whose k pairs are XOR-swizzled by (row >> 1) & 7.
+// Rows-contiguous: [k][row] with rows of DMA_KPR doubles (a pitch of 4 rows moves by
+// half of the 64 LDS banks, so the four lane groups of a fragment read hit disjoint
+// halves).
+//
+// A wave's loads, V = 16: KC the 8-row blocks 32 w + 8 c (c < 4), lane L the k pair
+// (L % 8) ^ swizzle of row L / 8 of its block; rows-contiguous the k rows 4 w + c,
+// lane L the rows 2 L, 2 L + 1.  The byte offsets from the tile's base at k = 0
+// (dma_base) are 32-bit; leading dimensions of 2^21 or more take the register
+// path of the last stage for all of them.
+// V = 4: KC the row pairs 32 w + 2 c (c < 16), lane L a half of a double of row L / 32;
+// rows-contiguous the k rows 4 w + c / 4, 32 rows at a time.
 constexpr int DMA_KPR = 132;
-// off: the lane's byte offsets from the tile's base at k = 0 (dma_base); the
-// launch checks that 128 rows stay within 32 bits
-template <bool KC>
-__device__ __forceinline__ void dma_offsets(int64_t ldx, int r0, int rows, int wave, int lane,
-                                            uint32_t (&off)[4], int (&dk)[4]) {
+template <bool KC, int V>
+struct DmaSrc {
+    // per load; V = 4 rows-contiguous: per 32 rows
+    static constexpr int NOFF = KC && V == 4 ? 16 : 4;
+    uint32_t off[NOFF];
+};
+template <bool KC, int V>
+__device__ __forceinline__ DmaSrc<KC, V> dma_offsets(int64_t ldx, int r0, int rows, int wave,
+                                                     int lane) {
+    DmaSrc<KC, V> s;
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {
-        if (KC) {
+    for (int c = 0; c < DmaSrc<KC, V>::NOFF; ++c) {
+        if (V == 16 && KC) {
             const int row = 32 * wave + 8 * c + (lane >> 3);
-            dk[c] = 2 * ((lane & 7) ^ ((row >> 1) & 7));
-            off[c] = 8u * ((uint32_t)ldx * (uint32_t)(min(r0 + row, rows - 1) - r0) + (uint32_t)dk[c]);
-        } else {
+            const int dk = 2 * ((lane & 7) ^ ((row >> 1) & 7));
+            s.off[c] = 8u * ((uint32_t)ldx * (uint32_t)(min(r0 + row, rows - 1) - r0) + (uint32_t)dk);
+        } else if (V == 16) {
             // rows is even here: the last pair is rows - 2, rows - 1
-            dk[c] = 4 * wave + c;
-            off[c] = 8u * ((uint32_t)(min(r0 + 2 * lane, rows - 2) - r0) + (uint32_t)ldx * (uint32_t)dk[c]);
+            s.off[c] = 8u * ((uint32_t)(min(r0 + 2 * lane, rows - 2) - r0) +
+                             (uint32_t)ldx * (uint32_t)(4 * wave + c));
+        } else if (KC) {
+            const int row = 32 * wave + 2 * c + (lane >> 5);
+            s.off[c] = 8u * ((uint32_t)ldx * (uint32_t)(min(r0 + row, rows - 1) - r0)) +
+                       4u * (((uint32_t)lane & 31u) ^ (4u * (c & 7)));
+        } else {
+            s.off[c] = 8u * (uint32_t)(min(r0 + 32 * c + (lane >> 1), rows - 1) - r0) + 4u * (lane & 1);
         }
     }
+    return s;
 }
 template <bool KC>
 __device__ __forceinline__ const char *dma_base(const double *X, int64_t ldx, int r0) {
     return reinterpret_cast<const char *>(X + (KC ? ldx * r0 : (int64_t)r0));
-}
-template <bool KC>
-__device__ __forceinline__ int dma_block(int wave, int c) {
-    return KC ? (32 * wave + 8 * c) * GKB : (4 * wave + c) * DMA_KPR;
 }
 // fragment of row `row` at the k pair 2 g4 + hh of a stage
 template <bool KC>
@@ -152,41 +152,56 @@ __host__ __device__ __forceinline__ d2_t dma_frag(const double *L, int row, int 
 }
 
 // one operand's full stage at k0 into the LDS buffer L, straight from global memory
-template <bool KC>
-__device__ __forceinline__ void dma_stage(const char *base, const uint32_t (&off)[4], int64_t ldx,
+template <bool KC, int V>
+__device__ __forceinline__ void dma_stage(const char *base, const DmaSrc<KC, V> &src, int64_t ldx,
                                           double *L, int wave, int k0) {
     // the builtin exists for the device pass only; the host pass never runs this
 #if defined(__HIP_DEVICE_COMPILE__)
-    const char *b = base + 8 * (KC ? (int64_t)k0 : ldx * k0);
+    typedef __attribute__((address_space(1))) const char gchar_t;
+    typedef __attribute__((address_space(1))) const void gvoid_t;
+    typedef __attribute__((address_space(3))) void lvoid_t;
+    gchar_t *b = (gchar_t *)(base + 8 * (KC ? (int64_t)k0 : ldx * k0));
+    if (V == 16) {
 #pragma unroll
-    for (int c = 0; c < 4; ++c)
-        __builtin_amdgcn_global_load_lds(
-            reinterpret_cast<const __attribute__((address_space(1))) void *>(
-                (__attribute__((address_space(1))) const char *)b + off[c]),
-            (__attribute__((address_space(3))) void *)(L + dma_block<KC>(wave, c)), 16, 0, 0);
+        for (int c = 0; c < 4; ++c)
+            __builtin_amdgcn_global_load_lds(
+                (gvoid_t *)(b + src.off[c]),
+                (lvoid_t *)(L + (KC ? (32 * wave + 8 * c) * GKB : (4 * wave + c) * DMA_KPR)), 16, 0,
+                0);
+    } else if (KC) {
+#pragma unroll
+        for (int c = 0; c < 16; ++c)
+            __builtin_amdgcn_global_load_lds((gvoid_t *)(b + src.off[c]),
+                                             (lvoid_t *)(L + (32 * wave + 2 * c) * GKB), 4, 0, 0);
+    } else {
+#pragma unroll
+        for (int c = 0; c < 16; ++c) {
+            const int kr = 4 * wave + (c >> 2);
+            __builtin_amdgcn_global_load_lds((gvoid_t *)(b + 8 * ldx * kr + src.off[c % DmaSrc<KC, V>::NOFF]),
+                                             (lvoid_t *)(L + kr * DMA_KPR + 32 * (c & 3)), 4, 0, 0);
+        }
+    }
 #endif
 }
 // the last stage when it has fewer than 16 k: through registers, zeros past kend
 template <bool KC>
-__device__ __forceinline__ void dma_stage_tail(const char *base, const uint32_t (&off)[4],
-                                               const int (&dk)[4], int64_t ldx, double *L, int wave,
-                                               int lane, int k0, int kend) {
-    const char *b = base + 8 * (KC ? (int64_t)k0 : ldx * k0);
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-        const double *p = reinterpret_cast<const double *>(b + off[c]);
-        const bool ok0 = k0 + dk[c] < kend, ok1 = KC ? k0 + dk[c] + 1 < kend : ok0;
-        d2_t v;
-        v.x = ok0 ? p[0] : 0.0;
-        v.y = ok1 ? p[1] : 0.0;
-        *reinterpret_cast<d2_t *>(L + dma_block<KC>(wave, c) + 2 * lane) = v;
+__device__ __forceinline__ void dma_stage_tail(const double *__restrict__ X, int64_t ldx, int r0,
+                                               int rows, double *L, int tid, int k0, int kend) {
+#pragma unroll 1
+    for (int u = 0; u < 8; ++u) {
+        const int e = tid + 256 * u;
+        const int row = KC ? e >> 4 : e & 127, kk = KC ? e & 15 : e >> 7;
+        const int64_t r = min(r0 + row, rows - 1);
+        const double v = k0 + kk < kend ? X[KC ? k0 + kk + ldx * r : r + ldx * (k0 + kk)] : 0.0;
+        L[KC ? row * GKB + 2 * ((kk >> 1) ^ ((row >> 1) & 7)) + (kk & 1) : kk * DMA_KPR + row] = v;
     }
 }
 
-template <bool TA, bool TB>
+template <bool TA, bool TB, int V>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_gemm_f64(const GemmArgs g) {
-    __shared__ __attribute__((aligned(16))) double sA[2][GT * KP];
-    __shared__ __attribute__((aligned(16))) double sB[2][GT * KP];
+    constexpr bool KCA = TA, KCB = !TB;   // operand contiguous in k
+    __shared__ __attribute__((aligned(16))) double sA[2][KCA ? GT * GKB : GKB * DMA_KPR];
+    __shared__ __attribute__((aligned(16))) double sB[2][KCB ? GT * GKB : GKB * DMA_KPR];
     const int item1 = (int)(blockIdx.x / (unsigned)g.ntiles);
     const int t = (int)(blockIdx.x - (unsigned)item1 * (unsigned)g.ntiles);
     const int item2 = (int)blockIdx.y;
@@ -230,176 +245,96 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
         for (int j = 0; j < 4; ++j) acc[i][j] = (d4_t){0.0, 0.0, 0.0, 0.0};
 
-    // pair q = tid + 256 i (i < 4) of a 128 x 16 panel: (row, k pair kp).
-    // Rows-contiguous operands: row q % 128 (fixed per thread), kp q / 128 =
-    // kp0 + 2 i; k-contiguous: row q / 8 = row0 + 32 i, kp q % 8 (fixed).  So
-    // per operand one base offset and one stride per i.
-    const int arow0 = TA ? (tid >> 3) : (tid & 127), akp0 = TA ? (tid & 7) : (tid >> 7);
-    const int brow0 = TB ? (tid & 127) : (tid >> 3), bkp0 = TB ? (tid >> 7) : (tid & 7);
-    const int64_t astep = TA ? 1 : lda, bstep = TB ? ldb : 1;   // per unit of k
-    const double *__restrict__ pa0 = A + (TA ? (int64_t)(2 * akp0) + lda * (m0 + arow0)
-                                             : (int64_t)(m0 + arow0) + lda * (2 * akp0));
-    const double *__restrict__ pb0 = B + (TB ? (int64_t)(n0 + brow0) + ldb * (2 * bkp0)
-                                             : (int64_t)(2 * bkp0) + ldb * (n0 + brow0));
-    const int64_t ai_step = TA ? 32 * lda : 4 * lda;   // per i
-    const int64_t bi_step = TB ? 4 * ldb : 32 * ldb;
-    const int as_lds = arow0 * KP + 2 * akp0, bs_lds = brow0 * KP + 2 * bkp0;
-    const int ai_lds = TA ? 32 * KP : 4, bi_lds = TB ? 4 : 32 * KP;
-
-    d2_t ra[4], rb[4];
-    auto gload = [&](int k0) {
-        const double *pa = pa0 + astep * k0, *pb = pb0 + bstep * k0;
+    if (kbeg < kend) {
+        const int rl = lane & 15, g4 = lane >> 4;
+        const DmaSrc<KCA, V> oa = dma_offsets<KCA, V>(lda, m0, m, wave, lane);
+        const DmaSrc<KCB, V> ob = dma_offsets<KCB, V>(ldb, n0, n, wave, lane);
+        const char *ba = dma_base<KCA>(A, lda, m0), *bb = dma_base<KCB>(B, ldb, n0);
+        auto stage = [&](int buf, int k0) {
+            dma_stage<KCA, V>(ba, oa, lda, sA[buf], wave, k0);
+            dma_stage<KCB, V>(bb, ob, ldb, sB[buf], wave, k0);
+        };
+        auto stage_tail = [&](int buf, int k0) {
+            dma_stage_tail<KCA>(A, lda, m0, m, sA[buf], tid, k0, kend);
+            dma_stage_tail<KCB>(B, ldb, n0, n, sB[buf], tid, k0, kend);
+        };
+        // one half of a stage: two k per lane
+        auto frags = [&](d2_t (&a)[4], d2_t (&b)[4], int buf, int hh) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const bool aok = m0 + arow0 + (TA ? 32 * i : 0) < m;
-            const int ka = k0 + 2 * akp0 + (TA ? 0 : 4 * i);
-            ra[i].x = (aok && ka < kend) ? pa[i * ai_step] : 0.0;
-            ra[i].y = (aok && ka + 1 < kend) ? pa[i * ai_step + astep] : 0.0;
-            const bool bok = n0 + brow0 + (TB ? 0 : 32 * i) < n;
-            const int kb = k0 + 2 * bkp0 + (TB ? 4 * i : 0);
-            rb[i].x = (bok && kb < kend) ? pb[i * bi_step] : 0.0;
-            rb[i].y = (bok && kb + 1 < kend) ? pb[i * bi_step + bstep] : 0.0;
-        }
-    };
-    auto lstore = [&](int buf) {
+            for (int i = 0; i < 4; ++i)
+                a[i] = dma_frag<KCA>(sA[buf], 64 * wm + 16 * i + rl, g4, hh);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            *reinterpret_cast<d2_t *>(&sA[buf][as_lds + i * ai_lds]) = ra[i];
-            *reinterpret_cast<d2_t *>(&sB[buf][bs_lds + i * bi_lds]) = rb[i];
-        }
-    };
-
-    if (g.dma) {
-        if (kbeg < kend) {
-            const int rl = lane & 15, g4 = lane >> 4;
-            constexpr bool KCA = TA, KCB = !TB;   // operand contiguous in k
-            uint32_t oa[4], ob[4];
-            int ka[4], kb[4];
-            dma_offsets<KCA>(lda, m0, m, wave, lane, oa, ka);
-            dma_offsets<KCB>(ldb, n0, n, wave, lane, ob, kb);
-            const char *ba = dma_base<KCA>(A, lda, m0), *bb = dma_base<KCB>(B, ldb, n0);
-            auto stage = [&](int buf, int k0) {
-                dma_stage<KCA>(ba, oa, lda, sA[buf], wave, k0);
-                dma_stage<KCB>(bb, ob, ldb, sB[buf], wave, k0);
-            };
-            auto stage_tail = [&](int buf, int k0) {
-                dma_stage_tail<KCA>(ba, oa, ka, lda, sA[buf], wave, lane, k0, kend);
-                dma_stage_tail<KCB>(bb, ob, kb, ldb, sB[buf], wave, lane, k0, kend);
-            };
-            // one half of a stage: two k per lane
-            auto frags = [&](d2_t (&a)[4], d2_t (&b)[4], int buf, int hh) {
+            for (int j = 0; j < 4; ++j)
+                b[j] = dma_frag<KCB>(sB[buf], 64 * wn + 16 * j + rl, g4, hh);
+        };
+        auto mma = [&](const d2_t (&a)[4], const d2_t (&b)[4]) {
+#pragma unroll
+            for (int st = 0; st < 2; ++st)
 #pragma unroll
                 for (int i = 0; i < 4; ++i)
-                    a[i] = dma_frag<KCA>(sA[buf], 64 * wm + 16 * i + rl, g4, hh);
 #pragma unroll
-                for (int j = 0; j < 4; ++j)
-                    b[j] = dma_frag<KCB>(sB[buf], 64 * wn + 16 * j + rl, g4, hh);
-            };
-            auto mma = [&](const d2_t (&a)[4], const d2_t (&b)[4]) {
-#pragma unroll
-                for (int st = 0; st < 2; ++st)
-#pragma unroll
-                    for (int i = 0; i < 4; ++i)
-#pragma unroll
-                        for (int j = 0; j < 4; ++j)
-                            acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(b[j][st], a[i][st],
-                                                                             acc[i][j], 0, 0, 0);
-            };
-            d2_t a0[4], b0[4], a1[4], b1[4];
-            // The fragments of either half of a stage are read while the other half
-            // is multiplied, one LDS read after each of the first MFMAs and then one
-            // load of the coming stage after each of the next.  The barrier stands
-            // between the halves: by then the next stage has landed and every wave
-            // has read the current one, whose buffer takes the loads of the stage
-            // after the next.  Bound by MFMA issue: TN 8192 x 8192 x 2048 73.0
-            // TFLOP/s, 4096^3 66.7, 3072^2 x 4096 (whose last 64 of 576 tiles run one
-            // per CU) 52 (68.5, 64.0 and 38-46 with all reads, then all loads, ahead
-            // of the stage's MFMAs).
-            const int nfull = (kend - kbeg) / GKB, ns = (kend - kbeg + GKB - 1) / GKB;
-            auto put = [&](int buf, int q) {
-                if (q < nfull)
-                    stage(buf, kbeg + GKB * q);
-                else if (q < ns)
-                    stage_tail(buf, kbeg + GKB * q);
-            };
-            put(0, 0);
-            __syncthreads();
-            put(1, 1);
-            frags(a0, b0, 0, 0);
-            int buf = 0, q = 0;
-            for (; q + 2 < nfull; ++q, buf ^= 1) {
-                frags(a1, b1, buf, 1);
-                mma(a0, b0);
-#pragma unroll
-                for (int u = 0; u < 8; ++u) {
-                    __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);     // MFMA
-                    __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);   // LDS read
-                }
-                __builtin_amdgcn_sched_group_barrier(0x8, 24, 0);
-                __builtin_amdgcn_sched_barrier(0);
-                __syncthreads();
-                frags(a0, b0, buf ^ 1, 0);
-                stage(buf, kbeg + GKB * (q + 2));
-                mma(a1, b1);
-#pragma unroll
-                for (int u = 0; u < 8; ++u) {
-                    __builtin_amdgcn_sched_group_barrier(0x8, 1, 1);
-                    __builtin_amdgcn_sched_group_barrier(0x100, 1, 1);
-                }
-#pragma unroll
-                for (int u = 0; u < 8; ++u) {
-                    __builtin_amdgcn_sched_group_barrier(0x8, 1, 1);
-                    __builtin_amdgcn_sched_group_barrier(0x20, 1, 1);   // global -> LDS
-                }
-                __builtin_amdgcn_sched_group_barrier(0x8, 16, 1);
-                __builtin_amdgcn_sched_barrier(0);
-            }
-            for (; q < ns; ++q, buf ^= 1) {
-                frags(a1, b1, buf, 1);
-                mma(a0, b0);
-                if (q + 1 < ns) {
-                    __syncthreads();
-                    put(buf, q + 2);
-                    frags(a0, b0, buf ^ 1, 0);
-                }
-                mma(a1, b1);
-            }
-        }
-    } else if (kbeg < kend) {
-        const int kq = 4 * (lane >> 4), rl = lane & 15;
-        gload(kbeg);
-        lstore(0);
+                    for (int j = 0; j < 4; ++j)
+                        acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(b[j][st], a[i][st],
+                                                                         acc[i][j], 0, 0, 0);
+        };
+        d2_t a0[4], b0[4], a1[4], b1[4];
+        // The fragments of either half of a stage are read while the other half
+        // is multiplied, one LDS read after each of the first MFMAs and then one
+        // load of the coming stage after each of the next.  The barrier stands
+        // between the halves: by then the next stage has landed and every wave
+        // has read the current one, whose buffer takes the loads of the stage
+        // after the next.  Bound by MFMA issue: TN 8192 x 8192 x 2048 73.0
+        // TFLOP/s, 4096^3 66.7, 3072^2 x 4096 (whose last 64 of 576 tiles run one
+        // per CU) 52 (68.5, 64.0 and 38-46 with all reads, then all loads, ahead
+        // of the stage's MFMAs).
+        const int nfull = g.far ? 0 : (kend - kbeg) / GKB, ns = (kend - kbeg + GKB - 1) / GKB;
+        auto put = [&](int buf, int q) {
+            if (q < nfull)
+                stage(buf, kbeg + GKB * q);
+            else if (q < ns)
+                stage_tail(buf, kbeg + GKB * q);
+        };
+        put(0, 0);
         __syncthreads();
-        if (kbeg + GKB < kend) gload(kbeg + GKB);
-        int buf = 0;
-        for (int k0 = kbeg; k0 < kend; k0 += GKB, buf ^= 1) {
-            // the stage in two halves of two k each; the next stage goes to the
-            // other buffer between them (that buffer was last read before the
-            // previous barrier), so its LDS stores overlap the second half's MFMAs
+        put(1, 1);
+        frags(a0, b0, 0, 0);
+        int buf = 0, q = 0;
+        for (; q + 2 < nfull; ++q, buf ^= 1) {
+            frags(a1, b1, buf, 1);
+            mma(a0, b0);
 #pragma unroll
-            for (int hh = 0; hh < 2; ++hh) {
-                d2_t a[4], b[4];
-#pragma unroll
-                for (int i = 0; i < 4; ++i)
-                    a[i] = *reinterpret_cast<const d2_t *>(
-                        &sA[buf][(64 * wm + 16 * i + rl) * KP + kq + 2 * hh]);
-#pragma unroll
-                for (int j = 0; j < 4; ++j)
-                    b[j] = *reinterpret_cast<const d2_t *>(
-                        &sB[buf][(64 * wn + 16 * j + rl) * KP + kq + 2 * hh]);
-                // C^T block = op(B)^T op(A)^T: rows of C along the lanes
-#pragma unroll
-                for (int st = 0; st < 2; ++st)
-#pragma unroll
-                    for (int i = 0; i < 4; ++i)
-#pragma unroll
-                        for (int j = 0; j < 4; ++j)
-                            acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(b[j][st], a[i][st],
-                                                                             acc[i][j], 0, 0, 0);
-                if (hh == 0 && k0 + GKB < kend) lstore(buf ^ 1);
+            for (int u = 0; u < 8; ++u) {
+                __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);     // MFMA
+                __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);   // LDS read
             }
+            __builtin_amdgcn_sched_group_barrier(0x8, 24, 0);
+            __builtin_amdgcn_sched_barrier(0);
             __syncthreads();
-            if (k0 + 2 * GKB < kend) gload(k0 + 2 * GKB);
+            frags(a0, b0, buf ^ 1, 0);
+            stage(buf, kbeg + GKB * (q + 2));
+            mma(a1, b1);
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+                __builtin_amdgcn_sched_group_barrier(0x8, 1, 1);
+                __builtin_amdgcn_sched_group_barrier(0x100, 1, 1);
+            }
+#pragma unroll
+            for (int u = 0; u < (V == 16 ? 8 : 16); ++u) {
+                __builtin_amdgcn_sched_group_barrier(0x8, 1, 1);
+                __builtin_amdgcn_sched_group_barrier(0x20, V == 16 ? 1 : 2, 1);   // global -> LDS
+            }
+            __builtin_amdgcn_sched_group_barrier(0x8, V == 16 ? 16 : 8, 1);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        for (; q < ns; ++q, buf ^= 1) {
+            frags(a1, b1, buf, 1);
+            mma(a0, b0);
+            if (q + 1 < ns) {
+                __syncthreads();
+                put(buf, q + 2);
+                frags(a0, b0, buf ^ 1, 0);
+            }
+            mma(a1, b1);
         }
     }
 
@@ -499,15 +434,16 @@ int launch_gemm_f64_batched(brpa_ctx *ctx, bool ta, bool tb, int64_t m, int64_t 
     g.scs1 = scs1;
     g.scs2 = scs2;
     g.P = nullptr;
-    // direct-to-LDS stages: 16-byte aligned sources (even leading dimensions and
-    // strides, aligned bases); a rows-contiguous operand also needs an even row
-    // count, so that its last row pair lies inside the matrix
-    g.dma = (lda % 2 == 0 && ldb % 2 == 0 && sA1 % 2 == 0 && sA2 % 2 == 0 && sB1 % 2 == 0 &&
-             sB2 % 2 == 0 && lda < (1 << 21) && ldb < (1 << 21) && (reinterpret_cast<uintptr_t>(A) & 15) == 0 &&
-             (reinterpret_cast<uintptr_t>(B) & 15) == 0 && (ta || m % 2 == 0) &&
-             (!tb || n % 2 == 0))
-                ? 1
-                : 0;
+    // 16 bytes per lane: aligned sources (even leading dimensions and strides, aligned
+    // bases) and 32-bit offsets within a tile; a rows-contiguous operand also needs
+    // an even row count, so that its last row pair lies inside the matrix.  Measured
+    // at 4097^3 with 4 bytes per lane: NN, NT, TT 51 TFLOP/s, TN 44 (through registers:
+    // 45 for all four)
+    g.far = lda >= (1 << 21) || ldb >= (1 << 21);
+    const bool wide = lda % 2 == 0 && ldb % 2 == 0 && sA1 % 2 == 0 && sA2 % 2 == 0 &&
+                      sB1 % 2 == 0 && sB2 % 2 == 0 && (reinterpret_cast<uintptr_t>(A) & 15) == 0 &&
+                      (reinterpret_cast<uintptr_t>(B) & 15) == 0 && (ta || m % 2 == 0) &&
+                      (!tb || n % 2 == 0);
     // split k when the last wave of tiles would leave much of the chip idle:
     // the split count s (<= 8, chunks of >= 256 k) minimises the modelled time
     // 1/eff(s) + (reduction traffic), eff(s) = tiles s / (slots ceil(tiles s /
@@ -549,14 +485,15 @@ int launch_gemm_f64_batched(brpa_ctx *ctx, bool ta, bool tb, int64_t m, int64_t 
     const dim3 grid((unsigned)(ntiles * nb1), (unsigned)nb2, (unsigned)g.nsplit), block(256);
     size_t slot = 0;
     BRPA_TRY(kstat_begin(ctx, &slot));
+    auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, block, 0, ctx->stream, g); };
     if (!ta && !tb)
-        hipLaunchKernelGGL((k_gemm_f64<false, false>), grid, block, 0, ctx->stream, g);
+        wide ? launch(k_gemm_f64<false, false, 16>) : launch(k_gemm_f64<false, false, 4>);
     else if (!ta && tb)
-        hipLaunchKernelGGL((k_gemm_f64<false, true>), grid, block, 0, ctx->stream, g);
+        wide ? launch(k_gemm_f64<false, true, 16>) : launch(k_gemm_f64<false, true, 4>);
     else if (ta && !tb)
-        hipLaunchKernelGGL((k_gemm_f64<true, false>), grid, block, 0, ctx->stream, g);
+        wide ? launch(k_gemm_f64<true, false, 16>) : launch(k_gemm_f64<true, false, 4>);
     else
-        hipLaunchKernelGGL((k_gemm_f64<true, true>), grid, block, 0, ctx->stream, g);
+        wide ? launch(k_gemm_f64<true, true, 16>) : launch(k_gemm_f64<true, true, 4>);
     LAUNCH_CHECK(ctx);
     if (g.nsplit > 1) {
         hipLaunchKernelGGL(k_gemm_reduce, dim3((unsigned)((m * n + 255) / 256)), dim3(256), 0,

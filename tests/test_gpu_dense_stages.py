@@ -39,3 +39,40 @@ def test_triangular_inverse(ctx, n):
     W = torch.empty((n, n), dtype=torch.float64, device="cuda").T
     ctx.dtrtri(Ud, W)
     assert np.array_equal(W.cpu().numpy() @ U, np.eye(n))
+
+
+@pytest.mark.parametrize("m,n,k", [(1, 1, 1), (127, 129, 31), (128, 128, 33), (129, 255, 48),
+                                   (257, 131, 79), (3, 260, 64)])
+@pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
+@pytest.mark.parametrize("off", [0, 1])
+def test_odd_leading_dimensions(ctx, m, n, k, ta, tb, off):
+    """Odd leading dimensions and operands that are only 8-byte aligned (4 bytes per
+    lane), rows and columns around the 128-row tiles."""
+    rng = np.random.default_rng(m + k)
+    A = rng.integers(-8, 9, (m, k)).astype(np.float64)
+    B = rng.integers(-8, 9, (k, n)).astype(np.float64)
+
+    def dev(x):
+        ld = x.shape[0] + 1 - x.shape[0] % 2 + 2 * off
+        buf = torch.full((x.shape[1] * ld + off,), np.nan, dtype=torch.float64, device="cuda")
+        v = buf[off:].view(x.shape[1], ld)
+        v[:, :x.shape[0]] = torch.from_numpy(np.ascontiguousarray(x.T)).cuda()
+        return v.T[:x.shape[0], :]
+
+    C = torch.full((n, m), np.nan, dtype=torch.float64, device="cuda").T
+    ctx.dgemm(dev(A.T if ta else A), dev(B.T if tb else B), C, transa=ta, transb=tb)
+    assert np.array_equal(C.cpu().numpy(), A @ B)
+
+
+def test_far_leading_dimension(ctx):
+    """A leading dimension beyond the 32-bit offsets of a tile (2^21 and more)."""
+    k, ld = 40, (1 << 21) + 1
+    rng = np.random.default_rng(0)
+    A = rng.integers(-8, 9, (k, 5)).astype(np.float64)
+    B = rng.integers(-8, 9, (k, 3)).astype(np.float64)
+    buf = torch.zeros((5, ld), dtype=torch.float64, device="cuda")
+    buf[:, :k] = torch.from_numpy(np.ascontiguousarray(A.T)).cuda()
+    Bd = torch.from_numpy(np.ascontiguousarray(B.T)).cuda().T
+    C = torch.full((3, 5), np.nan, dtype=torch.float64, device="cuda").T
+    ctx.dgemm(buf.T[:k, :], Bd, C, transa=True)
+    assert np.array_equal(C.cpu().numpy(), A.T @ B)
