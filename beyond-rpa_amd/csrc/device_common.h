@@ -61,14 +61,3 @@ __device__ __forceinline__ dd_t dd_add(dd_t a, dd_t b) {
     dd_t s = dd_add(a, b.hi);
     return dd_add(s, b.lo);
 }
-
-// XCD-aware block order.  Work-group ids are handed to the 8 XCDs round-robin
-// (id % 8), and each XCD has its own L2.  This bijection on [0, nblocks) gives
-// XCD x a contiguous range of logical work items, so tiles that share panels
-// (neighbouring items of one matrix) run on the same XCD and hit its L2.
-__device__ __forceinline__ int64_t xcd_remap(int64_t b, int64_t nblocks) {
-    constexpr int64_t NX = 8;
-    const int64_t q = nblocks / NX, rem = nblocks % NX;
-    const int64_t x = b % NX, r = b / NX;
-    return x * q + (x < rem ? x : rem) + r;
-}

@@ -140,10 +140,10 @@ int run_chunk(brpa_ctx *ctx, int precision, const std::vector<HostFrag> &fr, dou
         nsteps_max = std::max<int>(nsteps_max, (int)cdiv(fr[f].naux, CHOL_NB));
 
     // split-int8 product variant of every fragment (autotuner choice per size bucket)
-    std::vector<int> var(nfrag, I8V_T128);
+    std::vector<int> var(nfrag);
     for (int f = 0; f < nfrag; ++f) {
         const int c = ctx->i8_choice[tune_bucket(fr[f].naux)];
-        var[f] = ctx->tune_force >= 0 ? ctx->tune_force : (c >= 0 ? c : I8V_T128);
+        var[f] = ctx->tune_force >= 0 ? ctx->tune_force : (c >= 0 ? c : I8V_T128_XCD);
     }
     int64_t syrk_n[2] = {0, 0};
     for (int f = 0; f < nfrag; ++f)
@@ -496,7 +496,7 @@ int brpa_autotune(brpa_ctx *ctx, int precision, int64_t nfrag, const brpa_frag_t
         if (bucket[b].empty()) continue;
         std::vector<double> e(bucket[b].size()), e0;
         double best = 0.0;
-        int best_v = I8V_T128;
+        int best_v = I8V_T128_XCD;
         for (int v = 0; v < I8V_COUNT && rc == BRPA_OK; ++v) {
             ctx->tune_force = v;
             // the first run allocates and warms up; the second is timed

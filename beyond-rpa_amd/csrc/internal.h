@@ -191,7 +191,7 @@ struct FragDev {
     int Kpad, nblk;
     // split-int8 slices (only when precision == BRPA_SPLIT_I8)
     const double *sdtab;     // F x K, sqrt(c_w(k))
-    int8_t *sl8;             // F x NSLICE x N x Kpad8, per column P the Kpad8 rows contiguous
+    int8_t *sl8;             // F x NSLICE x Kpad8/64 x N x 64, per column P 64 rows contiguous
     double *scale8;          // F x N, column scale max_k |X_w[k][P]| / 127
     int Kpad8;
     // 1: the Cholesky also writes each factored 64x64 diagonal block back into
@@ -241,8 +241,8 @@ int launch_colscale_i8(brpa_ctx *, const FragDev *, const int64_t *pre, int nfra
                        const int64_t *pre_fin, int64_t total_fin);
 int launch_split_i8(brpa_ctx *, const FragDev *, const int64_t *pre, int nfrag, int64_t total);
 // split-int8 product kernel variants (chosen per fragment-size bucket by the
-// autotuner): 128x128 tiles in launch order, the same with one contiguous tile
-// range per XCD, 64x64 tiles
+// autotuner): 128x128 tiles in launch order, the same with chunks of 32 neighbouring
+// tiles per XCD (the default), 64x64 tiles
 enum { I8V_T128 = 0, I8V_T128_XCD = 1, I8V_T64 = 2, I8V_COUNT = 3 };
 int syrk_i8_tile(int variant);
 int launch_syrk_i8(brpa_ctx *, const FragDev *, const int64_t *pre, int nfrag, int64_t total,

@@ -18,7 +18,8 @@
 //
 //   k_colscale_i8  s_w[P] and the exact diagonal, one pass over R for all w
 //   k_split_i8     int8 slices of X_w, one read of R for all w
-//   k_syrk_i8      128x128 output tiles, 8 waves of 64x32, int8 MFMA
+//   k_syrk_i8_128  128x128 output tiles, 8 waves of 64x32, int8 MFMA
+//   k_syrk_i8_64   64x64 output tiles, 2 waves
 #include "device_common.h"
 #include "internal.h"
 
@@ -48,6 +49,7 @@ typedef int v4i_t __attribute__((ext_vector_type(4)));
 // work-group per 64 columns over all of K kept 29 of 256 CUs busy there (4809 us).
 // Over 32 fragments of the batch shapes: 1361 us, before 3359.
 constexpr int CS_WG = 16;       // frequencies per group of the split pass
+constexpr int KS8 = 64;         // k-values (bytes) per stage and slice of the product
 constexpr int CSF = 8;          // frequencies per register group of the column pass
 constexpr int CSR = 8;          // rows per step of a wave
 typedef __attribute__((address_space(4))) const double cdbl_t;
@@ -239,7 +241,8 @@ __global__ __launch_bounds__(256) void k_split_i8(const FragDev *__restrict__ fr
             }
 #pragma unroll
             for (int s = 0; s < NSLICE; ++s) {
-                int8_t *dst = F.sl8 + (((int64_t)w * NSLICE + s) * N + P) * Kp + k0 + r0;
+                int8_t *dst = F.sl8 + ((int64_t)w * NSLICE + s) * N * Kp +
+                              ((int64_t)((k0 + r0) / KS8) * N + P) * KS8 + r0 % KS8;
                 uint4 *d4 = reinterpret_cast<uint4 *>(dst);
                 d4[0] = make_uint4(pk[s][0], pk[s][1], pk[s][2], pk[s][3]);
                 d4[1] = make_uint4(pk[s][4], pk[s][5], pk[s][6], pk[s][7]);
@@ -261,6 +264,11 @@ int launch_split_i8(brpa_ctx *ctx, const FragDev *fr, const int64_t *pre, int nf
 // Product.  One TxT output tile pair (p-tile >= q-tile) of one frequency per
 // work-group; work-groups per fragment: F * npairs(ceil(N/T)).  The waves
 // own 64x32 sub-tiles: T = 128 -> 8 waves (2 x 4), T = 64 -> 2 waves (1 x 2).
+// Only the lower triangle of Pi is written (the Cholesky reads no other).
+//
+// The slices lie in memory as [w][slice][k / 64][column][64], so that the 16 columns
+// of a wave load are one contiguous KB (with the whole K of a column contiguous they
+// were 16 half cache lines: 6-9 % slower).
 //
 // v_mfma_i32_16x16x64_i8 lane layout (lane l, 16 bytes per operand):
 //   A[m = l%16][k = 16*(l/16) .. +15], B[k = 16*(l/16) .. +15][n = l%16],
@@ -273,7 +281,6 @@ int launch_split_i8(brpa_ctx *ctx, const FragDev *fr, const int64_t *pre, int nf
 // lane l lands in column l/4, slot l%4, and fetches k-piece
 // (l%4) ^ ((l/16)%4) of that column, so that the MFMA operand reads (16
 // columns at one k-piece per 16 lanes) hit 16 distinct 4-bank groups.
-constexpr int KS8 = 64;   // k-values (bytes) per stage and slice
 
 typedef __attribute__((address_space(3))) void lds_void_t;
 
@@ -281,9 +288,9 @@ __device__ __forceinline__ int swz8(int col_local, int piece) {
     return piece ^ ((col_local >> 2) & 3);
 }
 
-template <int T>
-__global__ __launch_bounds__((T / 64) * (T / 32) * 64) void k_syrk_i8(
-    const FragDev *__restrict__ fr, const int64_t *__restrict__ pre, int nfrag, int xcd) {
+__global__ __launch_bounds__(128) void k_syrk_i8_64(
+    const FragDev *__restrict__ fr, const int64_t *__restrict__ pre, int nfrag) {
+    constexpr int T = 64;
     constexpr int WJN = T / 32;                 // waves along columns
     constexpr int NW = (T / 64) * WJN;          // waves
     constexpr int GPS = T / 16;                 // 16-column groups per side and slice
@@ -292,8 +299,7 @@ __global__ __launch_bounds__((T / 64) * (T / 32) * 64) void k_syrk_i8(
     // [buffer][side][slice][column][slot] of 16-byte pieces
     __shared__ __attribute__((aligned(16))) uint4 sbuf[2][2][NSLICE][T][4];
     __shared__ int64_t s_pre[FIND_LDS_MAX + 1];
-    // xcd = 1: one contiguous range of tiles per XCD (see xcd_remap)
-    const int64_t b = xcd ? xcd_remap(blockIdx.x, gridDim.x) : (int64_t)blockIdx.x;
+    const int64_t b = blockIdx.x;
     const int f = find_frag_lds(pre, nfrag, b, s_pre);
     const FragDev &F = fr[f];
     const int N = F.N;
@@ -328,14 +334,14 @@ __global__ __launch_bounds__((T / 64) * (T / 32) * 64) void k_syrk_i8(
         const int side = id / LPS, sl = (id % LPS) / GPS, g = id % GPS;
         int P = (side ? q0 : p0) + 16 * g + lcol;
         P = P < N ? P : N - 1;
-        goff[t] = ((int64_t)sl * N + P) * Kp + 16 * lpiece;
+        goff[t] = (int64_t)sl * N * Kp + (int64_t)P * KS8 + 16 * lpiece;
     }
     auto issue = [&](int buf, int k0) {
 #pragma unroll
         for (int t = 0; t < LPW; ++t) {
             const int id = LPW * wave + t;
             const int side = id / LPS, sl = (id % LPS) / GPS, g = id % GPS;
-            __builtin_amdgcn_global_load_lds((const void *)(slw + goff[t] + k0),
+            __builtin_amdgcn_global_load_lds((const void *)(slw + goff[t] + (int64_t)k0 * N),
                                              (lds_void_t *)&sbuf[buf][side][sl][16 * g][0], 16, 0, 0);
         }
     };
@@ -403,7 +409,6 @@ __global__ __launch_bounds__((T / 64) * (T / 32) * 64) void k_syrk_i8(
 
     const double *scw = F.scale8 + (int64_t)w * N;
     double *C = F.Pi + (int64_t)w * N * N;
-    const bool diag = (tp == tq);
     const double c1 = 1.0 / 128.0, c2 = c1 * c1, c3 = c2 * c1;
 #pragma unroll
     for (int i = 0; i < 4; ++i)
@@ -414,15 +419,197 @@ __global__ __launch_bounds__((T / 64) * (T / 32) * 64) void k_syrk_i8(
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const int p = p0 + 64 * wi + 16 * i + 4 * (lane >> 4) + r;
-                if (p < N && q < N) {
+                if (p < N && q <= p) {
                     const double v = (double)L0[i][j][r] + c1 * (double)L1[i][j][r] +
                                      c2 * (double)L2[i][j][r] + c3 * (double)L3[i][j][r];
-                    const double out = v * (scw[p] * sq);
-                    C[(int64_t)p * N + q] = out;
-                    if (!diag) C[(int64_t)q * N + p] = out;
+                    C[(int64_t)p * N + q] = v * (scw[p] * sq);
                 }
             }
         }
+}
+
+// The 128x128 form: eight waves of 64x32, two stages of 64 k in LDS (one work-group
+// per CU, two waves per SIMD).  Of a stage's 80 MFMAs per wave, the 32 of slice 0 of
+// the p side run first, while the wave reads the other three p slices; the
+// barrier follows, since the stage's buffer has then been read by every wave, and the
+// loads of the stage after the next go into it.  The other 48 MFMAs cover those loads
+// and the reads of the next stage's first operands.  A wave above the diagonal of a
+// diagonal tile only stages.
+//
+// xcd: chunks of 32 consecutive tiles (which share panels) go to one XCD at a time,
+// so that its CUs find each other's panels in their L2, and the XCDs stay balanced
+// over fragments of different K (one contiguous range of the grid per XCD did not: 1.4
+// times slower on the batch).
+//
+// Bound by the int8 matrix rate and the LDS reads (24 KB per wave and stage).  Measured
+// at K = 10800, N = 1800, 24 frequencies: 4.19 ms with xcd, 4.43 without (200 and 190
+// TFLOP/s FP64-equivalent; 5.97 with one LDS read or wait ahead of each group of
+// MFMAs); 32 fragments of the batch shapes: 16.7 and 17.5 ms (23.8).
+constexpr int XCD_CHUNK = 32;
+__device__ __forceinline__ int64_t xcd_chunks(int64_t b, int64_t nblocks) {
+    constexpr int64_t R = 8 * XCD_CHUNK;
+    if (b >= nblocks / R * R) return b;
+    const int64_t x = b % 8, r = b / 8;
+    return (r / XCD_CHUNK * 8 + x) * XCD_CHUNK + r % XCD_CHUNK;
+}
+
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_syrk_i8_128(
+    const FragDev *__restrict__ fr, const int64_t *__restrict__ pre, int nfrag, int xcd) {
+    constexpr int T = 128;
+    // [buffer][side][slice][column][slot] of 16-byte pieces
+    __shared__ __attribute__((aligned(16))) uint4 sbuf[2][2][NSLICE][T][4];
+    __shared__ int64_t s_pre[FIND_LDS_MAX + 1];
+    const int64_t b = xcd ? xcd_chunks(blockIdx.x, gridDim.x) : (int64_t)blockIdx.x;
+    const int f = find_frag_lds(pre, nfrag, b, s_pre);
+    const FragDev &F = fr[f];
+    const int N = F.N;
+    const int nt = (N + T - 1) / T;
+    const int npairs = nt * (nt + 1) / 2;
+    const int64_t lb = b - (nfrag <= FIND_LDS_MAX ? s_pre[f] : pre[f]);
+    const int w = __builtin_amdgcn_readfirstlane((int)(lb / npairs));
+    const int pair = (int)(lb - (int64_t)w * npairs);
+    int tp, tq;
+    tri_decode(pair, tp, tq);
+    const int p0 = __builtin_amdgcn_readfirstlane(tp * T), q0 = __builtin_amdgcn_readfirstlane(tq * T);
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int wi = wave >> 2, wj = wave & 3;   // 64x32 block of the tile
+    const int64_t Kp = F.Kpad8;
+    const int8_t *slw = F.sl8 + (int64_t)w * NSLICE * N * Kp;
+
+    // A wave loads one slice of one side: 8 groups of 16 columns (1 KB per load; lane
+    // l lands in column l/4, slot l%4).  Columns past N repeat column N - 1: they only
+    // feed outputs that are never written.
+    const int side = wave >> 2, slice = wave & 3;
+    const int lpiece = (lane & 3) ^ ((lane >> 4) & 3);
+    uint32_t goff[8];
+#pragma unroll
+    for (int g = 0; g < 8; ++g)
+        goff[g] = (uint32_t)min((side ? q0 : p0) + 16 * g + (lane >> 2), N - 1) * KS8 + 16u * lpiece;
+    const int8_t *base = slw + (int64_t)slice * N * Kp;
+    auto issue = [&](int buf, int st) {
+#if defined(__HIP_DEVICE_COMPILE__)
+        typedef __attribute__((address_space(1))) const char gchar_t;
+        gchar_t *src = (gchar_t *)(base + (int64_t)st * KS8 * N);
+#pragma unroll
+        for (int g = 0; g < 8; ++g)
+            __builtin_amdgcn_global_load_lds(
+                (const __attribute__((address_space(1))) void *)(src + goff[g]),
+                (lds_void_t *)&sbuf[buf][side][slice][16 * g][0], 16, 0, 0);
+#endif
+    };
+    const int nst = (int)(Kp / KS8);
+    issue(0, 0);
+    if (tp == tq && 32 * wj > 64 * wi + 63) {
+        __syncthreads();
+        if (nst > 1) issue(1, 1);
+        for (int st = 0; st < nst; ++st) {
+            __syncthreads();
+            issue(st & 1, min(st + 2, nst - 1));
+        }
+        __builtin_amdgcn_s_waitcnt(0);
+        return;
+    }
+    // slice s of the wave's 16-column groups of the p side (four) and the q side (two)
+    const int fo = (lane & 15) * 4 + swz8(lane & 15, lane >> 4);
+    auto fragp = [&](v4i_t (&v)[4], int buf, int s) {
+        const uint4 *L = &sbuf[buf][0][s][64 * wi][0];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = __builtin_bit_cast(v4i_t, L[64 * i + fo]);
+    };
+    auto fragq = [&](v4i_t (&v)[2], int buf, int s) {
+        const uint4 *L = &sbuf[buf][1][s][32 * wj][0];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) v[j] = __builtin_bit_cast(v4i_t, L[64 * j + fo]);
+    };
+    v4i_t L0[4][2], L1[4][2], L2[4][2], L3[4][2];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) L0[i][j] = L1[i][j] = L2[i][j] = L3[i][j] = (v4i_t){0, 0, 0, 0};
+    auto mma = [&](const v4i_t (&a)[4], const v4i_t (&b)[2], v4i_t (&c)[4][2]) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+                c[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[i], b[j], c[i][j], 0, 0, 0);
+    };
+    v4i_t a0[4], a1[4], a2[4], a3[4], b0[2], b1[2], b2[2], b3[2];
+    __syncthreads();
+    if (nst > 1) issue(1, 1);
+    fragp(a0, 0, 0);
+    fragq(b0, 0, 0);
+    fragq(b1, 0, 1);
+    fragq(b2, 0, 2);
+    fragq(b3, 0, 3);
+    // the last stages load and read stage nst - 1 again, unused
+    for (int st = 0; st < nst; ++st) {
+        const int buf = st & 1;
+        fragp(a1, buf, 1);
+        fragp(a2, buf, 2);
+        fragp(a3, buf, 3);
+        mma(a0, b3, L3);
+        mma(a0, b2, L2);
+        mma(a0, b1, L1);
+        mma(a0, b0, L0);
+#pragma unroll
+        for (int u = 0; u < 12; ++u) {
+            __builtin_amdgcn_sched_group_barrier(0x8, 2, 0);     // MFMA
+            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);   // LDS read
+        }
+        __builtin_amdgcn_sched_group_barrier(0x8, 8, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        __syncthreads();
+        issue(buf, min(st + 2, nst - 1));
+        mma(a1, b2, L3);
+        mma(a1, b1, L2);
+        mma(a1, b0, L1);
+        mma(a2, b1, L3);
+        mma(a2, b0, L2);
+        mma(a3, b0, L3);
+        fragq(b3, buf ^ 1, 3);
+        fragp(a0, buf ^ 1, 0);
+        fragq(b2, buf ^ 1, 2);
+        fragq(b1, buf ^ 1, 1);
+        fragq(b0, buf ^ 1, 0);
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            __builtin_amdgcn_sched_group_barrier(0x8, 2, 1);
+            __builtin_amdgcn_sched_group_barrier(0x20, 1, 1);    // global -> LDS
+        }
+#pragma unroll
+        for (int u = 0; u < 10; ++u) {
+            __builtin_amdgcn_sched_group_barrier(0x8, 3, 1);
+            __builtin_amdgcn_sched_group_barrier(0x100, 1, 1);
+        }
+        __builtin_amdgcn_sched_group_barrier(0x8, 2, 1);
+        __builtin_amdgcn_sched_group_barrier(0x100, 2, 1);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    __builtin_amdgcn_s_waitcnt(0);   // no load into LDS outlives the work-group
+
+    const double *scw = F.scale8 + (int64_t)w * N;
+    double *C = F.Pi + (int64_t)w * N * N;
+    const double c1 = 1.0 / 128.0, c2 = c1 * c1, c3 = c2 * c1;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        double sp[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            sp[r] = scw[min(p0 + 64 * wi + 16 * i + 4 * (lane >> 4) + r, N - 1)];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const int q = q0 + 32 * wj + 16 * j + (lane & 15);
+            const double sq = scw[min(q, N - 1)];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int p = p0 + 64 * wi + 16 * i + 4 * (lane >> 4) + r;
+                const double v = (double)L0[i][j][r] + c1 * (double)L1[i][j][r] +
+                                 c2 * (double)L2[i][j][r] + c3 * (double)L3[i][j][r];
+                if (p < N && q <= p) C[(int64_t)p * N + q] = v * (sp[r] * sq);
+            }
+        }
+    }
 }
 
 int syrk_i8_tile(int variant) { return variant == I8V_T64 ? 64 : 128; }
@@ -432,16 +619,16 @@ int launch_syrk_i8(brpa_ctx *ctx, const FragDev *fr, const int64_t *pre, int nfr
     if (total <= 0) return BRPA_OK;
     switch (variant) {
     case I8V_T128:
-        hipLaunchKernelGGL(k_syrk_i8<128>, dim3((unsigned)total), dim3(512), 0, ctx->stream, fr,
+        hipLaunchKernelGGL(k_syrk_i8_128, dim3((unsigned)total), dim3(512), 0, ctx->stream, fr,
                            pre, nfrag, 0);
         break;
     case I8V_T128_XCD:
-        hipLaunchKernelGGL(k_syrk_i8<128>, dim3((unsigned)total), dim3(512), 0, ctx->stream, fr,
+        hipLaunchKernelGGL(k_syrk_i8_128, dim3((unsigned)total), dim3(512), 0, ctx->stream, fr,
                            pre, nfrag, 1);
         break;
     case I8V_T64:
-        hipLaunchKernelGGL(k_syrk_i8<64>, dim3((unsigned)total), dim3(128), 0, ctx->stream, fr,
-                           pre, nfrag, 0);
+        hipLaunchKernelGGL(k_syrk_i8_64, dim3((unsigned)total), dim3(128), 0, ctx->stream, fr,
+                           pre, nfrag);
         break;
     default:
         return brpa_fail(ctx, BRPA_ERR_ARG, "unknown split-int8 kernel variant %d", variant);

@@ -277,8 +277,8 @@ int brpa_ecrpa_batch(brpa_ctx *ctx, int precision, int64_t nfrag, const brpa_fra
                      double *ecrpa);
 
 /* Autotuner (no counterpart in the reference).  Times every tile variant of the
- * split-int8 product kernel (128x128 tiles, the same with one contiguous tile
- * range per XCD, 64x64 tiles) on the given fragments, separately for three
+ * split-int8 product kernel (128x128 tiles, the same with chunks of neighbouring
+ * tiles per XCD, 64x64 tiles) on the given fragments, separately for three
  * NAux buckets (< 640, < 1280, >= 1280), and keeps the fastest per bucket in
  * the context for later calls.  Other precisions have one kernel shape (no-op).
  * Runs the pipeline twice per variant and bucket (warm-up + timed). */
