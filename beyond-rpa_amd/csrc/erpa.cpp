@@ -82,10 +82,9 @@ int host_copy(brpa_ctx *ctx, double *dst, const double *src, int64_t n) {
 struct Counts {
     int64_t dtab, syrk, setdiag, split, syrk16, colscale8, split8;
     int64_t syrk8[I8V_COUNT];   // split-int8 product work-groups, per kernel variant
-    std::vector<int64_t> pdiag, trsm, update;   // per Cholesky step
 };
 
-Counts counts_of(const HostFrag &f, int nsteps_max, int precision, int i8_variant, bool quad) {
+Counts counts_of(const HostFrag &f, int precision, int i8_variant, bool quad) {
     Counts c;
     const int64_t K = f.nocc * f.nvir, N = f.naux, F = f.nfreqs;
     c.dtab = cdiv(F * K, 256);
@@ -101,15 +100,6 @@ Counts counts_of(const HostFrag &f, int nsteps_max, int precision, int i8_varian
     for (int v = 0; v < I8V_COUNT; ++v) {
         const int64_t t = cdiv(N, syrk_i8_tile(v));
         c.syrk8[v] = (i8 && v == i8_variant) ? F * (t * (t + 1) / 2) : 0;
-    }
-    c.pdiag.assign(nsteps_max, 0);
-    c.trsm.assign(nsteps_max, 0);
-    c.update.assign(nsteps_max, 0);
-    for (int j = 0; j < nsteps_max; ++j) {
-        int64_t j0 = (int64_t)j * CHOL_NB;
-        if (N > j0) c.pdiag[j] = F;
-        if (N > j0 + CHOL_NB) c.trsm[j] = F * (cdiv(N - j0, CHOL_NB) - 1);
-        c.update[j] = F * chol_upd_items(N, j);
     }
     return c;
 }
@@ -151,12 +141,12 @@ int run_chunk(brpa_ctx *ctx, int precision, const std::vector<HostFrag> &fr, dou
     const bool quad = syrk_quad(ctx, syrk_n[0], syrk_n[1]);
     std::vector<Counts> cnt(nfrag);
     for (int f = 0; f < nfrag; ++f)
-        cnt[f] = counts_of(fr[f], nsteps_max, precision, var[f], quad);
+        cnt[f] = counts_of(fr[f], precision, var[f], quad);
 
     // prefix arrays: [dtab, syrk, setdiag, split, syrk16, colscale8, split8,
-    //                 syrk8 per variant, pdiag_0..S-1, trsm_0..S-1, update_0..S-1]
+    //                 syrk8 per variant, the Cholesky's lists per step]
     constexpr int NFIX = 7 + I8V_COUNT;
-    const int nstage = NFIX + 3 * nsteps_max;
+    const int nstage = NFIX + CHOL_NLISTS * nsteps_max;
     std::vector<int64_t> pre((size_t)nstage * (nfrag + 1), 0);
     auto P = [&](int s) { return pre.data() + (size_t)s * (nfrag + 1); };
     for (int f = 0; f < nfrag; ++f) {
@@ -164,11 +154,11 @@ int run_chunk(brpa_ctx *ctx, int precision, const std::vector<HostFrag> &fr, dou
         int64_t v[NFIX] = {c.dtab,     c.syrk,     c.setdiag,  c.split,   c.syrk16,
                            c.colscale8, c.split8,  c.syrk8[0], c.syrk8[1], c.syrk8[2]};
         for (int s = 0; s < NFIX; ++s) P(s)[f + 1] = P(s)[f] + v[s];
-        for (int j = 0; j < nsteps_max; ++j) {
-            P(NFIX + j)[f + 1] = P(NFIX + j)[f] + c.pdiag[j];
-            P(NFIX + nsteps_max + j)[f + 1] = P(NFIX + nsteps_max + j)[f] + c.trsm[j];
-            P(NFIX + 2 * nsteps_max + j)[f + 1] = P(NFIX + 2 * nsteps_max + j)[f] + c.update[j];
-        }
+        for (int l = 0; l < CHOL_NLISTS; ++l)
+            for (int j = 0; j < nsteps_max; ++j) {
+                int64_t *p = P(NFIX + l * nsteps_max + j);
+                p[f + 1] = p[f] + chol_items(l, fr[f].naux, fr[f].nfreqs, j);
+            }
     }
 
     // Inputs reach the device through one upload of a pinned staging region
@@ -309,13 +299,7 @@ int run_chunk(brpa_ctx *ctx, int precision, const std::vector<HostFrag> &fr, dou
         const int diag_mode =
             precision == BRPA_SPLIT_BF16 ? 1 : (precision == BRPA_SPLIT_I8 ? 2 : 0);
         BRPA_TRY(launch_set_diag(ctx, d_fr, DP(2), nfrag, TOT(2), diag_mode));
-        for (int j = 0; j < nsteps_max; ++j) {
-            BRPA_TRY(launch_potrf_diag(ctx, d_fr, DP(NFIX + j), nfrag, TOT(NFIX + j), j));
-            BRPA_TRY(launch_trsm(ctx, d_fr, DP(NFIX + nsteps_max + j), nfrag,
-                                 TOT(NFIX + nsteps_max + j), j));
-            BRPA_TRY(launch_chol_update(ctx, d_fr, DP(NFIX + 2 * nsteps_max + j), nfrag,
-                                        TOT(NFIX + 2 * nsteps_max + j), j));
-        }
+        BRPA_TRY(launch_cholesky(ctx, d_fr, nfrag, nsteps_max, DP(NFIX), P(NFIX)));
         BRPA_TRY(se(BRPA_STAGE_CHOL));
         BRPA_TRY(launch_energy(ctx, d_fr, nfrag));
         BRPA_HIP(ctx, hipMemcpyAsync(h_dn, d_dn, dn_bytes, hipMemcpyDeviceToHost, ctx->stream));
@@ -443,26 +427,23 @@ int run_ecrpa(brpa_ctx *ctx, int precision, const std::vector<HostFrag> &fr, dou
 
 }  // namespace
 
-int64_t chol_pre_len(int64_t N) { return 3 * cdiv(N, CHOL_NB) * 2; }
+// Prefix sums [0, count] of the Cholesky's lists and steps for one fragment of F matrices
+static void chol_prefix(int64_t *pre, int64_t N, int64_t F) {
+    const int64_t nsteps = cdiv(N, CHOL_NB);
+    for (int l = 0; l < CHOL_NLISTS; ++l)
+        for (int64_t j = 0; j < nsteps; ++j) {
+            pre[2 * (l * nsteps + j)] = 0;
+            pre[2 * (l * nsteps + j) + 1] = chol_items(l, N, F, j);
+        }
+}
+
+int64_t chol_pre_len(int64_t N) { return CHOL_NLISTS * cdiv(N, CHOL_NB) * 2; }
 
 int chol_single(brpa_ctx *ctx, const FragDev *d_fr, int64_t *d_pre, int64_t N, int64_t F) {
-    const int nsteps = (int)cdiv(N, CHOL_NB);
-    // prefix arrays [0, count] per launch: pdiag_0..S-1, trsm_0..S-1, update_0..S-1
-    std::vector<int64_t> pre((size_t)chol_pre_len(N), 0);
-    for (int j = 0; j < nsteps; ++j) {
-        const int64_t j0 = (int64_t)j * CHOL_NB;
-        pre[2 * j + 1] = (N > j0) ? F : 0;
-        pre[2 * (nsteps + j) + 1] = (N > j0 + CHOL_NB) ? F * (cdiv(N - j0, CHOL_NB) - 1) : 0;
-        pre[2 * (2 * nsteps + j) + 1] = F * chol_upd_items(N, j);
-    }
+    std::vector<int64_t> pre((size_t)chol_pre_len(N));
+    chol_prefix(pre.data(), N, F);
     BRPA_TRY(copy_sync(ctx, d_pre, pre.data(), 8 * pre.size(), hipMemcpyHostToDevice));
-    for (int j = 0; j < nsteps; ++j) {
-        BRPA_TRY(launch_potrf_diag(ctx, d_fr, d_pre + 2 * j, 1, pre[2 * j + 1], j));
-        BRPA_TRY(launch_trsm(ctx, d_fr, d_pre + 2 * (nsteps + j), 1, pre[2 * (nsteps + j) + 1], j));
-        BRPA_TRY(launch_chol_update(ctx, d_fr, d_pre + 2 * (2 * nsteps + j), 1,
-                                    pre[2 * (2 * nsteps + j) + 1], j));
-    }
-    return BRPA_OK;
+    return launch_cholesky(ctx, d_fr, 1, (int)cdiv(N, CHOL_NB), d_pre, pre.data());
 }
 
 extern "C" {
@@ -647,17 +628,12 @@ struct StoredBufs {
     }
 };
 
-// Work-group prefix arrays [setdiag, pdiag_0..S-1, trsm_0..S-1, update_0..S-1]
-// of the blocked Cholesky of nf matrices of order N.
-static std::vector<int64_t> stored_prefix(int64_t N, int64_t nf, int nsteps) {
-    std::vector<int64_t> pre((size_t)(1 + 3 * nsteps) * 2, 0);
+// Work-group prefix arrays [setdiag, the Cholesky's lists] of nf matrices of order N.
+static std::vector<int64_t> stored_prefix(int64_t N, int64_t nf) {
+    std::vector<int64_t> pre((size_t)(2 + chol_pre_len(N)));
+    pre[0] = 0;
     pre[1] = cdiv(nf * N, 256);
-    for (int j = 0; j < nsteps; ++j) {
-        int64_t j0 = (int64_t)j * CHOL_NB;
-        pre[2 * (1 + j) + 1] = (N > j0) ? nf : 0;
-        pre[2 * (1 + nsteps + j) + 1] = (N > j0 + CHOL_NB) ? nf * (cdiv(N - j0, CHOL_NB) - 1) : 0;
-        pre[2 * (1 + 2 * nsteps + j) + 1] = nf * chol_upd_items(N, j);
-    }
+    chol_prefix(pre.data() + 2, N, nf);
     return pre;
 }
 
@@ -691,13 +667,7 @@ static int ecrpa_stored_run(brpa_ctx *ctx, StoredBufs &b, const std::vector<int6
     const int64_t *d_pre = b.d_pre;
     BRPA_HIP(ctx, hipEventRecord(ctx->ev0, ctx->stream));
     BRPA_TRY(launch_set_diag(ctx, d_fr, d_pre, 1, pre[1], 0));
-    for (int j = 0; j < nsteps; ++j) {
-        BRPA_TRY(launch_potrf_diag(ctx, d_fr, d_pre + 2 * (1 + j), 1, pre[2 * (1 + j) + 1], j));
-        BRPA_TRY(launch_trsm(ctx, d_fr, d_pre + 2 * (1 + nsteps + j), 1,
-                             pre[2 * (1 + nsteps + j) + 1], j));
-        BRPA_TRY(launch_chol_update(ctx, d_fr, d_pre + 2 * (1 + 2 * nsteps + j), 1,
-                                    pre[2 * (1 + 2 * nsteps + j) + 1], j));
-    }
+    BRPA_TRY(launch_cholesky(ctx, d_fr, 1, nsteps, d_pre + 2, pre.data() + 2));
     BRPA_TRY(launch_energy(ctx, d_fr, 1));
     BRPA_HIP(ctx, hipEventRecord(ctx->ev1, ctx->stream));
     std::vector<int> st(F);
@@ -723,7 +693,7 @@ static int ecrpa_stored(brpa_ctx *ctx, double *ecrpa, const double *piu, bool pa
     BRPA_HIP(ctx, hipSetDevice(ctx->device));
     const int64_t N = naux, F = nfreqs;
     const int nsteps = (int)cdiv(N, CHOL_NB);
-    const std::vector<int64_t> pre = stored_prefix(N, F, nsteps);
+    const std::vector<int64_t> pre = stored_prefix(N, F);
     const bool pk_host = packed && !is_device_ptr(piu);
     StoredBufs b;
     Arena count;
@@ -804,7 +774,7 @@ static int ecrpa_stored_noalloc(brpa_ctx *ctx, double *ecrpa, const double *piu,
     double ms_tot = 0.0;
     for (int64_t f0 = 0; f0 < F; f0 += fc) {
         const int64_t nf = std::min(fc, F - f0);
-        const std::vector<int64_t> pre = stored_prefix(N, nf, nsteps);
+        const std::vector<int64_t> pre = stored_prefix(N, nf);
         StoredBufs b;
         Arena ar;
         ar.base = base;

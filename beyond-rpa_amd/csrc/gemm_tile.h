@@ -1,0 +1,240 @@
+// One output tile of an FP64 product on v_mfma_f64_16x16x4_f64 by a work-group of four
+// waves (2 x 2): the loop of k_gemm_f64 and of the Cholesky's trailing update.
+#pragma once
+#include "device_common.h"
+
+constexpr int GKB = 16;    // k per LDS stage
+typedef double d2_t __attribute__((ext_vector_type(2)));
+
+// LDS layout of one operand's tile (ROWS rows, 128 or 64) and 16-k stage.  k-contiguous (KC): [row][k]
+// with unpadded 16-double rows whose k pairs are XOR-swizzled by (row >> 1) & 7.
+// Rows-contiguous: [k][row] with rows of DMA_KPR doubles (a pitch of 4 rows moves by
+// half of the 64 LDS banks, so the four lane groups of a fragment read hit disjoint
+// halves).
+//
+// A wave's loads, V = 16: KC the 8-row blocks ROWS / 4 w + 8 c, lane L the k pair
+// (L % 8) ^ swizzle of row L / 8 of its block; rows-contiguous (128 rows only) the k
+// rows 4 w + c, lane L the rows 2 L, 2 L + 1.  The byte offsets from the tile's base at k = 0
+// (dma_base) are 32-bit; leading dimensions of 2^21 or more take the register
+// path of the last stage for all of them.
+// V = 4: KC the row pairs ROWS / 4 w + 2 c, lane L a half of a double of row L / 32;
+// rows-contiguous the k rows 4 w + c / 4, 32 rows at a time.
+constexpr int DMA_KPR = 132;
+template <bool KC>
+constexpr int gemm_lds(int rows) {   // doubles of one stage
+    return KC ? rows * GKB : GKB * DMA_KPR;
+}
+template <bool KC, int V, int ROWS>
+struct DmaSrc {
+    static_assert(KC || ROWS == 128, "rows-contiguous operands have 128-row tiles");
+    static constexpr int NLOAD = V == 16 ? ROWS / 32 : ROWS / 8;   // loads per wave and stage
+    // per load; V = 4 rows-contiguous: per 32 rows
+    static constexpr int NOFF = !KC ? 4 : NLOAD;
+    uint32_t off[NOFF];
+};
+template <bool KC, int V, int ROWS>
+__device__ __forceinline__ DmaSrc<KC, V, ROWS> dma_offsets(int64_t ldx, int r0, int rows, int wave,
+                                                           int lane) {
+    DmaSrc<KC, V, ROWS> s;
+#pragma unroll
+    for (int c = 0; c < DmaSrc<KC, V, ROWS>::NOFF; ++c) {
+        if (V == 16 && KC) {
+            const int row = ROWS / 4 * wave + 8 * c + (lane >> 3);
+            const int dk = 2 * ((lane & 7) ^ ((row >> 1) & 7));
+            s.off[c] = 8u * ((uint32_t)ldx * (uint32_t)(min(r0 + row, rows - 1) - r0) + (uint32_t)dk);
+        } else if (V == 16) {
+            // rows is even here: the last pair is rows - 2, rows - 1
+            s.off[c] = 8u * ((uint32_t)(min(r0 + 2 * lane, rows - 2) - r0) +
+                             (uint32_t)ldx * (uint32_t)(4 * wave + c));
+        } else if (KC) {
+            const int row = ROWS / 4 * wave + 2 * c + (lane >> 5);
+            s.off[c] = 8u * ((uint32_t)ldx * (uint32_t)(min(r0 + row, rows - 1) - r0)) +
+                       4u * (((uint32_t)lane & 31u) ^ (4u * ((row >> 1) & 7)));
+        } else {
+            s.off[c] = 8u * (uint32_t)(min(r0 + 32 * c + (lane >> 1), rows - 1) - r0) + 4u * (lane & 1);
+        }
+    }
+    return s;
+}
+template <bool KC>
+__device__ __forceinline__ const char *dma_base(const double *X, int64_t ldx, int r0) {
+    return reinterpret_cast<const char *>(X + (KC ? ldx * r0 : (int64_t)r0));
+}
+// fragment of row `row` at the k pair 2 g4 + hh of a stage
+template <bool KC>
+__host__ __device__ __forceinline__ d2_t dma_frag(const double *L, int row, int g4, int hh) {
+    if (KC) {
+        const int kp = 2 * g4 + hh;
+        return *reinterpret_cast<const d2_t *>(&L[row * GKB + 2 * (kp ^ ((row >> 1) & 7))]);
+    }
+    const int kr = 4 * g4 + 2 * hh;
+    d2_t v;
+    v.x = L[kr * DMA_KPR + row];
+    v.y = L[(kr + 1) * DMA_KPR + row];
+    return v;
+}
+
+// one operand's full stage at k0 into the LDS buffer L, straight from global memory
+template <bool KC, int V, int ROWS>
+__device__ __forceinline__ void dma_stage(const char *base, const DmaSrc<KC, V, ROWS> &src,
+                                          int64_t ldx, double *L, int wave, int k0) {
+    // the builtin exists for the device pass only; the host pass never runs this
+#if defined(__HIP_DEVICE_COMPILE__)
+    typedef __attribute__((address_space(1))) const char gchar_t;
+    typedef __attribute__((address_space(1))) const void gvoid_t;
+    typedef __attribute__((address_space(3))) void lvoid_t;
+    gchar_t *b = (gchar_t *)(base + 8 * (KC ? (int64_t)k0 : ldx * k0));
+    if (V == 16) {
+#pragma unroll
+        for (int c = 0; c < DmaSrc<KC, V, ROWS>::NLOAD; ++c)
+            __builtin_amdgcn_global_load_lds(
+                (gvoid_t *)(b + src.off[c]),
+                (lvoid_t *)(L + (KC ? (ROWS / 4 * wave + 8 * c) * GKB : (4 * wave + c) * DMA_KPR)), 16, 0,
+                0);
+    } else if (KC) {
+#pragma unroll
+        for (int c = 0; c < DmaSrc<KC, V, ROWS>::NLOAD; ++c)
+            __builtin_amdgcn_global_load_lds((gvoid_t *)(b + src.off[c]),
+                                             (lvoid_t *)(L + (ROWS / 4 * wave + 2 * c) * GKB), 4,
+                                             0, 0);
+    } else {
+#pragma unroll
+        for (int c = 0; c < 16; ++c) {
+            const int kr = 4 * wave + (c >> 2);
+            __builtin_amdgcn_global_load_lds((gvoid_t *)(b + 8 * ldx * kr + src.off[c % DmaSrc<KC, V, ROWS>::NOFF]),
+                                             (lvoid_t *)(L + kr * DMA_KPR + 32 * (c & 3)), 4, 0, 0);
+        }
+    }
+#endif
+}
+// the last stage when it has fewer than 16 k: through registers, zeros past kend
+template <bool KC, int ROWS>
+__device__ __forceinline__ void dma_stage_tail(const double *__restrict__ X, int64_t ldx, int r0,
+                                               int rows, double *L, int tid, int k0, int kend) {
+#pragma unroll 1
+    for (int u = 0; u < ROWS / 16; ++u) {
+        const int e = tid + 256 * u;
+        const int row = KC ? e >> 4 : e & 127, kk = KC ? e & 15 : e >> 7;
+        const int64_t r = min(r0 + row, rows - 1);
+        const double v = k0 + kk < kend ? X[KC ? k0 + kk + ldx * r : r + ldx * (k0 + kk)] : 0.0;
+        L[KC ? row * GKB + 2 * ((kk >> 1) ^ ((row >> 1) & 7)) + (kk & 1) : kk * DMA_KPR + row] = v;
+    }
+}
+
+// acc += rows m0 .. of op(A) times columns n0 .. of op(B) over k in [kbeg, kend): wave
+// (wm, wn) = (wave / 2, wave % 2) holds the ROWS/2 x ROWS/2 block (wm, wn), acc[i][j][r]
+// = element (16 i + lane % 16, 16 j + lane / 16 + 4 r) of it.  m, n: rows of the whole
+// operands (past them the last row repeats).  far: leading dimensions beyond 32-bit
+// offsets.  Waves with active false only stage.  sA, sB: two stages each
+// (gemm_lds doubles per stage).
+//
+// The fragments of either half of a stage are read while the other half is
+// multiplied, one LDS read after each of the first MFMAs and then the loads of the
+// coming stage after the next ones.  The barrier stands between the halves: by then
+// the next stage has landed and every wave has read the current one, whose buffer
+// takes the loads of the stage after the next.  Bound by MFMA issue: TN 8192 x 8192 x
+// 2048 73.0 TFLOP/s, 4096^3 66.7, 3072^2 x 4096 (whose last 64 of 576 tiles run one
+// per CU) 52 (68.5, 64.0 and 38-46 with all reads, then all loads, ahead of the stage's
+// MFMAs).
+template <bool KCA, bool KCB, int V, int ROWS>
+__device__ __forceinline__ void gemm_tile(d4_t (&acc)[ROWS / 32][ROWS / 32],
+                                          const double *__restrict__ A, int64_t lda, int m0, int m,
+                                          const double *__restrict__ B, int64_t ldb, int n0, int n,
+                                          int kbeg, int kend, bool far, bool active, double *sA,
+                                          double *sB) {
+    constexpr int NB = ROWS / 32, SA = gemm_lds<KCA>(ROWS), SB = gemm_lds<KCB>(ROWS);
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave >> 1, wn = wave & 1;
+    const int rl = lane & 15, g4 = lane >> 4;
+    const auto oa = dma_offsets<KCA, V, ROWS>(lda, m0, m, wave, lane);
+    const auto ob = dma_offsets<KCB, V, ROWS>(ldb, n0, n, wave, lane);
+    const char *ba = dma_base<KCA>(A, lda, m0), *bb = dma_base<KCB>(B, ldb, n0);
+    const int nfull = far ? 0 : (kend - kbeg) / GKB, ns = (kend - kbeg + GKB - 1) / GKB;
+    auto stage = [&](int buf, int k0) {
+        dma_stage<KCA, V, ROWS>(ba, oa, lda, sA + buf * SA, wave, k0);
+        dma_stage<KCB, V, ROWS>(bb, ob, ldb, sB + buf * SB, wave, k0);
+    };
+    auto put = [&](int buf, int q) {
+        if (q < nfull) {
+            stage(buf, kbeg + GKB * q);
+        } else if (q < ns) {
+            dma_stage_tail<KCA, ROWS>(A, lda, m0, m, sA + buf * SA, tid, kbeg + GKB * q, kend);
+            dma_stage_tail<KCB, ROWS>(B, ldb, n0, n, sB + buf * SB, tid, kbeg + GKB * q, kend);
+        }
+    };
+    put(0, 0);
+    if (!active) {
+        __syncthreads();
+        put(1, 1);
+        for (int q = 0; q + 1 < ns; ++q) {
+            __syncthreads();
+            put(q & 1, q + 2);
+        }
+        return;
+    }
+    // one half of a stage: two k per lane
+    auto frags = [&](d2_t (&a)[NB], d2_t (&b)[NB], int buf, int hh) {
+#pragma unroll
+        for (int i = 0; i < NB; ++i)
+            a[i] = dma_frag<KCA>(sA + buf * SA, ROWS / 2 * wm + 16 * i + rl, g4, hh);
+#pragma unroll
+        for (int j = 0; j < NB; ++j)
+            b[j] = dma_frag<KCB>(sB + buf * SB, ROWS / 2 * wn + 16 * j + rl, g4, hh);
+    };
+    auto mma = [&](const d2_t (&a)[NB], const d2_t (&b)[NB]) {
+#pragma unroll
+        for (int st = 0; st < 2; ++st)
+#pragma unroll
+            for (int i = 0; i < NB; ++i)
+#pragma unroll
+                for (int j = 0; j < NB; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(b[j][st], a[i][st], acc[i][j], 0,
+                                                                     0, 0);
+    };
+    d2_t a0[NB], b0[NB], a1[NB], b1[NB];
+    __syncthreads();
+    put(1, 1);
+    frags(a0, b0, 0, 0);
+    constexpr int NM = 2 * NB * NB, NR = 2 * NB;      // MFMAs and LDS reads of a half
+    constexpr int NL = 2 * (V == 16 ? ROWS / 32 : ROWS / 8);   // loads of a stage per wave
+    constexpr int LG = NL < NM - NR ? NL : NM - NR;   // MFMAs they are spread over
+    int buf = 0, q = 0;
+    for (; q + 2 < nfull; ++q, buf ^= 1) {
+        frags(a1, b1, buf, 1);
+        mma(a0, b0);
+#pragma unroll
+        for (int u = 0; u < NR; ++u) {
+            __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);     // MFMA
+            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);   // LDS read
+        }
+        __builtin_amdgcn_sched_group_barrier(0x8, NM - NR, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        __syncthreads();
+        frags(a0, b0, buf ^ 1, 0);
+        stage(buf, kbeg + GKB * (q + 2));
+        mma(a1, b1);
+#pragma unroll
+        for (int u = 0; u < NR; ++u) {
+            __builtin_amdgcn_sched_group_barrier(0x8, 1, 1);
+            __builtin_amdgcn_sched_group_barrier(0x100, 1, 1);
+        }
+#pragma unroll
+        for (int u = 0; u < LG; ++u) {
+            __builtin_amdgcn_sched_group_barrier(0x8, 1, 1);
+            __builtin_amdgcn_sched_group_barrier(0x20, (NL + LG - 1) / LG, 1);   // global -> LDS
+        }
+        __builtin_amdgcn_sched_group_barrier(0x8, NM - NR - LG, 1);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    for (; q < ns; ++q, buf ^= 1) {
+        frags(a1, b1, buf, 1);
+        mma(a0, b0);
+        if (q + 1 < ns) {
+            __syncthreads();
+            put(buf, q + 2);
+            frags(a0, b0, buf ^ 1, 0);
+        }
+        mma(a1, b1);
+    }
+}

@@ -225,13 +225,13 @@ int launch_syrk_f64(brpa_ctx *, const FragDev *, const int64_t *pre, int nfrag, 
 // mode: 0 = Pi's own diagonal, 1 = split-BF16 partials, 2 = diag precomputed
 int launch_set_diag(brpa_ctx *, const FragDev *, const int64_t *pre, int nfrag, int64_t total,
                     int mode);
-int launch_potrf_diag(brpa_ctx *, const FragDev *, const int64_t *pre, int nfrag, int64_t total, int step);
-int launch_trsm(brpa_ctx *, const FragDev *, const int64_t *pre, int nfrag, int64_t total, int step);
-int launch_chol_update(brpa_ctx *, const FragDev *, const int64_t *pre, int nfrag, int64_t total, int step);
-// Work items per matrix of the trailing update after Cholesky step j (N x N):
-// the next 64-column strip inside an outer panel of CHOL_OUTER steps, the rest
-// of the trailing matrix after its last step.
-int64_t chol_upd_items(int64_t N, int64_t j);
+// Blocked Cholesky of every matrix of the fragments.  Work-groups per fragment, list
+// and 64-column step: chol_items; d_pre / h_pre: their prefix sums over the fragments on
+// the device and the host, [list][step][nfrag + 1].
+enum { CHOL_DIAG, CHOL_TRSM, CHOL_STRIP, CHOL_REST, CHOL_STEP, CHOL_NLISTS };
+int64_t chol_items(int list, int64_t N, int64_t F, int64_t j);
+int launch_cholesky(brpa_ctx *, const FragDev *, int nfrag, int nsteps, const int64_t *d_pre,
+                    const int64_t *h_pre);
 int launch_energy(brpa_ctx *, const FragDev *, int nfrag);
 int launch_fill_int(brpa_ctx *, int *p, int64_t n, int v);
 int launch_split(brpa_ctx *, const FragDev *, const int64_t *pre, int nfrag, int64_t total);

@@ -18,7 +18,7 @@
 //                       with strides (brpa_dtrsm)
 #include <algorithm>
 
-#include "device_common.h"
+#include "gemm_tile.h"
 #include "internal.h"
 
 #define LAUNCH_CHECK(ctx)                                                                      \
@@ -31,7 +31,6 @@
 
 namespace {
 constexpr int GT = 128;    // GEMM tile edge
-constexpr int GKB = 16;    // k per LDS stage
 constexpr int GGROUP = 8;  // tile rows per group of the tile order (panel reuse in L2)
 }
 
@@ -41,7 +40,7 @@ constexpr int GGROUP = 8;  // tile rows per group of the tile order (panel reuse
 //
 // Stages of 16 k go straight from global memory into LDS (global_load_lds, no
 // register staging and no LDS store instructions), double-buffered, in the
-// layouts at dma_offsets.  In a stage, lane l of a wave supplies the k values
+// layouts of gemm_tile.h.  In a stage, lane l of a wave supplies the k values
 // 4 (l / 16) .. +3 of its row to the four MFMA steps.  The k order inside a stage
 // is a permutation of the sum, the same for both operands.  The MFMA takes the B
 // fragment as its first operand, so the accumulator rows run along the lanes
@@ -85,123 +84,11 @@ struct GemmArgs {
     double *P;
 };
 
-namespace {
-typedef double d2_t __attribute__((ext_vector_type(2)));
-}
-
-// LDS layout of one operand's 128-row tile and 16-k stage.  k-contiguous (KC): [row][k]
-// with unpadded 16-double rows whose k pairs are XOR-swizzled by (row >> 1) & 7.
-// Rows-contiguous: [k][row] with rows of DMA_KPR doubles (a pitch of 4 rows moves by
-// half of the 64 LDS banks, so the four lane groups of a fragment read hit disjoint
-// halves).
-//
-// A wave's loads, V = 16: KC the 8-row blocks 32 w + 8 c (c < 4), lane L the k pair
-// (L % 8) ^ swizzle of row L / 8 of its block; rows-contiguous the k rows 4 w + c,
-// lane L the rows 2 L, 2 L + 1.  The byte offsets from the tile's base at k = 0
-// (dma_base) are 32-bit; leading dimensions of 2^21 or more take the register
-// path of the last stage for all of them.
-// V = 4: KC the row pairs 32 w + 2 c (c < 16), lane L a half of a double of row L / 32;
-// rows-contiguous the k rows 4 w + c / 4, 32 rows at a time.
-constexpr int DMA_KPR = 132;
-template <bool KC, int V>
-struct DmaSrc {
-    // per load; V = 4 rows-contiguous: per 32 rows
-    static constexpr int NOFF = KC && V == 4 ? 16 : 4;
-    uint32_t off[NOFF];
-};
-template <bool KC, int V>
-__device__ __forceinline__ DmaSrc<KC, V> dma_offsets(int64_t ldx, int r0, int rows, int wave,
-                                                     int lane) {
-    DmaSrc<KC, V> s;
-#pragma unroll
-    for (int c = 0; c < DmaSrc<KC, V>::NOFF; ++c) {
-        if (V == 16 && KC) {
-            const int row = 32 * wave + 8 * c + (lane >> 3);
-            const int dk = 2 * ((lane & 7) ^ ((row >> 1) & 7));
-            s.off[c] = 8u * ((uint32_t)ldx * (uint32_t)(min(r0 + row, rows - 1) - r0) + (uint32_t)dk);
-        } else if (V == 16) {
-            // rows is even here: the last pair is rows - 2, rows - 1
-            s.off[c] = 8u * ((uint32_t)(min(r0 + 2 * lane, rows - 2) - r0) +
-                             (uint32_t)ldx * (uint32_t)(4 * wave + c));
-        } else if (KC) {
-            const int row = 32 * wave + 2 * c + (lane >> 5);
-            s.off[c] = 8u * ((uint32_t)ldx * (uint32_t)(min(r0 + row, rows - 1) - r0)) +
-                       4u * (((uint32_t)lane & 31u) ^ (4u * (c & 7)));
-        } else {
-            s.off[c] = 8u * (uint32_t)(min(r0 + 32 * c + (lane >> 1), rows - 1) - r0) + 4u * (lane & 1);
-        }
-    }
-    return s;
-}
-template <bool KC>
-__device__ __forceinline__ const char *dma_base(const double *X, int64_t ldx, int r0) {
-    return reinterpret_cast<const char *>(X + (KC ? ldx * r0 : (int64_t)r0));
-}
-// fragment of row `row` at the k pair 2 g4 + hh of a stage
-template <bool KC>
-__host__ __device__ __forceinline__ d2_t dma_frag(const double *L, int row, int g4, int hh) {
-    if (KC) {
-        const int kp = 2 * g4 + hh;
-        return *reinterpret_cast<const d2_t *>(&L[row * GKB + 2 * (kp ^ ((row >> 1) & 7))]);
-    }
-    const int kr = 4 * g4 + 2 * hh;
-    d2_t v;
-    v.x = L[kr * DMA_KPR + row];
-    v.y = L[(kr + 1) * DMA_KPR + row];
-    return v;
-}
-
-// one operand's full stage at k0 into the LDS buffer L, straight from global memory
-template <bool KC, int V>
-__device__ __forceinline__ void dma_stage(const char *base, const DmaSrc<KC, V> &src, int64_t ldx,
-                                          double *L, int wave, int k0) {
-    // the builtin exists for the device pass only; the host pass never runs this
-#if defined(__HIP_DEVICE_COMPILE__)
-    typedef __attribute__((address_space(1))) const char gchar_t;
-    typedef __attribute__((address_space(1))) const void gvoid_t;
-    typedef __attribute__((address_space(3))) void lvoid_t;
-    gchar_t *b = (gchar_t *)(base + 8 * (KC ? (int64_t)k0 : ldx * k0));
-    if (V == 16) {
-#pragma unroll
-        for (int c = 0; c < 4; ++c)
-            __builtin_amdgcn_global_load_lds(
-                (gvoid_t *)(b + src.off[c]),
-                (lvoid_t *)(L + (KC ? (32 * wave + 8 * c) * GKB : (4 * wave + c) * DMA_KPR)), 16, 0,
-                0);
-    } else if (KC) {
-#pragma unroll
-        for (int c = 0; c < 16; ++c)
-            __builtin_amdgcn_global_load_lds((gvoid_t *)(b + src.off[c]),
-                                             (lvoid_t *)(L + (32 * wave + 2 * c) * GKB), 4, 0, 0);
-    } else {
-#pragma unroll
-        for (int c = 0; c < 16; ++c) {
-            const int kr = 4 * wave + (c >> 2);
-            __builtin_amdgcn_global_load_lds((gvoid_t *)(b + 8 * ldx * kr + src.off[c % DmaSrc<KC, V>::NOFF]),
-                                             (lvoid_t *)(L + kr * DMA_KPR + 32 * (c & 3)), 4, 0, 0);
-        }
-    }
-#endif
-}
-// the last stage when it has fewer than 16 k: through registers, zeros past kend
-template <bool KC>
-__device__ __forceinline__ void dma_stage_tail(const double *__restrict__ X, int64_t ldx, int r0,
-                                               int rows, double *L, int tid, int k0, int kend) {
-#pragma unroll 1
-    for (int u = 0; u < 8; ++u) {
-        const int e = tid + 256 * u;
-        const int row = KC ? e >> 4 : e & 127, kk = KC ? e & 15 : e >> 7;
-        const int64_t r = min(r0 + row, rows - 1);
-        const double v = k0 + kk < kend ? X[KC ? k0 + kk + ldx * r : r + ldx * (k0 + kk)] : 0.0;
-        L[KC ? row * GKB + 2 * ((kk >> 1) ^ ((row >> 1) & 7)) + (kk & 1) : kk * DMA_KPR + row] = v;
-    }
-}
-
 template <bool TA, bool TB, int V>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_gemm_f64(const GemmArgs g) {
     constexpr bool KCA = TA, KCB = !TB;   // operand contiguous in k
-    __shared__ __attribute__((aligned(16))) double sA[2][KCA ? GT * GKB : GKB * DMA_KPR];
-    __shared__ __attribute__((aligned(16))) double sB[2][KCB ? GT * GKB : GKB * DMA_KPR];
+    __shared__ __attribute__((aligned(16))) double sA[2][gemm_lds<KCA>(GT)];
+    __shared__ __attribute__((aligned(16))) double sB[2][gemm_lds<KCB>(GT)];
     const int item1 = (int)(blockIdx.x / (unsigned)g.ntiles);
     const int t = (int)(blockIdx.x - (unsigned)item1 * (unsigned)g.ntiles);
     const int item2 = (int)blockIdx.y;
@@ -245,98 +132,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
         for (int j = 0; j < 4; ++j) acc[i][j] = (d4_t){0.0, 0.0, 0.0, 0.0};
 
-    if (kbeg < kend) {
-        const int rl = lane & 15, g4 = lane >> 4;
-        const DmaSrc<KCA, V> oa = dma_offsets<KCA, V>(lda, m0, m, wave, lane);
-        const DmaSrc<KCB, V> ob = dma_offsets<KCB, V>(ldb, n0, n, wave, lane);
-        const char *ba = dma_base<KCA>(A, lda, m0), *bb = dma_base<KCB>(B, ldb, n0);
-        auto stage = [&](int buf, int k0) {
-            dma_stage<KCA, V>(ba, oa, lda, sA[buf], wave, k0);
-            dma_stage<KCB, V>(bb, ob, ldb, sB[buf], wave, k0);
-        };
-        auto stage_tail = [&](int buf, int k0) {
-            dma_stage_tail<KCA>(A, lda, m0, m, sA[buf], tid, k0, kend);
-            dma_stage_tail<KCB>(B, ldb, n0, n, sB[buf], tid, k0, kend);
-        };
-        // one half of a stage: two k per lane
-        auto frags = [&](d2_t (&a)[4], d2_t (&b)[4], int buf, int hh) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-                a[i] = dma_frag<KCA>(sA[buf], 64 * wm + 16 * i + rl, g4, hh);
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-                b[j] = dma_frag<KCB>(sB[buf], 64 * wn + 16 * j + rl, g4, hh);
-        };
-        auto mma = [&](const d2_t (&a)[4], const d2_t (&b)[4]) {
-#pragma unroll
-            for (int st = 0; st < 2; ++st)
-#pragma unroll
-                for (int i = 0; i < 4; ++i)
-#pragma unroll
-                    for (int j = 0; j < 4; ++j)
-                        acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(b[j][st], a[i][st],
-                                                                         acc[i][j], 0, 0, 0);
-        };
-        d2_t a0[4], b0[4], a1[4], b1[4];
-        // The fragments of either half of a stage are read while the other half
-        // is multiplied, one LDS read after each of the first MFMAs and then one
-        // load of the coming stage after each of the next.  The barrier stands
-        // between the halves: by then the next stage has landed and every wave
-        // has read the current one, whose buffer takes the loads of the stage
-        // after the next.  Bound by MFMA issue: TN 8192 x 8192 x 2048 73.0
-        // TFLOP/s, 4096^3 66.7, 3072^2 x 4096 (whose last 64 of 576 tiles run one
-        // per CU) 52 (68.5, 64.0 and 38-46 with all reads, then all loads, ahead
-        // of the stage's MFMAs).
-        const int nfull = g.far ? 0 : (kend - kbeg) / GKB, ns = (kend - kbeg + GKB - 1) / GKB;
-        auto put = [&](int buf, int q) {
-            if (q < nfull)
-                stage(buf, kbeg + GKB * q);
-            else if (q < ns)
-                stage_tail(buf, kbeg + GKB * q);
-        };
-        put(0, 0);
-        __syncthreads();
-        put(1, 1);
-        frags(a0, b0, 0, 0);
-        int buf = 0, q = 0;
-        for (; q + 2 < nfull; ++q, buf ^= 1) {
-            frags(a1, b1, buf, 1);
-            mma(a0, b0);
-#pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);     // MFMA
-                __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);   // LDS read
-            }
-            __builtin_amdgcn_sched_group_barrier(0x8, 24, 0);
-            __builtin_amdgcn_sched_barrier(0);
-            __syncthreads();
-            frags(a0, b0, buf ^ 1, 0);
-            stage(buf, kbeg + GKB * (q + 2));
-            mma(a1, b1);
-#pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                __builtin_amdgcn_sched_group_barrier(0x8, 1, 1);
-                __builtin_amdgcn_sched_group_barrier(0x100, 1, 1);
-            }
-#pragma unroll
-            for (int u = 0; u < (V == 16 ? 8 : 16); ++u) {
-                __builtin_amdgcn_sched_group_barrier(0x8, 1, 1);
-                __builtin_amdgcn_sched_group_barrier(0x20, V == 16 ? 1 : 2, 1);   // global -> LDS
-            }
-            __builtin_amdgcn_sched_group_barrier(0x8, V == 16 ? 16 : 8, 1);
-            __builtin_amdgcn_sched_barrier(0);
-        }
-        for (; q < ns; ++q, buf ^= 1) {
-            frags(a1, b1, buf, 1);
-            mma(a0, b0);
-            if (q + 1 < ns) {
-                __syncthreads();
-                put(buf, q + 2);
-                frags(a0, b0, buf ^ 1, 0);
-            }
-            mma(a1, b1);
-        }
-    }
+    if (kbeg < kend)
+        gemm_tile<KCA, KCB, V, GT>(acc, A, lda, m0, m, B, ldb, n0, n, kbeg, kend, g.far != 0, true,
+                                   sA[0], sB[0]);
 
     if (g.nsplit > 1) {
         // partial tile, reduced by k_gemm_reduce

@@ -7,12 +7,13 @@
 //   k_set_diag     diag_w (tr Pi, rpa_CC.f90:444-447); Pi_w[P][P] += 1 (448-450)
 //   k_potrf_diag   Cholesky + inverse of a 64x64 diagonal block (four waves)
 //   k_trsm         L21 = A21 L11^{-T} on MFMA
-//   k_chol_update  trailing update A22 -= L21 L21^T on MFMA
+//   k_chol_strip, k_chol_rest  trailing updates A22 -= L21 L21^T on MFMA
+//   k_chol_step    diagonal block, left-looking strip and L21 of a step in one launch
 //   k_energy       E = sum_w w/(2 pi) (2 sum log L_kk - tr Pi_w)  (rpa_CC.f90:451-453)
 //
 // All kernels walk a flattened work list over fragments: work-group b belongs
 // to fragment f with pre[f] <= b < pre[f+1].
-#include "device_common.h"
+#include "gemm_tile.h"
 #include "internal.h"
 
 #define LAUNCH_CHECK(ctx)                                                                      \
@@ -416,15 +417,16 @@ int launch_set_diag(brpa_ctx *ctx, const FragDev *fr, const int64_t *pre, int nf
 }
 
 // ---------------------------------------------------------------------------
-// Blocked right-looking Cholesky of A_w = 1 + Pi_w (lower triangle, row-major),
-// three launches per 64-column step j (j0 = 64 j):
+// Blocked Cholesky of A_w = 1 + Pi_w (lower triangle, row-major) in 64-column steps j
+// (j0 = 64 j), one launch per step for few matrices (k_chol_step), else three:
 //   k_potrf_diag   one work-group per matrix: factors the diagonal block in LDS,
 //                  writes its log-det partial and L11^{-1} (own buffer; A11
 //                  itself is never written back, so no work-group of the same
 //                  step can read a half-factored block)
 //   k_trsm         L21 = A21 L11^{-T} as a 64x64x64 MFMA product per row chunk
-//   k_chol_update  A22 -= L21 L21^T per lower 64x64 tile pair, MFMA
-// Work-groups per fragment: F (diag), F*(nchunks-1) (trsm), F*npairs (update).
+//   k_chol_strip   the next 64 columns of A22 -= L21 L21^T over the outer panel
+// and after every outer panel of four steps k_chol_rest, the rest of A22 (launch_cholesky).
+// Work-groups per fragment: chol_items.
 
 // C(64x64) = X Y^T with X, Y 64x64 in LDS; wave (qi,qj) owns a 32x32 quadrant,
 // acc[i][j][r] = C[32 qi + 16 i + l/16 + 4 r][32 qj + 16 j + l%16].
@@ -550,8 +552,8 @@ __device__ __forceinline__ double rcp_newton(double p) {
     return fma(fma(-p, x, 1.0), x, x);
 }
 
-// Diagonal block of step `step` of matrix w, one work-group of four waves per
-// matrix.  The 64 x 64 block sits in LDS as 4 x 4 blocks of 16:
+// Cholesky factor of a 64 x 64 block by one work-group of four waves.  The block sits in
+// LDS as 4 x 4 blocks of 16 (lower triangle; the upper one is scratch):
 //   panel p     wave 0: lane r holds row r of the 16 panel columns in registers
 //               and eliminates column by column.  The multiplier is a(r, c) /
 //               pivot, and the row of the pivot comes from lanes c+1 .. by
@@ -559,53 +561,140 @@ __device__ __forceinline__ double rcp_newton(double p) {
 //               square root lies between two pivots; the columns are scaled by
 //               1 / sqrt(pivot) at the end, all 16 at once.
 //   column p+1  waves 1-3: A(i, p+1) -= L(i, p) L(p+1, p)^T on MFMA
-//   the other blocks right of it by waves 1-3 while wave 0 runs panel p+1
-//   L11^{-1}    wave j: L(j, j)^{-1} by substitution (lane n: column n), then block
-//               column j on MFMA, X(i, j) = -X(i, i) sum_k L(i, k)
-//               X(k, j).  The accumulator layout of X(k, j) is the operand layout
-//               of the next product, so the column stays in registers.
-// Outputs: linv, log-det partial, status, optional L11 write-back.
+//   the other blocks right of it by waves 1-3 while wave 0 runs panel p+1, and after
+//               them work(p + 1), the caller's own
+//   L(p, p)^{-1}  from panel p itself, whose lanes 0 .. 15 would idle: rows of the
+//               identity below the block become those of L(p, p)^{-T}.  Panel 0 has no
+//               idle lanes; wave 2 inverts its block during panel 2.
+// chol_panels returns whether a pivot was not positive.
 //
 // Bound by latency: 64 pivots in a chain of readlane, reciprocal, multiply and
-// fma.  Measured per launch on MI355X: 17.7 us for 16 matrices, 20.7 us for 512
-// (61.3 and 65.4 us for one left-looking wave per matrix with rows of L from LDS,
+// fma.  Measured per k_potrf_diag launch on MI355X: 17.7 us for 16 matrices, 20.7 us for
+// 512 (61.3 and 65.4 us for one left-looking wave per matrix with rows of L from LDS,
 // the square root and division in the chain and the whole inverse by substitution).
-__global__ __launch_bounds__(256) void k_potrf_diag(const FragDev *__restrict__ fr,
-                                                   const int64_t *__restrict__ pre, int nfrag,
-                                                   int step) {
-    // row pitch 66 doubles: 16-byte aligned rows, 16 rows on 16 distinct 4-bank groups
-    constexpr int LP = CHOL_NB + 2;
-    constexpr int XP = 18;
-    __shared__ __attribute__((aligned(16))) double S[CHOL_NB][LP];
-    __shared__ __attribute__((aligned(16))) double Xd[4][16][XP];   // L(p, p)^{-1}
-    __shared__ double rdiag[CHOL_NB];
-    __shared__ int64_t s_pre[FIND_LDS_MAX + 1];
-    const int64_t b = blockIdx.x;
-    const int f = find_frag_lds(pre, nfrag, b, s_pre);
-    const int w = (int)(b - (nfrag <= FIND_LDS_MAX ? s_pre[f] : pre[f]));
-    const FragDev &F = fr[f];
-    const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-    const int N = F.N;
-    const int j0 = step * CHOL_NB;
-    const int nbj = min(CHOL_NB, N - j0);
-    double *A = F.Pi + (int64_t)w * N * N;
-    const gdouble_t *G = (const gdouble_t *)A;
-    // lower triangle only (the other one is never read); rows and columns past
-    // nbj are those of the identity
-    {
-        double v[16];
+constexpr int CH_LP = CHOL_NB + 2;   // row pitch: 16-byte aligned rows, 16 rows on 16 distinct 4-bank groups
+constexpr int CH_XP = 18;
+
+struct CholLds {
+    double S[CHOL_NB][CH_LP];
+    double Xd[4][16][CH_XP];   // L(p, p)^{-1}
+    double rdiag[CHOL_NB];
+};
+
+// the block at (j0, j0): lower triangle only; rows and columns past nbj are those of
+// the identity
+__device__ __forceinline__ void chol_load64(CholLds &T, const gdouble_t *G, int N, int j0, int nbj,
+                                            int wave, int lane) {
+    double v[16];
 #pragma unroll
-        for (int u = 0; u < 16; ++u) {
-            const int r = wave + 4 * u;
-            const bool in = r < nbj && lane <= r;
-            v[u] = G[in ? (int64_t)(j0 + r) * N + j0 + lane : 0];
-            v[u] = in ? v[u] : ((r >= nbj && lane == r) ? 1.0 : 0.0);
-        }
-#pragma unroll
-        for (int u = 0; u < 16; ++u) S[wave + 4 * u][lane] = v[u];
+    for (int u = 0; u < 16; ++u) {
+        const int r = wave + 4 * u;
+        const bool in = r < nbj && lane <= r;
+        v[u] = G[in ? (int64_t)(j0 + r) * N + j0 + lane : 0];
+        v[u] = in ? v[u] : ((r >= nbj && lane == r) ? 1.0 : 0.0);
     }
-    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < 16; ++u) T.S[wave + 4 * u][lane] = v[u];
+}
+
+// L(p, p)^{-1} by substitution (lane n: column n): x_i = (delta_in - sum_{k<i} L_ik x_k) / L_ii
+__device__ __forceinline__ void chol_invert16(CholLds &T, int p, int lane) {
+    const int l16 = lane & 15;
+    double x[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        double s0 = i == l16 ? 1.0 : 0.0, s1 = 0.0;
+#pragma unroll
+        for (int k = 0; k < i; k += 2) {
+            const d2v_t u = *reinterpret_cast<const d2v_t *>(&T.S[16 * p + i][16 * p + k]);
+            s0 = fma(-u.x, x[k], s0);
+            if (k + 1 < i) s1 = fma(-u.y, x[k + 1], s1);
+        }
+        x[i] = (s0 + s1) * T.rdiag[16 * p + i];
+    }
+    if (lane < 16)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) T.Xd[p][i][l16] = x[i];
+}
+
+// wave 0
+__device__ __forceinline__ bool chol_panels(CholLds &T, int lane) {
+    double(*S)[CH_LP] = T.S;
+    bool bad = false;
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+        double a[16];
+        d2v_t *row = reinterpret_cast<d2v_t *>(&S[lane][16 * p]);
+#pragma unroll
+        for (int t = 0; t < 8; ++t) {
+            const d2v_t u = row[t];
+            a[2 * t] = u.x;
+            a[2 * t + 1] = u.y;
+        }
+        if (p > 0 && lane < 16)
+#pragma unroll
+            for (int c = 0; c < 16; ++c) a[c] = lane == c ? 1.0 : 0.0;
+        double mypiv = 1.0;
+        bool inrange = true;
+#pragma unroll
+        for (int c = 0; c < 16; ++c) {
+            const double piv = wave_bcast(a[c], 16 * p + c);
+            inrange = inrange && piv >= 0x1p-1000 && piv <= 0x1p+1000;
+            const double m = a[c] * rcp_newton(piv);
+            mypiv = lane == 16 * p + c ? piv : mypiv;
+            // lanes above row j update entries that are never read
+#pragma unroll
+            for (int j = c + 1; j < 16; ++j)
+                a[j] = fma(-m, wave_bcast(a[c], 16 * p + j), a[j]);
+        }
+        if (!inrange) {
+            // a pivot that is not positive, or outside the range of rcp_newton: the
+            // panel again, on its columns in LDS, with divisions
+#pragma unroll 1
+            for (int c = 0; c < 16; ++c) {
+                const int pc = 16 * p + c;
+                double piv = S[pc][pc];
+                if (!(piv > 0.0) || !isfinite(piv)) {
+                    bad = true;
+                    piv = 1.0;
+                }
+                mypiv = lane == pc ? piv : mypiv;
+                const double m = S[lane][pc] / piv;
+#pragma unroll 1
+                for (int j = c + 1; j < 16; ++j)
+                    if (lane >= 16 * p + j)
+                        S[lane][16 * p + j] = fma(-m, S[16 * p + j][pc], S[lane][16 * p + j]);
+            }
+#pragma unroll
+            for (int t = 0; t < 8; ++t) {
+                const d2v_t u = row[t];
+                a[2 * t] = u.x;
+                a[2 * t + 1] = u.y;
+            }
+        }
+        const double d = sqrt(mypiv), rd = 1.0 / d;
+#pragma unroll
+        for (int c = 0; c < 16; ++c)
+            a[c] = lane == 16 * p + c ? d : a[c] * wave_bcast(rd, 16 * p + c);
+        if (lane >= 16 * p) {
+#pragma unroll
+            for (int t = 0; t < 8; ++t) row[t] = (d2v_t){a[2 * t], a[2 * t + 1]};
+            if (lane < 16 * p + 16) T.rdiag[lane] = rd;
+        } else if (lane < 16) {
+#pragma unroll
+            for (int c = 0; c < 16; ++c) T.Xd[p][c][lane] = a[c];
+        }
+        if (p > 0 && !inrange) chol_invert16(T, p, lane);
+        __syncthreads();
+        if (p < 3) __syncthreads();   // column p + 1
+    }
+    return bad;
+}
+
+// waves 1-3: the same barriers
+template <class Work>
+__device__ __forceinline__ void chol_blocks(CholLds &T, int wave, int lane, Work work) {
+    double(*S)[CH_LP] = T.S;
     const int l16 = lane & 15, g4 = lane >> 4;
     // S(i, j) -= L(i, p) L(j, p)^T for 16 x 16 blocks
     auto update = [&](int i, int j, int p) {
@@ -620,126 +709,32 @@ __global__ __launch_bounds__(256) void k_potrf_diag(const FragDev *__restrict__ 
 #pragma unroll
         for (int r = 0; r < 4; ++r) S[16 * i + g4 + 4 * r][16 * j + l16] = acc[r];
     };
-    // column l16 of L(p, p)^{-1}: x_i = (delta_in - sum_{k<i} L_ik x_k) / L_ii
-    auto invert = [&](int p) {
-        double x[16];
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            double s0 = i == l16 ? 1.0 : 0.0, s1 = 0.0;
-#pragma unroll
-            for (int k = 0; k < i; k += 2) {
-                const d2v_t u = *reinterpret_cast<const d2v_t *>(&S[16 * p + i][16 * p + k]);
-                s0 = fma(-u.x, x[k], s0);
-                if (k + 1 < i) s1 = fma(-u.y, x[k + 1], s1);
-            }
-            x[i] = (s0 + s1) * rdiag[16 * p + i];
-        }
-        if (lane < 16)
-#pragma unroll
-            for (int i = 0; i < 16; ++i) Xd[p][i][l16] = x[i];
-    };
-    int bad = 0;
 #pragma unroll
     for (int p = 0; p < 4; ++p) {
-        if (wave == 0) {
-            double a[16];
-            d2v_t *row = reinterpret_cast<d2v_t *>(&S[lane][16 * p]);
-#pragma unroll
-            for (int t = 0; t < 8; ++t) {
-                const d2v_t u = row[t];
-                a[2 * t] = u.x;
-                a[2 * t + 1] = u.y;
-            }
-            double mypiv = 1.0;
-            bool inrange = true;
-#pragma unroll
-            for (int c = 0; c < 16; ++c) {
-                const double piv = wave_bcast(a[c], 16 * p + c);
-                inrange = inrange && piv >= 0x1p-1000 && piv <= 0x1p+1000;
-                const double m = a[c] * rcp_newton(piv);
-                mypiv = lane == 16 * p + c ? piv : mypiv;
-                // lanes above row j update entries of the upper triangle, never read
-#pragma unroll
-                for (int j = c + 1; j < 16; ++j)
-                    a[j] = fma(-m, wave_bcast(a[c], 16 * p + j), a[j]);
-            }
-            if (!inrange) {
-                // a pivot that is not positive, or outside the range of rcp_newton: the
-                // panel again, on its columns in LDS, with divisions
-#pragma unroll 1
-                for (int c = 0; c < 16; ++c) {
-                    const int pc = 16 * p + c;
-                    double piv = S[pc][pc];
-                    if (!(piv > 0.0) || !isfinite(piv)) {
-                        bad = 1;
-                        piv = 1.0;
-                    }
-                    mypiv = lane == pc ? piv : mypiv;
-                    const double m = S[lane][pc] / piv;
-#pragma unroll 1
-                    for (int j = c + 1; j < 16; ++j)
-                        if (lane >= 16 * p + j)
-                            S[lane][16 * p + j] = fma(-m, S[16 * p + j][pc], S[lane][16 * p + j]);
-                }
-#pragma unroll
-                for (int t = 0; t < 8; ++t) {
-                    const d2v_t u = row[t];
-                    a[2 * t] = u.x;
-                    a[2 * t + 1] = u.y;
-                }
-            }
-            const double d = sqrt(mypiv), rd = 1.0 / d;
-#pragma unroll
-            for (int c = 0; c < 16; ++c)
-                a[c] = lane == 16 * p + c ? d : a[c] * wave_bcast(rd, 16 * p + c);
-            if (lane >= 16 * p) {
-#pragma unroll
-                for (int t = 0; t < 8; ++t) row[t] = (d2v_t){a[2 * t], a[2 * t + 1]};
-                if (lane < 16 * p + 16) rdiag[lane] = rd;
-            }
-        } else {
-            // panel p - 1: the blocks right of column p
-            if (p == 1) update(wave == 1 ? 2 : 3, wave == 3 ? 3 : 2, 0);
-            if (p == 2 && wave == 1) update(3, 3, 1);
-        }
+        // panel p - 1: the blocks right of column p
+        if (p == 1) update(wave == 1 ? 2 : 3, wave == 3 ? 3 : 2, 0);
+        if (p == 2 && wave == 1) update(3, 3, 1);
+        if (p == 2 && wave == 2) chol_invert16(T, 0, lane);
+        work(p);
         __syncthreads();
         if (p < 3) {
             if (wave > p) update(wave, p + 1, p);
             __syncthreads();
         }
     }
-    double *linv = F.linv + (int64_t)w * CHOL_NB * CHOL_NB;
-    invert(wave);
-    if (wave == 3) {
-        // log-det partial: one log per lane, then a fixed butterfly in double-double
-        dd_t sl = {lane < nbj ? log(S[lane][lane]) : 0.0, 0.0};
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) {
-            const dd_t o = {__shfl_xor(sl.hi, off), __shfl_xor(sl.lo, off)};
-            sl = dd_add(sl, o);
-        }
-        if (lane == 0) {
-            double *part = F.ldpart + ((int64_t)w * F.nsteps + step) * 2;
-            part[0] = sl.hi;
-            part[1] = sl.lo;
-        }
-    }
-    if (F.keep_l11) {
-        // the factored block back into Pi (lower triangle and diagonal); no
-        // other work item reads this diagonal block
-        for (int r = wave; r < nbj; r += 4)
-            if (lane <= r) A[(int64_t)(j0 + r) * N + j0 + lane] = S[r][lane];
-    }
-    __syncthreads();
-    // block column `wave` of L11^{-1}; x[k] holds X(k, wave) as l16 = column,
-    // g4 + 4 r = row, which is also the B operand of step r
-    d4_t x[4];
+}
+
+// Block column `wave` of L11^{-1} on MFMA from the inverses of the diagonal blocks, X(i, j)
+// = -X(i, i) sum_k L(i, k) X(k, j); x[k] holds X(k, wave) as l16 = column, g4 + 4 r = row,
+// which is also the B operand of step r, so the column stays in registers.
+__device__ __forceinline__ void chol_inverse64(const CholLds &T, int wave, int lane, d4_t (&x)[4]) {
+    const int l16 = lane & 15, g4 = lane >> 4;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         x[i] = (d4_t){0.0, 0.0, 0.0, 0.0};
         if (i == wave) {
 #pragma unroll
-            for (int r = 0; r < 4; ++r) x[i][r] = Xd[i][g4 + 4 * r][l16];
+            for (int r = 0; r < 4; ++r) x[i][r] = T.Xd[i][g4 + 4 * r][l16];
         } else if (i > wave) {
             d4_t t = (d4_t){0.0, 0.0, 0.0, 0.0};
 #pragma unroll
@@ -747,27 +742,272 @@ __global__ __launch_bounds__(256) void k_potrf_diag(const FragDev *__restrict__ 
                 if (k >= wave)
 #pragma unroll
                     for (int s = 0; s < 4; ++s)
-                        t = __builtin_amdgcn_mfma_f64_16x16x4f64(S[16 * i + l16][16 * k + 4 * s + g4],
-                                                                 x[k][s], t, 0, 0, 0);
+                        t = __builtin_amdgcn_mfma_f64_16x16x4f64(
+                            T.S[16 * i + l16][16 * k + 4 * s + g4], x[k][s], t, 0, 0, 0);
 #pragma unroll
             for (int s = 0; s < 4; ++s)
-                x[i] = __builtin_amdgcn_mfma_f64_16x16x4f64(-Xd[i][l16][4 * s + g4], t[s], x[i], 0,
+                x[i] = __builtin_amdgcn_mfma_f64_16x16x4f64(-T.Xd[i][l16][4 * s + g4], t[s], x[i], 0,
                                                             0, 0);
         }
+    }
+}
+
+// log-det partial of the block: one log per lane, then a fixed butterfly in double-double
+__device__ __forceinline__ void chol_logdet(const CholLds &T, const FragDev &F, int w, int step,
+                                            int nbj, int lane) {
+    dd_t sl = {lane < nbj ? log(T.S[lane][lane]) : 0.0, 0.0};
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+        const dd_t o = {__shfl_xor(sl.hi, off), __shfl_xor(sl.lo, off)};
+        sl = dd_add(sl, o);
+    }
+    if (lane == 0) {
+        double *part = F.ldpart + ((int64_t)w * F.nsteps + step) * 2;
+        part[0] = sl.hi;
+        part[1] = sl.lo;
+    }
+}
+
+// Diagonal block of step `step` of matrix w, one work-group per matrix: linv, log-det
+// partial, status, optional L11 write-back.
+__global__ __launch_bounds__(256) void k_potrf_diag(const FragDev *__restrict__ fr,
+                                                   const int64_t *__restrict__ pre, int nfrag,
+                                                   int step) {
+    __shared__ __attribute__((aligned(16))) CholLds T;
+    __shared__ int64_t s_pre[FIND_LDS_MAX + 1];
+    const int64_t b = blockIdx.x;
+    const int f = find_frag_lds(pre, nfrag, b, s_pre);
+    const int w = (int)(b - (nfrag <= FIND_LDS_MAX ? s_pre[f] : pre[f]));
+    const FragDev &F = fr[f];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int N = F.N;
+    const int j0 = step * CHOL_NB;
+    const int nbj = min(CHOL_NB, N - j0);
+    double *A = F.Pi + (int64_t)w * N * N;
+    chol_load64(T, (const gdouble_t *)A, N, j0, nbj, wave, lane);
+    __syncthreads();
+    bool bad = false;
+    if (wave == 0)
+        bad = chol_panels(T, lane);
+    else
+        chol_blocks(T, wave, lane, [](int) {});
+    if (wave == 3) chol_logdet(T, F, w, step, nbj, lane);
+    if (F.keep_l11) {
+        // the factored block back into Pi (lower triangle and diagonal); no
+        // other work item reads this diagonal block
+        for (int r = wave; r < nbj; r += 4)
+            if (lane <= r) A[(int64_t)(j0 + r) * N + j0 + lane] = T.S[r][lane];
+    }
+    d4_t x[4];
+    chol_inverse64(T, wave, lane, x);
+    double *linv = F.linv + (int64_t)w * CHOL_NB * CHOL_NB;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
 #pragma unroll
         for (int r = 0; r < 4; ++r)
-            linv[(16 * i + g4 + 4 * r) * CHOL_NB + 16 * wave + l16] = x[i][r];
-    }
+            linv[(16 * i + (lane >> 4) + 4 * r) * CHOL_NB + 16 * wave + (lane & 15)] = x[i][r];
     if (threadIdx.x == 0 && bad) F.status[w] = 1;
 }
 
-int launch_potrf_diag(brpa_ctx *ctx, const FragDev *fr, const int64_t *pre, int nfrag,
-                      int64_t total, int step) {
-    if (total <= 0) return BRPA_OK;
-    hipLaunchKernelGGL(k_potrf_diag, dim3(grid1(total)), dim3(256), 0, ctx->stream, fr, pre, nfrag,
-                       step);
-    LAUNCH_CHECK(ctx);
-    return BRPA_OK;
+// One step of the Cholesky in one launch, for launches of few matrices: work-group (w, r)
+// takes the 64 rows from j0 + 64 r of the step's 64 columns.  Every one factors the
+// diagonal block itself (wave 0, bound by latency, on CUs that would be idle); meanwhile
+// waves 1-3 apply the outer panel's earlier columns to their rows (left-looking, rank 64
+// s_in, operands straight from L2).  Then L21 = B L11^{-T}, and the work-groups
+// within the outer panel bring their own diagonal block up to date, so that the
+// next step finds it complete.
+// 14 us for the first step of an outer panel, 18 us for the fourth (k_potrf_diag, k_trsm
+// and k_chol_strip: 37 to 51 us at N = 400).
+// r = 0 writes the log-det partial and the status.  No work-group may see a half-factored
+// block, so with keep_l11 it leaves L11 in linv and copies it into Pi in the next
+// step (pend: the previous step did so); the matrix's last step writes it at once.
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_chol_step(
+    const FragDev *__restrict__ fr, const int64_t *__restrict__ pre, int nfrag, int step, int pend) {
+    __shared__ __attribute__((aligned(16))) CholLds T;
+    // B, and before it the waves' own stages of 96 rows x 16 columns
+    __shared__ __attribute__((aligned(16))) double sm[3 * 96 * 16];
+    static_assert(CHOL_NB * CH_LP <= 3 * 96 * 16, "B fits");
+    double(*sB)[CH_LP] = reinterpret_cast<double(*)[CH_LP]>(sm);
+    const int64_t b = blockIdx.x;
+    const int f = __builtin_amdgcn_readfirstlane(find_frag(pre, nfrag, b));
+    const FragDev &F = fr[f];
+    const int N = F.N;
+    const int j0 = step * CHOL_NB;
+    const int nrb = (N - j0 + CHOL_NB - 1) / CHOL_NB;
+    const int64_t lb = b - pre[f];
+    const int w = __builtin_amdgcn_readfirstlane((int)(lb / nrb));
+    const int rb = __builtin_amdgcn_readfirstlane((int)(lb - (int64_t)w * nrb));
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int l16 = lane & 15, g4 = lane >> 4;
+    const int nbj = min(CHOL_NB, N - j0);
+    const int s_in = step % CHOL_OUTER, kbase = j0 - s_in * CHOL_NB;
+    double *A = F.Pi + (int64_t)w * N * N;
+    const gdouble_t *G = (const gdouble_t *)A;
+    gdouble_mut_t *GM = (gdouble_mut_t *)A;
+    double *linv = F.linv + (int64_t)w * CHOL_NB * CHOL_NB;
+    chol_load64(T, G, N, j0, nbj, wave, lane);
+    if (rb == 0) {
+        if (pend && F.keep_l11)
+            for (int r = wave; r < CHOL_NB; r += 4)
+                if (lane <= r) GM[(int64_t)(j0 - CHOL_NB + r) * N + j0 - CHOL_NB + lane] =
+                    linv[r * CHOL_NB + lane];
+        __syncthreads();
+        bool bad = false;
+        if (wave == 0)
+            bad = chol_panels(T, lane);
+        else
+            chol_blocks(T, wave, lane, [](int) {});
+        if (wave == 3) chol_logdet(T, F, w, step, nbj, lane);
+        if (F.keep_l11) {
+            const bool last = nrb == 1;
+            for (int r = wave; r < nbj; r += 4)
+                if (lane <= r) {
+                    if (last)
+                        GM[(int64_t)(j0 + r) * N + j0 + lane] = T.S[r][lane];
+                    else
+                        linv[r * CHOL_NB + lane] = T.S[r][lane];
+                }
+        }
+        if (threadIdx.x == 0 && bad) F.status[w] = 1;
+        return;
+    }
+    const int R0 = j0 + CHOL_NB * rb;
+    if (wave == 0) {
+        __syncthreads();
+        chol_panels(T, lane);
+    } else {
+        // Waves 1-3, v = wave - 1: block row v of B and the blocks (3, v) and, for the last
+        // wave, (3, 3); acc = sum P_r P_d^T - A
+        const int v = wave - 1;
+        d4_t acc[6];
+        auto brow = [&](int q) { return q < 4 ? v : 3; };
+        auto bcol = [&](int q) { return q < 4 ? q : (q == 4 ? v : 3); };
+        const int nq = wave == 3 ? 6 : 5;
+#pragma unroll
+        for (int q = 0; q < 6; ++q)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int row = R0 + 16 * brow(q) + g4 + 4 * r;
+                acc[q][r] = -G[(int64_t)min(row, N - 1) * N + j0 + 16 * bcol(q) + l16];
+            }
+        // 16 columns of the outer panel, rows of blocks v and 3 of the work-group and of the
+        // diagonal block's four: four rows per load, then through LDS (k pairs swizzled as in
+        // gemm_tile.h), the wave's own rows only, so without a barrier.  Straight into the
+        // MFMA layout, 16 rows x 32 bytes per load, 4500 cycles per 16 columns instead
+        // of 3000.
+        double *st = sm + 96 * 16 * v;
+        double x[6][4];
+        uint32_t roff[2][4];
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                roff[h][q] = (uint32_t)min((h == 0 ? 16 * v : 48) + 4 * q + g4, N - 1 - R0) * (uint32_t)N + l16;
+        auto fetch = [&](int g) {
+            const gdouble_t *pr = G + (int64_t)R0 * N + kbase + 16 * g;
+            const gdouble_t *pd = G + (int64_t)j0 * N + kbase + 16 * g;
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) x[h][q] = pr[roff[h][q]];
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    x[2 + i][q] = pd[(int64_t)(16 * i + 4 * q) * N + (uint32_t)(g4 * N + l16)];
+        };
+        if (s_in > 0) fetch(0);
+        __syncthreads();
+        chol_blocks(T, wave, lane, [&](int p) {
+            for (int g = p * s_in; g < (p + 1) * s_in; ++g) {
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+                for (int i = 0; i < 6; ++i)
+#pragma unroll
+                    for (int q = 0; q < 4; ++q)
+                        st[(16 * i + 4 * q + g4) * 16 + 2 * ((l16 >> 1) ^ (2 * q + (g4 >> 1))) + (l16 & 1)] =
+                            x[i][q];
+                fetch(min(g + 1, 4 * s_in - 1));
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                auto frag = [&](int i, int h) {
+                    return *reinterpret_cast<const d2v_t *>(
+                        &st[(16 * i + l16) * 16 + 2 * ((2 * g4 + h) ^ (l16 >> 1))]);
+                };
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    d2v_t fr[6];
+#pragma unroll
+                    for (int i = 0; i < 6; ++i) fr[i] = frag(i, h);
+                    const d2v_t dv = frag(2 + v, h);
+#pragma unroll
+                    for (int k = 0; k < 2; ++k) {
+#pragma unroll
+                        for (int q = 0; q < 4; ++q)
+                            acc[q] = __builtin_amdgcn_mfma_f64_16x16x4f64(fr[0][k], fr[2 + q][k], acc[q], 0, 0, 0);
+                        acc[4] = __builtin_amdgcn_mfma_f64_16x16x4f64(fr[1][k], dv[k], acc[4], 0, 0, 0);
+                        if (nq == 6)
+                            acc[5] = __builtin_amdgcn_mfma_f64_16x16x4f64(fr[1][k], fr[5][k], acc[5], 0, 0, 0);
+                    }
+                }
+            }
+        });
+#pragma unroll
+        for (int q = 0; q < 6; ++q)
+            if (q < nq)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) sB[16 * brow(q) + g4 + 4 * r][16 * bcol(q) + l16] = -acc[q][r];
+    }
+    __syncthreads();
+    // Block row `wave` of L21, transposed: X_c = L(c, c)^{-1} (B_c^T - sum_{k<c} L(c, k) X_k),
+    // X_k as l16 = row, g4 + 4 r = column, which is also the B operand of step r.
+    // 3100 cycles; by way of the whole L11^{-1} 7900.
+    d4_t l21[4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+        d4_t t;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) t[r] = sB[16 * wave + l16][16 * c + g4 + 4 * r];
+#pragma unroll
+        for (int k = 0; k < c; ++k)
+#pragma unroll
+            for (int s = 0; s < 4; ++s)
+                t = __builtin_amdgcn_mfma_f64_16x16x4f64(-T.S[16 * c + l16][16 * k + 4 * s + g4],
+                                                         l21[k][s], t, 0, 0, 0);
+        l21[c] = (d4_t){0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+            l21[c] = __builtin_amdgcn_mfma_f64_16x16x4f64(T.Xd[c][l16][4 * s + g4], t[s], l21[c], 0, 0, 0);
+    }
+    // through the wave's own rows of B to whole rows
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) sB[16 * wave + l16][16 * c + g4 + 4 * r] = l21[c][r];
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+        const int row = R0 + 16 * wave + r;
+        if (row < N) GM[(int64_t)row * N + j0 + lane] = sB[16 * wave + r][lane];
+    }
+    if (rb > CHOL_OUTER - 1 - s_in) return;
+    // the work-group's own diagonal block -= L21 L21^T (lower blocks)
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        if (j > wave) break;
+        d4_t t = (d4_t){0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int s = 0; s < 16; ++s)
+            t = __builtin_amdgcn_mfma_f64_16x16x4f64(sB[16 * wave + l16][4 * s + g4],
+                                                     sB[16 * j + l16][4 * s + g4], t, 0, 0, 0);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int row = R0 + 16 * wave + g4 + 4 * r, col = R0 + 16 * j + l16;
+            if (row < N && col <= row) GM[(int64_t)row * N + col] -= t[r];
+        }
+    }
 }
 
 __global__ __launch_bounds__(256) void k_trsm(const FragDev *__restrict__ fr,
@@ -784,41 +1024,32 @@ __global__ __launch_bounds__(256) void k_trsm(const FragDev *__restrict__ fr,
     trsm_body<256>(F, w, step, r, sB, sL, threadIdx.x);
 }
 
-int launch_trsm(brpa_ctx *ctx, const FragDev *fr, const int64_t *pre, int nfrag, int64_t total,
-                int step) {
-    if (total <= 0) return BRPA_OK;
-    hipLaunchKernelGGL(k_trsm, dim3(grid1(total)), dim3(256), 0, ctx->stream, fr, pre, nfrag, step);
-    LAUNCH_CHECK(ctx);
-    return BRPA_OK;
-}
-
-constexpr int UPD_T = 128;   // trailing-update super-tile edge
+// Trailing updates.  Outer panels of CHOL_OUTER steps (256 columns): step s of an outer
+// panel (s = step % CHOL_OUTER) updates, for s < CHOL_OUTER - 1, only the next
+// 64-column strip (rows >= t0 = j0 + 64, columns t0 .. t0+63) with the panels of steps
+// step-s .. step (rank 64 (s+1): the strip has seen no panel of this outer panel yet;
+// k_chol_strip); the last step updates the rest of the trailing matrix with all
+// CHOL_OUTER panels (rank 256; k_chol_rest), so A22 is read and written once per outer
+// panel.
+constexpr int UPD_T = 128;   // strip rows per work-group
+constexpr int REST_T = 64;   // tile edge of the rest
 constexpr int UPD_KH = 16;   // panel columns per LDS phase
 
-// Trailing update of one 128 x 128 super-tile (TI >= TJ in 128-row units of the
-// trailing matrix that starts at t0 = j0 + 64): C -= P_i P_j^T over the panel
-// columns of the current outer panel (see below), C preloaded into the
-// accumulators.  Four waves of 64 x 64 (two work-groups per CU, two waves per
-// SIMD); waves entirely above the diagonal of a diagonal super-tile skip their
-// products; element writes keep col <= row.  The panels pass through LDS in
-// phases of 16 columns as [row][k] (pitch 18 doubles), double-buffered with one
-// barrier per phase; every thread moves pairs of consecutive columns (one
-// ds_write_b128), and in a phase lane group l/16 supplies the k values
-// 4 (l/16) .. +3 of its row to the four MFMA steps (a permutation of the
-// phase's k, the same for both operands), two ds_read_b128 per 16-row block.
-// The MFMA takes the P_i fragment first, so the accumulator columns run along
-// the lanes and the row-major C is read and written coalesced.
-template <bool STRIP>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_chol_update(
+// A 128 x 64 piece of the strip, the four waves as 2 x 2 blocks of 64 x 32, C preloaded
+// into the accumulators.  The panels pass through LDS in phases of 16 columns as
+// [row][k] (pitch 18 doubles), double-buffered with one barrier per phase; every thread
+// moves pairs of consecutive columns (one ds_write_b128), and in a phase lane group
+// l/16 supplies the k values 4 (l/16) .. +3 of its row to the four MFMA steps (a
+// permutation of the phase's k, the same for both operands), two ds_read_b128 per
+// 16-row block.  The MFMA takes the P_i fragment first, so the accumulator columns run
+// along the lanes and the row-major C is read and written coalesced.
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_chol_strip(
     const FragDev *__restrict__ fr, const int64_t *__restrict__ pre, int nfrag, int step) {
-    // STRIP: the 64-column strip of a step inside an outer panel; the 128 x 64
-    // tile is split over the four waves as 2 x 2 blocks of 64 x 32.  Otherwise
-    // 128 x 128 tiles, four waves of 64 x 64.
-    constexpr int WC = STRIP ? 32 : 64;    // columns per wave
+    constexpr int WC = 32;                 // columns per wave
     constexpr int NJ = WC / 16;            // 16-column MFMA blocks per wave
     constexpr int KPU = UPD_KH + 2;
     __shared__ __attribute__((aligned(16))) double sI[2][UPD_T * KPU];
-    __shared__ __attribute__((aligned(16))) double sJ[2][UPD_T * KPU];
+    __shared__ __attribute__((aligned(16))) double sJ[2][CHOL_NB * KPU];
     __shared__ int64_t s_pre[FIND_LDS_MAX + 1];
     int64_t b = blockIdx.x;
     int f = find_frag_lds(pre, nfrag, b, s_pre);
@@ -827,42 +1058,24 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     const int j0 = step * CHOL_NB;
     const int t0 = j0 + CHOL_NB;
     const int nt = (N - t0 + UPD_T - 1) / UPD_T;
-    // Outer panels of CHOL_OUTER steps (256 columns): step s of an outer panel
-    // (s = step % CHOL_OUTER) updates, for s < CHOL_OUTER - 1, only the next
-    // 64-column strip (rows >= t0, columns t0 .. t0+63) with the panels of
-    // steps step-s .. step (rank 64 (s+1): the strip has seen no panel of this
-    // outer panel yet); the last step updates the rest of the trailing matrix
-    // with all CHOL_OUTER panels (rank 256), so A22 is read and written once
-    // per outer panel.  Work items: nt row tiles (strip) or nt(nt+1)/2 tile
-    // pairs (rest).
     const int s_in = step % CHOL_OUTER;
-    constexpr bool strip = STRIP;
     const int kbase = j0 - s_in * CHOL_NB;    // first panel column
     const int nph = (s_in + 1) * CHOL_NB / UPD_KH;
-    const int colmax = strip ? min(N, t0 + CHOL_NB) : N;   // C columns < colmax
-    const int nitems = strip ? nt : nt * (nt + 1) / 2;
+    const int colmax = min(N, t0 + CHOL_NB);   // C columns < colmax
     int64_t lb = b - (nfrag <= FIND_LDS_MAX ? s_pre[f] : pre[f]);
-    const int w = (int)(lb / nitems), item = (int)(lb - (int64_t)w * nitems);
-    int ti, tj;
-    if (strip) {
-        ti = item;
-        tj = 0;
-    } else {
-        tri_decode(item, ti, tj);
-    }
+    const int w = (int)(lb / nt), ti = (int)(lb - (int64_t)w * nt);
     double *A = F.Pi + (int64_t)w * N * N;
     const gdouble_t *G = (const gdouble_t *)A;
-    const int Ri = t0 + UPD_T * ti, Rj = t0 + UPD_T * tj;
+    const int Ri = t0 + UPD_T * ti, Rj = t0;
     const int tid = threadIdx.x;
     const int wave = tid >> 6, lane = tid & 63;
     const int wm = wave >> 1, wn = wave & 1;   // rows 64*wm.., cols WC*wn..
     const int r0 = 64 * wm, c0 = WC * wn;
-    const bool active = !(ti == tj && c0 > r0 + 63) && Ri + r0 < N && Rj + c0 < colmax;
+    const bool active = Ri + r0 < N && Rj + c0 < colmax;
 
-    // phase h (h < nph): rows Ri.. / Rj.. (128 each) x columns kbase + 16 h .. + 16
-    // (all < t0 <= N); pair q = tid + 256 u (u < 4): row q / 8, columns
-    // 2 (q % 8) + {0, 1}
-    d2v_t vi[4], vj[4];
+    // phase h (h < nph): rows Ri.. (128) / Rj.. (64) x columns kbase + 16 h .. + 16
+    // (all < t0 <= N); pair q = tid + 256 u: row q / 8, columns 2 (q % 8) + {0, 1}
+    d2v_t vi[4], vj[2];
     auto gload = [&](int h) {
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
@@ -870,12 +1083,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             const int r = q >> 3, col = kbase + UPD_KH * h + 2 * (q & 7);
             const bool oki = Ri + r < N, okj = Rj + r < N;
             const gdouble_t *pi = G + (oki ? (int64_t)(Ri + r) * N + col : 0);
-            const gdouble_t *pj = G + (okj ? (int64_t)(Rj + r) * N + col : 0);
-            const double i0 = pi[0], i1 = pi[1], ja = pj[0], jb = pj[1];
+            const double i0 = pi[0], i1 = pi[1];
             vi[u].x = oki ? i0 : 0.0;
             vi[u].y = oki ? i1 : 0.0;
-            vj[u].x = okj ? ja : 0.0;
-            vj[u].y = okj ? jb : 0.0;
+            if (u < 2) {
+                const gdouble_t *pj = G + (okj ? (int64_t)(Rj + r) * N + col : 0);
+                const double ja = pj[0], jb = pj[1];
+                vj[u].x = okj ? ja : 0.0;
+                vj[u].y = okj ? jb : 0.0;
+            }
         }
     };
     auto lstore = [&](int buf) {
@@ -884,7 +1100,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             const int q = tid + 256 * u;
             const int o = (q >> 3) * KPU + 2 * (q & 7);
             *reinterpret_cast<d2v_t *>(&sI[buf][o]) = vi[u];
-            *reinterpret_cast<d2v_t *>(&sJ[buf][o]) = vj[u];
+            if (u < 2) *reinterpret_cast<d2v_t *>(&sJ[buf][o]) = vj[u];
         }
     };
 
@@ -892,9 +1108,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     lstore(0);
     __syncthreads();
     if (nph > 1) gload(1);
-    // the C tile into the accumulators: D[q] = C(row = 16 i + lane/16 * 4 + q ...)
-    // in MFMA order, element (row r0 + 16 i + 4 (lane/16) + q, col c0 + 16 j + lane%16)
-    // (out-of-range / upper elements read A[0], then 0)
+    // the C tile into the accumulators: element (row r0 + 16 i + lane/16 + 4 q, col c0 +
+    // 16 j + lane%16) (out-of-range / upper elements read A[0], then 0)
     d4_t acc[4][NJ];
 #pragma unroll
     for (int i = 0; i < 4; ++i)
@@ -954,23 +1169,105 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             }
 }
 
-int64_t chol_upd_items(int64_t N, int64_t j) {
-    const int64_t t0 = (j + 1) * CHOL_NB;
-    if (N <= t0) return 0;
-    const int64_t t = (N - t0 + UPD_T - 1) / UPD_T;
-    return (j % CHOL_OUTER != CHOL_OUTER - 1) ? t : t * (t + 1) / 2;
+// Rank-256 update of the trailing matrix, one 64 x 64 tile (ti >= tj) per work-group:
+// C -= P_i P_j^T by the loop of k_gemm_f64 (both panels are rows of A, contiguous in
+// k), then one read and write of C's lower part.  Bound by the MFMA pipe where the
+// launch is large (2.1 ms at N = 1800, 24 frequencies, 24 fragments) and by the length of
+// one tile's loop where it is small.  Four work-groups per CU hide each other's C
+// pass, which the 128 x 128 tiles of two per CU did not.  Average launch: N = 400, 16 matrices
+// 21 us; N = 1800, 24 matrices 137 us; 24 x 24 of N up to 1800 706 us (128 x 128 tiles:
+// 54, 191, 935; register-staged 128 x 128 tiles with C preloaded: 50, 194, 890).
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) void k_chol_rest(
+    const FragDev *__restrict__ fr, const int64_t *__restrict__ pre, int nfrag, int step) {
+    constexpr int T = REST_T;
+    __shared__ __attribute__((aligned(16))) double sA[2 * gemm_lds<true>(T)];
+    __shared__ __attribute__((aligned(16))) double sB[2 * gemm_lds<true>(T)];
+    const int64_t b = blockIdx.x;
+    const int f = __builtin_amdgcn_readfirstlane(find_frag(pre, nfrag, b));
+    const FragDev &F = fr[f];
+    const int N = F.N;
+    const int t0 = (step + 1) * CHOL_NB, kbase = t0 - CHOL_OUTER * CHOL_NB;
+    const int nt = (N - t0 + T - 1) / T, nitems = nt * (nt + 1) / 2;
+    const int64_t lb = b - pre[f];
+    const int w = __builtin_amdgcn_readfirstlane((int)(lb / nitems));
+    int ti, tj;
+    tri_decode((int)(lb - (int64_t)w * nitems), ti, tj);
+    const int Ri = t0 + T * __builtin_amdgcn_readfirstlane(ti);
+    const int Rj = t0 + T * __builtin_amdgcn_readfirstlane(tj);
+    double *A = F.Pi + (int64_t)w * N * N;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    // the wave's block: columns Rj + T/2 wm .., rows Ri + T/2 wn ..
+    const int c0 = Rj + T / 2 * (wave >> 1), r0 = Ri + T / 2 * (wave & 1);
+    const bool active = r0 < N && c0 < N && c0 < r0 + T / 2;
+    constexpr int NB = T / 32;
+    d4_t acc[NB][NB];
+#pragma unroll
+    for (int i = 0; i < NB; ++i)
+#pragma unroll
+        for (int j = 0; j < NB; ++j) acc[i][j] = (d4_t){0.0, 0.0, 0.0, 0.0};
+    if (N % 2 == 0 && (reinterpret_cast<uintptr_t>(A) & 15) == 0)
+        gemm_tile<true, true, 16, T>(acc, A, N, Rj, N, A, N, Ri, N, kbase, t0, false, active, sA, sB);
+    else
+        gemm_tile<true, true, 4, T>(acc, A, N, Rj, N, A, N, Ri, N, kbase, t0, false, active, sA, sB);
+    if (!active) return;
+    gdouble_mut_t *C = (gdouble_mut_t *)A;
+#pragma unroll
+    for (int j = 0; j < NB; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int row = r0 + 16 * j + (lane >> 4) + 4 * r;
+#pragma unroll
+            for (int i = 0; i < NB; ++i) {
+                const int col = c0 + 16 * i + (lane & 15);
+                if (row < N && col <= row) C[(int64_t)row * N + col] -= acc[i][j][r];
+            }
+        }
 }
 
-int launch_chol_update(brpa_ctx *ctx, const FragDev *fr, const int64_t *pre, int nfrag,
-                       int64_t total, int step) {
-    if (total <= 0) return BRPA_OK;
-    if (step % CHOL_OUTER != CHOL_OUTER - 1)
-        hipLaunchKernelGGL(k_chol_update<true>, dim3(grid1(total)), dim3(256), 0, ctx->stream, fr,
-                           pre, nfrag, step);
-    else
-        hipLaunchKernelGGL(k_chol_update<false>, dim3(grid1(total)), dim3(256), 0, ctx->stream, fr,
-                           pre, nfrag, step);
-    LAUNCH_CHECK(ctx);
+int64_t chol_items(int list, int64_t N, int64_t F, int64_t j) {
+    const int64_t j0 = j * CHOL_NB, t0 = j0 + CHOL_NB;
+    const bool rest = j % CHOL_OUTER == CHOL_OUTER - 1;
+    auto tiles = [&](int64_t t) { return N > t0 ? (N - t0 + t - 1) / t : 0; };
+    switch (list) {
+    case CHOL_DIAG: return N > j0 ? F : 0;
+    case CHOL_TRSM: return F * tiles(CHOL_NB);
+    case CHOL_STRIP: return rest ? 0 : F * tiles(UPD_T);
+    case CHOL_REST: return rest ? F * tiles(REST_T) * (tiles(REST_T) + 1) / 2 : 0;
+    default: return N > j0 ? F * (1 + tiles(CHOL_NB)) : 0;   // CHOL_STEP
+    }
+}
+
+int launch_cholesky(brpa_ctx *ctx, const FragDev *fr, int nfrag, int nsteps, const int64_t *d_pre,
+                    const int64_t *h_pre) {
+    const int64_t ncu = ctx->ncu > 0 ? ctx->ncu : 256;
+    bool fused = false, pend = false;
+    for (int j = 0; j < nsteps; ++j) {
+        auto at = [&](int list) { return ((int64_t)list * nsteps + j) * (nfrag + 1); };
+        auto total = [&](int list) { return h_pre[at(list) + nfrag]; };
+        auto launch = [&](auto kernel, int list, auto... extra) -> int {
+            if (total(list) <= 0) return BRPA_OK;
+            hipLaunchKernelGGL(kernel, dim3(grid1(total(list))), dim3(256), 0, ctx->stream, fr,
+                               d_pre + at(list), nfrag, j, extra...);
+            LAUNCH_CHECK(ctx);
+            return BRPA_OK;
+        };
+        // From the first outer panel on whose steps have at most four work-groups per CU (two
+        // rounds of the resident ones) one launch per step.  ERPA of N = 400 / 16 matrices,
+        // N = 1053 / 16 and N = 1800 / 24: 411, 2762 and 7471 us with three launches throughout,
+        // 333, 2524 and 7254 us with a line at two per CU, 333, 2526 and 7163 us at four,
+        // no different at eight and sixteen.
+        if (j % CHOL_OUTER == 0 && !fused) fused = total(CHOL_STEP) <= 4 * ncu;
+        if (fused) {
+            BRPA_TRY(launch(k_chol_step, CHOL_STEP, pend ? 1 : 0));
+            pend = true;
+        } else {
+            BRPA_TRY(launch(k_potrf_diag, CHOL_DIAG));
+            BRPA_TRY(launch(k_trsm, CHOL_TRSM));
+            BRPA_TRY(launch(k_chol_strip, CHOL_STRIP));
+        }
+        BRPA_TRY(launch(k_chol_rest, CHOL_REST));
+    }
     return BRPA_OK;
 }
 
