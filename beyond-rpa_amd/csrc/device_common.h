@@ -22,6 +22,16 @@ __device__ __forceinline__ int find_frag(const int64_t *__restrict__ pre, int nf
     return lo;
 }
 
+// Block b of a grid in chunks of 32 consecutive blocks per XCD (blocks go to the eight XCDs
+// in turn): tiles that share panels find them in one XCD's L2.
+constexpr int XCD_CHUNK = 32;
+__device__ __forceinline__ int64_t xcd_chunks(int64_t b, int64_t nblocks) {
+    constexpr int64_t R = 8 * XCD_CHUNK;
+    if (b >= nblocks / R * R) return b;
+    const int64_t x = b % 8, r = b / 8;
+    return (r / XCD_CHUNK * 8 + x) * XCD_CHUNK + r % XCD_CHUNK;
+}
+
 // The same search on a copy of pre staged in LDS (one parallel load instead of
 // a chain of dependent global loads; matters for small work-groups).  Every
 // thread of the work-group must call it (it synchronises).

@@ -110,11 +110,11 @@ size_t frag_bytes(const HostFrag &h, int precision) {
     size_t b = 8 * (F * K + F * N * N + 4 * F * N + 64 * F + F * CHOL_NB * CHOL_NB) + 8 * K * N;
     if (precision == BRPA_SPLIT_BF16) {
         size_t kpad = cdiv(K, SPLIT_KB) * SPLIT_KB;
-        b += 2 * F * NSLICE * N * kpad + (4 + 16) * F * (kpad / SPLIT_KB) * N;
+        b += 2 * F * NSLICE * N * kpad + SL_PAD + (4 + 16) * F * (kpad / SPLIT_KB) * N;
     }
     if (precision == BRPA_SPLIT_I8) {
         size_t kpad = cdiv(K, I8_KB) * I8_KB;
-        b += F * NSLICE * N * kpad + 8 * F * N + 8 * F * K + 24 * cdiv(K, CS_ROWS) * F * N;
+        b += F * NSLICE * N * kpad + SL_PAD + 8 * F * N + 8 * F * K + 24 * cdiv(K, CS_ROWS) * F * N;
     }
     return b;
 }
@@ -222,14 +222,14 @@ int run_chunk(brpa_ctx *ctx, int precision, const std::vector<HostFrag> &fr, dou
             d.Kpad = (int)(cdiv(K, SPLIT_KB) * SPLIT_KB);
             d.nblk = d.Kpad / SPLIT_KB;
             if (precision == BRPA_SPLIT_BF16) {
-                d.sl = ar.take<uint16_t>((size_t)F * NSLICE * N * d.Kpad);
+                d.sl = ar.take<uint16_t>((size_t)F * NSLICE * N * d.Kpad + SL_PAD / 2);
                 d.scale = ar.take<float>((size_t)F * d.nblk * N);
                 d.dpart = ar.take<double>((size_t)F * d.nblk * N * 2);
             }
             d.Kpad8 = (int)(cdiv(K, I8_KB) * I8_KB);
             if (precision == BRPA_SPLIT_I8) {
                 d.sdtab = ar.take<double>((size_t)F * K);
-                d.sl8 = ar.take<int8_t>((size_t)F * NSLICE * N * d.Kpad8);
+                d.sl8 = ar.take<int8_t>((size_t)F * NSLICE * N * d.Kpad8 + SL_PAD);
                 d.scale8 = ar.take<double>((size_t)F * N);
                 d.dpart = ar.take<double>((size_t)cdiv(K, CS_ROWS) * F * N * 3);
             }

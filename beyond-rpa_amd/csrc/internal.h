@@ -186,7 +186,7 @@ struct FragDev {
     int nocc, nvir;
     const double *eocc, *evir, *freqs;   // device copies
     // split-BF16 slices (only when precision == BRPA_SPLIT_BF16)
-    uint16_t *sl;            // F x NSLICE x N x Kpad, per column P the Kpad rows contiguous
+    uint16_t *sl;            // F x NSLICE x Kpad/32 x N x 32, per column P 32 rows contiguous
     float *scale;            // F x nblk x N, block scale 2^(e-8)
     int Kpad, nblk;
     // split-int8 slices (only when precision == BRPA_SPLIT_I8)
@@ -206,6 +206,7 @@ constexpr int CHOL_OUTER = 4; // Cholesky steps per outer panel of the trailing 
 constexpr int SYRK_T = 64;    // FP64 SYRK tile
 constexpr int SPLIT_KB = 128; // split-BF16 exactness block (rows per scale)
 constexpr int NSLICE = 4;     // bf16 (or int8) slices per FP64 value in the split forms
+constexpr int SL_PAD = 128 * 64;  // bytes a product may read past its slices: 64 of each column of a tile
 constexpr int I8_KB = 128;    // split-int8: rows per split work-group (Kpad8 is a multiple)
 constexpr int CS_ROWS = 512;   // split-int8: rows per work-group of the column pass
 constexpr int I8_KMAX = 65536;// split-int8: largest K with exact int32 level sums

@@ -441,23 +441,20 @@ __global__ __launch_bounds__(128) void k_syrk_i8_64(
 // over fragments of different K (one contiguous range of the grid per XCD did not: 1.4
 // times slower on the batch).
 //
-// Bound by the int8 matrix rate and the LDS reads (24 KB per wave and stage).  Measured
-// at K = 10800, N = 1800, 24 frequencies: 4.19 ms with xcd, 4.43 without (200 and 190
-// TFLOP/s FP64-equivalent; 5.97 with one LDS read or wait ahead of each group of
-// MFMAs); 32 fragments of the batch shapes: 16.7 and 17.5 ms (23.8).
-constexpr int XCD_CHUNK = 32;
-__device__ __forceinline__ int64_t xcd_chunks(int64_t b, int64_t nblocks) {
-    constexpr int64_t R = 8 * XCD_CHUNK;
-    if (b >= nblocks / R * R) return b;
-    const int64_t x = b % 8, r = b / 8;
-    return (r / XCD_CHUNK * 8 + x) * XCD_CHUNK + r % XCD_CHUNK;
-}
-
+// Bound by the int8 matrix rate at the clock that it runs at (1.8 GHz under this load),
+// then the LDS reads (24 KB per wave and stage).  Measured at K = 10800, N = 1800, 24
+// frequencies: 3.80 ms (221 TFLOP/s FP64-equivalent; 4.19 ms with both stages in one
+// array, where the compiler made the first read after the loads wait for them, 4.43
+// without xcd, 5.97 with one LDS read or wait ahead of each group of MFMAs); 32
+// fragments of the batch shapes: 14.7 ms (16.5, 17.5, 23.8).  Loads of later stages into L2
+// ahead of their use made it no faster.
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_syrk_i8_128(
     const FragDev *__restrict__ fr, const int64_t *__restrict__ pre, int nfrag, int xcd) {
     constexpr int T = 128;
-    // [buffer][side][slice][column][slot] of 16-byte pieces
-    __shared__ __attribute__((aligned(16))) uint4 sbuf[2][2][NSLICE][T][4];
+    // [side][slice][column][slot] of 16-byte pieces.  Two arrays and not one with an
+    // index: the compiler then knows that a read of one does not wait for the loads into the
+    // other.
+    __shared__ __attribute__((aligned(16))) uint4 sb0[2][NSLICE][T][4], sb1[2][NSLICE][T][4];
     __shared__ int64_t s_pre[FIND_LDS_MAX + 1];
     const int64_t b = xcd ? xcd_chunks(blockIdx.x, gridDim.x) : (int64_t)blockIdx.x;
     const int f = find_frag_lds(pre, nfrag, b, s_pre);
@@ -478,24 +475,28 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     const int8_t *slw = F.sl8 + (int64_t)w * NSLICE * N * Kp;
 
     // A wave loads one slice of one side: 8 groups of 16 columns (1 KB per load; lane
-    // l lands in column l/4, slot l%4).  Columns past N repeat column N - 1: they only
-    // feed outputs that are never written.
+    // l lands in column l/4, slot l%4).  Columns past N are whatever follows (the
+    // allocation ends with SL_PAD spare bytes): they only feed outputs that are never
+    // written.
     const int side = wave >> 2, slice = wave & 3;
     const int lpiece = (lane & 3) ^ ((lane >> 4) & 3);
-    uint32_t goff[8];
-#pragma unroll
-    for (int g = 0; g < 8; ++g)
-        goff[g] = (uint32_t)min((side ? q0 : p0) + 16 * g + (lane >> 2), N - 1) * KS8 + 16u * lpiece;
-    const int8_t *base = slw + (int64_t)slice * N * Kp;
+    const uint32_t goff = (uint32_t)((side ? q0 : p0) + (lane >> 2)) * KS8 + 16u * lpiece;
+    const char *base = (const char *)(slw + (int64_t)slice * N * Kp);
     auto issue = [&](int buf, int st) {
 #if defined(__HIP_DEVICE_COMPILE__)
         typedef __attribute__((address_space(1))) const char gchar_t;
-        gchar_t *src = (gchar_t *)(base + (int64_t)st * KS8 * N);
+        // the load's constant offset counts for both addresses: four groups per base
 #pragma unroll
-        for (int g = 0; g < 8; ++g)
-            __builtin_amdgcn_global_load_lds(
-                (const __attribute__((address_space(1))) void *)(src + goff[g]),
-                (lds_void_t *)&sbuf[buf][side][slice][16 * g][0], 16, 0, 0);
+        for (int h = 0; h < 2; ++h) {
+            const char *src = base + ((int64_t)st * KS8 * N + 64 * KS8 * h);
+            asm("" : "+s"(src));   // a scalar base, the lane's offset in 32 bits
+            auto *from = (const __attribute__((address_space(1))) void *)((gchar_t *)src + goff);
+            auto *to = (lds_void_t *)(buf ? &sb1[side][slice][64 * h][0] : &sb0[side][slice][64 * h][0]);
+            __builtin_amdgcn_global_load_lds(from, to, 16, 0, 0);
+            __builtin_amdgcn_global_load_lds(from, to, 16, 1024, 0);
+            __builtin_amdgcn_global_load_lds(from, to, 16, 2048, 0);
+            __builtin_amdgcn_global_load_lds(from, to, 16, 3072, 0);
+        }
 #endif
     };
     const int nst = (int)(Kp / KS8);
@@ -513,12 +514,12 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     // slice s of the wave's 16-column groups of the p side (four) and the q side (two)
     const int fo = (lane & 15) * 4 + swz8(lane & 15, lane >> 4);
     auto fragp = [&](v4i_t (&v)[4], int buf, int s) {
-        const uint4 *L = &sbuf[buf][0][s][64 * wi][0];
+        const uint4 *L = buf ? &sb1[0][s][64 * wi][0] : &sb0[0][s][64 * wi][0];
 #pragma unroll
         for (int i = 0; i < 4; ++i) v[i] = __builtin_bit_cast(v4i_t, L[64 * i + fo]);
     };
     auto fragq = [&](v4i_t (&v)[2], int buf, int s) {
-        const uint4 *L = &sbuf[buf][1][s][32 * wj][0];
+        const uint4 *L = buf ? &sb1[1][s][32 * wj][0] : &sb0[1][s][32 * wj][0];
 #pragma unroll
         for (int j = 0; j < 2; ++j) v[j] = __builtin_bit_cast(v4i_t, L[64 * j + fo]);
     };
@@ -543,8 +544,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     fragq(b2, 0, 2);
     fragq(b3, 0, 3);
     // the last stages load and read stage nst - 1 again, unused
-    for (int st = 0; st < nst; ++st) {
-        const int buf = st & 1;
+    auto stage = [&](int buf, int st) {
         fragp(a1, buf, 1);
         fragp(a2, buf, 2);
         fragp(a3, buf, 3);
@@ -585,6 +585,10 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         __builtin_amdgcn_sched_group_barrier(0x8, 2, 1);
         __builtin_amdgcn_sched_group_barrier(0x100, 2, 1);
         __builtin_amdgcn_sched_barrier(0);
+    };
+    for (int st = 0; st < nst; st += 2) {   // Kpad8 is a multiple of 128: an even number
+        stage(0, st);
+        stage(1, st + 1);
     }
     __builtin_amdgcn_s_waitcnt(0);   // no load into LDS outlives the work-group
 
