@@ -28,9 +28,11 @@ template <bool KC, int V, int ROWS>
 struct DmaSrc {
     static_assert(KC || ROWS == 128, "rows-contiguous operands have 128-row tiles");
     static constexpr int NLOAD = V == 16 ? ROWS / 32 : ROWS / 8;   // loads per wave and stage
-    // per load; V = 4 rows-contiguous: per 32 rows
-    static constexpr int NOFF = !KC ? 4 : NLOAD;
+    // per load; V = 4 rows-contiguous: per 32 rows; V = 4 KC: only the lane's part, since 16
+    // offsets per operand and wave do not fit beside the accumulators
+    static constexpr int NOFF = !KC ? 4 : (V == 4 ? 1 : NLOAD);
     uint32_t off[NOFF];
+    int last;   // V = 4 KC: the last row of the operand, from the wave's first one
 };
 template <bool KC, int V, int ROWS>
 __device__ __forceinline__ DmaSrc<KC, V, ROWS> dma_offsets(int64_t ldx, int r0, int rows, int wave,
@@ -47,9 +49,8 @@ __device__ __forceinline__ DmaSrc<KC, V, ROWS> dma_offsets(int64_t ldx, int r0, 
             s.off[c] = 8u * ((uint32_t)(min(r0 + 2 * lane, rows - 2) - r0) +
                              (uint32_t)ldx * (uint32_t)(4 * wave + c));
         } else if (KC) {
-            const int row = ROWS / 4 * wave + 2 * c + (lane >> 5);
-            s.off[c] = 8u * ((uint32_t)ldx * (uint32_t)(min(r0 + row, rows - 1) - r0)) +
-                       4u * (((uint32_t)lane & 31u) ^ (4u * ((row >> 1) & 7)));
+            s.off[c] = 4u * ((uint32_t)lane & 31u);
+            s.last = rows - 1 - r0 - ROWS / 4 * wave;
         } else {
             s.off[c] = 8u * (uint32_t)(min(r0 + 32 * c + (lane >> 1), rows - 1) - r0) + 4u * (lane & 1);
         }
@@ -92,11 +93,20 @@ __device__ __forceinline__ void dma_stage(const char *base, const DmaSrc<KC, V, 
                 (lvoid_t *)(L + (KC ? (ROWS / 4 * wave + 8 * c) * GKB : (4 * wave + c) * DMA_KPR)), 16, 0,
                 0);
     } else if (KC) {
+        static_assert(!KC || V != 4 || (ROWS / 8) % 8 == 0, "a wave's swizzle starts at 0");
+        // rows 2c and 2c + 1 of the wave's; the offset is made here (volatile: not kept)
+        int last = src.last;
+        asm volatile("" : "+s"(last));
+        const uint32_t first = (uint32_t)(ROWS / 4 * wave), ld8 = 8u * (uint32_t)ldx;
+        const bool odd = threadIdx.x & 32;
 #pragma unroll
-        for (int c = 0; c < DmaSrc<KC, V, ROWS>::NLOAD; ++c)
-            __builtin_amdgcn_global_load_lds((gvoid_t *)(b + src.off[c]),
-                                             (lvoid_t *)(L + (ROWS / 4 * wave + 2 * c) * GKB), 4,
-                                             0, 0);
+        for (int c = 0; c < DmaSrc<KC, V, ROWS>::NLOAD; ++c) {
+            const uint32_t ra = ld8 * (first + (uint32_t)min(2 * c, last)),
+                           rb = ld8 * (first + (uint32_t)min(2 * c + 1, last));
+            const uint32_t off = (odd ? rb : ra) + (src.off[0] ^ (16u * (c & 7)));
+            __builtin_amdgcn_global_load_lds((gvoid_t *)(b + off),
+                                             (lvoid_t *)(L + (ROWS / 4 * wave + 2 * c) * GKB), 4, 0, 0);
+        }
     } else {
 #pragma unroll
         for (int c = 0; c < 16; ++c) {
@@ -125,7 +135,7 @@ __device__ __forceinline__ void dma_stage_tail(const double *__restrict__ X, int
 // (wm, wn) = (wave / 2, wave % 2) holds the ROWS/2 x ROWS/2 block (wm, wn), acc[i][j][r]
 // = element (16 i + lane % 16, 16 j + lane / 16 + 4 r) of it.  m, n: rows of the whole
 // operands (past them the last row repeats).  far: leading dimensions beyond 32-bit
-// offsets.  Waves with active false only stage.  sA, sB: two stages each
+// offsets.  Waves with active false only stage.  sA0/1, sB0/1: the two stages of each operand
 // (gemm_lds doubles per stage).
 //
 // The fragments of either half of a stage are read while the other half is
@@ -140,9 +150,9 @@ template <bool KCA, bool KCB, int V, int ROWS>
 __device__ __forceinline__ void gemm_tile(d4_t (&acc)[ROWS / 32][ROWS / 32],
                                           const double *__restrict__ A, int64_t lda, int m0, int m,
                                           const double *__restrict__ B, int64_t ldb, int n0, int n,
-                                          int kbeg, int kend, bool far, bool active, double *sA,
-                                          double *sB) {
-    constexpr int NB = ROWS / 32, SA = gemm_lds<KCA>(ROWS), SB = gemm_lds<KCB>(ROWS);
+                                          int kbeg, int kend, bool far, bool active, double *sA0,
+                                          double *sA1, double *sB0, double *sB1) {
+    constexpr int NB = ROWS / 32;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave >> 1, wn = wave & 1;
@@ -152,15 +162,15 @@ __device__ __forceinline__ void gemm_tile(d4_t (&acc)[ROWS / 32][ROWS / 32],
     const char *ba = dma_base<KCA>(A, lda, m0), *bb = dma_base<KCB>(B, ldb, n0);
     const int nfull = far ? 0 : (kend - kbeg) / GKB, ns = (kend - kbeg + GKB - 1) / GKB;
     auto stage = [&](int buf, int k0) {
-        dma_stage<KCA, V, ROWS>(ba, oa, lda, sA + buf * SA, wave, k0);
-        dma_stage<KCB, V, ROWS>(bb, ob, ldb, sB + buf * SB, wave, k0);
+        dma_stage<KCA, V, ROWS>(ba, oa, lda, buf ? sA1 : sA0, wave, k0);
+        dma_stage<KCB, V, ROWS>(bb, ob, ldb, buf ? sB1 : sB0, wave, k0);
     };
     auto put = [&](int buf, int q) {
         if (q < nfull) {
             stage(buf, kbeg + GKB * q);
         } else if (q < ns) {
-            dma_stage_tail<KCA, ROWS>(A, lda, m0, m, sA + buf * SA, tid, kbeg + GKB * q, kend);
-            dma_stage_tail<KCB, ROWS>(B, ldb, n0, n, sB + buf * SB, tid, kbeg + GKB * q, kend);
+            dma_stage_tail<KCA, ROWS>(A, lda, m0, m, buf ? sA1 : sA0, tid, kbeg + GKB * q, kend);
+            dma_stage_tail<KCB, ROWS>(B, ldb, n0, n, buf ? sB1 : sB0, tid, kbeg + GKB * q, kend);
         }
     };
     put(0, 0);
@@ -177,10 +187,10 @@ __device__ __forceinline__ void gemm_tile(d4_t (&acc)[ROWS / 32][ROWS / 32],
     auto frags = [&](d2_t (&a)[NB], d2_t (&b)[NB], int buf, int hh) {
 #pragma unroll
         for (int i = 0; i < NB; ++i)
-            a[i] = dma_frag<KCA>(sA + buf * SA, ROWS / 2 * wm + 16 * i + rl, g4, hh);
+            a[i] = dma_frag<KCA>(buf ? sA1 : sA0, ROWS / 2 * wm + 16 * i + rl, g4, hh);
 #pragma unroll
         for (int j = 0; j < NB; ++j)
-            b[j] = dma_frag<KCB>(sB + buf * SB, ROWS / 2 * wn + 16 * j + rl, g4, hh);
+            b[j] = dma_frag<KCB>(buf ? sB1 : sB0, ROWS / 2 * wn + 16 * j + rl, g4, hh);
     };
     auto mma = [&](const d2_t (&a)[NB], const d2_t (&b)[NB]) {
 #pragma unroll
@@ -199,8 +209,9 @@ __device__ __forceinline__ void gemm_tile(d4_t (&acc)[ROWS / 32][ROWS / 32],
     constexpr int NM = 2 * NB * NB, NR = 2 * NB;      // MFMAs and LDS reads of a half
     constexpr int NL = 2 * (V == 16 ? ROWS / 32 : ROWS / 8);   // loads of a stage per wave
     constexpr int LG = NL < NM - NR ? NL : NM - NR;   // MFMAs they are spread over
-    int buf = 0, q = 0;
-    for (; q + 2 < nfull; ++q, buf ^= 1) {
+    // with buf constant the compiler knows that a read of one stage does not wait for the loads
+    // into the other
+    auto step = [&](int buf, int q) {
         frags(a1, b1, buf, 1);
         mma(a0, b0);
 #pragma unroll
@@ -226,7 +237,13 @@ __device__ __forceinline__ void gemm_tile(d4_t (&acc)[ROWS / 32][ROWS / 32],
         }
         __builtin_amdgcn_sched_group_barrier(0x8, NM - NR - LG, 1);
         __builtin_amdgcn_sched_barrier(0);
+    };
+    int q = 0;
+    for (; q + 3 < nfull; q += 2) {
+        step(0, q);
+        step(1, q + 1);
     }
+    int buf = 0;
     for (; q < ns; ++q, buf ^= 1) {
         frags(a1, b1, buf, 1);
         mma(a0, b0);

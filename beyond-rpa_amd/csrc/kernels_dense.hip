@@ -87,8 +87,8 @@ struct GemmArgs {
 template <bool TA, bool TB, int V>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_gemm_f64(const GemmArgs g) {
     constexpr bool KCA = TA, KCB = !TB;   // operand contiguous in k
-    __shared__ __attribute__((aligned(16))) double sA[2][gemm_lds<KCA>(GT)];
-    __shared__ __attribute__((aligned(16))) double sB[2][gemm_lds<KCB>(GT)];
+    __shared__ __attribute__((aligned(16))) double sA0[gemm_lds<KCA>(GT)], sA1[gemm_lds<KCA>(GT)];
+    __shared__ __attribute__((aligned(16))) double sB0[gemm_lds<KCB>(GT)], sB1[gemm_lds<KCB>(GT)];
     const int item1 = (int)(blockIdx.x / (unsigned)g.ntiles);
     const int t = (int)(blockIdx.x - (unsigned)item1 * (unsigned)g.ntiles);
     const int item2 = (int)blockIdx.y;
@@ -134,7 +134,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 
     if (kbeg < kend)
         gemm_tile<KCA, KCB, V, GT>(acc, A, lda, m0, m, B, ldb, n0, n, kbeg, kend, g.far != 0, true,
-                                   sA[0], sB[0]);
+                                   sA0, sA1, sB0, sB1);
 
     if (g.nsplit > 1) {
         // partial tile, reduced by k_gemm_reduce
@@ -235,7 +235,7 @@ int launch_gemm_f64_batched(brpa_ctx *ctx, bool ta, bool tb, int64_t m, int64_t 
     // 16 bytes per lane: aligned sources (even leading dimensions and strides, aligned
     // bases) and 32-bit offsets within a tile; a rows-contiguous operand also needs
     // an even row count, so that its last row pair lies inside the matrix.  Measured
-    // at 4097^3 with 4 bytes per lane: NN, NT, TT 51 TFLOP/s, TN 44 (through registers:
+    // at 4097^3 with 4 bytes per lane: NN, NT, TT 51 TFLOP/s, TN 50 (through registers:
     // 45 for all four)
     g.far = lda >= (1 << 21) || ldb >= (1 << 21);
     const bool wide = lda % 2 == 0 && ldb % 2 == 0 && sA1 % 2 == 0 && sA2 % 2 == 0 &&

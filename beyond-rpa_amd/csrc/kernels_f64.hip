@@ -1175,13 +1175,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 // launch is large (2.1 ms at N = 1800, 24 frequencies, 24 fragments) and by the length of
 // one tile's loop where it is small.  Four work-groups per CU hide each other's C
 // pass, which the 128 x 128 tiles of two per CU did not.  Average launch: N = 400, 16 matrices
-// 21 us; N = 1800, 24 matrices 137 us; 24 x 24 of N up to 1800 706 us (128 x 128 tiles:
+// 21 us; N = 1800, 24 matrices 137 us; 24 x 24 of N up to 1800 676 us (128 x 128 tiles:
 // 54, 191, 935; register-staged 128 x 128 tiles with C preloaded: 50, 194, 890).
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) void k_chol_rest(
     const FragDev *__restrict__ fr, const int64_t *__restrict__ pre, int nfrag, int step) {
     constexpr int T = REST_T;
-    __shared__ __attribute__((aligned(16))) double sA[2 * gemm_lds<true>(T)];
-    __shared__ __attribute__((aligned(16))) double sB[2 * gemm_lds<true>(T)];
+    __shared__ __attribute__((aligned(16))) double sA0[gemm_lds<true>(T)], sA1[gemm_lds<true>(T)];
+    __shared__ __attribute__((aligned(16))) double sB0[gemm_lds<true>(T)], sB1[gemm_lds<true>(T)];
     const int64_t b = blockIdx.x;
     const int f = __builtin_amdgcn_readfirstlane(find_frag(pre, nfrag, b));
     const FragDev &F = fr[f];
@@ -1207,9 +1207,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
 #pragma unroll
         for (int j = 0; j < NB; ++j) acc[i][j] = (d4_t){0.0, 0.0, 0.0, 0.0};
     if (N % 2 == 0 && (reinterpret_cast<uintptr_t>(A) & 15) == 0)
-        gemm_tile<true, true, 16, T>(acc, A, N, Rj, N, A, N, Ri, N, kbase, t0, false, active, sA, sB);
+        gemm_tile<true, true, 16, T>(acc, A, N, Rj, N, A, N, Ri, N, kbase, t0, false, active, sA0, sA1,
+                                     sB0, sB1);
     else
-        gemm_tile<true, true, 4, T>(acc, A, N, Rj, N, A, N, Ri, N, kbase, t0, false, active, sA, sB);
+        gemm_tile<true, true, 4, T>(acc, A, N, Rj, N, A, N, Ri, N, kbase, t0, false, active, sA0, sA1,
+                                     sB0, sB1);
     if (!active) return;
     gdouble_mut_t *C = (gdouble_mut_t *)A;
 #pragma unroll
