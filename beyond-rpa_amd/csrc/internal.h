@@ -48,7 +48,6 @@ struct brpa_ctx {
     // contraction (kept apart from the workspace, which that call may regrow)
     double *x_V = nullptr, *x_B = nullptr;
     size_t x_V_cap = 0, x_B_cap = 0;
-    bool mbpt3_chol = false;   // the last MBPT3-1 factored -X by Cholesky (else eigenpairs)
     // pinned bounce buffer of the small completed copies (copy_sync), kBounceBytes
     void *bounce = nullptr;
     // pinned host staging of the batched E_RPA path (uploads and results)
@@ -248,6 +247,13 @@ enum { I8V_T128 = 0, I8V_T128_XCD = 1, I8V_T64 = 2, I8V_COUNT = 3 };
 int syrk_i8_tile(int variant);
 int launch_syrk_i8(brpa_ctx *, const FragDev *, const int64_t *pre, int nfrag, int64_t total,
                    int variant);
+
+// SOSEX contraction in the explicit ov space, E = -alpha sum (aj|bi) (V X V^T)(ai, bj), with
+// X = diag(hB) (host), or VX (device, NT2 x K column-major like V) = X V^T given; and
+// whether it is the cheaper form
+bool sosex_prefers_explicit(int precision, int64_t o, int64_t v, int64_t N, int64_t nt);
+int sosex_explicit(brpa_ctx *, double *ec, double alpha, const double *V, const double *hB,
+                   const double *VX, const double *R, int64_t o, int64_t v, int64_t N, int64_t nt);
 
 // Blocked Cholesky of the F matrices d_fr->Pi (1 + Pi already formed) of one
 // fragment, in place on ctx->stream; status/linv/ldpart of the descriptor

@@ -15,10 +15,13 @@
 // until B = I, when X = A/2 (getrf/getri and dgemm on the device; once
 // |B - 1|_F <= 1/4 the inverse-free Newton-Schulz step, all dgemm).  X is the
 // derivative of the amplitudes with the coupling strength in the V basis and
-// is negative definite in practice: -X = U'^T U' by the library's Cholesky
-// gives V X V^T = -(V U'^T)(V U'^T)^T, so the trace is the SOSEX contraction
-// of V'' = V U'^T with B'' = -1 (brpa_sosex, FP64 or split-int8); a Cholesky
-// breakdown falls back to the eigenpairs of X (rocSOLVER dsyevd).
+// is negative semidefinite up to rounding.  The trace is the SOSEX contraction of V X V^T:
+// where the explicit ov form is the cheaper one it takes X as it is (sosex_explicit;
+// NT2 = 1200: 0.5 ms, the eigenpairs below 37 ms, which a rounding-level
+// positive eigenvalue asked for).  The pair forms need a factor: -X = U'^T U' by the
+// library's Cholesky gives V X V^T = -(V U'^T)(V U'^T)^T, so V'' = V U'^T with B'' = -1
+// (brpa_sosex, FP64 or split-int8); a Cholesky breakdown falls back to the eigenpairs
+// of X (rocSOLVER dsyevd).
 //
 // MBPT3-2 runs as T~_k(c, i v + a) = T(ci, ak) = sum_mu (V A)(ci, mu) V(ak, mu)
 // (strided-batched dgemm over i) and M_k = R^T T~_k^T (N x v), E = 2 sum_k |M_k|_F^2:
@@ -31,7 +34,7 @@
 #include <cstring>
 #include <vector>
 
-#include "internal.h"
+#include "dense.h"
 
 int rocblas_handle_of(brpa_ctx *ctx, void **h);
 int launch_col_scale(brpa_ctx *, double *out, const double *in, const double *s, int64_t m,
@@ -274,7 +277,24 @@ int brpa_mbpt3_1(brpa_ctx *ctx, int precision, double *ec_exchange, const double
     }
     if (!conv)
         return brpa_fail(ctx, BRPA_ERR_SOLVER, "brpa_mbpt3_1: Lyapunov iteration did not converge");
-    // X = Am / 2.  Factor -X = U'^T U' (Cholesky on T1 = -X)
+    const bool keep = ctx->stage_keep;
+    auto end_stage = [&]() -> int {
+        BRPA_TRY(stage_end(ctx, BRPA_STAGE_MBPT3));
+        BRPA_HIP(ctx, hipStreamSynchronize(ctx->stream));
+        BRPA_TRY(stage_collect(ctx, BRPA_STAGE_MBPT3));
+        ctx->stage_launches[BRPA_STAGE_MBPT3] = iters;   // reported as the sign-iteration steps
+        return BRPA_OK;
+    };
+    BRPA_TRY(grow(ctx, &ctx->x_V, &ctx->x_V_cap, (size_t)K * n));
+    // X = Am / 2
+    if (sosex_prefers_explicit(precision, nocc, nvir, N, n)) {
+        BRPA_TRY(dense_gemm(ctx, false, false, n, K, n, 0.5, Am, n, dV, n, 0.0, ctx->x_V, n));
+        BRPA_TRY(end_stage());
+        // V and R as the caller gave them: the workspace copies may not survive the
+        // contraction's own workspace
+        return sosex_explicit(ctx, ec_exchange, 1.0, V, nullptr, ctx->x_V, R, nocc, nvir, N, n);
+    }
+    // Factor -X = U'^T U' (Cholesky on T1 = -X)
     BRPA_HIP(ctx, hipMemcpyAsync(T1, Am, 8 * n * n, hipMemcpyDeviceToDevice, ctx->stream));
     BRPA_TRY(launch_scale(ctx, T1, -0.5, n * n));
     fm.Pi = T1;
@@ -287,7 +307,6 @@ int brpa_mbpt3_1(brpa_ctx *ctx, int precision, double *ec_exchange, const double
     BRPA_TRY(chol_single(ctx, dfm, dchol, n, 1));
     int st = 0;
     BRPA_TRY(copy_sync(ctx, &st, fm.status, sizeof(int), hipMemcpyDeviceToHost));
-    BRPA_TRY(grow(ctx, &ctx->x_V, &ctx->x_V_cap, (size_t)K * n));
     BRPA_TRY(grow(ctx, &ctx->x_B, &ctx->x_B_cap, (size_t)n));
     if (st == 0) {
         // V X V^T = -(V U'^T)(V U'^T)^T; store V''^T = U' V^T as C V''[ai][mu]
@@ -309,13 +328,8 @@ int brpa_mbpt3_1(brpa_ctx *ctx, int precision, double *ec_exchange, const double
         BRPA_TRY(gemm(ctx, h, true, false, n, K, n, 1.0, T1, n, dV, n, 0.0, ctx->x_V, n));
         BRPA_HIP(ctx, hipMemcpyAsync(ctx->x_B, ev_x, 8 * n, hipMemcpyDeviceToDevice, ctx->stream));
     }
-    BRPA_TRY(stage_end(ctx, BRPA_STAGE_MBPT3));
-    BRPA_HIP(ctx, hipStreamSynchronize(ctx->stream));
-    BRPA_TRY(stage_collect(ctx, BRPA_STAGE_MBPT3));
-    ctx->stage_launches[BRPA_STAGE_MBPT3] = iters;   // reported as the sign-iteration steps
-    ctx->mbpt3_chol = (st == 0);
+    BRPA_TRY(end_stage());
     // E = -sum (aj|bi) (V'' diag(B'') V''^T)(ai, bj): the SOSEX contraction with alpha = 1
-    const bool keep = ctx->stage_keep;
     ctx->stage_keep = true;
     // R as the caller gave it: the workspace copy may not survive brpa_sosex's own workspace
     int rc = brpa_sosex(ctx, precision, ec_exchange, 1.0, ctx->x_V, ctx->x_B, R, nocc, nvir, naux,

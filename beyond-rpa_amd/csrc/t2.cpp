@@ -692,7 +692,7 @@ int t2_build(brpa_ctx *ctx, int precision, const double *R, int64_t naux, const 
 namespace {
 
 // SOSEX in the explicit ov space: E = -alpha sum_{aibj} (ai|bj) T(aj, bi) with
-// G = R R^T and T = V diag(B) V^T formed block by block on the library's GEMM,
+// G = R R^T and T = V X V^T (X = diag(B), or any symmetric X given as VX) formed block by block on the library's GEMM,
 // K^2 (N + NT2) flop for both, then contracted by k_sosex_contract.  Blocks are
 // pairs I <= J of occupied ranges of at most kSosexBlock ov rows, so a block pair
 // needs 2 x 8 kSosexBlock^2 bytes (4.3 GB); on I = J only the tiles on or above
@@ -705,6 +705,8 @@ constexpr int64_t kSosexBlock = 16384;
 // pair products at 60 of their own flop counts.  The ratio of the flop counts is
 // about v (N + NT2) / (2 N NT2), so the pair forms remain for few amplitude
 // vectors (NT2 below ~ v / 2).
+}  // namespace
+
 bool sosex_prefers_explicit(int precision, int64_t o, int64_t v, int64_t N, int64_t nt) {
     const double K = (double)o * (double)v;
     const double ex = K * K * ((double)N + (double)nt) / 60.0;
@@ -713,9 +715,8 @@ bool sosex_prefers_explicit(int precision, int64_t o, int64_t v, int64_t N, int6
     return ex < pr && v <= kSosexBlock;
 }
 
-int sosex_explicit(brpa_ctx *ctx, double *ec, double alpha, const double *V,
-                   const std::vector<double> &hB, const double *R, int64_t o, int64_t v, int64_t N,
-                   int64_t nt) {
+int sosex_explicit(brpa_ctx *ctx, double *ec, double alpha, const double *V, const double *hB,
+                   const double *VX, const double *R, int64_t o, int64_t v, int64_t N, int64_t nt) {
     const int64_t K = o * v;
     const bool rdev = is_device_ptr(R), vdev = is_device_ptr(V);
     const int64_t ob = std::min(o, std::max<int64_t>(1, kSosexBlock / v)), bs = ob * v;
@@ -725,8 +726,8 @@ int sosex_explicit(brpa_ctx *ctx, double *ec, double alpha, const double *V,
     auto layout = [&](Arena &ar) {
         dR = rdev ? const_cast<double *>(R) : ar.take<double>(K * N);
         dV = vdev ? const_cast<double *>(V) : ar.take<double>(K * nt);
-        dB = ar.take<double>(nt);
-        VB = ar.take<double>(K * nt);
+        dB = VX ? nullptr : ar.take<double>(nt);
+        VB = VX ? const_cast<double *>(VX) : ar.take<double>(K * nt);
         G = ar.take<double>(bs * bs);
         M = ar.take<double>(bs * bs);
         part = ar.take<double>(cdiv(o, ob) * K);
@@ -738,7 +739,7 @@ int sosex_explicit(brpa_ctx *ctx, double *ec, double alpha, const double *V,
     layout(ar);
     if (!rdev) BRPA_TRY(to_device(ctx, dR, R, 8 * K * N));
     if (!vdev) BRPA_TRY(to_device(ctx, dV, V, 8 * K * nt));
-    BRPA_TRY(copy_sync(ctx, dB, hB.data(), 8 * nt, hipMemcpyHostToDevice));
+    if (!VX) BRPA_TRY(copy_sync(ctx, dB, hB, 8 * nt, hipMemcpyHostToDevice));
     struct SplitLend {
         brpa_ctx *c;
         ~SplitLend() {
@@ -753,7 +754,7 @@ int sosex_explicit(brpa_ctx *ctx, double *ec, double alpha, const double *V,
     BRPA_TRY(stage_begin(ctx, BRPA_STAGE_SOSEX));
     // R and V are column-major N x K and NT2 x K here: every product is TN, both
     // operands contiguous in k
-    BRPA_TRY(launch_row_scale(ctx, VB, dV, dB, nt, K));
+    if (!VX) BRPA_TRY(launch_row_scale(ctx, VB, dV, dB, nt, K));
     int64_t np = 0;
     for (int64_t i0 = 0; i0 < o; i0 += ob) {
         const int64_t ni = std::min(ob, o - i0), mi = ni * v;
@@ -787,8 +788,6 @@ int sosex_explicit(brpa_ctx *ctx, double *ec, double alpha, const double *V,
     *ec = (double)(-(long double)alpha * s);
     return BRPA_OK;
 }
-
-}  // namespace
 
 extern "C" {
 
@@ -1016,7 +1015,7 @@ int brpa_sosex(brpa_ctx *ctx, int precision, double *ec_exchange, double alpha, 
     std::vector<double> hB(nt);
     for (int64_t k = 0; k < nt; ++k) hB[k] = s2_operator ? hA[k] / (1.0 - 4.0 * hA[k] * hA[k]) : hA[k];
     if (sosex_prefers_explicit(precision, o, v, N, nt))
-        return sosex_explicit(ctx, ec_exchange, alpha, V, hB, R, o, v, N, nt);
+        return sosex_explicit(ctx, ec_exchange, alpha, V, hB.data(), nullptr, R, o, v, N, nt);
     const bool rdev = is_device_ptr(R), vdev = is_device_ptr(V);
     if (precision == BRPA_SPLIT_I8) {
         // fused split-int8 pair kernel: 5 int8 slices per value, 15 products,
