@@ -12,7 +12,7 @@
 // Schur form, so here the equation is solved by the scaled matrix-sign
 // (Newton) iteration, which keeps Bk^T X + X Bk = Ak at every step:
 //   B <- (cB + (cB)^-1)/2,  A <- (cA + c^-1 B^-T A B^-1)/2,  c = sqrt(|B^-1|_F/|B|_F),
-// until B = I, when X = A/2 (getrf/getri and dgemm on the device; once
+// until B = I, when X = A/2 (the inverse by Cholesky of B^T B and refinement, else getrf/getri; once
 // |B - 1|_F <= 1/4 the inverse-free Newton-Schulz step, all dgemm).  X is the
 // derivative of the amplitudes with the coupling strength in the V basis and
 // is negative semidefinite up to rounding.  The trace is the SOSEX contraction of V X V^T:
@@ -158,13 +158,11 @@ int brpa_mbpt3_1(brpa_ctx *ctx, int precision, double *ec_exchange, const double
     for (double x : d)
         if (!std::isfinite(x)) return brpa_fail(ctx, BRPA_ERR_NONFINITE, "brpa_mbpt3_1: non-finite input");
     const bool vdev = is_device_ptr(V), adev = is_device_ptr(A), rdev = is_device_ptr(R);
-    const int64_t nsteps = (n + CHOL_NB - 1) / CHOL_NB;
     const double *dV = V, *dA = A, *dR = R;
     double *dd, *W, *U, *Dm, *Vd, *Am, *Bm, *Bi, *T1, *ev_x, *work;
     int *ipiv, *info;
-    int64_t *dchol;
-    FragDev fm{};
-    FragDev *dfm = nullptr;
+    double *Fi, *tw;
+    DenseChol ch;
     auto layout = [&](Arena &ar) {
         if (!vdev) dV = ar.take<double>(K * n);
         if (!adev) dA = ar.take<double>(n);
@@ -182,11 +180,9 @@ int brpa_mbpt3_1(brpa_ctx *ctx, int precision, double *ec_exchange, const double
         work = ar.take<double>(n);
         ipiv = ar.take<int>(n);
         info = ar.take<int>(2);
-        dfm = ar.take<FragDev>(1);
-        fm.linv = ar.take<double>(CHOL_NB * CHOL_NB);
-        fm.ldpart = ar.take<double>(nsteps * 2);
-        fm.status = ar.take<int>(1);
-        dchol = ar.take<int64_t>(chol_pre_len(n));
+        Fi = ar.take<double>(n * n);
+        tw = ar.take<double>(trinv_scratch(n));
+        ch.layout(ar, n);
     };
     Arena count, ar;
     layout(count);
@@ -210,6 +206,38 @@ int brpa_mbpt3_1(brpa_ctx *ctx, int precision, double *ec_exchange, const double
     BRPA_TRY(gemm(ctx, h, false, true, n, n, K, 1.0, dV, n, Vd, n, 0.0, Dm, n));
     BRPA_TRY(launch_mbpt3_ab(ctx, Dm, U, dA, n, Am, Bm));
     // Bm^T X + X Bm = Am by the scaled sign iteration; Am -> 2X, Bm -> I
+    // Bi = Bm^{-1} by the Cholesky factor of Bm^T Bm = F^T F, Bi = F^{-1} F^{-T} Bm^T (relative
+    // error of order cond(Bm)^2 eps), and steps Bi <- Bi + Bi (1 - Bm Bi), which square
+    // the residual r = |1 - Bm Bi|_F, until the last one started from r <= 1e-9.  Not
+    // inverted (then LU decides): a breakdown, or r not down there after three steps.
+    // Matrix products instead of rocSOLVER's column by column getrf / getri: 6.1 ms less per
+    // inverse at n = 1200 (four inverses: MBPT3-1 of 33 to 9 ms).
+    auto inverse = [&](bool *done) -> int {
+        *done = false;
+        BRPA_TRY(dense_syrk(ctx, true, n, n, 1.0, Bm, n, 0.0, T1, n));
+        bool okc = false;
+        BRPA_TRY(ch.run(ctx, T1, n, &okc));
+        if (!okc) return BRPA_OK;
+        BRPA_TRY(dense_trinv(ctx, n, T1, n, 0, Fi, n, 0, 1, tw));
+        BRPA_TRY(launch_gemm_f64_batched(ctx, true, true, n, n, n, 1.0, Fi, n, 0, 0, Bm, n, 0, 0, 0.0,
+                                         T1, n, 0, 0, 1, 1, false, TRI_A_LOWER, nullptr, 0, 0));
+        BRPA_TRY(launch_gemm_f64_batched(ctx, false, false, n, n, n, 1.0, Fi, n, 0, 0, T1, n, 0, 0,
+                                         0.0, Bi, n, 0, 0, 1, 1, false, TRI_A_UPPER, nullptr, 0, 0));
+        for (int t = 0; t < 3; ++t) {
+            BRPA_TRY(dense_gemm(ctx, false, false, n, n, n, -1.0, Bm, n, Bi, n, 0.0, T1, n));
+            BRPA_TRY(launch_add_diag(ctx, T1, n, 1.0));
+            double r = 0.0;
+            BRPA_TRY(nrm2(ctx, h, T1, n * n, &r));
+            if (!(r < 0.5)) return BRPA_OK;
+            BRPA_HIP(ctx, hipMemcpyAsync(Fi, Bi, 8 * n * n, hipMemcpyDeviceToDevice, ctx->stream));
+            BRPA_TRY(dense_gemm(ctx, false, false, n, n, n, 1.0, Fi, n, T1, n, 1.0, Bi, n));
+            if (r <= 1e-9) {
+                *done = true;
+                return BRPA_OK;
+            }
+        }
+        return BRPA_OK;
+    };
     const double tol = 1e-12 * std::sqrt((double)n);
     bool conv = false;
     int iters = 0;
@@ -241,9 +269,11 @@ int brpa_mbpt3_1(brpa_ctx *ctx, int precision, double *ec_exchange, const double
             iters = it + 1;
             continue;
         }
-        BRPA_HIP(ctx, hipMemcpyAsync(Bi, Bm, 8 * n * n, hipMemcpyDeviceToDevice, ctx->stream));
+        bool inverted = false;
+        BRPA_TRY(inverse(&inverted));
         int hinfo[2] = {0, 0};
-        {
+        if (!inverted) {
+            BRPA_HIP(ctx, hipMemcpyAsync(Bi, Bm, 8 * n * n, hipMemcpyDeviceToDevice, ctx->stream));
             std::lock_guard<std::mutex> lk(solver_mutex());
             BRPA_TRY(rbc(ctx, rocsolver_dgetrf(h, (rocblas_int)n, (rocblas_int)n, Bi,
                                                (rocblas_int)n, ipiv, info),
@@ -297,18 +327,10 @@ int brpa_mbpt3_1(brpa_ctx *ctx, int precision, double *ec_exchange, const double
     // Factor -X = U'^T U' (Cholesky on T1 = -X)
     BRPA_HIP(ctx, hipMemcpyAsync(T1, Am, 8 * n * n, hipMemcpyDeviceToDevice, ctx->stream));
     BRPA_TRY(launch_scale(ctx, T1, -0.5, n * n));
-    fm.Pi = T1;
-    fm.N = (int)n;
-    fm.F = 1;
-    fm.nsteps = (int)nsteps;
-    fm.keep_l11 = 1;
-    BRPA_TRY(launch_fill_int(ctx, fm.status, 1, 0));
-    BRPA_TRY(copy_sync(ctx, dfm, &fm, sizeof(FragDev), hipMemcpyHostToDevice));
-    BRPA_TRY(chol_single(ctx, dfm, dchol, n, 1));
-    int st = 0;
-    BRPA_TRY(copy_sync(ctx, &st, fm.status, sizeof(int), hipMemcpyDeviceToHost));
+    bool chol = false;
+    BRPA_TRY(ch.run(ctx, T1, n, &chol));
     BRPA_TRY(grow(ctx, &ctx->x_B, &ctx->x_B_cap, (size_t)n));
-    if (st == 0) {
+    if (chol) {
         // V X V^T = -(V U'^T)(V U'^T)^T; store V''^T = U' V^T as C V''[ai][mu]
         BRPA_TRY(launch_zero_lower(ctx, T1, n));
         BRPA_TRY(gemm(ctx, h, false, false, n, K, n, 1.0, T1, n, dV, n, 0.0, ctx->x_V, n));

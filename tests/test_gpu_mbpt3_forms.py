@@ -26,3 +26,20 @@ def test_forms(ctx, nt, prec):
     assert abs(ctx.mbpt3_1(V, A, f.R, f.eocc, f.evir, precision=prec) - ref) <= tol
     Vd, Rd = torch.from_numpy(V).cuda(), torch.from_numpy(f.R).cuda()
     assert abs(ctx.mbpt3_1(Vd, A, Rd, f.eocc, f.evir, precision=prec) - ref) <= tol
+
+
+@pytest.mark.parametrize("spread,size", [(1e2, 0.1), (1e8, 0.1), (1e2, 30.0), (1e2, 3e3)])
+def test_inverses(ctx, spread, size):
+    """The inverses of the sign iteration at condition numbers of B where the Cholesky of
+    B^T B suffices, needs refinement and breaks down (LU).  A backward-stable solution is
+    off by about cond(B) n u; ten times that."""
+    o, v, n, nt = 4, 30, 50, 70
+    rng = np.random.default_rng(3)
+    R = size * rng.standard_normal((o * v, n))
+    eocc, evir = -np.geomspace(1e-3, 1e-3 * spread, o)[::-1], np.geomspace(1e-3, 1e-3 * spread, v)
+    V = np.linalg.qr(rng.standard_normal((o * v, nt)))[0]
+    A = -np.linspace(0.2, 0.01, nt)
+    ref = mbpt3.mbpt3_1(R, V, A, o, v, eocc, evir)
+    cond = np.linalg.cond(mbpt3.mbpt3_1_matrices(R, V, A, eocc, evir)[1])
+    e = ctx.mbpt3_1(V, A, R, eocc, evir)
+    assert abs(e - ref) <= (1e-10 + 10 * cond * nt * 2.0 ** -53) * abs(ref)
