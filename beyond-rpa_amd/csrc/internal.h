@@ -222,6 +222,9 @@ int64_t syrk_items(int64_t N, int64_t F, bool quad);
 bool syrk_quad(const brpa_ctx *, int64_t wide_total, int64_t quad_total);
 int launch_syrk_f64(brpa_ctx *, const FragDev *, const int64_t *pre, int nfrag, int64_t total,
                     bool quad, bool both);
+// P += sum_q S_q, N x N matrices S_q = S + q N^2 of which only the lower triangle is
+// given
+int launch_syrk_acc(brpa_ctx *, double *P, const double *S, int64_t N, int nq);
 // mode: 0 = Pi's own diagonal, 1 = split-BF16 partials, 2 = diag precomputed
 int launch_set_diag(brpa_ctx *, const FragDev *, const int64_t *pre, int nfrag, int64_t total,
                     int mode);

@@ -154,7 +154,8 @@ __device__ __forceinline__ void syrk_stage_tail(const double *__restrict__ R, in
 
 template <int V, bool QUAD, bool DIAG>
 __device__ __forceinline__ void syrk_f64_tile(const FragDev &F, int w0, int tp, int tq, int both,
-                                              double *__restrict__ sA, double *__restrict__ sB) {
+                                              double *__restrict__ sA0, double *__restrict__ sA1,
+                                              double *__restrict__ sB0, double *__restrict__ sB1) {
     const double *__restrict__ R = F.R;
     const int K = F.K, N = F.N;
     const int tid = threadIdx.x, lane = tid & 63;
@@ -173,15 +174,15 @@ __device__ __forceinline__ void syrk_f64_tile(const FragDev &F, int w0, int tp, 
     const int nfull = K / KB, ns = (K + KB - 1) / KB;
     auto stage = [&](int buf, int q) {
         const int64_t o = 8 * (int64_t)N * (KB * q);
-        syrk_stage<V>(pa, ba + o, N, sA + buf * SYRK_P, wave);
-        if (!DIAG) syrk_stage<V>(pb, bb + o, N, sB + buf * SYRK_P, wave);
+        syrk_stage<V>(pa, ba + o, N, buf ? sA1 : sA0, wave);
+        if (!DIAG) syrk_stage<V>(pb, bb + o, N, buf ? sB1 : sB0, wave);
     };
     auto put = [&](int buf, int q) {
         if (q < nfull) {
             stage(buf, q);
         } else if (q < ns) {
-            syrk_stage_tail(R, K, N, KB * q, p0, sA + buf * SYRK_P, tid);
-            if (!DIAG) syrk_stage_tail(R, K, N, KB * q, q0, sB + buf * SYRK_P, tid);
+            syrk_stage_tail(R, K, N, KB * q, p0, buf ? sA1 : sA0, tid);
+            if (!DIAG) syrk_stage_tail(R, K, N, KB * q, q0, buf ? sB1 : sB0, tid);
         }
     };
     put(0, 0);
@@ -203,8 +204,8 @@ __device__ __forceinline__ void syrk_f64_tile(const FragDev &F, int w0, int tp, 
     // has its low bit flipped
     const int x0 = g4 * SYRK_T + rl + 16 * (g4 & 1), x1 = g4 * SYRK_T + rl - 16 * (g4 & 1);
     auto frags = [&](double (&a)[2][NB], double (&b)[2][NB], int buf, int h) {
-        const double *LA = sA + buf * SYRK_P + 16 * bi;
-        const double *LB = (DIAG ? sA : sB) + buf * SYRK_P + 16 * bj;
+        const double *LA = (buf ? sA1 : sA0) + 16 * bi;
+        const double *LB = (DIAG ? (buf ? sA1 : sA0) : (buf ? sB1 : sB0)) + 16 * bj;
 #pragma unroll
         for (int s = 0; s < 2; ++s) {
 #pragma unroll
@@ -227,70 +228,79 @@ __device__ __forceinline__ void syrk_f64_tile(const FragDev &F, int w0, int tp, 
                         acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(x, b[s][j], acc[i][j], 0, 0, 0);
             }
     };
-    // c_w of the lane's four rows of stage q
+    // c_w of the lane's rows of stage q: two for either half
     const gdouble_t *dt = (const gdouble_t *)F.dtab + (int64_t)w * K;
-    auto coef = [&](double (&d)[4], int q) {
+    auto coef = [&](double (&d)[4], int q, int h) {
 #pragma unroll
-        for (int s = 0; s < 4; ++s) {
+        for (int s = 2 * h; s < 2 * h + 2; ++s) {
             const int k = KB * q + 4 * s + g4;
             d[s] = dt[min(k, K - 1)];   // rows past K are zero
         }
     };
-    double a0[2][NB], b0[2][NB], a1[2][NB], b1[2][NB], dv[4], dn[4];
-    coef(dv, 0);
+    double a0[2][NB], b0[2][NB], a1[2][NB], b1[2][NB], de[4], dd[4];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        coef(de, 0, h);
+        coef(dd, min(1, ns - 1), h);
+    }
     __syncthreads();
     put(1, 1);
     frags(a0, b0, 0, 0);
-    int buf = 0, q = 0;
-    for (; q + 2 < nfull; ++q, buf ^= 1) {
-        coef(dn, q + 1);
+    // buf constant, arrays of their own: as in gemm_tile.h.  d: c_w of this stage, replaced by
+    // that of the stage after the next as soon as it is used; loaded one stage ahead, just before
+    // the barrier that waits for it, it held up the quad form at every stage (K = 3620, N =
+    // 905 in seven chunks: 97 us instead of 86).
+    auto step = [&](int buf, int q, double (&d)[4]) {
         frags(a1, b1, buf, 1);
-        mma(a0, b0, dv[0], dv[1]);
-        if (!QUAD) {
-            constexpr int NM = DIAG ? 20 : 32;
+        mma(a0, b0, d[0], d[1]);
+        constexpr int NM = QUAD ? 8 : (DIAG ? 20 : 32), NR = QUAD ? 4 : 8;
 #pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);     // MFMA
-                __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);   // LDS read
-            }
-            __builtin_amdgcn_sched_group_barrier(0x8, NM - 8, 0);
-            __builtin_amdgcn_sched_barrier(0);
+        for (int u = 0; u < NR; ++u) {
+            __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);     // MFMA
+            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);   // LDS read
         }
+        __builtin_amdgcn_sched_group_barrier(0x8, NM - NR, 0);
+        __builtin_amdgcn_sched_barrier(0);
         __syncthreads();
         frags(a0, b0, buf ^ 1, 0);
+        coef(d, q + 2, 0);
         stage(buf, q + 2);
-        mma(a1, b1, dv[2], dv[3]);
-        if (!QUAD) {
-            constexpr int NM = DIAG ? 20 : 32, NL = (V == 16 ? 2 : 8) * (DIAG ? 1 : 2);
-            constexpr int NL1 = NL < NM - 8 ? NL : NM - 8;
+        mma(a1, b1, d[2], d[3]);
+        constexpr int NL = 2 + (V == 16 ? 2 : 8) * (DIAG ? 1 : 2);
+        constexpr int NL1 = NL < NM - NR ? NL : NM - NR;
 #pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                __builtin_amdgcn_sched_group_barrier(0x8, 1, 1);
-                __builtin_amdgcn_sched_group_barrier(0x100, 1, 1);
-            }
-#pragma unroll
-            for (int u = 0; u < NL1; ++u) {
-                __builtin_amdgcn_sched_group_barrier(0x8, 1, 1);
-                __builtin_amdgcn_sched_group_barrier(0x20, 1, 1);    // global -> LDS
-            }
-            __builtin_amdgcn_sched_group_barrier(0x8, NM - 8 - NL1, 1);
-            __builtin_amdgcn_sched_barrier(0);
+        for (int u = 0; u < NR; ++u) {
+            __builtin_amdgcn_sched_group_barrier(0x8, 1, 1);
+            __builtin_amdgcn_sched_group_barrier(0x100, 1, 1);
         }
 #pragma unroll
-        for (int s = 0; s < 4; ++s) dv[s] = dn[s];
+        for (int u = 0; u < NL1; ++u) {
+            __builtin_amdgcn_sched_group_barrier(0x8, 1, 1);
+            __builtin_amdgcn_sched_group_barrier(0x20, (NL + NL1 - 1) / NL1, 1);   // global loads
+        }
+        __builtin_amdgcn_sched_group_barrier(0x8, NM - NR - NL1, 1);
+        __builtin_amdgcn_sched_barrier(0);
+        coef(d, q + 2, 1);
+    };
+    int q = 0;
+    for (; q + 3 < nfull; q += 2) {
+        step(0, q, de);
+        step(1, q + 1, dd);
     }
+    int buf = 0;
     for (; q < ns; ++q, buf ^= 1) {
-        coef(dn, min(q + 1, ns - 1));
         frags(a1, b1, buf, 1);
-        mma(a0, b0, dv[0], dv[1]);
+        mma(a0, b0, de[0], de[1]);
         if (q + 1 < ns) {
             __syncthreads();
             put(buf, q + 2);
             frags(a0, b0, buf ^ 1, 0);
         }
-        mma(a1, b1, dv[2], dv[3]);
+        mma(a1, b1, de[2], de[3]);
 #pragma unroll
-        for (int s = 0; s < 4; ++s) dv[s] = dn[s];
+        for (int s = 0; s < 4; ++s) de[s] = dd[s];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) coef(dd, min(q + 2, ns - 1), h);
     }
 
     gdouble_mut_t *C = (gdouble_mut_t *)(F.Pi + (int64_t)w * N * N);
@@ -317,8 +327,7 @@ __device__ __forceinline__ void syrk_f64_tile(const FragDev &F, int w0, int tp, 
 template <bool QUAD>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, QUAD ? 4 : 2))) void
 k_syrk_f64(const FragDev *__restrict__ fr, const int64_t *__restrict__ pre, int nfrag, int both) {
-    __shared__ __attribute__((aligned(16))) double sA[2 * SYRK_P];
-    __shared__ __attribute__((aligned(16))) double sB[2 * SYRK_P];
+    __shared__ __attribute__((aligned(16))) double sA0[SYRK_P], sA1[SYRK_P], sB0[SYRK_P], sB1[SYRK_P];
     int64_t b = blockIdx.x;
     int f = find_frag(pre, nfrag, b);
     const FragDev &F = fr[f];
@@ -332,14 +341,14 @@ k_syrk_f64(const FragDev *__restrict__ fr, const int64_t *__restrict__ pre, int 
     const bool wide = F.N % 2 == 0 && (reinterpret_cast<uintptr_t>(F.R) & 15) == 0;
     if (tp == tq) {
         if (wide)
-            syrk_f64_tile<16, QUAD, true>(F, w0, tp, tq, both, sA, sB);
+            syrk_f64_tile<16, QUAD, true>(F, w0, tp, tq, both, sA0, sA1, sB0, sB1);
         else
-            syrk_f64_tile<4, QUAD, true>(F, w0, tp, tq, both, sA, sB);
+            syrk_f64_tile<4, QUAD, true>(F, w0, tp, tq, both, sA0, sA1, sB0, sB1);
     } else {
         if (wide)
-            syrk_f64_tile<16, QUAD, false>(F, w0, tp, tq, both, sA, sB);
+            syrk_f64_tile<16, QUAD, false>(F, w0, tp, tq, both, sA0, sA1, sB0, sB1);
         else
-            syrk_f64_tile<4, QUAD, false>(F, w0, tp, tq, both, sA, sB);
+            syrk_f64_tile<4, QUAD, false>(F, w0, tp, tq, both, sA0, sA1, sB0, sB1);
     }
 }
 
@@ -369,6 +378,55 @@ int launch_syrk_f64(brpa_ctx *ctx, const FragDev *fr, const int64_t *pre, int nf
     else
         hipLaunchKernelGGL(k_syrk_f64<false>, dim3(grid1(total)), dim3(256), 0, ctx->stream, fr,
                            pre, nfrag, both ? 1 : 0);
+    LAUNCH_CHECK(ctx);
+    return BRPA_OK;
+}
+
+// 16 rows of a 64 x 64 tile pair per work-group: the sum of the partial tiles is added
+// to P as it is and, off the diagonal, transposed through LDS.  Bound by memory:
+// (nq / 2 + 2) N^2 doubles: 11 us at N = 905, nq = 7 (30 us with a whole tile pair per
+// work-group).
+__global__ __launch_bounds__(256) void k_syrk_acc(double *__restrict__ P,
+                                                 const double *__restrict__ S, int N, int nq) {
+    __shared__ double sT[16][65];
+    int ti, tj;
+    tri_decode((int)blockIdx.x >> 2, ti, tj);
+    const int c = threadIdx.x & 63, r0 = threadIdx.x >> 6;
+    const int row0 = 64 * ti + 16 * ((int)blockIdx.x & 3), col = 64 * tj + c;
+    const int64_t NN = (int64_t)N * N;
+    double s[4] = {0.0, 0.0, 0.0, 0.0}, p[4] = {0.0, 0.0, 0.0, 0.0};
+    int64_t e[4];
+    bool ok[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int row = row0 + r0 + 4 * i;
+        ok[i] = row < N && col <= row;
+        e[i] = ok[i] ? (int64_t)row * N + col : 0;
+        p[i] = P[e[i]];
+    }
+#pragma unroll 4
+    for (int q = 0; q < nq; ++q)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) s[i] += S[q * NN + e[i]];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        if (ok[i]) P[e[i]] = p[i] + s[i];
+        sT[r0 + 4 * i][c] = s[i];
+    }
+    __syncthreads();
+    // rows of the transposed tile: 16 columns each
+    const int tc = threadIdx.x & 15, tr = threadIdx.x >> 4;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int r = 64 * tj + tr + 16 * i, cc = row0 + tc;
+        if (cc < N && r < cc) P[(int64_t)r * N + cc] += sT[tc][tr + 16 * i];
+    }
+}
+
+int launch_syrk_acc(brpa_ctx *ctx, double *P, const double *S, int64_t N, int nq) {
+    const int64_t nt = (N + 63) / 64;
+    hipLaunchKernelGGL(k_syrk_acc, dim3(grid1(2 * nt * (nt + 1))), dim3(256), 0, ctx->stream, P, S,
+                       (int)N, nq);
     LAUNCH_CHECK(ctx);
     return BRPA_OK;
 }
