@@ -559,34 +559,68 @@ int brpa_gpiug_mo(brpa_ctx *ctx, double *gpiug, const double *crg, int64_t naux,
             c[i * nvir + a] = prefactor * (d / (d * d + freq * freq));
         }
     const bool rdev = is_device_ptr(crg), pdev = is_device_ptr(gpiug);
-    void *hv = nullptr;
-    BRPA_TRY(rocblas_handle_of(ctx, &hv));
-    rocblas_handle h = static_cast<rocblas_handle>(hv);
+    // GPiUG += CRG diag(W) CRG^T, half of it on the SYRK of the E_RPA pipeline.  One
+    // frequency alone has few tiles, so the rows of R are cut into nk chunks, each a work
+    // list entry with a partial product of its own, and k_syrk_acc adds them to both
+    // triangles: enough chunks for three work-groups per CU (N = 905, K = 3620, twelve calls and
+    // the rest of the MO route: 2693 us with one per CU, 2492 two, 2486 three, 2480 six), of
+    // 256 rows or more, and partial products of no more than R's own size.  Fewer rows than N: the reference's own
+    // shape (rpa_core_MO.f90:398-402), DCRG = CRG diag(W) and one plain dgemm.
+    // N = 905, K = 3620: 143 us by way of DCRG, 96 us.
+    const int64_t ncu = ctx->ncu > 0 ? ctx->ncu : 256, tiles = syrk_items(N, 1, true);
+    const int64_t nk = std::min({cdiv(3 * ncu, tiles), K / 256 + 1, K / N});
+    const int64_t kc = nk > 0 ? cdiv(cdiv(K, nk), 16) * 16 : 0;
+    const int64_t ne = nk > 0 ? cdiv(K, kc) : 0;   // work list entries
+    const size_t upn = sizeof(FragDev) * ne + 8 * (ne + 1) + 8 * K;
     Arena count;
-    count.take<double>(K);
-    count.take<double>(K * N);
+    count.take<char>(upn);
+    count.take<double>(nk > 0 ? ne * N * N : K * N);
     if (!rdev) count.take<double>(K * N);
     if (!pdev) count.take<double>(N * N);
     Arena ar;
     BRPA_TRY(ws_reserve(ctx, count.off, &ar));
-    double *dc = ar.take<double>(K);
-    double *dW = ar.take<double>(K * N);
+    char *d_up = ar.take<char>(upn);
+    double *dW = ar.take<double>(nk > 0 ? ne * N * N : K * N);
     const double *dR = rdev ? crg : ar.take<double>(K * N);
     double *dP = pdev ? gpiug : ar.take<double>(N * N);
-    BRPA_TRY(copy_sync(ctx, dc, c.data(), 8 * K, hipMemcpyHostToDevice));
+    const double *dc = reinterpret_cast<double *>(d_up + sizeof(FragDev) * ne + 8 * (ne + 1));
+    std::vector<char> up(upn);
+    FragDev *fe = reinterpret_cast<FragDev *>(up.data());
+    int64_t *pre = reinterpret_cast<int64_t *>(up.data() + sizeof(FragDev) * ne);
+    pre[0] = 0;
+    for (int64_t q = 0; q < ne; ++q) {
+        FragDev d{};
+        d.R = dR + q * kc * N;
+        d.dtab = dc + q * kc;
+        d.Pi = dW + q * N * N;
+        d.K = (int)std::min(kc, K - q * kc);
+        d.N = (int)N;
+        d.F = 1;
+        fe[q] = d;
+        pre[q + 1] = pre[q] + tiles;
+    }
+    std::memcpy(pre + ne + 1, c.data(), 8 * K);
+    BRPA_TRY(copy_sync(ctx, d_up, up.data(), upn, hipMemcpyHostToDevice));
     if (!rdev) BRPA_TRY(to_device(ctx, const_cast<double *>(dR), crg, 8 * K * N));
     if (!pdev) BRPA_TRY(to_device(ctx, dP, gpiug, 8 * N * N));
     BRPA_HIP(ctx, hipEventRecord(ctx->ev0, ctx->stream));
-    // the reference's own shape (rpa_core_MO.f90:398-402): DCRG = CRG diag(W),
-    // then GPiUG += CRG DCRG^T as one plain dgemm (column-major N x K operands)
-    BRPA_TRY(launch_col_scale(ctx, dW, dR, dc, N, K));
-    const double one = 1.0;
-    const rocblas_status st =
-        rocblas_dgemm(h, rocblas_operation_none, rocblas_operation_transpose, (rocblas_int)N,
-                      (rocblas_int)N, (rocblas_int)K, &one, dR, (rocblas_int)N, dW, (rocblas_int)N,
-                      &one, dP, (rocblas_int)N);
-    if (st != rocblas_status_success)
-        return brpa_fail(ctx, BRPA_ERR_SOLVER, "rocblas_dgemm failed: rocblas status %d", (int)st);
+    if (nk > 0) {
+        BRPA_TRY(launch_syrk_f64(ctx, reinterpret_cast<FragDev *>(d_up),
+                                 reinterpret_cast<int64_t *>(d_up + sizeof(FragDev) * ne), (int)ne,
+                                 pre[ne], true, false));
+        BRPA_TRY(launch_syrk_acc(ctx, dP, dW, N, (int)ne));
+    } else {
+        void *hv = nullptr;
+        BRPA_TRY(rocblas_handle_of(ctx, &hv));
+        rocblas_handle h = static_cast<rocblas_handle>(hv);
+        BRPA_TRY(launch_col_scale(ctx, dW, dR, dc, N, K));
+        const double one = 1.0;
+        const rocblas_status st = rocblas_dgemm(
+            h, rocblas_operation_none, rocblas_operation_transpose, (rocblas_int)N, (rocblas_int)N,
+            (rocblas_int)K, &one, dR, (rocblas_int)N, dW, (rocblas_int)N, &one, dP, (rocblas_int)N);
+        if (st != rocblas_status_success)
+            return brpa_fail(ctx, BRPA_ERR_SOLVER, "rocblas_dgemm failed: rocblas status %d", (int)st);
+    }
     BRPA_HIP(ctx, hipEventRecord(ctx->ev1, ctx->stream));
     if (!pdev) BRPA_TRY(from_device(ctx, gpiug, dP, 8 * N * N));
     BRPA_HIP(ctx, hipStreamSynchronize(ctx->stream));
