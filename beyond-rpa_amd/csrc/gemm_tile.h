@@ -12,50 +12,46 @@ typedef double d2_t __attribute__((ext_vector_type(2)));
 // half of the 64 LDS banks, so the four lane groups of a fragment read hit disjoint
 // halves).
 //
-// A wave's loads, V = 16: KC the 8-row blocks ROWS / 4 w + 8 c, lane L the k pair
-// (L % 8) ^ swizzle of row L / 8 of its block; rows-contiguous (128 rows only) the k
-// rows 4 w + c, lane L the rows 2 L, 2 L + 1.  The byte offsets from the tile's base at k = 0
-// (dma_base) are 32-bit; leading dimensions of 2^21 or more take the register
-// path of the last stage for all of them.
-// V = 4: KC the row pairs ROWS / 4 w + 2 c, lane L a half of a double of row L / 32;
-// rows-contiguous the k rows 4 w + c / 4, 32 rows at a time.
+// A wave's loads, 16 bytes per lane (which need no more than the 4-byte alignment of every
+// vector load, so odd leading dimensions take them too): KC the 8-row blocks ROWS / 4 w +
+// 8 c, lane L the k pair (L % 8) ^ swizzle of row L / 8 of its block; rows-contiguous (128
+// rows only) the k rows 4 w + c, lane L the rows 2 L, 2 L + 1.  The byte offsets from the
+// tile's base at k = 0 (dma_base) are 32-bit; leading dimensions of 2^21 or more take
+// the register path of the last stage for all of them.
 constexpr int DMA_KPR = 132;
 template <bool KC>
 constexpr int gemm_lds(int rows) {   // doubles of one stage
     return KC ? rows * GKB : GKB * DMA_KPR;
 }
-template <bool KC, int V, int ROWS>
+template <bool KC, int ROWS>
 struct DmaSrc {
     static_assert(KC || ROWS == 128, "rows-contiguous operands have 128-row tiles");
-    static constexpr int NLOAD = V == 16 ? ROWS / 32 : ROWS / 8;   // loads per wave and stage
-    // per load; V = 4 rows-contiguous: per 32 rows; V = 4 KC: only the lane's part, since 16
-    // offsets per operand and wave do not fit beside the accumulators
-    static constexpr int NOFF = !KC ? 4 : (V == 4 ? 1 : NLOAD);
-    uint32_t off[NOFF];
-    int last;   // V = 4 KC: the last row of the operand, from the wave's first one
+    static constexpr int NLOAD = ROWS / 32;   // loads per wave and stage
+    uint32_t off[NLOAD];
 };
-template <bool KC, int V, int ROWS>
-__device__ __forceinline__ DmaSrc<KC, V, ROWS> dma_offsets(int64_t ldx, int r0, int rows, int wave,
-                                                           int lane) {
-    DmaSrc<KC, V, ROWS> s;
+template <bool KC, int ROWS>
+__device__ __forceinline__ DmaSrc<KC, ROWS> dma_offsets(int64_t ldx, int r0, int rows, int wave,
+                                                       int lane) {
+    DmaSrc<KC, ROWS> s;
 #pragma unroll
-    for (int c = 0; c < DmaSrc<KC, V, ROWS>::NOFF; ++c) {
-        if (V == 16 && KC) {
+    for (int c = 0; c < DmaSrc<KC, ROWS>::NLOAD; ++c) {
+        if (KC) {
             const int row = ROWS / 4 * wave + 8 * c + (lane >> 3);
             const int dk = 2 * ((lane & 7) ^ ((row >> 1) & 7));
             s.off[c] = 8u * ((uint32_t)ldx * (uint32_t)(min(r0 + row, rows - 1) - r0) + (uint32_t)dk);
-        } else if (V == 16) {
-            // rows is even here: the last pair is rows - 2, rows - 1
-            s.off[c] = 8u * ((uint32_t)(min(r0 + 2 * lane, rows - 2) - r0) +
-                             (uint32_t)ldx * (uint32_t)(4 * wave + c));
-        } else if (KC) {
-            s.off[c] = 4u * ((uint32_t)lane & 31u);
-            s.last = rows - 1 - r0 - ROWS / 4 * wave;
         } else {
-            s.off[c] = 8u * (uint32_t)(min(r0 + 32 * c + (lane >> 1), rows - 1) - r0) + 4u * (lane & 1);
+            // the pair of the last row of an odd count ends in the next k's first row
+            // (dma_over)
+            s.off[c] = 8u * ((uint32_t)(min(r0 + 2 * lane, (rows - 1) & ~1) - r0) +
+                             (uint32_t)ldx * (uint32_t)(4 * wave + c));
         }
     }
     return s;
+}
+// whether a full stage that ends with the last k of all reads past the operand's end
+template <bool KC, int ROWS>
+__device__ __forceinline__ bool dma_over(int r0, int rows) {
+    return !KC && (rows & 1) && r0 + ROWS > rows;
 }
 template <bool KC>
 __device__ __forceinline__ const char *dma_base(const double *X, int64_t ldx, int r0) {
@@ -76,48 +72,24 @@ __host__ __device__ __forceinline__ d2_t dma_frag(const double *L, int row, int 
 }
 
 // one operand's full stage at k0 into the LDS buffer L, straight from global memory
-template <bool KC, int V, int ROWS>
-__device__ __forceinline__ void dma_stage(const char *base, const DmaSrc<KC, V, ROWS> &src,
-                                          int64_t ldx, double *L, int wave, int k0) {
+template <bool KC, int ROWS>
+__device__ __forceinline__ void dma_stage(const char *base, const DmaSrc<KC, ROWS> &src, int64_t ldx,
+                                          double *L, int wave, int k0) {
     // the builtin exists for the device pass only; the host pass never runs this
 #if defined(__HIP_DEVICE_COMPILE__)
     typedef __attribute__((address_space(1))) const char gchar_t;
     typedef __attribute__((address_space(1))) const void gvoid_t;
     typedef __attribute__((address_space(3))) void lvoid_t;
     gchar_t *b = (gchar_t *)(base + 8 * (KC ? (int64_t)k0 : ldx * k0));
-    if (V == 16) {
 #pragma unroll
-        for (int c = 0; c < DmaSrc<KC, V, ROWS>::NLOAD; ++c)
-            __builtin_amdgcn_global_load_lds(
-                (gvoid_t *)(b + src.off[c]),
-                (lvoid_t *)(L + (KC ? (ROWS / 4 * wave + 8 * c) * GKB : (4 * wave + c) * DMA_KPR)), 16, 0,
-                0);
-    } else if (KC) {
-        static_assert(!KC || V != 4 || (ROWS / 8) % 8 == 0, "a wave's swizzle starts at 0");
-        // rows 2c and 2c + 1 of the wave's; the offset is made here (volatile: not kept)
-        int last = src.last;
-        asm volatile("" : "+s"(last));
-        const uint32_t first = (uint32_t)(ROWS / 4 * wave), ld8 = 8u * (uint32_t)ldx;
-        const bool odd = threadIdx.x & 32;
-#pragma unroll
-        for (int c = 0; c < DmaSrc<KC, V, ROWS>::NLOAD; ++c) {
-            const uint32_t ra = ld8 * (first + (uint32_t)min(2 * c, last)),
-                           rb = ld8 * (first + (uint32_t)min(2 * c + 1, last));
-            const uint32_t off = (odd ? rb : ra) + (src.off[0] ^ (16u * (c & 7)));
-            __builtin_amdgcn_global_load_lds((gvoid_t *)(b + off),
-                                             (lvoid_t *)(L + (ROWS / 4 * wave + 2 * c) * GKB), 4, 0, 0);
-        }
-    } else {
-#pragma unroll
-        for (int c = 0; c < 16; ++c) {
-            const int kr = 4 * wave + (c >> 2);
-            __builtin_amdgcn_global_load_lds((gvoid_t *)(b + 8 * ldx * kr + src.off[c % DmaSrc<KC, V, ROWS>::NOFF]),
-                                             (lvoid_t *)(L + kr * DMA_KPR + 32 * (c & 3)), 4, 0, 0);
-        }
-    }
+    for (int c = 0; c < DmaSrc<KC, ROWS>::NLOAD; ++c)
+        __builtin_amdgcn_global_load_lds(
+            (gvoid_t *)(b + src.off[c]),
+            (lvoid_t *)(L + (KC ? (ROWS / 4 * wave + 8 * c) * GKB : (4 * wave + c) * DMA_KPR)), 16, 0, 0);
 #endif
 }
-// the last stage when it has fewer than 16 k: through registers, zeros past kend
+// the last stage when it has fewer than 16 k, or may not be read past its end: through
+// registers, zeros past kend
 template <bool KC, int ROWS>
 __device__ __forceinline__ void dma_stage_tail(const double *__restrict__ X, int64_t ldx, int r0,
                                                int rows, double *L, int tid, int k0, int kend) {
@@ -131,7 +103,7 @@ __device__ __forceinline__ void dma_stage_tail(const double *__restrict__ X, int
     }
 }
 
-// acc += rows m0 .. of op(A) times columns n0 .. of op(B) over k in [kbeg, kend): wave
+// acc += rows m0 .. of op(A) times columns n0 .. of op(B) over k in [kbeg, kend) of [0, k): wave
 // (wm, wn) = (wave / 2, wave % 2) holds the ROWS/2 x ROWS/2 block (wm, wn), acc[i][j][r]
 // = element (16 i + lane % 16, 16 j + lane / 16 + 4 r) of it.  m, n: rows of the whole
 // operands (past them the last row repeats).  far: leading dimensions beyond 32-bit
@@ -143,27 +115,29 @@ __device__ __forceinline__ void dma_stage_tail(const double *__restrict__ X, int
 // coming stage after the next ones.  The barrier stands between the halves: by then
 // the next stage has landed and every wave has read the current one, whose buffer
 // takes the loads of the stage after the next.  Bound by MFMA issue: TN 8192 x 8192 x
-// 2048 73.0 TFLOP/s, 4096^3 66.7, 3072^2 x 4096 (whose last 64 of 576 tiles run one
+// 2048 73.0 TFLOP/s, 4096^3 68.0, 4097^3 56 (50 with four bytes per lane for odd
+// leading dimensions), 3072^2 x 4096 (whose last 64 of 576 tiles run one
 // per CU) 52 (68.5, 64.0 and 38-46 with all reads, then all loads, ahead of the stage's
 // MFMAs).
-template <bool KCA, bool KCB, int V, int ROWS>
+template <bool KCA, bool KCB, int ROWS>
 __device__ __forceinline__ void gemm_tile(d4_t (&acc)[ROWS / 32][ROWS / 32],
                                           const double *__restrict__ A, int64_t lda, int m0, int m,
                                           const double *__restrict__ B, int64_t ldb, int n0, int n,
-                                          int kbeg, int kend, bool far, bool active, double *sA0,
+                                          int kbeg, int kend, int k, bool far, bool active, double *sA0,
                                           double *sA1, double *sB0, double *sB1) {
     constexpr int NB = ROWS / 32;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave >> 1, wn = wave & 1;
     const int rl = lane & 15, g4 = lane >> 4;
-    const auto oa = dma_offsets<KCA, V, ROWS>(lda, m0, m, wave, lane);
-    const auto ob = dma_offsets<KCB, V, ROWS>(ldb, n0, n, wave, lane);
+    const auto oa = dma_offsets<KCA, ROWS>(lda, m0, m, wave, lane);
+    const auto ob = dma_offsets<KCB, ROWS>(ldb, n0, n, wave, lane);
     const char *ba = dma_base<KCA>(A, lda, m0), *bb = dma_base<KCB>(B, ldb, n0);
-    const int nfull = far ? 0 : (kend - kbeg) / GKB, ns = (kend - kbeg + GKB - 1) / GKB;
+    const bool over = kend == k && (dma_over<KCA, ROWS>(m0, m) || dma_over<KCB, ROWS>(n0, n));
+    const int nfull = far ? 0 : (kend - kbeg - (over ? 1 : 0)) / GKB, ns = (kend - kbeg + GKB - 1) / GKB;
     auto stage = [&](int buf, int k0) {
-        dma_stage<KCA, V, ROWS>(ba, oa, lda, buf ? sA1 : sA0, wave, k0);
-        dma_stage<KCB, V, ROWS>(bb, ob, ldb, buf ? sB1 : sB0, wave, k0);
+        dma_stage<KCA, ROWS>(ba, oa, lda, buf ? sA1 : sA0, wave, k0);
+        dma_stage<KCB, ROWS>(bb, ob, ldb, buf ? sB1 : sB0, wave, k0);
     };
     auto put = [&](int buf, int q) {
         if (q < nfull) {
@@ -207,7 +181,7 @@ __device__ __forceinline__ void gemm_tile(d4_t (&acc)[ROWS / 32][ROWS / 32],
     put(1, 1);
     frags(a0, b0, 0, 0);
     constexpr int NM = 2 * NB * NB, NR = 2 * NB;      // MFMAs and LDS reads of a half
-    constexpr int NL = 2 * (V == 16 ? ROWS / 32 : ROWS / 8);   // loads of a stage per wave
+    constexpr int NL = 2 * (ROWS / 32);   // loads of a stage per wave
     constexpr int LG = NL < NM - NR ? NL : NM - NR;   // MFMAs they are spread over
     // with buf constant the compiler knows that a read of one stage does not wait for the loads
     // into the other

@@ -61,11 +61,9 @@ constexpr int GGROUP = 8;  // tile rows per group of the tile order (panel reuse
 // Split k (nsplit > 1, one item only): work-group z takes the z-th chunk of k
 // and writes its partial tile to P + z m n (ld m); k_gemm_reduce then adds the
 // partials in order and applies alpha, cs and beta.
-// V: bytes per lane of the loads.  16 (1 KB per wave instruction) with even leading
-// dimensions and strides, 16-byte aligned operands and, for an operand contiguous in
-// rows, an even row count; 4 (256 bytes) otherwise.  Rows past m (n) repeat the last
-// row (pair): they only reach products that are not stored.  A last stage with fewer
-// than 16 k goes through registers with zeros past kend.
+// Rows past m (n) repeat the last row (pair): they only reach products that are not
+// stored.  A last stage with fewer than 16 k, or whose loads would end past the
+// operand, goes through registers with zeros past kend.
 struct GemmArgs {
     int m, n, k;
     int mt, nt, ntiles;
@@ -84,7 +82,7 @@ struct GemmArgs {
     double *P;
 };
 
-template <bool TA, bool TB, int V>
+template <bool TA, bool TB>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_gemm_f64(const GemmArgs g) {
     constexpr bool KCA = TA, KCB = !TB;   // operand contiguous in k
     __shared__ __attribute__((aligned(16))) double sA0[gemm_lds<KCA>(GT)], sA1[gemm_lds<KCA>(GT)];
@@ -133,7 +131,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         for (int j = 0; j < 4; ++j) acc[i][j] = (d4_t){0.0, 0.0, 0.0, 0.0};
 
     if (kbeg < kend)
-        gemm_tile<KCA, KCB, V, GT>(acc, A, lda, m0, m, B, ldb, n0, n, kbeg, kend, g.far != 0, true,
+        gemm_tile<KCA, KCB, GT>(acc, A, lda, m0, m, B, ldb, n0, n, kbeg, kend, g.k, g.far != 0, true,
                                    sA0, sA1, sB0, sB1);
 
     if (g.nsplit > 1) {
@@ -232,16 +230,8 @@ int launch_gemm_f64_batched(brpa_ctx *ctx, bool ta, bool tb, int64_t m, int64_t 
     g.scs1 = scs1;
     g.scs2 = scs2;
     g.P = nullptr;
-    // 16 bytes per lane: aligned sources (even leading dimensions and strides, aligned
-    // bases) and 32-bit offsets within a tile; a rows-contiguous operand also needs
-    // an even row count, so that its last row pair lies inside the matrix.  Measured
-    // at 4097^3 with 4 bytes per lane: NN, NT, TT 51 TFLOP/s, TN 50 (through registers:
-    // 45 for all four)
+    // 32-bit byte offsets within a tile
     g.far = lda >= (1 << 21) || ldb >= (1 << 21);
-    const bool wide = lda % 2 == 0 && ldb % 2 == 0 && sA1 % 2 == 0 && sA2 % 2 == 0 &&
-                      sB1 % 2 == 0 && sB2 % 2 == 0 && (reinterpret_cast<uintptr_t>(A) & 15) == 0 &&
-                      (reinterpret_cast<uintptr_t>(B) & 15) == 0 && (ta || m % 2 == 0) &&
-                      (!tb || n % 2 == 0);
     // split k when the last wave of tiles would leave much of the chip idle:
     // the split count s (<= 8, chunks of >= 256 k) minimises the modelled time
     // 1/eff(s) + (reduction traffic), eff(s) = tiles s / (slots ceil(tiles s /
@@ -285,13 +275,13 @@ int launch_gemm_f64_batched(brpa_ctx *ctx, bool ta, bool tb, int64_t m, int64_t 
     BRPA_TRY(kstat_begin(ctx, &slot));
     auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, block, 0, ctx->stream, g); };
     if (!ta && !tb)
-        wide ? launch(k_gemm_f64<false, false, 16>) : launch(k_gemm_f64<false, false, 4>);
+        launch(k_gemm_f64<false, false>);
     else if (!ta && tb)
-        wide ? launch(k_gemm_f64<false, true, 16>) : launch(k_gemm_f64<false, true, 4>);
+        launch(k_gemm_f64<false, true>);
     else if (ta && !tb)
-        wide ? launch(k_gemm_f64<true, false, 16>) : launch(k_gemm_f64<true, false, 4>);
+        launch(k_gemm_f64<true, false>);
     else
-        wide ? launch(k_gemm_f64<true, true, 16>) : launch(k_gemm_f64<true, true, 4>);
+        launch(k_gemm_f64<true, true>);
     LAUNCH_CHECK(ctx);
     if (g.nsplit > 1) {
         hipLaunchKernelGGL(k_gemm_reduce, dim3((unsigned)((m * n + 255) / 256)), dim3(256), 0,

@@ -71,75 +71,49 @@ int launch_dtab(brpa_ctx *ctx, const FragDev *fr, const int64_t *pre, int nfrag,
 //   quad  (QUAD = true)   one frequency: wave (w/2, w%2) computes a 32x32 quadrant,
 //         for launches whose wide form would not fill the chip (syrk_quad)
 //
-// The stages go straight from global memory into LDS, double-buffered, rows of 64
-// doubles with the 16-double blocks of odd rows swapped in pairs, so that the four
-// lane groups of an operand read (four consecutive rows) hit both halves of the 64
-// banks.  An even N and a 16-byte aligned R take 16 bytes per lane (V = 16), others
-// 4 bytes (V = 4, four times the load instructions).  Columns past N repeat the last
-// one (pair): they only reach products that are not stored.  A last stage with fewer
-// than 16 rows goes through registers with zeros past K.  A diagonal tile needs one
-// panel and the blocks i >= j only.
+// The stages go straight from global memory into LDS (16 bytes per lane), double-buffered,
+// rows of 64 doubles with the 16-double blocks of odd rows swapped in pairs, so that the
+// four lane groups of an operand read (four consecutive rows) hit both halves of the 64
+// banks.  Columns past N repeat the last pair: they only reach products that are not
+// stored.  A last stage with fewer than 16 rows, or one whose loads would end past R,
+// goes through registers with zeros past K.  A diagonal tile needs one panel and the
+// blocks i >= j only.
 //
 // Bound by MFMA issue.  The reads of one half of a stage run while the other half is
 // multiplied, the barrier stands between the halves (as in k_gemm_f64).  Measured at
-// K = 19200, N = 2400, 16 frequencies: 64.1 TFLOP/s (56.2 with register-staged
-// stages between two barriers); K = 10800, N = 1800, 24 frequencies: 60.9 (51.1),
-// N = 1801: 59.3 (50.9).
+// K = 19200, N = 2400, 16 frequencies: 64.9 TFLOP/s (56.2 with register-staged
+// stages between two barriers).  A batch of 12 fragments, half of them with odd N: 23.9
+// ms with four bytes per lane for those, 23.4.
 constexpr int KB = 16;                    // rows of R per LDS stage
 constexpr int SYRK_P = KB * SYRK_T;       // doubles per panel stage
 
 struct SyrkPanel {
-    uint32_t off[4];   // V = 16: the two loads of a wave; V = 4: [half][row parity]
+    uint32_t off[2];   // the two loads of a wave
 };
 
 // byte offsets from R + k0 N + c0 of the lane's part of a wave's loads
-template <int V>
 __device__ __forceinline__ SyrkPanel syrk_panel(int N, int c0, int wave, int lane) {
     SyrkPanel p;
-    if (V == 16) {
 #pragma unroll
-        for (int t = 0; t < 2; ++t) {
-            const int kr = 4 * wave + 2 * t + (lane >> 5);
-            const int c = 2 * ((lane & 31) ^ (8 * (kr & 1)));
-            p.off[t] = 8u * ((uint32_t)kr * (uint32_t)N + (uint32_t)(min(c0 + c, N - 2) - c0));
-        }
-    } else {
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const int c = (32 * (q >> 1) + (lane >> 1)) ^ (16 * (q & 1));
-            p.off[q] = 8u * (uint32_t)(min(c0 + c, N - 1) - c0) + 4u * (lane & 1);
-        }
+    for (int t = 0; t < 2; ++t) {
+        const int kr = 4 * wave + 2 * t + (lane >> 5);
+        const int c = 2 * ((lane & 31) ^ (8 * (kr & 1)));
+        p.off[t] = 8u * ((uint32_t)kr * (uint32_t)N + (uint32_t)(min(c0 + c, (N - 1) & ~1) - c0));
     }
     return p;
 }
 
-template <int V>
-__device__ __forceinline__ void syrk_stage(const SyrkPanel &p, const char *base, int N, double *L,
-                                           int wave) {
+__device__ __forceinline__ void syrk_stage(const SyrkPanel &p, const char *base, double *L, int wave) {
 #if defined(__HIP_DEVICE_COMPILE__)
     typedef __attribute__((address_space(1))) const char gchar_t;
     typedef __attribute__((address_space(3))) void lvoid_t;
-    if (V == 16) {
 #pragma unroll
-        for (int t = 0; t < 2; ++t)
-            __builtin_amdgcn_global_load_lds(
-                (const __attribute__((address_space(1))) void *)((gchar_t *)base + p.off[t]),
-                (lvoid_t *)(L + (4 * wave + 2 * t) * SYRK_T), 16, 0, 0);
-    } else {
-#pragma unroll
-        for (int t = 0; t < 8; ++t) {
-            const int kr = 4 * wave + (t >> 1);
-            __builtin_amdgcn_global_load_lds(
-                (const __attribute__((address_space(1))) void *)((gchar_t *)base +
-                                                                 8 * (int64_t)N * kr +
-                                                                 p.off[2 * (t & 1) + ((t >> 1) & 1)]),
-                (lvoid_t *)(L + kr * SYRK_T + 32 * (t & 1)), 4, 0, 0);
-        }
-    }
+    for (int t = 0; t < 2; ++t)
+        __builtin_amdgcn_global_load_lds(
+            (const __attribute__((address_space(1))) void *)((gchar_t *)base + p.off[t]),
+            (lvoid_t *)(L + (4 * wave + 2 * t) * SYRK_T), 16, 0, 0);
 #endif
 }
-
-// rows k0 .. K - 1 (fewer than 16) of a panel, zeros below
 __device__ __forceinline__ void syrk_stage_tail(const double *__restrict__ R, int K, int N, int k0,
                                                 int c0, double *L, int tid) {
     const gdouble_t *G = (const gdouble_t *)R;
@@ -152,7 +126,7 @@ __device__ __forceinline__ void syrk_stage_tail(const double *__restrict__ R, in
     }
 }
 
-template <int V, bool QUAD, bool DIAG>
+template <bool QUAD, bool DIAG>
 __device__ __forceinline__ void syrk_f64_tile(const FragDev &F, int w0, int tp, int tq, int both,
                                               double *__restrict__ sA0, double *__restrict__ sA1,
                                               double *__restrict__ sB0, double *__restrict__ sB1) {
@@ -167,15 +141,17 @@ __device__ __forceinline__ void syrk_f64_tile(const FragDev &F, int w0, int tp, 
     // waves past the last frequency, and the quadrant above the diagonal, only stage
     const bool active = w < F.F && !(QUAD && DIAG && bj > bi);
     const int rl = lane & 15, g4 = lane >> 4;
-    const SyrkPanel pa = syrk_panel<V>(N, p0, wave, lane);
-    const SyrkPanel pb = DIAG ? pa : syrk_panel<V>(N, q0, wave, lane);
+    const SyrkPanel pa = syrk_panel(N, p0, wave, lane);
+    const SyrkPanel pb = DIAG ? pa : syrk_panel(N, q0, wave, lane);
     const char *ba = reinterpret_cast<const char *>(R + p0);
     const char *bb = reinterpret_cast<const char *>(R + q0);
-    const int nfull = K / KB, ns = (K + KB - 1) / KB;
+    // with an odd N the last column's pair of row K - 1 would end past R
+    const bool over = (N & 1) && p0 + SYRK_T > N;
+    const int nfull = (K - (over ? 1 : 0)) / KB, ns = (K + KB - 1) / KB;
     auto stage = [&](int buf, int q) {
         const int64_t o = 8 * (int64_t)N * (KB * q);
-        syrk_stage<V>(pa, ba + o, N, buf ? sA1 : sA0, wave);
-        if (!DIAG) syrk_stage<V>(pb, bb + o, N, buf ? sB1 : sB0, wave);
+        syrk_stage(pa, ba + o, buf ? sA1 : sA0, wave);
+        if (!DIAG) syrk_stage(pb, bb + o, buf ? sB1 : sB0, wave);
     };
     auto put = [&](int buf, int q) {
         if (q < nfull) {
@@ -266,7 +242,7 @@ __device__ __forceinline__ void syrk_f64_tile(const FragDev &F, int w0, int tp, 
         coef(d, q + 2, 0);
         stage(buf, q + 2);
         mma(a1, b1, d[2], d[3]);
-        constexpr int NL = 2 + (V == 16 ? 2 : 8) * (DIAG ? 1 : 2);
+        constexpr int NL = 2 + 2 * (DIAG ? 1 : 2);
         constexpr int NL1 = NL < NM - NR ? NL : NM - NR;
 #pragma unroll
         for (int u = 0; u < NR; ++u) {
@@ -338,18 +314,10 @@ k_syrk_f64(const FragDev *__restrict__ fr, const int64_t *__restrict__ pre, int 
     int tp, tq;
     tri_decode(pair, tp, tq);
     const int w0 = QUAD ? g : 4 * g;
-    const bool wide = F.N % 2 == 0 && (reinterpret_cast<uintptr_t>(F.R) & 15) == 0;
-    if (tp == tq) {
-        if (wide)
-            syrk_f64_tile<16, QUAD, true>(F, w0, tp, tq, both, sA0, sA1, sB0, sB1);
-        else
-            syrk_f64_tile<4, QUAD, true>(F, w0, tp, tq, both, sA0, sA1, sB0, sB1);
-    } else {
-        if (wide)
-            syrk_f64_tile<16, QUAD, false>(F, w0, tp, tq, both, sA0, sA1, sB0, sB1);
-        else
-            syrk_f64_tile<4, QUAD, false>(F, w0, tp, tq, both, sA0, sA1, sB0, sB1);
-    }
+    if (tp == tq)
+        syrk_f64_tile<QUAD, true>(F, w0, tp, tq, both, sA0, sA1, sB0, sB1);
+    else
+        syrk_f64_tile<QUAD, false>(F, w0, tp, tq, both, sA0, sA1, sB0, sB1);
 }
 
 int64_t syrk_items(int64_t N, int64_t F, bool quad) {
@@ -1264,12 +1232,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
     for (int i = 0; i < NB; ++i)
 #pragma unroll
         for (int j = 0; j < NB; ++j) acc[i][j] = (d4_t){0.0, 0.0, 0.0, 0.0};
-    if (N % 2 == 0 && (reinterpret_cast<uintptr_t>(A) & 15) == 0)
-        gemm_tile<true, true, 16, T>(acc, A, N, Rj, N, A, N, Ri, N, kbase, t0, false, active, sA0, sA1,
-                                     sB0, sB1);
-    else
-        gemm_tile<true, true, 4, T>(acc, A, N, Rj, N, A, N, Ri, N, kbase, t0, false, active, sA0, sA1,
-                                     sB0, sB1);
+    gemm_tile<true, true, T>(acc, A, N, Rj, N, A, N, Ri, N, kbase, t0, t0, false, active, sA0, sA1, sB0,
+                             sB1);
     if (!active) return;
     gdouble_mut_t *C = (gdouble_mut_t *)A;
 #pragma unroll
