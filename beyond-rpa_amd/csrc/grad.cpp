@@ -9,31 +9,22 @@
 // The frequency grid is held fixed.  Pi_k is recomputed here (FP64 MFMA SYRK),
 // not kept from the forward pass.  (1 + Pi_k)^{-1} = U_k^{-1} U_k^{-T} for all k
 // at once: the library's batched blocked Cholesky (1 + Pi_k = U_k^T U_k, U_k the
-// column-major upper triangle), rocBLAS's batched triangular inverse and one
-// strided-batched dgemm; then R (1 + Pi_k)^{-1} by one dgemm per frequency.
-#include <rocblas/rocblas.h>
-
+// column-major upper triangle), its batched triangular inverse and one batched product of
+// triangles; then R (1 + Pi_k)^{-1} by one product per frequency.
 #include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <vector>
 
-#include "internal.h"
+#include "dense.h"
 
 int launch_grad_acc(brpa_ctx *, const double *X, const double *Rc, int64_t N, int64_t K,
                     const double *c, const double *dc, double coef, double *dR, double *dd);
 int launch_fill(brpa_ctx *, double *p, int64_t n, double v);
-int rocblas_handle_of(brpa_ctx *ctx, void **h);
-int launch_zero_lower(brpa_ctx *, double *M, int64_t n);
 
 namespace {
 constexpr double kPi = 3.14159265358979323846;
 int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
-int rb(brpa_ctx *ctx, rocblas_status st, const char *what) {
-    if (st != rocblas_status_success)
-        return brpa_fail(ctx, BRPA_ERR_SOLVER, "%s failed: rocblas status %d", what, (int)st);
-    return BRPA_OK;
-}
 }  // namespace
 
 extern "C" int brpa_ecrpa_grad(brpa_ctx *ctx, const double *R, int64_t naux, const double *eocc,
@@ -64,9 +55,6 @@ extern "C" int brpa_ecrpa_grad(brpa_ctx *ctx, const double *R, int64_t naux, con
     if (!(*std::min_element(ev.begin(), ev.end()) - *std::max_element(eo.begin(), eo.end()) > 0.0))
         return brpa_fail(ctx, BRPA_ERR_GAP, "Found invalid orbital energy gap.");
     BRPA_HIP(ctx, hipSetDevice(ctx->device));
-    void *hv_ = nullptr;
-    BRPA_TRY(rocblas_handle_of(ctx, &hv_));
-    rocblas_handle h = static_cast<rocblas_handle>(hv_);
 
     // c_k and dc_k/dd per (k, ai)
     std::vector<double> cc(F * K), dcc(F * K);
@@ -90,6 +78,8 @@ extern "C" int brpa_ecrpa_grad(brpa_ctx *ctx, const double *R, int64_t naux, con
     double *dRd, *ddR, *dc, *ddc, *X, *dd;
     double *Uinv;
     int64_t *dchol;
+    // matrices per batch of the triangular inverse: its scratch is X
+    const int64_t nbi = std::max<int64_t>(1, std::min(F, K * N / trinv_scratch(N)));
     auto layout = [&](Arena &ar) {
         dfd = ar.take<FragDev>(1);
         dpre = ar.take<int64_t>(pre.size());
@@ -104,7 +94,7 @@ extern "C" int brpa_ecrpa_grad(brpa_ctx *ctx, const double *R, int64_t naux, con
         fd.evir = ar.take<double>(nvir);
         dc = ar.take<double>(F * K);
         ddc = ar.take<double>(F * K);
-        X = ar.take<double>(K * N);
+        X = ar.take<double>(std::max(K * N, nbi * trinv_scratch(N)));
         dd = ar.take<double>(K);
         fd.linv = ar.take<double>(F * CHOL_NB * CHOL_NB);
         fd.ldpart = ar.take<double>(F * nsteps * 2);
@@ -147,28 +137,19 @@ extern "C" int brpa_ecrpa_grad(brpa_ctx *ctx, const double *R, int64_t naux, con
     BRPA_TRY(launch_fill(ctx, dd, K, 0.0));
     BRPA_TRY(launch_fill_int(ctx, fd.status, F, 0));
     BRPA_TRY(chol_single(ctx, dfd, dchol, N, F));
-    BRPA_TRY(rb(ctx,
-                rocblas_dtrtri_strided_batched(h, rocblas_fill_upper, rocblas_diagonal_non_unit,
-                                               (rocblas_int)N, fd.Pi, (rocblas_int)N, N * N, Uinv,
-                                               (rocblas_int)N, N * N, (rocblas_int)F),
-                "rocblas_dtrtri_strided_batched"));
-    for (int64_t k = 0; k < F; ++k) BRPA_TRY(launch_zero_lower(ctx, Uinv + k * N * N, N));
-    // M_k = U_k^{-1} U_k^{-T} (full, symmetric) in place of Pi_k
-    const double one = 1.0, zero = 0.0;
-    BRPA_TRY(rb(ctx,
-                rocblas_dgemm_strided_batched(h, rocblas_operation_none, rocblas_operation_transpose,
-                                              (rocblas_int)N, (rocblas_int)N, (rocblas_int)N, &one,
-                                              Uinv, (rocblas_int)N, N * N, Uinv, (rocblas_int)N,
-                                              N * N, &zero, fd.Pi, (rocblas_int)N, N * N,
-                                              (rocblas_int)F),
-                "rocblas_dgemm_strided_batched"));
+    // M_k = U_k^{-1} U_k^{-T} in place of Pi_k: the batched triangular inverse, and of
+    // each product the tiles on or above the diagonal, from k = their column on
+    for (int64_t k = 0; k < F; k += nbi)
+        BRPA_TRY(dense_trinv(ctx, N, fd.Pi + k * N * N, N, N * N, Uinv + k * N * N, N, N * N,
+                             std::min(nbi, F - k), X));
+    BRPA_TRY(launch_gemm_f64_batched(ctx, false, true, N, N, N, 1.0, Uinv, N, N * N, 0, Uinv, N,
+                                     N * N, 0, 0.0, fd.Pi, N, N * N, 0, F, 1, true, TRI_B_LOWER,
+                                     nullptr, 0, 0));
     for (int64_t k = 0; k < F; ++k) {
         // X(N x K) = M_k Rc
-        BRPA_TRY(rb(ctx,
-                    rocblas_dgemm(h, rocblas_operation_none, rocblas_operation_none, (rocblas_int)N,
-                                  (rocblas_int)K, (rocblas_int)N, &one, fd.Pi + k * N * N,
-                                  (rocblas_int)N, dRd, (rocblas_int)N, &zero, X, (rocblas_int)N),
-                    "rocblas_dgemm"));
+        double *M = fd.Pi + k * N * N;
+        BRPA_TRY(dense_symm_fill(ctx, M, N));
+        BRPA_TRY(dense_gemm(ctx, true, false, N, K, N, 1.0, M, N, dRd, N, 0.0, X, N));
         BRPA_TRY(launch_grad_acc(ctx, X, dRd, N, K, dc + k * K, ddc + k * K,
                                  fw[k] / (2.0 * kPi), ddR, dd));
     }
