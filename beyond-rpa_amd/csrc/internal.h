@@ -231,7 +231,7 @@ int launch_set_diag(brpa_ctx *, const FragDev *, const int64_t *pre, int nfrag, 
 // Blocked Cholesky of every matrix of the fragments.  Work-groups per fragment, list
 // and 64-column step: chol_items; d_pre / h_pre: their prefix sums over the fragments on
 // the device and the host, [list][step][nfrag + 1].
-enum { CHOL_DIAG, CHOL_TRSM, CHOL_STRIP, CHOL_REST, CHOL_STEP, CHOL_NLISTS };
+enum { CHOL_DIAG, CHOL_PANEL, CHOL_REST, CHOL_STEP, CHOL_NLISTS };
 int64_t chol_items(int list, int64_t N, int64_t F, int64_t j);
 int launch_cholesky(brpa_ctx *, const FragDev *, int nfrag, int nsteps, const int64_t *d_pre,
                     const int64_t *h_pre);

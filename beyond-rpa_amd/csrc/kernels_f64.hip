@@ -6,8 +6,8 @@
 //                  frequency's tile  (dgemm of rpa_core_MO.f90:402)
 //   k_set_diag     diag_w (tr Pi, rpa_CC.f90:444-447); Pi_w[P][P] += 1 (448-450)
 //   k_potrf_diag   Cholesky + inverse of a 64x64 diagonal block (four waves)
-//   k_trsm         L21 = A21 L11^{-T} on MFMA
-//   k_chol_strip, k_chol_rest  trailing updates A22 -= L21 L21^T on MFMA
+//   k_chol_panel   left-looking update of a 64-column strip and L21 = B L11^{-T}
+//   k_chol_rest    rank-256 update of the rest of the trailing matrix
 //   k_chol_step    diagonal block, left-looking strip and L21 of a step in one launch
 //   k_energy       E = sum_w w/(2 pi) (2 sum log L_kk - tr Pi_w)  (rpa_CC.f90:451-453)
 //
@@ -444,44 +444,15 @@ int launch_set_diag(brpa_ctx *ctx, const FragDev *fr, const int64_t *pre, int nf
 
 // ---------------------------------------------------------------------------
 // Blocked Cholesky of A_w = 1 + Pi_w (lower triangle, row-major) in 64-column steps j
-// (j0 = 64 j), one launch per step for few matrices (k_chol_step), else three:
+// (j0 = 64 j), one launch per step for few matrices (k_chol_step), else two:
 //   k_potrf_diag   one work-group per matrix: factors the diagonal block in LDS,
 //                  writes its log-det partial and L11^{-1} (own buffer; A11
 //                  itself is never written back, so no work-group of the same
 //                  step can read a half-factored block)
-//   k_trsm         L21 = A21 L11^{-T} as a 64x64x64 MFMA product per row chunk
-//   k_chol_strip   the next 64 columns of A22 -= L21 L21^T over the outer panel
+//   k_chol_panel   64 rows of the step's columns: the outer panel's earlier columns
+//                  applied, then L21
 // and after every outer panel of four steps k_chol_rest, the rest of A22 (launch_cholesky).
 // Work-groups per fragment: chol_items.
-
-// C(64x64) = X Y^T with X, Y 64x64 in LDS; wave (qi,qj) owns a 32x32 quadrant,
-// acc[i][j][r] = C[32 qi + 16 i + l/16 + 4 r][32 qj + 16 j + l%16].
-// X Y^T of two 64 x 64 LDS panels on MFMA, 4 waves of 32 x 32 (wave = tid / 64 < 4).
-__device__ __forceinline__ void mma64_xyt(const double (*sX)[CHOL_NB + 1],
-                                          const double (*sY)[CHOL_NB + 1], d4_t acc[2][2],
-                                          int tid) {
-    const int wave = tid >> 6, lane = tid & 63;
-    const int qi = wave >> 1, qj = wave & 1;
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) acc[i][j] = (d4_t){0.0, 0.0, 0.0, 0.0};
-#pragma unroll 4
-    for (int kk = 0; kk < CHOL_NB; kk += 4) {
-        const int kc = kk + (lane >> 4);
-        double a[2], bv[2];
-#pragma unroll
-        for (int i = 0; i < 2; ++i) a[i] = sX[32 * qi + 16 * i + (lane & 15)][kc];
-#pragma unroll
-        for (int j = 0; j < 2; ++j) bv[j] = sY[32 * qj + 16 * j + (lane & 15)][kc];
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-#pragma unroll
-            for (int j = 0; j < 2; ++j)
-                acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i], bv[j], acc[i][j], 0, 0, 0);
-    }
-}
-
 
 template <int ROWS, int THREADS, int NP>
 __device__ __forceinline__ void load_panels64(double (*const *s)[CHOL_NB + 1],
@@ -523,43 +494,7 @@ __device__ __forceinline__ void load_panel64(double (*s)[CHOL_NB + 1], const dou
 // calls the body (the barriers are uniform) and the work is guarded by the
 // thread index.
 
-// L21 chunk r (rows j0 + 64 r ..) of step `step`: L21 = A21 L11^{-T} on MFMA
-// (waves 0..3).  sB, sL: [64][65] LDS.
-template <int NT>
-__device__ __forceinline__ void trsm_body(const FragDev &F, int w, int step, int r, double (*sB)[CHOL_NB + 1],
-                          double (*sL)[CHOL_NB + 1], int tid) {
-    static_assert(NT >= 256 && NT % 256 == 0, "work-group too small");
-    const int N = F.N;
-    const int j0 = step * CHOL_NB;
-    double *A = F.Pi + (int64_t)w * N * N;
-    const double *linv = F.linv + (int64_t)w * CHOL_NB * CHOL_NB;
-    const int R0 = j0 + CHOL_NB * r;
-    load_panel64<CHOL_NB, NT>(sB, A, N, R0, N, j0, N, tid);
-    load_panel64<CHOL_NB, NT>(sL, linv, CHOL_NB, 0, CHOL_NB, 0, CHOL_NB, tid);
-    __syncthreads();
-    if (tid < 256) {
-        d4_t acc[2][2];
-        mma64_xyt(sB, sL, acc, tid);   // L21[i][c] = sum_k A21[i][k] Linv[c][k]
-        const int wave = tid >> 6, lane = tid & 63, qi = wave >> 1, qj = wave & 1;
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-#pragma unroll
-            for (int j = 0; j < 2; ++j)
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    int row = R0 + 32 * qi + 16 * i + (lane >> 4) + 4 * q;
-                    int col = 32 * qj + 16 * j + (lane & 15);
-                    if (row < N) A[(int64_t)row * N + j0 + col] = acc[i][j][q];
-                }
-    }
-}
-
 // Number of L21 chunks of step j.
-__device__ __forceinline__ int trsm_chunks(int N, int j) {
-    const int j0 = j * CHOL_NB;
-    return N > j0 + CHOL_NB ? (N - j0 + CHOL_NB - 1) / CHOL_NB - 1 : 0;
-}
-
 // ---------------------------------------------------------------------------
 // Per-step kernels (flat work lists over fragments and frequencies)
 
@@ -843,8 +778,8 @@ __global__ __launch_bounds__(256) void k_potrf_diag(const FragDev *__restrict__ 
 // s_in, operands straight from L2).  Then L21 = B L11^{-T}, and the work-groups
 // within the outer panel bring their own diagonal block up to date, so that the
 // next step finds it complete.
-// 14 us for the first step of an outer panel, 18 us for the fourth (k_potrf_diag, k_trsm
-// and k_chol_strip: 37 to 51 us at N = 400).
+// 14 us for the first step of an outer panel, 18 us for the fourth (in three launches 37 to
+// 51 us at N = 400).
 // r = 0 writes the log-det partial and the status.  No work-group may see a half-factored
 // block, so with keep_l11 it leaves L11 in linv and copies it into Pi in the next
 // step (pend: the previous step did so); the matrix's last step writes it at once.
@@ -1036,164 +971,117 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     }
 }
 
-__global__ __launch_bounds__(256) void k_trsm(const FragDev *__restrict__ fr,
-                                             const int64_t *__restrict__ pre, int nfrag, int step) {
-    __shared__ double sB[CHOL_NB][CHOL_NB + 1];
-    __shared__ double sL[CHOL_NB][CHOL_NB + 1];
-    __shared__ int64_t s_pre[FIND_LDS_MAX + 1];
-    const int64_t b = blockIdx.x;
-    const int f = find_frag_lds(pre, nfrag, b, s_pre);
-    const FragDev &F = fr[f];
-    const int nsub = trsm_chunks(F.N, step);
-    const int64_t lb = b - (nfrag <= FIND_LDS_MAX ? s_pre[f] : pre[f]);
-    const int w = (int)(lb / nsub), r = 1 + (int)(lb - (int64_t)w * nsub);
-    trsm_body<256>(F, w, step, r, sB, sL, threadIdx.x);
-}
-
-// Trailing updates.  Outer panels of CHOL_OUTER steps (256 columns): step s of an outer
-// panel (s = step % CHOL_OUTER) updates, for s < CHOL_OUTER - 1, only the next
-// 64-column strip (rows >= t0 = j0 + 64, columns t0 .. t0+63) with the panels of steps
-// step-s .. step (rank 64 (s+1): the strip has seen no panel of this outer panel yet;
-// k_chol_strip); the last step updates the rest of the trailing matrix with all
-// CHOL_OUTER panels (rank 256; k_chol_rest), so A22 is read and written once per outer
-// panel.
-constexpr int UPD_T = 128;   // strip rows per work-group
-constexpr int REST_T = 64;   // tile edge of the rest
-constexpr int UPD_KH = 16;   // panel columns per LDS phase
-
-// A 128 x 64 piece of the strip, the four waves as 2 x 2 blocks of 64 x 32, C preloaded
-// into the accumulators.  The panels pass through LDS in phases of 16 columns as
-// [row][k] (pitch 18 doubles), double-buffered with one barrier per phase; every thread
-// moves pairs of consecutive columns (one ds_write_b128), and in a phase lane group
-// l/16 supplies the k values 4 (l/16) .. +3 of its row to the four MFMA steps (a
-// permutation of the phase's k, the same for both operands), two ds_read_b128 per
-// 16-row block.  The MFMA takes the P_i fragment first, so the accumulator columns run
-// along the lanes and the row-major C is read and written coalesced.
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_chol_strip(
+// One step's 64 rows from j0 + 64 r of its 64 columns, for launches of many matrices (the
+// diagonal block is k_potrf_diag's): B = A - sum P_r P_d^T over the outer panel's earlier
+// columns by the loop of k_gemm_f64 (left-looking, rank 64 s_in), L21 = B L11^{-T} with the
+// inverse in LDS, and within the outer panel the update of the work-group's own diagonal
+// block, so that the next k_potrf_diag finds it complete.  B passes from the product to the
+// solve in the product's stage buffers, 16 rows in each: 66 KB of LDS, two
+// work-groups per CU.  Bound by the latencies between its short phases: 32 fragments of
+// the batch shapes, 20 launches, 3.1 ms (a strip kernel that kept C in memory and a
+// triangular solve of its own: 4.0 ms).
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_chol_panel(
     const FragDev *__restrict__ fr, const int64_t *__restrict__ pre, int nfrag, int step) {
-    constexpr int WC = 32;                 // columns per wave
-    constexpr int NJ = WC / 16;            // 16-column MFMA blocks per wave
-    constexpr int KPU = UPD_KH + 2;
-    __shared__ __attribute__((aligned(16))) double sI[2][UPD_T * KPU];
-    __shared__ __attribute__((aligned(16))) double sJ[2][CHOL_NB * KPU];
-    __shared__ int64_t s_pre[FIND_LDS_MAX + 1];
-    int64_t b = blockIdx.x;
-    int f = find_frag_lds(pre, nfrag, b, s_pre);
+    constexpr int T = CHOL_NB;
+    static_assert(gemm_lds<true>(T) == 16 * T, "a stage buffer holds 16 rows of B");
+    __shared__ __attribute__((aligned(16))) double sA0[gemm_lds<true>(T)], sA1[gemm_lds<true>(T)];
+    __shared__ __attribute__((aligned(16))) double sB0[gemm_lds<true>(T)], sB1[gemm_lds<true>(T)];
+    __shared__ __attribute__((aligned(16))) double sL[T][CH_LP];
+    const int64_t b = blockIdx.x;
+    const int f = __builtin_amdgcn_readfirstlane(find_frag(pre, nfrag, b));
     const FragDev &F = fr[f];
     const int N = F.N;
     const int j0 = step * CHOL_NB;
-    const int t0 = j0 + CHOL_NB;
-    const int nt = (N - t0 + UPD_T - 1) / UPD_T;
-    const int s_in = step % CHOL_OUTER;
-    const int kbase = j0 - s_in * CHOL_NB;    // first panel column
-    const int nph = (s_in + 1) * CHOL_NB / UPD_KH;
-    const int colmax = min(N, t0 + CHOL_NB);   // C columns < colmax
-    int64_t lb = b - (nfrag <= FIND_LDS_MAX ? s_pre[f] : pre[f]);
-    const int w = (int)(lb / nt), ti = (int)(lb - (int64_t)w * nt);
+    const int nrb = (N - j0 + CHOL_NB - 1) / CHOL_NB - 1;
+    const int64_t lb = b - pre[f];
+    const int w = __builtin_amdgcn_readfirstlane((int)(lb / nrb));
+    const int rb = 1 + __builtin_amdgcn_readfirstlane((int)(lb - (int64_t)w * nrb));
+    const int R0 = j0 + CHOL_NB * rb;
+    const int s_in = step % CHOL_OUTER, kbase = j0 - s_in * CHOL_NB;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int l16 = lane & 15, g4 = lane >> 4, wm = wave >> 1, wn = wave & 1;
     double *A = F.Pi + (int64_t)w * N * N;
-    const gdouble_t *G = (const gdouble_t *)A;
-    const int Ri = t0 + UPD_T * ti, Rj = t0;
-    const int tid = threadIdx.x;
-    const int wave = tid >> 6, lane = tid & 63;
-    const int wm = wave >> 1, wn = wave & 1;   // rows 64*wm.., cols WC*wn..
-    const int r0 = 64 * wm, c0 = WC * wn;
-    const bool active = Ri + r0 < N && Rj + c0 < colmax;
-
-    // phase h (h < nph): rows Ri.. (128) / Rj.. (64) x columns kbase + 16 h .. + 16
-    // (all < t0 <= N); pair q = tid + 256 u: row q / 8, columns 2 (q % 8) + {0, 1}
-    d2v_t vi[4], vj[2];
-    auto gload = [&](int h) {
+    gdouble_mut_t *G = (gdouble_mut_t *)A;
+    const gdouble_t *linv = (const gdouble_t *)F.linv + (int64_t)w * CHOL_NB * CHOL_NB;
+    // B in accumulator layout: row 32 wn + 16 j + g4 + 4 r, column 32 wm + 16 i + l16
+    d4_t a[2][2], acc[2][2];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int q = tid + 256 * u;
-            const int r = q >> 3, col = kbase + UPD_KH * h + 2 * (q & 7);
-            const bool oki = Ri + r < N, okj = Rj + r < N;
-            const gdouble_t *pi = G + (oki ? (int64_t)(Ri + r) * N + col : 0);
-            const double i0 = pi[0], i1 = pi[1];
-            vi[u].x = oki ? i0 : 0.0;
-            vi[u].y = oki ? i1 : 0.0;
-            if (u < 2) {
-                const gdouble_t *pj = G + (okj ? (int64_t)(Rj + r) * N + col : 0);
-                const double ja = pj[0], jb = pj[1];
-                vj[u].x = okj ? ja : 0.0;
-                vj[u].y = okj ? jb : 0.0;
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int row = min(R0 + 32 * wn + 16 * j + g4 + 4 * r, N - 1);
+                a[i][j][r] = G[(int64_t)row * N + j0 + 32 * wm + 16 * i + l16];
+                acc[i][j][r] = 0.0;
             }
-        }
-    };
-    auto lstore = [&](int buf) {
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int q = tid + 256 * u;
-            const int o = (q >> 3) * KPU + 2 * (q & 7);
-            *reinterpret_cast<d2v_t *>(&sI[buf][o]) = vi[u];
-            if (u < 2) *reinterpret_cast<d2v_t *>(&sJ[buf][o]) = vj[u];
-        }
-    };
-
-    gload(0);
-    lstore(0);
-    __syncthreads();
-    if (nph > 1) gload(1);
-    // the C tile into the accumulators: element (row r0 + 16 i + lane/16 + 4 q, col c0 +
-    // 16 j + lane%16) (out-of-range / upper elements read A[0], then 0)
-    d4_t acc[4][NJ];
+    for (int r = 0; r < 16; ++r) sL[4 * r + wave][lane] = linv[(4 * r + wave) * CHOL_NB + lane];
+    if (s_in > 0)
+        gemm_tile<true, true, T>(acc, A, N, j0, N, A, N, R0, N, kbase, j0, j0, false, true, sA0, sA1, sB0,
+                                 sB1);
+    __syncthreads();   // the stage buffers are read
+    // row q of B's block row c, columns XOR-swizzled by 4 q
+    auto rows = [&](int c) { return c < 2 ? (c == 0 ? sA0 : sA1) : (c == 2 ? sB0 : sB1); };
+    auto at = [](int q, int col) { return q * CHOL_NB + (col ^ (4 * q)); };
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int j = 0; j < 2; ++j) {
+        double *L = rows(2 * wn + j);
 #pragma unroll
-        for (int j = 0; j < NJ; ++j)
+        for (int i = 0; i < 2; ++i)
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const int row = Ri + r0 + 16 * i + (lane >> 4) + 4 * q;
-                const int col = Rj + c0 + 16 * j + (lane & 15);
-                const bool ok = active && row < N && col < colmax && col <= row;
-                const double v = G[ok ? (int64_t)row * N + col : 0];
-                acc[i][j][q] = ok ? v : 0.0;
-            }
-    const int kq = 4 * (lane >> 4), rl = lane & 15;
-    int buf = 0;
-    for (int h = 0; h < nph; ++h, buf ^= 1) {
-        if (active) {
-            // two halves of two MFMA steps (one ds_read_b128 per operand block
-            // and half: the register budget)
-#pragma unroll
-            for (int hh = 0; hh < 2; ++hh) {
-                d2v_t a[4], bv[NJ];
-#pragma unroll
-                for (int i = 0; i < 4; ++i)
-                    a[i] = -*reinterpret_cast<const d2v_t *>(
-                        &sI[buf][(r0 + 16 * i + rl) * KPU + kq + 2 * hh]);
-#pragma unroll
-                for (int j = 0; j < NJ; ++j)
-                    bv[j] = *reinterpret_cast<const d2v_t *>(
-                        &sJ[buf][(c0 + 16 * j + rl) * KPU + kq + 2 * hh]);
-#pragma unroll
-                for (int st = 0; st < 2; ++st)
-#pragma unroll
-                    for (int i = 0; i < 4; ++i)
-#pragma unroll
-                        for (int j = 0; j < NJ; ++j)
-                            acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i][st], bv[j][st],
-                                                                             acc[i][j], 0, 0, 0);
-            }
-        }
-        // the other buffer was last read before the previous barrier
-        if (h + 1 < nph) lstore(buf ^ 1);
-        __syncthreads();
-        if (h + 2 < nph) gload(h + 2);
+            for (int r = 0; r < 4; ++r)
+                L[at(g4 + 4 * r, 32 * wm + 16 * i + l16)] = a[i][j][r] - acc[i][j][r];
     }
-    if (!active) return;
+    __syncthreads();
+    // block row `wave` of L21, transposed: X_c = sum_{k <= c} L11^{-1}(c, k) B_k^T
+    double *own = rows(wave);
+    d4_t bt[4], x[4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int c = 0; c < 4; ++c)
 #pragma unroll
-        for (int j = 0; j < NJ; ++j)
+        for (int r = 0; r < 4; ++r) bt[c][r] = own[at(l16, 16 * c + g4 + 4 * r)];
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const int row = Ri + r0 + 16 * i + (lane >> 4) + 4 * q;
-                const int col = Rj + c0 + 16 * j + (lane & 15);
-                if (row < N && col < colmax && col <= row)
-                    ((gdouble_mut_t *)A)[(int64_t)row * N + col] = acc[i][j][q];
-            }
+    for (int c = 0; c < 4; ++c) {
+        x[c] = (d4_t){0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int k = 0; k <= c; ++k)
+#pragma unroll
+            for (int s = 0; s < 4; ++s)
+                x[c] = __builtin_amdgcn_mfma_f64_16x16x4f64(sL[16 * c + l16][16 * k + 4 * s + g4],
+                                                            bt[k][s], x[c], 0, 0, 0);
+    }
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) own[at(l16, 16 * c + g4 + 4 * r)] = x[c][r];
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+        const int row = R0 + 16 * wave + r;
+        if (row < N) G[(int64_t)row * N + j0 + lane] = own[at(r, lane)];
+    }
+    if (rb > CHOL_OUTER - 1 - s_in) return;
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        if (j > wave) break;
+        const double *oj = rows(j);
+        d4_t t = (d4_t){0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int s = 0; s < 16; ++s)
+            t = __builtin_amdgcn_mfma_f64_16x16x4f64(own[at(l16, 4 * s + g4)], oj[at(l16, 4 * s + g4)], t,
+                                                     0, 0, 0);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int row = R0 + 16 * wave + g4 + 4 * r, col = R0 + 16 * j + l16;
+            if (row < N && col <= row) G[(int64_t)row * N + col] -= t[r];
+        }
+    }
 }
+
+constexpr int REST_T = 64;   // tile edge of the rest
 
 // Rank-256 update of the trailing matrix, one 64 x 64 tile (ti >= tj) per work-group:
 // C -= P_i P_j^T by the loop of k_gemm_f64 (both panels are rows of A, contiguous in
@@ -1255,8 +1143,7 @@ int64_t chol_items(int list, int64_t N, int64_t F, int64_t j) {
     auto tiles = [&](int64_t t) { return N > t0 ? (N - t0 + t - 1) / t : 0; };
     switch (list) {
     case CHOL_DIAG: return N > j0 ? F : 0;
-    case CHOL_TRSM: return F * tiles(CHOL_NB);
-    case CHOL_STRIP: return rest ? 0 : F * tiles(UPD_T);
+    case CHOL_PANEL: return F * tiles(CHOL_NB);
     case CHOL_REST: return rest ? F * tiles(REST_T) * (tiles(REST_T) + 1) / 2 : 0;
     default: return N > j0 ? F * (1 + tiles(CHOL_NB)) : 0;   // CHOL_STEP
     }
@@ -1278,7 +1165,7 @@ int launch_cholesky(brpa_ctx *ctx, const FragDev *fr, int nfrag, int nsteps, con
         };
         // From the first outer panel on whose steps have at most four work-groups per CU (two
         // rounds of the resident ones) one launch per step.  ERPA of N = 400 / 16 matrices,
-        // N = 1053 / 16 and N = 1800 / 24: 411, 2762 and 7471 us with three launches throughout,
+        // N = 1053 / 16 and N = 1800 / 24: 411, 2762 and 7471 us with separate launches throughout,
         // 333, 2524 and 7254 us with a line at two per CU, 333, 2526 and 7163 us at four,
         // no different at eight and sixteen.
         if (j % CHOL_OUTER == 0 && !fused) fused = total(CHOL_STEP) <= 4 * ncu;
@@ -1287,8 +1174,7 @@ int launch_cholesky(brpa_ctx *ctx, const FragDev *fr, int nfrag, int nsteps, con
             pend = true;
         } else {
             BRPA_TRY(launch(k_potrf_diag, CHOL_DIAG));
-            BRPA_TRY(launch(k_trsm, CHOL_TRSM));
-            BRPA_TRY(launch(k_chol_strip, CHOL_STRIP));
+            BRPA_TRY(launch(k_chol_panel, CHOL_PANEL));
         }
         BRPA_TRY(launch(k_chol_rest, CHOL_REST));
     }
