@@ -379,8 +379,8 @@ def bench_thc(a):
     pi_flops = syrk_flops(o, v, n, nf)
     r_tf = r_flops / (st_r * 1e-3) / 1e12
     pi_tf = pi_flops / (st_pi * 1e-3) / 1e12
-    dom = ("k_syrk_f64", pi_tf, st_pi) if st_pi >= st_r else ("k_thc_r", r_tf, st_r)
-    oth = ("k_thc_r", r_tf, st_r) if dom[0] == "k_syrk_f64" else ("k_syrk_f64", pi_tf, st_pi)
+    dom = ("k_syrk_f64", pi_tf, st_pi) if st_pi >= st_r else ("k_gemm_f64", r_tf, st_r)
+    oth = ("k_gemm_f64", r_tf, st_r) if dom[0] == "k_syrk_f64" else ("k_syrk_f64", pi_tf, st_pi)
     out = {"metric": "THC-route Pi(u) build (R from the THC factors, then Pi of all 16 "
                      "frequencies) of one fragment o=36, v=300, NAux=1800, NGridTHC=4032",
            "value": round(dt * 1e3, 3), "unit": "ms", "n_gpus": 1, "steps": a.steps,

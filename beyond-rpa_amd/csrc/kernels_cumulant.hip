@@ -175,7 +175,7 @@ __global__ __launch_bounds__(256) void k_thc_1b2g_reduce(const double *__restric
 __global__ __launch_bounds__(256) void k_thc_pairs(const double *__restrict__ Y,
                                                    const double *__restrict__ X, int G, int v,
                                                    double *__restrict__ P, int64_t ldp) {
-    const int g = blockIdx.x * 256 + threadIdx.x, c = blockIdx.y;
+    const int g = blockIdx.y * 256 + threadIdx.x, c = blockIdx.x;
     if (g >= G) return;
     const int j = c / v, a = c - j * v;
     P[g + ldp * c] = Y[g + (int64_t)G * a] * X[g + (int64_t)G * j];
@@ -331,7 +331,7 @@ __global__ __launch_bounds__(256) void k_thc_terms(const double *__restrict__ pa
 
 int launch_thc_pairs(brpa_ctx *ctx, const double *Y, const double *X, int64_t G, int64_t v,
                      int64_t o, double *P, int64_t ldp) {
-    hipLaunchKernelGGL(k_thc_pairs, dim3((unsigned)((G + 255) / 256), (unsigned)(v * o)), dim3(256),
+    hipLaunchKernelGGL(k_thc_pairs, dim3((unsigned)(v * o), (unsigned)((G + 255) / 256)), dim3(256),
                        0, ctx->stream, Y, X, (int)G, (int)v, P, ldp);
     LAUNCH_CHECK(ctx);
     return BRPA_OK;

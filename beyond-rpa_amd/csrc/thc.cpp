@@ -4,19 +4,21 @@
 //
 // The reference walks ai in blocks of MaxBlockDim to bound its memory: per
 // block it forms Xgab = Xga o Xgi (ngrid x block), R_block = Zgk^T Xgab, and
-// one dgemm per frequency.  Here R is produced whole, once, into HBM by
-// k_thc_r (the Hadamard product formed in the operand loader), and all
-// frequencies of Pi(u) come from one FP64 MFMA SYRK launch that stages each R
-// tile once for four frequencies (k_syrk_f64).
+// one dgemm per frequency.  Here R is produced whole, once, into HBM: the products
+// X(g, a) X(g, i) of as many occupied i as fit 512 MB (k_thc_pairs), then R by the
+// library's GEMM (at o = 36, v = 300, N = 1800, 4032 grid points 2.5 ms; a kernel that
+// formed the products in its operand loader, between two barriers per stage, took
+// 3.2).  All frequencies of Pi(u) come from one FP64 MFMA SYRK launch that stages each
+// R tile once for four frequencies (k_syrk_f64).
 #include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <vector>
 
-#include "internal.h"
+#include "dense.h"
 
-int launch_thc_r(brpa_ctx *, const double *Xa, const double *Xi, const double *Z, int64_t G,
-                 int64_t nocc, int64_t nvir, int64_t N, double *R);
+int launch_thc_pairs(brpa_ctx *, const double *Y, const double *X, int64_t G, int64_t v, int64_t o,
+                     double *P, int64_t ldp);
 int launch_axpy(brpa_ctx *, double *y, const double *x, int64_t n);
 int launch_fill(brpa_ctx *, double *x, int64_t n, double v);
 
@@ -47,6 +49,9 @@ int brpa_thc_piu(brpa_ctx *ctx, double *PiU, double *Rkai, const double *Xga, co
     const int64_t K = nocc * nvir, N = naux, F = nfreqs, G = ngrid;
     if (K > INT32_MAX || N > 65536 || F > 4096)
         return brpa_fail(ctx, BRPA_ERR_ARG, "brpa_thc_piu: sizes beyond the supported range");
+    if (G * std::max(std::max(nocc, nvir), N) + 64 > INT32_MAX)
+        return brpa_fail(ctx, BRPA_ERR_ARG,
+                         "THC R: ngrid x max(nocc, nvir, naux) must stay below 2^31 elements");
     BRPA_HIP(ctx, hipSetDevice(ctx->device));
     std::vector<double> eo, ev, fx;
     BRPA_TRY(host_copy(ctx, eo, eocc, nocc));
@@ -89,7 +94,11 @@ int brpa_thc_piu(brpa_ctx *ctx, double *PiU, double *Rkai, const double *Xga, co
     FragDev *dfd = nullptr;
     int64_t *dpre = nullptr;
     const double *dXa = Xga, *dXi = Xgi, *dZ = Zgk;
-    double *dR = nullptr, *dP = nullptr, *dOut = nullptr;
+    double *dR = nullptr, *dP = nullptr, *dOut = nullptr, *H = nullptr, *splitws = nullptr;
+    // occupied orbitals per product, leading dimension of H, split-k partials (up to 4 of R)
+    const int64_t gp = G + (G & 1);
+    const int64_t ni = std::max<int64_t>(1, std::min(nocc, ((int64_t)1 << 26) / (gp * nvir)));
+    const int64_t nsplit = std::min<int64_t>(4 * ni * nvir * N, (int64_t)1 << 26);
     auto layout = [&](Arena &ar) {
         dfd = ar.take<FragDev>(1);
         dpre = ar.take<int64_t>(2);
@@ -100,6 +109,8 @@ int brpa_thc_piu(brpa_ctx *ctx, double *PiU, double *Rkai, const double *Xga, co
         dR = rdev ? Rkai : ar.take<double>(K * N);
         dP = direct ? PiU : ar.take<double>(F * N * N);
         dOut = (accumulate && !pdev) ? ar.take<double>(F * N * N) : nullptr;
+        H = ar.take<double>(gp * ni * nvir);
+        splitws = ar.take<double>(nsplit);
     };
     Arena count;
     layout(count);
@@ -124,7 +135,23 @@ int brpa_thc_piu(brpa_ctx *ctx, double *PiU, double *Rkai, const double *Xga, co
 
     BRPA_HIP(ctx, hipEventRecord(ctx->ev0, ctx->stream));
     BRPA_TRY(stage_begin(ctx, BRPA_STAGE_THC_R));
-    BRPA_TRY(launch_thc_r(ctx, dXa, dXi, dZ, G, nocc, nvir, N, dR));
+    {
+        struct SplitLend {
+            brpa_ctx *c;
+            ~SplitLend() {
+                c->split_ws = nullptr;
+                c->split_ws_cap = 0;
+            }
+        } lend{ctx};
+        ctx->split_ws = splitws;
+        ctx->split_ws_cap = (size_t)nsplit;
+        kstat_drop(ctx);
+        for (int64_t i = 0; i < nocc; i += ni) {
+            const int64_t m = std::min(ni, nocc - i) * nvir;
+            BRPA_TRY(launch_thc_pairs(ctx, dXa, dXi + i * G, G, nvir, m / nvir, H, gp));
+            BRPA_TRY(dense_gemm(ctx, true, false, N, m, G, 1.0, dZ, G, H, gp, 0.0, dR + i * nvir * N, N));
+        }
+    }
     BRPA_TRY(stage_end(ctx, BRPA_STAGE_THC_R));
     BRPA_TRY(stage_begin(ctx, BRPA_STAGE_THC_PI));
     BRPA_TRY(launch_syrk_f64(ctx, dfd, dpre, 1, total, quad, true));
@@ -142,6 +169,7 @@ int brpa_thc_piu(brpa_ctx *ctx, double *PiU, double *Rkai, const double *Xga, co
     BRPA_HIP(ctx, hipStreamSynchronize(ctx->stream));
     BRPA_TRY(stage_collect(ctx, BRPA_STAGE_THC_R));
     BRPA_TRY(stage_collect(ctx, BRPA_STAGE_THC_PI));
+    BRPA_TRY(kstat_collect(ctx));
     float ms = 0.f;
     BRPA_HIP(ctx, hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1));
     ctx->last_kernel_ms = ms;
