@@ -157,6 +157,14 @@ int brpa_thc_1b2g(brpa_ctx *ctx, const double *Zgh, const double *Xgi, const dou
         BRPA_TRY(launch_thc_1b2g(ctx, YU, dX, dZ, G, o, m, part, yxu_diag ? dD : nullptr, mu0, S));
     }
     BRPA_HIP(ctx, hipEventRecord(ctx->ev1, ctx->stream));
+    // While the device works: the pages of a host diagonal are touched (their contents stay),
+    // so that the copy at the end does not fault them in one by one.  G = 4032, 2100
+    // vectors, 68 MB of fresh pages: 35.3 ms without, 32.7.
+    if (yxu_diag && !ddev)
+        for (size_t b = 0, n = 8 * (size_t)(G * nt); b < n; b += 4096) {
+            volatile char *p = reinterpret_cast<char *>(yxu_diag) + b;
+            *p = *p;
+        }
     kstat_drop(ctx);
     std::vector<double> hs(2 * nt);
     BRPA_TRY(copy_sync(ctx, hs.data(), S, 8 * 2 * nt, hipMemcpyDeviceToHost));
