@@ -498,13 +498,6 @@ __device__ __forceinline__ void load_panel64(double (*s)[CHOL_NB + 1], const dou
 // ---------------------------------------------------------------------------
 // Per-step kernels (flat work lists over fragments and frequencies)
 
-// lane `l`'s value of v, broadcast to the whole wave (two 32-bit readlanes)
-__device__ __forceinline__ double wave_bcast(double v, int l) {
-    const int lo = __builtin_amdgcn_readlane(__double2loint(v), l);
-    const int hi = __builtin_amdgcn_readlane(__double2hiint(v), l);
-    return __hiloint2double(hi, lo);
-}
-
 // 1 / p for p within 2^-1000 .. 2^1000: the hardware estimate and two Newton
 // steps (5 dependent instructions instead of the ~12 of a division)
 __device__ __forceinline__ double rcp_newton(double p) {
@@ -516,11 +509,12 @@ __device__ __forceinline__ double rcp_newton(double p) {
 // Cholesky factor of a 64 x 64 block by one work-group of four waves.  The block sits in
 // LDS as 4 x 4 blocks of 16 (lower triangle; the upper one is scratch):
 //   panel p     wave 0: lane r holds row r of the 16 panel columns in registers
-//               and eliminates column by column.  The multiplier is a(r, c) /
-//               pivot, and the row of the pivot comes from lanes c+1 .. by
-//               readlane (the block is symmetric), so no LDS access and no
-//               square root lies between two pivots; the columns are scaled by
-//               1 / sqrt(pivot) at the end, all 16 at once.
+//               and eliminates column by column.  Beside it every row of 16 lanes holds
+//               the 16 pivot rows, so that the row of the pivot comes by the
+//               row_newbcast operand of the multiply-add itself (by readlane it took two
+//               reads, a wait and the multiply-add), and neither LDS access nor square
+//               root lies between two pivots; the columns are scaled by 1 / sqrt(pivot)
+//               at the end, all 16 at once.
 //   column p+1  waves 1-3: A(i, p+1) -= L(i, p) L(p+1, p)^T on MFMA
 //   the other blocks right of it by waves 1-3 while wave 0 runs panel p+1, and after
 //               them work(p + 1), the caller's own
@@ -529,10 +523,11 @@ __device__ __forceinline__ double rcp_newton(double p) {
 //               idle lanes; wave 2 inverts its block during panel 2.
 // chol_panels returns whether a pivot was not positive.
 //
-// Bound by latency: 64 pivots in a chain of readlane, reciprocal, multiply and
-// fma.  Measured per k_potrf_diag launch on MI355X: 17.7 us for 16 matrices, 20.7 us for
-// 512 (61.3 and 65.4 us for one left-looking wave per matrix with rows of L from LDS,
-// the square root and division in the chain and the whole inverse by substitution).
+// Bound by latency: 64 pivots in a chain of broadcast, reciprocal, multiply and
+// multiply-add.  Measured on MI355X: 21300 cycles for the four panels (26600 by
+// readlane); a k_potrf_diag launch of 16 matrices 15 us (17.7; 61.3 for one left-looking
+// wave per matrix with rows of L from LDS, the square root and division in the chain
+// and the whole inverse by substitution).
 constexpr int CH_LP = CHOL_NB + 2;   // row pitch: 16-byte aligned rows, 16 rows on 16 distinct 4-bank groups
 constexpr int CH_XP = 18;
 
@@ -578,36 +573,122 @@ __device__ __forceinline__ void chol_invert16(CholLds &T, int p, int lane) {
         for (int i = 0; i < 16; ++i) T.Xd[p][i][l16] = x[i];
 }
 
+// x + y * (v of lane j of the lane's row of 16), for columns J .. J + n - 1 of the pivot
+// rows d and of the lane's own row a.  The s_nop keeps the two wait states between a
+// vector write of dc and its cross-lane read.
+#define CHOL_DPP(x, y, j) \
+    "v_fmac_f64_dpp %[" x "], %[dc], %[" y "] row_newbcast:%[" j "] row_mask:0xf bank_mask:0xf\n\t"
+template <int J, int NJ>
+__device__ __forceinline__ void chol_eliminate(double (&d)[16], double (&a)[16], double dc, double md,
+                                               double ma) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    if constexpr (NJ >= 5) {
+        asm("s_nop 1\n\t"
+            CHOL_DPP("d0", "md", "j0") CHOL_DPP("a0", "ma", "j0")
+            CHOL_DPP("d1", "md", "j1") CHOL_DPP("a1", "ma", "j1")
+            CHOL_DPP("d2", "md", "j2") CHOL_DPP("a2", "ma", "j2")
+            CHOL_DPP("d3", "md", "j3") CHOL_DPP("a3", "ma", "j3")
+            CHOL_DPP("d4", "md", "j4") CHOL_DPP("a4", "ma", "j4")
+            : [d0] "+&v"(d[J + 0]), [a0] "+&v"(a[J + 0]), [d1] "+&v"(d[J + 1]), [a1] "+&v"(a[J + 1]), [d2] "+&v"(d[J + 2]), [a2] "+&v"(a[J + 2]), [d3] "+&v"(d[J + 3]), [a3] "+&v"(a[J + 3]), [d4] "+&v"(d[J + 4]), [a4] "+&v"(a[J + 4])
+            : [dc] "v"(dc), [md] "v"(md), [ma] "v"(ma), [j0] "n"(J + 0), [j1] "n"(J + 1), [j2] "n"(J + 2), [j3] "n"(J + 3), [j4] "n"(J + 4));
+        chol_eliminate<J + 5, NJ - 5>(d, a, dc, md, ma);
+    } else if constexpr (NJ == 4) {
+        asm("s_nop 1\n\t"
+            CHOL_DPP("d0", "md", "j0") CHOL_DPP("a0", "ma", "j0")
+            CHOL_DPP("d1", "md", "j1") CHOL_DPP("a1", "ma", "j1")
+            CHOL_DPP("d2", "md", "j2") CHOL_DPP("a2", "ma", "j2")
+            CHOL_DPP("d3", "md", "j3") CHOL_DPP("a3", "ma", "j3")
+            : [d0] "+&v"(d[J + 0]), [a0] "+&v"(a[J + 0]), [d1] "+&v"(d[J + 1]), [a1] "+&v"(a[J + 1]), [d2] "+&v"(d[J + 2]), [a2] "+&v"(a[J + 2]), [d3] "+&v"(d[J + 3]), [a3] "+&v"(a[J + 3])
+            : [dc] "v"(dc), [md] "v"(md), [ma] "v"(ma), [j0] "n"(J + 0), [j1] "n"(J + 1), [j2] "n"(J + 2), [j3] "n"(J + 3));
+    } else if constexpr (NJ == 3) {
+        asm("s_nop 1\n\t"
+            CHOL_DPP("d0", "md", "j0") CHOL_DPP("a0", "ma", "j0")
+            CHOL_DPP("d1", "md", "j1") CHOL_DPP("a1", "ma", "j1")
+            CHOL_DPP("d2", "md", "j2") CHOL_DPP("a2", "ma", "j2")
+            : [d0] "+&v"(d[J + 0]), [a0] "+&v"(a[J + 0]), [d1] "+&v"(d[J + 1]), [a1] "+&v"(a[J + 1]), [d2] "+&v"(d[J + 2]), [a2] "+&v"(a[J + 2])
+            : [dc] "v"(dc), [md] "v"(md), [ma] "v"(ma), [j0] "n"(J + 0), [j1] "n"(J + 1), [j2] "n"(J + 2));
+    } else if constexpr (NJ == 2) {
+        asm("s_nop 1\n\t"
+            CHOL_DPP("d0", "md", "j0") CHOL_DPP("a0", "ma", "j0")
+            CHOL_DPP("d1", "md", "j1") CHOL_DPP("a1", "ma", "j1")
+            : [d0] "+&v"(d[J + 0]), [a0] "+&v"(a[J + 0]), [d1] "+&v"(d[J + 1]), [a1] "+&v"(a[J + 1])
+            : [dc] "v"(dc), [md] "v"(md), [ma] "v"(ma), [j0] "n"(J + 0), [j1] "n"(J + 1));
+    } else if constexpr (NJ == 1) {
+        asm("s_nop 1\n\t"
+            CHOL_DPP("d0", "md", "j0") CHOL_DPP("a0", "ma", "j0")
+            : [d0] "+&v"(d[J + 0]), [a0] "+&v"(a[J + 0])
+            : [dc] "v"(dc), [md] "v"(md), [ma] "v"(ma), [j0] "n"(J + 0));
+    }
+#endif
+}
+#undef CHOL_DPP
+// v of lane J of the lane's row of 16
+template <int J>
+__device__ __forceinline__ double row_bcast(double v) {
+    double x = v;
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm("s_nop 1\n\tv_mov_b64_dpp %0, %1 row_newbcast:%2 row_mask:0xf bank_mask:0xf"
+        : "=v"(x)
+        : "v"(v), "n"(J));
+#endif
+    return x;
+}
+// Pivot C: its reciprocal rp is given; that of pivot C + 1 (rcp_newton, in steps) is made
+// between the eliminations, five columns at a time.
+template <int C>
+__device__ __forceinline__ void chol_pivots(double (&d)[16], double (&a)[16], double piv, double rp,
+                                            double &mypiv, bool &inrange, int l16) {
+    inrange = inrange && piv >= 0x1p-1000 && piv <= 0x1p+1000;
+    mypiv = l16 == C ? piv : mypiv;
+    if constexpr (C < 15) {
+        constexpr int R = 15 - C, N1 = R < 5 ? R : 5, N2 = R - N1 < 5 ? R - N1 : 5, N3 = R - N1 - N2;
+        const double ma = -(a[C] * rp), md = -(d[C] * rp);
+        chol_eliminate<C + 1, N1>(d, a, d[C], md, ma);
+        const double p1 = row_bcast<C + 1>(d[C + 1]);
+        double r1 = __builtin_amdgcn_rcp(p1);
+        __builtin_amdgcn_sched_barrier(0);
+        chol_eliminate<C + 1 + N1, N2>(d, a, d[C], md, ma);
+        r1 = fma(fma(-p1, r1, 1.0), r1, r1);
+        __builtin_amdgcn_sched_barrier(0);
+        chol_eliminate<C + 1 + N1 + N2, N3>(d, a, d[C], md, ma);
+        r1 = fma(fma(-p1, r1, 1.0), r1, r1);
+        chol_pivots<C + 1>(d, a, p1, r1, mypiv, inrange, l16);
+    }
+}
+template <int C>
+__device__ __forceinline__ void chol_scale(double (&a)[16], double rd, double diag, int own) {
+    const double r = row_bcast<C>(rd);
+    a[C] = own == C ? diag : a[C] * r;
+    if constexpr (C < 15) chol_scale<C + 1>(a, rd, diag, own);
+}
+
 // wave 0
 __device__ __forceinline__ bool chol_panels(CholLds &T, int lane) {
     double(*S)[CH_LP] = T.S;
+    const int l16 = lane & 15;
     bool bad = false;
 #pragma unroll
     for (int p = 0; p < 4; ++p) {
-        double a[16];
+        // a: the lane's row; d: row l16 of the diagonal block, in every row of 16 lanes
+        double a[16], d[16];
         d2v_t *row = reinterpret_cast<d2v_t *>(&S[lane][16 * p]);
+        const d2v_t *drow = reinterpret_cast<const d2v_t *>(&S[16 * p + l16][16 * p]);
 #pragma unroll
         for (int t = 0; t < 8; ++t) {
-            const d2v_t u = row[t];
+            const d2v_t u = row[t], x = drow[t];
             a[2 * t] = u.x;
             a[2 * t + 1] = u.y;
+            d[2 * t] = x.x;
+            d[2 * t + 1] = x.y;
         }
         if (p > 0 && lane < 16)
 #pragma unroll
             for (int c = 0; c < 16; ++c) a[c] = lane == c ? 1.0 : 0.0;
         double mypiv = 1.0;
         bool inrange = true;
-#pragma unroll
-        for (int c = 0; c < 16; ++c) {
-            const double piv = wave_bcast(a[c], 16 * p + c);
-            inrange = inrange && piv >= 0x1p-1000 && piv <= 0x1p+1000;
-            const double m = a[c] * rcp_newton(piv);
-            mypiv = lane == 16 * p + c ? piv : mypiv;
-            // lanes above row j update entries that are never read
-#pragma unroll
-            for (int j = c + 1; j < 16; ++j)
-                a[j] = fma(-m, wave_bcast(a[c], 16 * p + j), a[j]);
-        }
+        // lanes above row j update entries that are never read
+        const double p0 = row_bcast<0>(d[0]);
+        chol_pivots<0>(d, a, p0, rcp_newton(p0), mypiv, inrange, l16);
         if (!inrange) {
             // a pivot that is not positive, or outside the range of rcp_newton: the
             // panel again, on its columns in LDS, with divisions
@@ -619,7 +700,7 @@ __device__ __forceinline__ bool chol_panels(CholLds &T, int lane) {
                     bad = true;
                     piv = 1.0;
                 }
-                mypiv = lane == pc ? piv : mypiv;
+                mypiv = l16 == c ? piv : mypiv;
                 const double m = S[lane][pc] / piv;
 #pragma unroll 1
                 for (int j = c + 1; j < 16; ++j)
@@ -633,10 +714,8 @@ __device__ __forceinline__ bool chol_panels(CholLds &T, int lane) {
                 a[2 * t + 1] = u.y;
             }
         }
-        const double d = sqrt(mypiv), rd = 1.0 / d;
-#pragma unroll
-        for (int c = 0; c < 16; ++c)
-            a[c] = lane == 16 * p + c ? d : a[c] * wave_bcast(rd, 16 * p + c);
+        const double sd = sqrt(mypiv), rd = 1.0 / sd;
+        chol_scale<0>(a, rd, sd, lane - 16 * p);
         if (lane >= 16 * p) {
 #pragma unroll
             for (int t = 0; t < 8; ++t) row[t] = (d2v_t){a[2 * t], a[2 * t + 1]};
