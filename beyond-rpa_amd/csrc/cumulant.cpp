@@ -81,7 +81,8 @@ int brpa_thc_1b2g(brpa_ctx *ctx, const double *Zgh, const double *Xgi, const dou
                udev = is_device_ptr(Uaim), ddev = yxu_diag && is_device_ptr(yxu_diag);
     const double *dZ = Zgh, *dX = Xgi, *dY = Yga, *dU = Uaim;
     double *YU, *part, *S, *dD = yxu_diag;
-    double *Zp = nullptr, *P, *ZP, *Q, *W, *D, *Up = nullptr, *DU;
+    double *Zp = nullptr, *P, *ZP, *Q, *W, *D, *Up = nullptr, *DU, *splitws = nullptr;
+    const int64_t nsplit = (int64_t)1 << 24;   // the GEMM's split-k partials: 128 MB
     auto layout = [&](Arena &ar) {
         if (!zdev) dZ = ar.take<double>(G * G);
         if (!xdev) dX = ar.take<double>(G * o);
@@ -100,6 +101,7 @@ int brpa_thc_1b2g(brpa_ctx *ctx, const double *Zgh, const double *Xgi, const dou
         W = ar.take<double>(K * K);
         D = ar.take<double>(kp * K);
         DU = ar.take<double>(K * nt);
+        splitws = ar.take<double>(nsplit);
     };
     Arena count, ar;
     layout(count);
@@ -120,7 +122,16 @@ int brpa_thc_1b2g(brpa_ctx *ctx, const double *Zgh, const double *Xgi, const dou
                  : brpa_fail(ctx, BRPA_ERR_SOLVER, "rocblas_set_stream failed"));
     BRPA_HIP(ctx, hipEventRecord(ctx->ev0, ctx->stream));
     const double one = 1.0, zero = 0.0;
+    struct SplitLend {
+        brpa_ctx *c;
+        ~SplitLend() {
+            c->split_ws = nullptr;
+            c->split_ws_cap = 0;
+        }
+    } lend{ctx};
     if (ex) {
+        ctx->split_ws = splitws;
+        ctx->split_ws_cap = (size_t)nsplit;
         const double *Zs = dZ;
         if (Zp) {
             BRPA_HIP(ctx, hipMemcpy2DAsync(Zp, 8 * gp, dZ, 8 * G, 8 * G, G, hipMemcpyDeviceToDevice,

@@ -69,6 +69,7 @@ struct GemmArgs {
     int mt, nt, ntiles;
     int upper, tri, nb1;
     int nsplit, kchunk;
+    int tail0, tsplit;   // tiles from tail0 on in tsplit chunks of k each (1: none)
     int far;   // a leading dimension too large for 32-bit offsets: every stage through registers
     double alpha, beta;
     const double *A;
@@ -82,15 +83,7 @@ struct GemmArgs {
     double *P;
 };
 
-template <bool TA, bool TB>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_gemm_f64(const GemmArgs g) {
-    constexpr bool KCA = TA, KCB = !TB;   // operand contiguous in k
-    __shared__ __attribute__((aligned(16))) double sA0[gemm_lds<KCA>(GT)], sA1[gemm_lds<KCA>(GT)];
-    __shared__ __attribute__((aligned(16))) double sB0[gemm_lds<KCB>(GT)], sB1[gemm_lds<KCB>(GT)];
-    const int item1 = (int)(blockIdx.x / (unsigned)g.ntiles);
-    const int t = (int)(blockIdx.x - (unsigned)item1 * (unsigned)g.ntiles);
-    const int item2 = (int)blockIdx.y;
-    int ti, tj;
+__device__ __forceinline__ void gemm_tile_of(const GemmArgs &g, int t, int &ti, int &tj) {
     if (g.upper) {
         // upper tiles ti <= tj in column order: tj (tj+1)/2 + ti
         tri_decode(t, tj, ti);
@@ -105,6 +98,22 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         if (g.tri == TRI_B_UPPER) tj = g.nt - 1 - tj;
         else if (g.tri == TRI_A_LOWER) ti = g.mt - 1 - ti;
     }
+}
+
+// TAIL: with the last tiles' k split (tsplit > 1, one item)
+template <bool TA, bool TB, bool TAIL>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_gemm_f64(const GemmArgs g) {
+    constexpr bool KCA = TA, KCB = !TB;   // operand contiguous in k
+    __shared__ __attribute__((aligned(16))) double sA0[gemm_lds<KCA>(GT)], sA1[gemm_lds<KCA>(GT)];
+    __shared__ __attribute__((aligned(16))) double sB0[gemm_lds<KCB>(GT)], sB1[gemm_lds<KCB>(GT)];
+    const bool tail = TAIL && (int)blockIdx.x >= g.tail0;
+    const int tt = (int)blockIdx.x - g.tail0, tz = tail ? tt % g.tsplit : 0;
+    const int item1 = TAIL ? 0 : (int)(blockIdx.x / (unsigned)g.ntiles);
+    const int t = tail ? g.tail0 + tt / g.tsplit
+                       : (int)(blockIdx.x - (unsigned)item1 * (unsigned)g.ntiles);
+    const int item2 = (int)blockIdx.y;
+    int ti, tj;
+    gemm_tile_of(g, t, ti, tj);
     const double *__restrict__ A = g.A + item1 * g.sA1 + item2 * g.sA2;
     const double *__restrict__ B = g.B + item1 * g.sB1 + item2 * g.sB2;
     const int m = g.m, n = g.n;
@@ -122,6 +131,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         const int z = (int)blockIdx.z;
         kbeg = max(kbeg, z * g.kchunk);
         kend = min(kend, (z + 1) * g.kchunk);
+    }
+    if (tail) {
+        kbeg = tz * g.kchunk;
+        kend = min(kend, kbeg + g.kchunk);
     }
 
     d4_t acc[4][4];
@@ -149,6 +162,19 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
                     if (col < n) P[(int64_t)row + (int64_t)m * col] = acc[i][j][r];
                 }
         }
+        return;
+    }
+    if (tail) {
+        // partial tile, whole, reduced by k_gemm_reduce_tail
+        double *P = g.P + (int64_t)tt * (GT * GT);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    P[64 * wm + 16 * i + (lane & 15) + GT * (64 * wn + 16 * j + (lane >> 4) + 4 * r)] =
+                        acc[i][j][r];
         return;
     }
     double *__restrict__ C = g.C + item1 * g.sC1 + item2 * g.sC2;
@@ -186,6 +212,23 @@ __global__ __launch_bounds__(256) void k_gemm_reduce(const GemmArgs g) {
     double v = g.alpha * s;
     if (g.cs) v *= g.cs[col];
     double *p = g.C + (int64_t)row + g.ldc * col;
+    *p = g.beta == 0.0 ? v : fma(g.beta, *p, v);
+}
+
+// the tail's partial tiles in order, 256 elements of a tile per work-group
+__global__ __launch_bounds__(256) void k_gemm_reduce_tail(const GemmArgs g) {
+    constexpr int PER = GT * GT / 256;
+    const int q = (int)blockIdx.x / PER, e = ((int)blockIdx.x % PER) * 256 + (int)threadIdx.x;
+    int ti, tj;
+    gemm_tile_of(g, g.tail0 + q, ti, tj);
+    const int row = ti * GT + e % GT, col = tj * GT + e / GT;
+    if (row >= g.m || col >= g.n) return;
+    const double *P = g.P + (int64_t)q * g.tsplit * (GT * GT) + e;
+    double s = 0.0;
+    for (int z = 0; z < g.tsplit; ++z) s += P[(int64_t)z * (GT * GT)];
+    double *p = g.C + (int64_t)row + g.ldc * col;
+    double v = g.alpha * s;
+    if (g.cs) v *= g.cs[col];
     *p = g.beta == 0.0 ? v : fma(g.beta, *p, v);
 }
 
@@ -237,7 +280,12 @@ int launch_gemm_f64_batched(brpa_ctx *ctx, bool ta, bool tb, int64_t m, int64_t 
     // 1/eff(s) + (reduction traffic), eff(s) = tiles s / (slots ceil(tiles s /
     // slots)) with two work-groups per CU; partials in the context's split
     // scratch (set by the caller for the duration of a call)
-    g.nsplit = 1;
+    // Or only the tiles after the last full round of slots, L of them, in s <= slots / L
+    // chunks: (rounds + 1 / s) slots / tiles instead of 1 / eff(1).
+    // THC 1b2g (2720 and 3655 tiles on 512 slots) 33.4 ms whole, 32.8 with its tails split;
+    // THC R (1275 tiles) 11.9 and 11.8 ms.
+    g.nsplit = g.tsplit = 1;
+    g.tail0 = (int)ntiles;
     g.kchunk = g.k;
     const int64_t wgs = ntiles * nb1 * nb2;
     if (nb1 == 1 && nb2 == 1 && ctx->split_ws && g.k >= 512) {
@@ -263,29 +311,47 @@ int launch_gemm_f64_batched(brpa_ctx *ctx, bool ta, bool tb, int64_t m, int64_t 
                 bs = sp;
             }
         }
-        if (bs > 1) {
+        const int64_t full = wgs / (int64_t)slots * (int64_t)slots, L = wgs - full;
+        const int64_t ts = L > 0 && full > 0 && tri == TRI_NONE
+                               ? std::min<int64_t>({8, (int64_t)slots / L, g.k / 256,
+                                                    (int64_t)(ctx->split_ws_cap / (size_t)(L * GT * GT))})
+                               : 1;
+        if (ts > 1 && (full / slots + 1.0 / ts) * slots / wgs + 48.0 * (ts + 1) / g.k * L / wgs < best - 1e-9) {
+            g.tsplit = (int)ts;
+            g.tail0 = (int)full;
+            const int64_t chunk = ((g.k + ts - 1) / ts + GKB - 1) / GKB * GKB;
+            g.tsplit = (int)((g.k + chunk - 1) / chunk);
+            g.kchunk = (int)chunk;
+            g.P = ctx->split_ws;
+        } else if (bs > 1) {
             const int64_t chunk = ((g.k + bs - 1) / bs + GKB - 1) / GKB * GKB;
             g.nsplit = (int)((g.k + chunk - 1) / chunk);
             g.kchunk = (int)chunk;
             g.P = ctx->split_ws;
         }
     }
-    const dim3 grid((unsigned)(ntiles * nb1), (unsigned)nb2, (unsigned)g.nsplit), block(256);
+    const int64_t gx = g.tsplit > 1 ? g.tail0 + (ntiles - g.tail0) * g.tsplit : ntiles * nb1;
+    const dim3 grid((unsigned)gx, (unsigned)nb2, (unsigned)g.nsplit), block(256);
     size_t slot = 0;
     BRPA_TRY(kstat_begin(ctx, &slot));
     auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, block, 0, ctx->stream, g); };
     if (!ta && !tb)
-        launch(k_gemm_f64<false, false>);
+        g.tsplit > 1 ? launch(k_gemm_f64<false, false, true>) : launch(k_gemm_f64<false, false, false>);
     else if (!ta && tb)
-        launch(k_gemm_f64<false, true>);
+        g.tsplit > 1 ? launch(k_gemm_f64<false, true, true>) : launch(k_gemm_f64<false, true, false>);
     else if (ta && !tb)
-        launch(k_gemm_f64<true, false>);
+        g.tsplit > 1 ? launch(k_gemm_f64<true, false, true>) : launch(k_gemm_f64<true, false, false>);
     else
-        launch(k_gemm_f64<true, true>);
+        g.tsplit > 1 ? launch(k_gemm_f64<true, true, true>) : launch(k_gemm_f64<true, true, false>);
     LAUNCH_CHECK(ctx);
     if (g.nsplit > 1) {
         hipLaunchKernelGGL(k_gemm_reduce, dim3((unsigned)((m * n + 255) / 256)), dim3(256), 0,
                            ctx->stream, g);
+        LAUNCH_CHECK(ctx);
+    }
+    if (g.tsplit > 1) {
+        hipLaunchKernelGGL(k_gemm_reduce_tail, dim3((unsigned)((ntiles - g.tail0) * (GT * GT / 256))),
+                           dim3(256), 0, ctx->stream, g);
         LAUNCH_CHECK(ctx);
     }
     // algorithmic flop: 2 m n k, n (n + 1) k on the triangle of a SYRK, m n k
