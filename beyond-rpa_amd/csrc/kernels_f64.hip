@@ -525,7 +525,7 @@ __device__ __forceinline__ double rcp_newton(double p) {
 //
 // Bound by latency: 64 pivots in a chain of broadcast, reciprocal, multiply and
 // multiply-add.  Measured on MI355X: 21300 cycles for the four panels (26600 by
-// readlane); a k_potrf_diag launch of 16 matrices 15 us (17.7; 61.3 for one left-looking
+// readlane); a k_potrf_diag launch of 160 matrices 15 us (17.7; 61.3 for one left-looking
 // wave per matrix with rows of L from LDS, the square root and division in the chain
 // and the whole inverse by substitution).
 constexpr int CH_LP = CHOL_NB + 2;   // row pitch: 16-byte aligned rows, 16 rows on 16 distinct 4-bank groups
@@ -857,8 +857,9 @@ __global__ __launch_bounds__(256) void k_potrf_diag(const FragDev *__restrict__ 
 // s_in, operands straight from L2).  Then L21 = B L11^{-T}, and the work-groups
 // within the outer panel bring their own diagonal block up to date, so that the
 // next step finds it complete.
-// 14 us for the first step of an outer panel, 18 us for the fourth (in three launches 37 to
-// 51 us at N = 400).
+// N = 400, 16 matrices: 22 to 26 us a step of the first outer panel, 13 us the last one;
+// E_RPA of o = 8, v = 72 with three launches a step 451 us, with this kernel and k_chol_rest
+// 331.
 // r = 0 writes the log-det partial and the status.  No work-group may see a half-factored
 // block, so with keep_l11 it leaves L11 in linv and copies it into Pi in the next
 // step (pend: the previous step did so); the matrix's last step writes it at once.

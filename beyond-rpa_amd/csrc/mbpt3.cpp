@@ -17,7 +17,7 @@
 // derivative of the amplitudes with the coupling strength in the V basis and
 // is negative semidefinite up to rounding.  The trace is the SOSEX contraction of V X V^T:
 // where the explicit ov form is the cheaper one it takes X as it is (sosex_explicit;
-// NT2 = 1200: 0.5 ms, the eigenpairs below 37 ms, which a rounding-level
+// NT2 = 1200: 28 ms less than with the eigenpairs below, which a rounding-level
 // positive eigenvalue asked for).  The pair forms need a factor: -X = U'^T U' by the
 // library's Cholesky gives V X V^T = -(V U'^T)(V U'^T)^T, so V'' = V U'^T with B'' = -1
 // (brpa_sosex, FP64 or split-int8); a Cholesky breakdown falls back to the eigenpairs
@@ -211,7 +211,7 @@ int brpa_mbpt3_1(brpa_ctx *ctx, int precision, double *ec_exchange, const double
     // the residual r = |1 - Bm Bi|_F, until the last one started from r <= 1e-9.  Not
     // inverted (then LU decides): a breakdown, or r not down there after three steps.
     // Matrix products instead of rocSOLVER's column by column getrf / getri: 6.1 ms less per
-    // inverse at n = 1200 (four inverses: MBPT3-1 of 33 to 9 ms).
+    // inverse at n = 1200 (four inverses: MBPT3-1 of 36 to 12 ms).
     auto inverse = [&](bool *done) -> int {
         *done = false;
         BRPA_TRY(dense_syrk(ctx, true, n, n, 1.0, Bm, n, 0.0, T1, n));
