@@ -75,23 +75,6 @@ int launch_row_scale(brpa_ctx *ctx, double *out, const double *in, const double 
     return BRPA_OK;
 }
 
-// io(r, c) += a * s[r] * in(r, c)
-__global__ void k_row_scale_acc(double *__restrict__ io, const double *__restrict__ in,
-                                const double *__restrict__ s, double a, int64_t m, int64_t n) {
-    int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (e >= m * n) return;
-    io[e] = fma(a * s[e % m], in[e], io[e]);
-}
-
-int launch_row_scale_acc(brpa_ctx *ctx, double *io, const double *in, const double *s, double a,
-                         int64_t m, int64_t n) {
-    if (m * n <= 0) return BRPA_OK;
-    hipLaunchKernelGGL(k_row_scale_acc, dim3(nblocks(m * n)), dim3(256), 0, ctx->stream, io, in, s,
-                       a, m, n);
-    LAUNCH_CHECK(ctx);
-    return BRPA_OK;
-}
-
 // W(:, j) = U(:, c0 + j) / sqrt(ev[c0 + j]) for j < nt  (rpa_CC_Doubles.f90:610-614)
 __global__ void k_select_scale(double *__restrict__ W, const double *__restrict__ U,
                                const double *__restrict__ ev, int64_t m, int64_t c0, int64_t nt) {

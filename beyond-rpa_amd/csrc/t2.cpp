@@ -27,8 +27,6 @@
 int launch_guess(brpa_ctx *, double *O, int64_t m, int64_t n, uint64_t seed);
 int launch_normalize_columns(brpa_ctx *, double *X, int64_t m, int64_t n);
 int launch_row_scale(brpa_ctx *, double *out, const double *in, const double *s, int64_t m, int64_t n);
-int launch_row_scale_acc(brpa_ctx *, double *io, const double *in, const double *s, double a,
-                         int64_t m, int64_t n);
 int launch_select_scale(brpa_ctx *, double *W, const double *U, const double *ev, int64_t m,
                         int64_t c0, int64_t nt);
 int launch_col_scale(brpa_ctx *, double *out, const double *in, const double *s, int64_t m,
@@ -258,6 +256,14 @@ int t2_build(brpa_ctx *ctx, int precision, const double *R, int64_t naux, const 
     const int64_t nsteps = cdiv(N, CHOL_NB);
     FragDev fd{};
     double *dR = nullptr, *dchi, *omega, *tmp, *iom, *Y, *Sm, *sev, *sE, *Uinv, *Rt;
+    double *DG = nullptr, *dcoef = nullptr, *tinv = nullptr, *splitws = nullptr;
+    // FP64, NG < o*v: chi_k is folded into Rt_k and the F matrices are stacked to one
+    // (F N) x K matrix, so that I Omega and T^T I T are two products each over kf
+    // frequencies at a time (all of them, unless N kf NG passes 16 M elements)
+    // instead of two per frequency.
+    const bool stack = !split && !over;
+    const int64_t kf = std::max<int64_t>(1, std::min<int64_t>(F, (16 << 20) / (N * NG)));
+    const int64_t nsplit = stack ? 16 << 20 : 0;   // split-k partials of k_gemm_f64
     int *dinfo;
     int64_t *dchol = nullptr, *dchol2 = nullptr;
     FragDev fm{};                  // one dense matrix for the library's Cholesky
@@ -282,7 +288,7 @@ int t2_build(brpa_ctx *ctx, int precision, const double *R, int64_t naux, const 
         fd.dtab = ar.take<double>(F * K);
         fd.Pi = ar.take<double>(F * N * N);
         Uinv = ar.take<double>(F * N * N);
-        Rt = ar.take<double>(F * K * N);
+        Rt = ar.take<double>(std::max(F * K * N, trinv_scratch(N)));
         fd.diag = ar.take<double>(F * N);
         fd.weights = ar.take<double>(F);
         fd.freqs = ar.take<double>(F);
@@ -294,7 +300,13 @@ int t2_build(brpa_ctx *ctx, int precision, const double *R, int64_t naux, const 
         // Gram matrix of the other side; no Y and no split operands
         tmp = ar.take<double>(over ? K * K : K * NG);
         iom = ar.take<double>(K * NG);
-        Y = over ? nullptr : ar.take<double>(N * NG);
+        Y = over ? nullptr : ar.take<double>((stack ? kf : 1) * N * NG);
+        if (stack) {
+            DG = ar.take<double>(kf * N * NG);
+            dcoef = ar.take<double>(F * N);
+            splitws = ar.take<double>(nsplit);
+        }
+        if (!over) tinv = ar.take<double>(trinv_scratch(NG));
         Sm = ar.take<double>(nd * nd);
         sev = ar.take<double>(nd);
         sE = ar.take<double>(nd);
@@ -348,6 +360,21 @@ int t2_build(brpa_ctx *ctx, int precision, const double *R, int64_t naux, const 
                        hipMemcpyHostToDevice));
     BRPA_TRY(copy_sync(ctx, dchi, chi.data(), 8 * F * K, hipMemcpyHostToDevice));
     if (over) BRPA_TRY(copy_sync(ctx, chis, hchis.data(), 8 * F * K, hipMemcpyHostToDevice));
+    if (stack) {
+        std::vector<double> hcoef(F * N);
+        for (int64_t k = 0; k < F; ++k)
+            std::fill_n(hcoef.begin() + k * N, N, -fw[k] * lambda / (4.0 * kPi));
+        BRPA_TRY(copy_sync(ctx, dcoef, hcoef.data(), 8 * F * N, hipMemcpyHostToDevice));
+    }
+    struct SplitLend {
+        brpa_ctx *c;
+        ~SplitLend() {
+            c->split_ws = nullptr;
+            c->split_ws_cap = 0;
+        }
+    } lend{ctx};
+    ctx->split_ws = splitws;
+    ctx->split_ws_cap = (size_t)nsplit;
     BRPA_TRY(copy_sync(ctx, dfd, &fd, sizeof(FragDev), hipMemcpyHostToDevice));
     BRPA_TRY(copy_sync(ctx, dpre, pre.data(), 8 * pre.size(), hipMemcpyHostToDevice));
     BRPA_HIP(ctx, hipEventRecord(ctx->ev0, ctx->stream));
@@ -368,24 +395,24 @@ int t2_build(brpa_ctx *ctx, int precision, const double *R, int64_t naux, const 
     BRPA_TRY(launch_set_diag(ctx, dfd, dpre + 4, 1, pre[5], 0));
     // all F factors in one batched blocked Cholesky (the library's own kernels).
     // The factor L is the lower triangle of the row-major matrix, i.e. the
-    // upper triangle U = L^T of the column-major view the solvers below read
-    // (A = U^T U): hence rocblas_fill_upper there.
+    // upper triangle U = L^T of the column-major view (A = U^T U).
     BRPA_TRY(chol_single(ctx, dfd, dchol, N, F));
     // Rt_k = R U_k^-1 (C Rt_k[ai][P], the layout of R), so that
     // R (1 + l Pi_k)^-1 R^T = Rt_k Rt_k^T: no triangular solves in the
     // frequency loops.  Column-major Rt_k^T = U_k^-T Rc with U_k^-1 from the
-    // batched triangular inverse, its lower triangle cleared for the GEMM.
-    BRPA_TRY(rb_check(ctx,
-                      rocblas_dtrtri_strided_batched(h, rocblas_fill_upper,
-                                                     rocblas_diagonal_non_unit, (rocblas_int)N,
-                                                     fd.Pi, (rocblas_int)N, N * N, Uinv,
-                                                     (rocblas_int)N, N * N, (rocblas_int)F),
-                      "rocblas_dtrtri_strided_batched"));
-    for (int64_t k = 0; k < F; ++k) {
-        BRPA_TRY(launch_zero_lower(ctx, Uinv + k * N * N, N));
-        BRPA_TRY(gemm(ctx, h, true, false, N, K, N, 1.0, Uinv + k * N * N, N, dR, N, 0.0,
-                      Rt + k * K * N, N));
-    }
+    // batched triangular inverse (scratch: Rt itself, written next), all k in one product.
+    // With the stacked products below, F = 12, N = 400, K = 2250, NG = 1200: 35.5 ms by
+    // rocBLAS's batched trtri, dtrsm and two products per k each, 34.4 ms here (30 of them
+    // the final eigensolve).
+    const int64_t nbi = std::max<int64_t>(1, std::min(F, F * K / N));
+    for (int64_t k = 0; k < F; k += nbi)
+        BRPA_TRY(dense_trinv(ctx, N, fd.Pi + k * N * N, N, N * N, Uinv + k * N * N, N, N * N,
+                             std::min(nbi, F - k), Rt));
+    // stacked: rows k N .. of the (F N) x K matrix, columns scaled by chi_k
+    const int64_t FN = F * N;
+    BRPA_TRY(launch_gemm_f64_batched(ctx, true, false, N, K, N, 1.0, Uinv, N, N * N, 0, dR, N, 0, 0,
+                                     0.0, Rt, stack ? FN : N, stack ? N : K * N, 0, F, 1, false,
+                                     TRI_A_LOWER, stack ? dchi : nullptr, stack ? K : 0, 0));
     BRPA_TRY(stage_end(ctx, BRPA_STAGE_T2_PI));
 
     // Cholesky factor of one dense n x n matrix M in place with the same
@@ -413,7 +440,6 @@ int t2_build(brpa_ctx *ctx, int precision, const double *R, int64_t naux, const 
             if (staged[st]) BRPA_TRY(stage_collect(ctx, st));
         return kstat_collect(ctx);
     };
-    const double one = 1.0;
     int64_t nt = 0;
     double *Tkeep = iom;    // K x nt orthonormal basis of the kept subspace
     bool ident = false;     // the kept subspace is the whole ov space, T = 1
@@ -486,14 +512,14 @@ int t2_build(brpa_ctx *ctx, int precision, const double *R, int64_t naux, const 
         BRPA_TRY(begin(BRPA_STAGE_T2_IOMEGA));
         BRPA_TRY(launch_guess(ctx, omega, K, NG, seed));
         BRPA_TRY(launch_normalize_columns(ctx, omega, K, NG));
-        BRPA_HIP(ctx, hipMemsetAsync(iom, 0, 8 * K * NG, ctx->stream));
-        // frequency-independent operand of the split form, once per fragment
-        if (split) BRPA_TRY(launch_colslice_i8(ctx, omega, K, K, NG, nullptr, Kp, scOT, SOT));
-        for (int64_t k = 0; k < F; ++k) {
-            const double *ck = dchi + k * K;
-            const double coef = -fw[k] * lambda / (4.0 * kPi);
-            const double *Rtk = Rt + k * K * N;
-            if (split) {
+        if (split) {
+            BRPA_HIP(ctx, hipMemsetAsync(iom, 0, 8 * K * NG, ctx->stream));
+            // frequency-independent operand of the split form, once per fragment
+            BRPA_TRY(launch_colslice_i8(ctx, omega, K, K, NG, nullptr, Kp, scOT, SOT));
+            for (int64_t k = 0; k < F; ++k) {
+                const double *ck = dchi + k * K;
+                const double coef = -fw[k] * lambda / (4.0 * kPi);
+                const double *Rtk = Rt + k * K * N;
                 // Y = (chi_k Rt_k)^T Omega, I Omega += coef chi_k Rt_k Y; the chi_k Rt_k
                 // slices are kept for T^T I T
                 int8_t *SCRk = SCR + k * 5 * N * Kp;
@@ -505,12 +531,16 @@ int t2_build(brpa_ctx *ctx, int precision, const double *R, int64_t naux, const 
                 BRPA_TRY(launch_colslice_i8(ctx, Y, N, N, NG, nullptr, Np, scY, SY));
                 BRPA_TRY(launch_gemm_i8(ctx, SRR, scRR, K, SY, scY, NG, Np, coef, ck, 1.0, iom, 1,
                                         K, N));
-                continue;
             }
-            BRPA_TRY(launch_row_scale(ctx, tmp, omega, ck, K, NG));
-            BRPA_TRY(gemm(ctx, h, false, false, N, NG, K, 1.0, Rtk, N, tmp, K, 0.0, Y, N));
-            BRPA_TRY(gemm(ctx, h, true, false, K, NG, N, 1.0, Rtk, N, Y, N, 0.0, tmp, K));
-            BRPA_TRY(launch_row_scale_acc(ctx, iom, tmp, ck, coef, K, NG));
+        }
+        for (int64_t k = 0; stack && k < F; k += kf) {
+            // Y^T = Omega^T (chi Rt)^T diag(coef), I Omega += (chi Rt) Y
+            const int64_t nr = std::min(kf, F - k) * N;
+            BRPA_TRY(launch_gemm_f64_batched(ctx, true, true, NG, nr, K, 1.0, omega, K, 0, 0,
+                                             Rt + k * N, FN, 0, 0, 0.0, Y, NG, 0, 0, 1, 1, false,
+                                             TRI_NONE, dcoef + k * N, 0, 0));
+            BRPA_TRY(dense_gemm(ctx, true, true, K, NG, nr, 1.0, Rt + k * N, FN, Y, NG,
+                                k == 0 ? 0.0 : 1.0, iom, K));
         }
         BRPA_TRY(launch_normalize_columns(ctx, iom, K, NG));
         BRPA_TRY(stage_end(ctx, BRPA_STAGE_T2_IOMEGA));
@@ -529,8 +559,8 @@ int t2_build(brpa_ctx *ctx, int precision, const double *R, int64_t naux, const 
         // restores orthonormality to O(eps kappa(X1)^2) -- never worse than the
         // eps s_max / s_min of the reference's own eigenvector basis.
         BRPA_TRY(begin(BRPA_STAGE_T2_BASIS));
-        // Gram matrices as full GEMMs: rocBLAS dgemm takes a third of dsyrk's time here
-        BRPA_TRY(gemm(ctx, h, true, false, NG, NG, K, 1.0, iom, K, iom, K, 0.0, Sm, NG));
+        // upper triangles (the ones the Cholesky reads) by the library's SYRK
+        BRPA_TRY(dense_syrk(ctx, true, NG, K, 1.0, iom, K, 0.0, Sm, NG));
         bool cholqr = false;
         BRPA_TRY(launch_add_diag(ctx, Sm, NG, -cutoff));
         BRPA_TRY(chol_dense(Sm, NG, &cholqr));
@@ -538,21 +568,19 @@ int t2_build(brpa_ctx *ctx, int precision, const double *R, int64_t naux, const 
             nt = NG;
             for (int pass = 0; pass < 2; ++pass) {
                 if (pass > 0) {
-                    BRPA_TRY(gemm(ctx, h, true, false, NG, NG, K, 1.0, iom, K, iom, K, 0.0, Sm,
-                                  NG));
+                    BRPA_TRY(dense_syrk(ctx, true, NG, K, 1.0, iom, K, 0.0, Sm, NG));
                     bool okp = false;
                     BRPA_TRY(chol_dense(Sm, NG, &okp));
                     if (!okp)
                         return brpa_fail(ctx, BRPA_ERR_SOLVER,
                                          "Cholesky-QR pass %d of the T2 basis broke down", pass);
                 }
-                // X <- X U^{-1}, so that X^T X = 1
-                BRPA_TRY(rb_check(ctx,
-                                  rocblas_dtrsm(h, rocblas_side_right, rocblas_fill_upper,
-                                                rocblas_operation_none, rocblas_diagonal_non_unit,
-                                                (rocblas_int)K, (rocblas_int)NG, &one, Sm,
-                                                (rocblas_int)NG, iom, (rocblas_int)K),
-                                  "rocblas_dtrsm"));
+                // X <- X U^{-1}, so that X^T X = 1, by the inverse and one triangular product
+                BRPA_TRY(dense_trinv(ctx, NG, Sm, NG, 0, omega, NG, 0, 1, tinv));
+                BRPA_TRY(launch_gemm_f64_batched(ctx, false, false, K, NG, NG, 1.0, iom, K, 0, 0,
+                                                 omega, NG, 0, 0, 0.0, tmp, K, 0, 0, 1, 1, false,
+                                                 TRI_B_UPPER, nullptr, 0, 0));
+                std::swap(iom, tmp);   // back in place after the second pass
             }
         } else {
             BRPA_TRY(begin(BRPA_STAGE_T2_EIG));
@@ -571,7 +599,7 @@ int t2_build(brpa_ctx *ctx, int precision, const double *R, int64_t naux, const 
         if (nt > 0) {
             // T = (I Omega) U_s s^{-1/2}; TIT = T^T I T (rpa_CC_MIM_v5, 425-488)
             double *T = tmp;               // K x nt
-            double *G = Y;                 // N x nt
+            double *G = Y;                 // N x nt, or nt x (kf N)
             if (!cholqr) {
                 double *Wm = omega;        // NG x nt   (omega no longer needed)
                 BRPA_TRY(launch_select_scale(ctx, Wm, Sm, sev, NG, NG - nt, nt));
@@ -583,21 +611,24 @@ int t2_build(brpa_ctx *ctx, int precision, const double *R, int64_t naux, const 
             BRPA_TRY(begin(BRPA_STAGE_T2_TIT));
             if (split)
                 BRPA_TRY(launch_colslice_i8(ctx, Tkeep, K, K, nt, nullptr, Kp, scOT, SOT));
-            for (int64_t k = 0; k < F; ++k) {
-                const double *ck = dchi + k * K;
-                if (split) {
-                    // G = (chi_k Rt_k)^T T
-                    BRPA_TRY(launch_gemm_i8(ctx, SCR + k * 5 * N * Kp, scCR + k * N, N, SOT, scOT,
-                                            nt, Kp, 1.0, nullptr, 0.0, G, 1, N, K));
-                } else {
-                    BRPA_TRY(launch_row_scale(ctx, T, Tkeep, ck, K, nt));
-                    BRPA_TRY(gemm(ctx, h, false, false, N, nt, K, 1.0, Rt + k * K * N, N, T, K,
-                                  0.0, G, N));
-                }
-                // G = Rt_k^T chi_k T = U_k^-T R^T chi_k T, so G^T G = T^T chi R (1 + l Pi_k)^-1 R^T chi T
+            for (int64_t k = 0; split && k < F; ++k) {
+                // G = (chi_k Rt_k)^T T = U_k^-T R^T chi_k T, so G^T G = T^T chi R (1 + l Pi_k)^-1 R^T chi T
+                BRPA_TRY(launch_gemm_i8(ctx, SCR + k * 5 * N * Kp, scCR + k * N, N, SOT, scOT, nt,
+                                        Kp, 1.0, nullptr, 0.0, G, 1, N, K));
                 BRPA_TRY(gemm(ctx, h, true, false, nt, nt, N, -fw[k] * lambda / (4.0 * kPi), G, N,
                               G, N, k == 0 ? 0.0 : 1.0, TIT, nt));
             }
+            for (int64_t k = 0; stack && k < F; k += kf) {
+                // the same with G^T = T^T (chi Rt)^T of kf frequencies: G^T diag(coef) G
+                const int64_t nr = std::min(kf, F - k) * N;
+                BRPA_TRY(dense_gemm(ctx, true, true, nt, nr, K, 1.0, Tkeep, K, Rt + k * N, FN, 0.0,
+                                    G, nt));
+                BRPA_TRY(launch_col_scale(ctx, DG, G, dcoef + k * N, nt, nr));
+                BRPA_TRY(launch_gemm_f64_batched(ctx, false, true, nt, nt, nr, 1.0, G, nt, 0, 0, DG,
+                                                 nt, 0, 0, k == 0 ? 0.0 : 1.0, TIT, nt, 0, 0, 1, 1,
+                                                 true, TRI_NONE, nullptr, 0, 0));
+            }
+            if (stack) BRPA_TRY(dense_symm_fill(ctx, TIT, nt));
             BRPA_TRY(stage_end(ctx, BRPA_STAGE_T2_TIT));
         } else {
             BRPA_TRY(stage_end(ctx, BRPA_STAGE_T2_BASIS));
