@@ -161,7 +161,8 @@ int brpa_mbpt3_1(brpa_ctx *ctx, int precision, double *ec_exchange, const double
     const double *dV = V, *dA = A, *dR = R;
     double *dd, *W, *U, *Dm, *Vd, *Am, *Bm, *Bi, *T1, *ev_x, *work;
     int *ipiv, *info;
-    double *Fi, *tw;
+    double *Fi, *tw, *splitws;
+    const int64_t nsplit = 16 << 20;   // split-k partials of k_gemm_f64
     DenseChol ch;
     auto layout = [&](Arena &ar) {
         if (!vdev) dV = ar.take<double>(K * n);
@@ -182,6 +183,7 @@ int brpa_mbpt3_1(brpa_ctx *ctx, int precision, double *ec_exchange, const double
         info = ar.take<int>(2);
         Fi = ar.take<double>(n * n);
         tw = ar.take<double>(trinv_scratch(n));
+        splitws = ar.take<double>(nsplit);
         ch.layout(ar, n);
     };
     Arena count, ar;
@@ -197,6 +199,17 @@ int brpa_mbpt3_1(brpa_ctx *ctx, int precision, double *ec_exchange, const double
     BRPA_TRY(copy_sync(ctx, dd, d.data(), 8 * K, hipMemcpyHostToDevice));
     stage_reset(ctx);
     BRPA_TRY(stage_begin(ctx, BRPA_STAGE_MBPT3));
+    // k of the n x n products is split (100 tiles at n = 1200: 11.5 ms without, 9.65 with)
+    struct SplitLend {
+        brpa_ctx *c;
+        void end() {
+            c->split_ws = nullptr;
+            c->split_ws_cap = 0;
+        }
+        ~SplitLend() { end(); }
+    } lend{ctx};
+    ctx->split_ws = splitws;
+    ctx->split_ws_cap = (size_t)nsplit;
     // V is C V[ai][mu] = column-major n x K (V^T); R is column-major N x K (R^T)
     // W = R^T V (N x n), U = W^T W (rpa_CC_Ukl 178-207)
     BRPA_TRY(gemm(ctx, h, false, true, N, n, K, 1.0, dR, N, dV, n, 0.0, W, N));
@@ -211,7 +224,7 @@ int brpa_mbpt3_1(brpa_ctx *ctx, int precision, double *ec_exchange, const double
     // the residual r = |1 - Bm Bi|_F, until the last one started from r <= 1e-9.  Not
     // inverted (then LU decides): a breakdown, or r not down there after three steps.
     // Matrix products instead of rocSOLVER's column by column getrf / getri: 6.1 ms less per
-    // inverse at n = 1200 (four inverses: MBPT3-1 of 36 to 12 ms).
+    // inverse at n = 1200 (four inverses: MBPT3-1 of 36 to 11.5 ms).
     auto inverse = [&](bool *done) -> int {
         *done = false;
         BRPA_TRY(dense_syrk(ctx, true, n, n, 1.0, Bm, n, 0.0, T1, n));
@@ -309,6 +322,7 @@ int brpa_mbpt3_1(brpa_ctx *ctx, int precision, double *ec_exchange, const double
         return brpa_fail(ctx, BRPA_ERR_SOLVER, "brpa_mbpt3_1: Lyapunov iteration did not converge");
     const bool keep = ctx->stage_keep;
     auto end_stage = [&]() -> int {
+        lend.end();   // the contraction has a workspace of its own
         BRPA_TRY(stage_end(ctx, BRPA_STAGE_MBPT3));
         BRPA_HIP(ctx, hipStreamSynchronize(ctx->stream));
         BRPA_TRY(stage_collect(ctx, BRPA_STAGE_MBPT3));
