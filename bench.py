@@ -83,8 +83,9 @@ def chol_flops(n, nf):
 
 def bench_sosex(a):
     """SOSEX contraction of one large fragment (o=64, v=600, NAux=3200, 16
-    frequencies, amplitudes with NGuess = 3 NAux built once in FP64): FP64
-    (rocBLAS pair GEMMs) vs the fused split-int8 kernel, |dE| between them."""
+    frequencies, amplitudes with NGuess = 3 NAux built once in FP64) at either
+    precision; with this many vectors both take the explicit (ai|bj) and T blocks
+    on the FP64 GEMM, so |dE| between them is zero."""
     import math
 
     import numpy as np
@@ -114,23 +115,23 @@ def bench_sosex(a):
         res[prec] = (e, (time.perf_counter() - t) / a.steps, kms / a.steps)
         print("# %s: E_x %.10f  %.1f ms/step (kernels %.1f ms)" % (prec, e, res[prec][1] * 1e3,
                                                                   res[prec][2]), file=sys.stderr)
-    flops = 2.0 * 2 * (o * (o + 1) // 2) * n * nt * v   # two W GEMMs per pair (i >= j)
+    flops = 1.0 * o * v * (o * v + 1) * (n + nt)   # (ai|bj) and T, the half of each
     e8, dt8, k8 = res["split_i8"]
     e64, dt64, k64 = res["fp64"]
     out = {"metric": "E_SOSEX contraction time, split-int8 vs FP64 at |dE|<=1e-7 Ha",
            "value": round(dt8 * 1e3, 3), "unit": "ms", "n_gpus": 1, "steps": a.steps,
            "warmup": a.warmup, "ms_per_step": round(dt8 * 1e3, 3), "higher_is_better": False,
            "scaling": "strong", "vs_baseline": None,
-           "dtype": "i8 (5-slice split, 15 products, exact i32 acc) + f64 tile sums",
+           "dtype": "f64",
            "data": "synthetic (seeded PCG64, brpa.synth)",
            "config": {"workload": "SOSEX of one fragment o=64, v=600, NAux=3200, 16 "
                                   "frequencies, NT2=%d" % nt},
            "fp64_ms": round(dt64 * 1e3, 3), "speedup_vs_fp64": round(dt64 / dt8, 3),
            "abs_dE_vs_fp64_Ha": abs(e8 - e64), "E_x_fp64": e64,
            "roofline": {"bound": "mfma", "achieved": round(flops / (k8 * 1e-3) / 1e12, 3),
-                        "peak": round(PEAK_I8_TOPS / 15, 3), "unit": "TFLOP/s",
-                        "frac": round(flops / (k8 * 1e-3) / 1e12 / (PEAK_I8_TOPS / 15), 4),
-                        "traffic": None, "kernel": "k_sosex_i8 (+ slicing)",
+                        "peak": PEAK_FP64_TFLOPS, "unit": "TFLOP/s",
+                        "frac": round(flops / (k8 * 1e-3) / 1e12 / PEAK_FP64_TFLOPS, 4),
+                        "traffic": None, "kernel": "k_gemm_f64 (+ k_sosex_contract)",
                         "fp64_achieved": round(flops / (k64 * 1e-3) / 1e12, 3)}}
     print(json.dumps(out))
 
@@ -456,7 +457,7 @@ def bench_mbpt3(a):
     K = o * v
     r1 = res["mbpt3_1_split_i8"]
     # algorithmic FP64 flop of the MBPT3-1 core: W, U, D, then per sign step the
-    # Newton step's getrf + getri (2 n^3) and two GEMMs (4 n^3); the final
+    # Newton step's inverse (2 n^3) and two GEMMs (4 n^3); the final
     # Newton-Schulz steps (six GEMMs) are counted at the same 6 n^3
     core_flops = 2.0 * K * n * nt + 2.0 * n * nt * nt + 2.0 * K * nt * nt \
         + 6.0 * nt ** 3 * max(r1["sign_iterations"], 1)
@@ -505,7 +506,7 @@ def bench_mbpt3(a):
            "value": round(total, 3), "unit": "ms", "n_gpus": 1, "steps": a.steps,
            "warmup": a.warmup, "ms_per_step": round(total, 3), "higher_is_better": False,
            "scaling": "strong", "vs_baseline": None,
-           "dtype": "f64 (Lyapunov, MBPT3-2) + i8 split (MBPT3-1 contraction)",
+           "dtype": "f64",
            "data": "synthetic (seeded PCG64, brpa.synth)",
            "config": {"workload": "MBPT3 exchange of one fragment o=64, v=600, NAux=3200, 16 "
                                   "frequencies, NT2=%d" % nt},
@@ -641,7 +642,10 @@ def bench_thc1b2g(a):
     torch.cuda.synchronize()
     dt = (time.perf_counter() - t) / a.steps
     kms /= a.steps
-    flops = 2.0 * g * g * o * nt + 2.0 * g * v * o * nt      # M tiles (both orders) + YU
+    # the explicit pair form: Z P, P^T (Z P) (half), Z XX, D U, and YU
+    K = o * v
+    flops = 2.0 * g * g * K + 1.0 * g * K * K + 1.0 * g * g * o * (o + 1) \
+        + 2.0 * K * K * nt + 2.0 * g * K * nt
     tf = flops / (kms * 1e-3) / 1e12
     cpu = None
     if a.cpu_seconds > 0:
@@ -663,7 +667,7 @@ def bench_thc1b2g(a):
            "Ec1b_half": 0.5 * e1, "Ec2g": e2,
            "roofline": {"bound": "mfma", "achieved": round(tf, 3), "peak": PEAK_FP64_TFLOPS,
                         "unit": "TFLOP/s", "frac": round(tf / PEAK_FP64_TFLOPS, 4),
-                        "traffic": None, "kernel": "k_thc_1b2g (+ YU dgemm)",
+                        "traffic": None, "kernel": "k_gemm_f64 (explicit pair products, + YU dgemm)",
                         "kernel_ms_per_step": round(kms, 3)},
            "cpu_baseline": None if cpu is None else {
                "value": round(cpu * 1e3, 1), "unit": "ms", "cores": _cpu_threads(),
@@ -856,7 +860,7 @@ def main():
         kernel, peak = PI_KERNEL[a.precision]
         achieved = tot_syrk / (stage_ms["pi"] * 1e-3) / 1e12
     else:
-        kernel, peak = "k_potrf_diag+k_trsm+k_chol_update", PEAK_FP64_TFLOPS
+        kernel, peak = "k_potrf_diag+k_chol_panel+k_chol_rest", PEAK_FP64_TFLOPS
         achieved = tot_chol / (stage_ms["chol"] * 1e-3) / 1e12
     # the committed PMC runs cover the default batch (256 fragments, 16 frequencies)
     traffic = (pmc_traffic(kernel + "<128>")
