@@ -79,7 +79,7 @@ extern "C" int brpa_ecrpa_grad(brpa_ctx *ctx, const double *R, int64_t naux, con
     double *Uinv;
     int64_t *dchol;
     // matrices per batch of the triangular inverse: its scratch is X
-    const int64_t nbi = std::max<int64_t>(1, std::min(F, K * N / trinv_scratch(N)));
+    const int64_t nbi = std::max<int64_t>(1, std::min<int64_t>({F, K * N / trinv_scratch(N), 65535}));
     auto layout = [&](Arena &ar) {
         dfd = ar.take<FragDev>(1);
         dpre = ar.take<int64_t>(pre.size());

@@ -263,7 +263,7 @@ int t2_build(brpa_ctx *ctx, int precision, const double *R, int64_t naux, const 
     // instead of two per frequency.
     const bool stack = !split && !over;
     const int64_t kf = std::max<int64_t>(1, std::min<int64_t>(F, (16 << 20) / (N * NG)));
-    const int64_t nsplit = stack ? 16 << 20 : 0;   // split-k partials of k_gemm_f64
+    const int64_t nsplit = over ? 0 : 16 << 20;   // split-k partials of k_gemm_f64
     int *dinfo;
     int64_t *dchol = nullptr, *dchol2 = nullptr;
     FragDev fm{};                  // one dense matrix for the library's Cholesky
@@ -304,9 +304,11 @@ int t2_build(brpa_ctx *ctx, int precision, const double *R, int64_t naux, const 
         if (stack) {
             DG = ar.take<double>(kf * N * NG);
             dcoef = ar.take<double>(F * N);
+        }
+        if (!over) {
+            tinv = ar.take<double>(trinv_scratch(NG));
             splitws = ar.take<double>(nsplit);
         }
-        if (!over) tinv = ar.take<double>(trinv_scratch(NG));
         Sm = ar.take<double>(nd * nd);
         sev = ar.take<double>(nd);
         sE = ar.take<double>(nd);
@@ -404,7 +406,7 @@ int t2_build(brpa_ctx *ctx, int precision, const double *R, int64_t naux, const 
     // With the stacked products below, F = 12, N = 400, K = 2250, NG = 1200: 35.5 ms by
     // rocBLAS's batched trtri, dtrsm and two products per k each, 34.4 ms here (30 of them
     // the final eigensolve).
-    const int64_t nbi = std::max<int64_t>(1, std::min(F, F * K / N));
+    const int64_t nbi = std::max<int64_t>(1, std::min<int64_t>({F, F * K / N, 65535}));
     for (int64_t k = 0; k < F; k += nbi)
         BRPA_TRY(dense_trinv(ctx, N, fd.Pi + k * N * N, N, N * N, Uinv + k * N * N, N, N * N,
                              std::min(nbi, F - k), Rt));

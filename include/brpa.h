@@ -404,8 +404,9 @@ int brpa_ao_mo(brpa_ctx *ctx, double *CRG, const double *RG, int64_t nvecs, int6
  * a Cholesky factor of 1 + l Pi(u) built from R.  Guess vectors: uniform
  * (-1/2, 1/2) from a SplitMix64 counter hash of (seed, column, row), columns
  * normalised (the reference draws them from gfortran's RNG, 571-588).
- * precision: BRPA_FP64 (the drop-in: FP64 GEMMs; up to 384 MB of device scratch
- * beside the operands, or two naux x nguess blocks) or BRPA_SPLIT_I8: the
+ * precision: BRPA_FP64 (the drop-in: FP64 GEMMs; beside the operands 128 MB of
+ * device scratch, an nguess x nguess block, and two more of 128 MB or
+ * naux x nguess) or BRPA_SPLIT_I8: the
  * amplitude contractions R^T chi_k Omega, R Y_k and R^T chi_k T run as
  * split-int8 GEMMs (5 int8 slices per value, 15 products, exact int32 level
  * sums, FP64 combination; nocc*nvir <= 65536); Pi(u), the Cholesky factors,
