@@ -79,7 +79,21 @@ extern "C" int brpa_ecrpa_grad(brpa_ctx *ctx, const double *R, int64_t naux, con
     double *Uinv;
     int64_t *dchol;
     // matrices per batch of the triangular inverse: its scratch is X
-    const int64_t nbi = std::max<int64_t>(1, std::min<int64_t>({F, K * N / trinv_scratch(N), 65535}));
+    // frequencies per product M_k R^T: the number with the fewest rounds of tiles (two
+    // work-groups per CU) over all F, within 2 GB of X.  N = 2400, K = 19200, F = 16: 2850
+    // tiles each, 6 rounds of 512 (0.93 full); five together 28 (0.99): the gradient 122.6
+    // and 119.0 ms.
+    const int64_t slots = 2 * (ctx->ncu > 0 ? ctx->ncu : 256);
+    const int64_t tiles = cdiv(N, 128) * cdiv(K, 128);
+    int64_t kb = 1, rounds = INT64_MAX;
+    for (int64_t b = 1; b <= F && (b == 1 || b * K * N <= (int64_t)1 << 28); ++b) {
+        const int64_t r = F / b * cdiv(b * tiles, slots) + cdiv(F % b * tiles, slots);
+        if (r < rounds) {
+            rounds = r;
+            kb = b;
+        }
+    }
+    const int64_t nbi = std::max<int64_t>(1, std::min<int64_t>({F, kb * K * N / trinv_scratch(N), 65535}));
     auto layout = [&](Arena &ar) {
         dfd = ar.take<FragDev>(1);
         dpre = ar.take<int64_t>(pre.size());
@@ -94,7 +108,7 @@ extern "C" int brpa_ecrpa_grad(brpa_ctx *ctx, const double *R, int64_t naux, con
         fd.evir = ar.take<double>(nvir);
         dc = ar.take<double>(F * K);
         ddc = ar.take<double>(F * K);
-        X = ar.take<double>(std::max(K * N, nbi * trinv_scratch(N)));
+        X = ar.take<double>(std::max(kb * K * N, nbi * trinv_scratch(N)));
         dd = ar.take<double>(K);
         fd.linv = ar.take<double>(F * CHOL_NB * CHOL_NB);
         fd.ldpart = ar.take<double>(F * nsteps * 2);
@@ -145,13 +159,16 @@ extern "C" int brpa_ecrpa_grad(brpa_ctx *ctx, const double *R, int64_t naux, con
     BRPA_TRY(launch_gemm_f64_batched(ctx, false, true, N, N, N, 1.0, Uinv, N, N * N, 0, Uinv, N,
                                      N * N, 0, 0.0, fd.Pi, N, N * N, 0, F, 1, true, TRI_B_LOWER,
                                      nullptr, 0, 0));
-    for (int64_t k = 0; k < F; ++k) {
-        // X(N x K) = M_k Rc
-        double *M = fd.Pi + k * N * N;
-        BRPA_TRY(dense_symm_fill(ctx, M, N));
-        BRPA_TRY(dense_gemm(ctx, true, false, N, K, N, 1.0, M, N, dRd, N, 0.0, X, N));
-        BRPA_TRY(launch_grad_acc(ctx, X, dRd, N, K, dc + k * K, ddc + k * K,
-                                 fw[k] / (2.0 * kPi), ddR, dd));
+    for (int64_t k = 0; k < F; ++k) BRPA_TRY(dense_symm_fill(ctx, fd.Pi + k * N * N, N));
+    for (int64_t k0 = 0; k0 < F; k0 += kb) {
+        // X_k (N x K) = M_k Rc
+        const int64_t nb = std::min(kb, F - k0);
+        BRPA_TRY(launch_gemm_f64_batched(ctx, true, false, N, K, N, 1.0, fd.Pi + k0 * N * N, N, N * N,
+                                         0, dRd, N, 0, 0, 0.0, X, N, K * N, 0, nb, 1, false, TRI_NONE,
+                                         nullptr, 0, 0));
+        for (int64_t k = k0; k < k0 + nb; ++k)
+            BRPA_TRY(launch_grad_acc(ctx, X + (k - k0) * K * N, dRd, N, K, dc + k * K, ddc + k * K,
+                                     fw[k] / (2.0 * kPi), ddR, dd));
     }
     BRPA_HIP(ctx, hipEventRecord(ctx->ev1, s));
     std::vector<double> hdd(K);
