@@ -863,7 +863,7 @@ def main():
         kernel, peak = "k_potrf_diag+k_chol_panel+k_chol_rest", PEAK_FP64_TFLOPS
         achieved = tot_chol / (stage_ms["chol"] * 1e-3) / 1e12
     # the committed PMC runs cover the default batch (256 fragments, 16 frequencies)
-    traffic = (pmc_traffic(kernel + "_128")
+    traffic = (pmc_traffic(kernel + "<128>")
                if kernel == "k_syrk_i8" and a.nfrag == 256 and a.nfreqs == 16 else None)
     roofline_erpa = {"bound": "mfma", "achieved": round(achieved, 3), "peak": round(peak, 3),
                 "unit": "TFLOP/s", "frac": round(achieved / peak, 4), "traffic": traffic,
