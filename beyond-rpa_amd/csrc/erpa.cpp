@@ -662,9 +662,12 @@ struct StoredBufs {
     }
 };
 
-// Work-group prefix arrays [setdiag, the Cholesky's lists] of nf matrices of order N.
+// Work-group prefix arrays [setdiag, the Cholesky's lists] of nf matrices of order N, and
+// their length
+static size_t stored_pre_len(int64_t N) { return (size_t)(2 + chol_pre_len(N)); }
+
 static std::vector<int64_t> stored_prefix(int64_t N, int64_t nf) {
-    std::vector<int64_t> pre((size_t)(2 + chol_pre_len(N)));
+    std::vector<int64_t> pre(stored_pre_len(N));
     pre[0] = 0;
     pre[1] = cdiv(nf * N, 256);
     chol_prefix(pre.data() + 2, N, nf);
@@ -770,6 +773,23 @@ int noalloc_setup(int device) {
     return BRPA_OK;
 }
 
+// Bytes of the scratch array that nf matrices of order N take (pk_host: packed host
+// input), and the largest chunk of F frequencies that fits it (0: not even one)
+size_t noalloc_bytes(int64_t N, int64_t nf, bool pk_host) {
+    StoredBufs t;
+    Arena count;
+    t.layout(count, N, nf, (int)cdiv(N, CHOL_NB), stored_pre_len(N), pk_host);
+    return count.off;
+}
+int64_t noalloc_chunk(int64_t N, int64_t F, bool pk_host) {
+    auto fits = [&](int64_t nf) { return noalloc_bytes(N, nf, pk_host) <= kNoallocBytes; };
+    if (!fits(1)) return 0;
+    int64_t fc = F;
+    while (fc > 1 && !fits(fc)) fc = std::max<int64_t>(1, fc / 2);
+    while (fc < F && fits(fc + 1)) ++fc;
+    return fc;
+}
+
 static int ecrpa_stored_noalloc(brpa_ctx *ctx, double *ecrpa, const double *piu, bool packed,
                                 const double *weights, int64_t nfreqs, int64_t naux, double *eu,
                                 const char *who) {
@@ -788,21 +808,12 @@ static int ecrpa_stored_noalloc(brpa_ctx *ctx, double *ecrpa, const double *piu,
     const int64_t N = naux, F = nfreqs;
     const int nsteps = (int)cdiv(N, CHOL_NB);
     const bool pk_host = packed && !is_device_ptr(piu);
-    // the largest frequency chunk whose buffers fit the scratch array
-    auto bytes_for = [&](int64_t nf) {
-        StoredBufs t;
-        Arena count;
-        t.layout(count, N, nf, nsteps, (size_t)(1 + 3 * nsteps) * 2, pk_host);
-        return count.off;
-    };
-    if (bytes_for(1) > kNoallocBytes)
+    const int64_t fc = noalloc_chunk(N, F, pk_host);
+    if (fc <= 0)
         return brpa_fail(ctx, BRPA_ERR_ARG,
                          "%s: NAux = %lld needs %zu bytes of scratch per frequency, beyond the "
                          "%zu-byte scratch array of the allocation-free entry point",
-                         who, (long long)N, bytes_for(1), kNoallocBytes);
-    int64_t fc = F;
-    while (fc > 1 && bytes_for(fc) > kNoallocBytes) fc = std::max<int64_t>(1, fc / 2);
-    while (fc < F && bytes_for(fc + 1) <= kNoallocBytes) ++fc;
+                         who, (long long)N, noalloc_bytes(N, 1, pk_host), kNoallocBytes);
     const int64_t msize = packed ? N * (N + 1) / 2 : N * N;
     long double etot = 0.0L;
     double ms_tot = 0.0;
@@ -813,6 +824,9 @@ static int ecrpa_stored_noalloc(brpa_ctx *ctx, double *ecrpa, const double *piu,
         Arena ar;
         ar.base = base;
         b.layout(ar, N, nf, nsteps, pre.size(), pk_host);
+        if (ar.off > kNoallocBytes)
+            return brpa_fail(ctx, BRPA_ERR_INTERNAL, "%s: %zu bytes laid out in %zu", who, ar.off,
+                             kNoallocBytes);
         // the chunk's energy comes back to the host (the run ends with a
         // completed copy, so e is final on return)
         double e = 0.0;
