@@ -52,9 +52,7 @@ int brpa_exchange_batch(brpa_ctx *ctx, int precision, int64_t nfrag, const brpa_
     // on the whole chip 14.2 s, 2 workers on CU halves 14.7 s; 3, 6 and 8
     // workers on CU shares were slower still.  Other counts share the chip.
     // Workers made for another worker count are replaced.
-    const char *esh = getenv("EX_SH");
-    const int nshares = esh ? atoi(esh) : nworkers == 4 ? 4 : 1;
-    if (const char *e = getenv("EX_RST")) if (atoi(e) != ctx->ex_rst) { ctx->ex_rst = atoi(e); for (brpa_ctx *w : ctx->workers) brpa_ctx_destroy(w); ctx->workers.clear(); }
+    const int nshares = nworkers == 4 ? 4 : 1;
     if ((int)ctx->workers.size() != nworkers) {
         for (brpa_ctx *w : ctx->workers) brpa_ctx_destroy(w);
         ctx->workers.clear();

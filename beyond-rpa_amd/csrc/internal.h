@@ -48,7 +48,6 @@ struct brpa_ctx {
     // contraction (kept apart from the workspace, which that call may regrow)
     double *x_V = nullptr, *x_B = nullptr;
     size_t x_V_cap = 0, x_B_cap = 0;
-    int ex_rst = 0;
     // pinned bounce buffer of the small completed copies (copy_sync), kBounceBytes
     void *bounce = nullptr;
     // pinned host staging of the batched E_RPA path (uploads and results)
