@@ -122,6 +122,7 @@ int brpa_thc_1b2g(brpa_ctx *ctx, const double *Zgh, const double *Xgi, const dou
                  : brpa_fail(ctx, BRPA_ERR_SOLVER, "rocblas_set_stream failed"));
     BRPA_HIP(ctx, hipEventRecord(ctx->ev0, ctx->stream));
     const double one = 1.0, zero = 0.0;
+    const KstatDrop kdrop{ctx};
     struct SplitLend {
         brpa_ctx *c;
         ~SplitLend() {
@@ -176,7 +177,6 @@ int brpa_thc_1b2g(brpa_ctx *ctx, const double *Zgh, const double *Xgi, const dou
             volatile char *p = reinterpret_cast<char *>(yxu_diag) + b;
             *p = *p;
         }
-    kstat_drop(ctx);
     std::vector<double> hs(2 * nt);
     BRPA_TRY(copy_sync(ctx, hs.data(), S, 8 * 2 * nt, hipMemcpyDeviceToHost));
     if (yxu_diag && !ddev) BRPA_TRY(copy_sync(ctx, yxu_diag, dD, 8 * G * nt, hipMemcpyDeviceToHost));

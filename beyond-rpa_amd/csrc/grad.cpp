@@ -55,6 +55,7 @@ extern "C" int brpa_ecrpa_grad(brpa_ctx *ctx, const double *R, int64_t naux, con
     if (!(*std::min_element(ev.begin(), ev.end()) - *std::max_element(eo.begin(), eo.end()) > 0.0))
         return brpa_fail(ctx, BRPA_ERR_GAP, "Found invalid orbital energy gap.");
     BRPA_HIP(ctx, hipSetDevice(ctx->device));
+    const KstatDrop kdrop{ctx};
 
     // c_k and dc_k/dd per (k, ai)
     std::vector<double> cc(F * K), dcc(F * K);

@@ -117,6 +117,12 @@ int kstat_begin(brpa_ctx *ctx, size_t *slot);
 int kstat_end(brpa_ctx *ctx, size_t slot, int kernel, double flops);
 int kstat_collect(brpa_ctx *ctx);
 void kstat_drop(brpa_ctx *ctx);
+// Drops the pairs of a call that reports no kernel times, however the call ends (they
+// would pile up in the context from call to call)
+struct KstatDrop {
+    brpa_ctx *ctx;
+    ~KstatDrop() { kstat_drop(ctx); }
+};
 
 // One lock for every rocSOLVER call of the library: contexts driven from
 // several host threads (the exchange batch's workers) take turns in it.

@@ -145,6 +145,7 @@ int brpa_mbpt3_1(brpa_ctx *ctx, int precision, double *ec_exchange, const double
     void *hv = nullptr;
     BRPA_TRY(rocblas_handle_of(ctx, &hv));
     rocblas_handle h = static_cast<rocblas_handle>(hv);
+    const KstatDrop kdrop{ctx};
     std::vector<double> eo(nocc), ev(nvir), d(K);
     auto hostv = [&](std::vector<double> &out, const double *p, int64_t m) -> int {
         if (is_device_ptr(p)) return copy_sync(ctx, out.data(), p, 8 * m, hipMemcpyDeviceToHost);
