@@ -1,6 +1,7 @@
 // Context, workspace and error plumbing of the C ABI.
 #include <cstdarg>
 #include <cstdio>
+#include <cstdlib>
 #include <cstring>
 
 #include "internal.h"
@@ -72,6 +73,29 @@ int copy_sync(brpa_ctx *ctx, void *dst, const void *src, size_t bytes, hipMemcpy
     return BRPA_OK;
 }
 
+// what ws_reserve allocates for `bytes`
+static size_t ws_growth(size_t bytes) { return bytes + bytes / 8 + (64u << 20); }
+
+int ws_budget(const brpa_ctx *ctx, size_t *bytes) {
+    if (const char *e = std::getenv("BRPA_WS_BUDGET_GB")) {
+        *bytes = (size_t)(std::atof(e) * (1ull << 30));
+        return BRPA_OK;
+    }
+    size_t free_b = 0, total_b = 0;
+    if (hipMemGetInfo(&free_b, &total_b) != hipSuccess) {
+        (void)hipGetLastError();
+        return BRPA_ERR_HIP;
+    }
+    *bytes = (free_b + ctx->ws_cap) / 4 * 3;
+    return BRPA_OK;
+}
+
+bool ws_affords(const brpa_ctx *ctx, size_t bytes) {
+    size_t budget = 0;
+    return bytes <= ctx->ws_cap ||
+           (ws_budget(ctx, &budget) == BRPA_OK && ws_growth(bytes) <= budget);
+}
+
 int ws_reserve(brpa_ctx *ctx, size_t bytes, Arena *arena) {
     if (bytes > ctx->ws_cap) {
         BRPA_HIP(ctx, hipStreamSynchronize(ctx->stream));
@@ -81,7 +105,7 @@ int ws_reserve(brpa_ctx *ctx, size_t bytes, Arena *arena) {
             ctx->ws = nullptr;
             ctx->ws_cap = 0;
         }
-        size_t cap = bytes + bytes / 8 + (64u << 20);
+        size_t cap = ws_growth(bytes);
         hipError_t e = hipMalloc(&ctx->ws, cap);
         if (e != hipSuccess) {
             (void)hipGetLastError();

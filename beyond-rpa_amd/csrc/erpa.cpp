@@ -385,7 +385,7 @@ int run_chunk(brpa_ctx *ctx, int precision, const std::vector<HostFrag> &fr, dou
 }
 
 // Validates every fragment, then runs the pipeline in chunks whose device
-// workspace stays under the budget (BRPA_WS_BUDGET_GB, default 64 GiB).
+// workspace stays under ws_budget.
 int run_ecrpa(brpa_ctx *ctx, int precision, const std::vector<HostFrag> &fr, double *energies,
               double *const *eu_out) {
     if (precision != BRPA_FP64 && precision != BRPA_SPLIT_BF16 && precision != BRPA_SPLIT_I8)
@@ -399,16 +399,9 @@ int run_ecrpa(brpa_ctx *ctx, int precision, const std::vector<HostFrag> &fr, dou
                              (long long)f, (long long)(fr[f].nocc * fr[f].nvir), I8_KMAX);
     }
     BRPA_HIP(ctx, hipSetDevice(ctx->device));
-    // workspace budget: BRPA_WS_BUDGET_GB, else 3/4 of the device memory that is
-    // free now plus what the context already holds
-    size_t budget;
-    if (const char *e = std::getenv("BRPA_WS_BUDGET_GB")) {
-        budget = (size_t)(std::atof(e) * (1ull << 30));
-    } else {
-        size_t free_b = 0, total_b = 0;
-        BRPA_HIP(ctx, hipMemGetInfo(&free_b, &total_b));
-        budget = (free_b + ctx->ws_cap) / 4 * 3;
-    }
+    size_t budget = 0;
+    if (ws_budget(ctx, &budget) != BRPA_OK)
+        return brpa_fail(ctx, BRPA_ERR_HIP, "hipMemGetInfo failed");
     double ms = 0.0;
     stage_reset(ctx);
     ctx->last_graph_captures = ctx->last_graph_replays = 0;

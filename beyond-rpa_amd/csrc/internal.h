@@ -157,6 +157,13 @@ struct Arena {
     }
 };
 int ws_reserve(brpa_ctx *ctx, size_t bytes, Arena *arena);
+// Workspace budget of the calls that have a choice: BRPA_WS_BUDGET_GB, else 3/4 of the
+// device memory that is free now plus what the context already holds.
+int ws_budget(const brpa_ctx *ctx, size_t *bytes);
+// Whether a form that is faster but takes a workspace of `bytes` may be chosen: the context
+// holds that much already, or growing to it stays under the budget.  Otherwise the
+// call takes its form with less scratch, so that it runs wherever that one fits.
+bool ws_affords(const brpa_ctx *ctx, size_t bytes);
 bool is_device_ptr(const void *p);
 // Copy n elements of a host-or-device array into device memory dst.
 int to_device(brpa_ctx *ctx, void *dst, const void *src, size_t bytes);
@@ -259,7 +266,8 @@ int launch_syrk_i8(brpa_ctx *, const FragDev *, const int64_t *pre, int nfrag, i
 
 // SOSEX contraction in the explicit ov space, E = -alpha sum (aj|bi) (V X V^T)(ai, bj), with
 // X = diag(hB) (host), or VX (device, NT2 x K column-major like V) = X V^T given; and
-// whether it is the cheaper form
+// whether it is the cheaper form, and its workspace
+size_t sosex_explicit_bytes(bool rdev, bool vdev, bool vx, int64_t o, int64_t v, int64_t N, int64_t nt);
 bool sosex_prefers_explicit(int precision, int64_t o, int64_t v, int64_t N, int64_t nt);
 int sosex_explicit(brpa_ctx *, double *ec, double alpha, const double *V, const double *hB,
                    const double *VX, const double *R, int64_t o, int64_t v, int64_t N, int64_t nt);

@@ -332,7 +332,8 @@ int brpa_mbpt3_1(brpa_ctx *ctx, int precision, double *ec_exchange, const double
     };
     BRPA_TRY(grow(ctx, &ctx->x_V, &ctx->x_V_cap, (size_t)K * n));
     // X = Am / 2
-    if (sosex_prefers_explicit(precision, nocc, nvir, N, n)) {
+    if (sosex_prefers_explicit(precision, nocc, nvir, N, n) &&
+        ws_affords(ctx, sosex_explicit_bytes(rdev, vdev, true, nocc, nvir, N, n))) {
         BRPA_TRY(dense_gemm(ctx, false, false, n, K, n, 0.5, Am, n, dV, n, 0.0, ctx->x_V, n));
         BRPA_TRY(end_stage());
         // V and R as the caller gave them: the workspace copies may not survive the

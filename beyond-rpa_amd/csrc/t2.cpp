@@ -748,31 +748,50 @@ bool sosex_prefers_explicit(int precision, int64_t o, int64_t v, int64_t N, int6
     return ex < pr && v <= kSosexBlock;
 }
 
-int sosex_explicit(brpa_ctx *ctx, double *ec, double alpha, const double *V, const double *hB,
-                   const double *VX, const double *R, int64_t o, int64_t v, int64_t N, int64_t nt) {
-    const int64_t K = o * v;
-    const bool rdev = is_device_ptr(R), vdev = is_device_ptr(V);
-    const int64_t ob = std::min(o, std::max<int64_t>(1, kSosexBlock / v)), bs = ob * v;
-    // split-k partial tiles (up to 8) for blocks that leave the chip idle
-    const int64_t nsplit = std::min<int64_t>(8 * bs * bs, (int64_t)1 << 27);
-    double *dR, *dV, *dB, *VB, *G, *M, *part, *splitws;
-    auto layout = [&](Arena &ar) {
-        dR = rdev ? const_cast<double *>(R) : ar.take<double>(K * N);
-        dV = vdev ? const_cast<double *>(V) : ar.take<double>(K * nt);
-        dB = VX ? nullptr : ar.take<double>(nt);
-        VB = VX ? const_cast<double *>(VX) : ar.take<double>(K * nt);
+namespace {
+struct SosexExplicit {
+    int64_t ob, bs, nsplit;   // occupied orbitals and ov rows per block, split-k partials
+    double *R, *V, *B, *VB, *G, *M, *part, *splitws;
+    // rdev, vdev: R and V are device memory; vx: so is V X
+    void layout(Arena &ar, bool rdev, bool vdev, bool vx, int64_t o, int64_t v, int64_t N, int64_t nt) {
+        const int64_t K = o * v;
+        ob = std::min(o, std::max<int64_t>(1, kSosexBlock / v));
+        bs = ob * v;
+        // partial tiles (up to 8) for blocks that leave the chip idle
+        nsplit = std::min<int64_t>(8 * bs * bs, (int64_t)1 << 27);
+        R = rdev ? nullptr : ar.take<double>(K * N);
+        V = vdev ? nullptr : ar.take<double>(K * nt);
+        B = vx ? nullptr : ar.take<double>(nt);
+        VB = vx ? nullptr : ar.take<double>(K * nt);
         G = ar.take<double>(bs * bs);
         M = ar.take<double>(bs * bs);
         part = ar.take<double>(cdiv(o, ob) * K);
         splitws = ar.take<double>(nsplit);
-    };
-    Arena count, ar;
-    layout(count);
-    BRPA_TRY(ws_reserve(ctx, count.off, &ar));
-    layout(ar);
-    if (!rdev) BRPA_TRY(to_device(ctx, dR, R, 8 * K * N));
-    if (!vdev) BRPA_TRY(to_device(ctx, dV, V, 8 * K * nt));
-    if (!VX) BRPA_TRY(copy_sync(ctx, dB, hB, 8 * nt, hipMemcpyHostToDevice));
+    }
+};
+}  // namespace
+
+size_t sosex_explicit_bytes(bool rdev, bool vdev, bool vx, int64_t o, int64_t v, int64_t N, int64_t nt) {
+    SosexExplicit b;
+    Arena count;
+    b.layout(count, rdev, vdev, vx, o, v, N, nt);
+    return count.off;
+}
+
+int sosex_explicit(brpa_ctx *ctx, double *ec, double alpha, const double *V, const double *hB,
+                   const double *VX, const double *R, int64_t o, int64_t v, int64_t N, int64_t nt) {
+    const int64_t K = o * v;
+    const bool rdev = is_device_ptr(R), vdev = is_device_ptr(V);
+    SosexExplicit b;
+    Arena ar;
+    BRPA_TRY(ws_reserve(ctx, sosex_explicit_bytes(rdev, vdev, VX != nullptr, o, v, N, nt), &ar));
+    b.layout(ar, rdev, vdev, VX != nullptr, o, v, N, nt);
+    const int64_t ob = b.ob;
+    const double *dR = rdev ? R : b.R, *dV = vdev ? V : b.V;
+    double *VB = VX ? const_cast<double *>(VX) : b.VB, *G = b.G, *M = b.M, *part = b.part;
+    if (!rdev) BRPA_TRY(to_device(ctx, b.R, R, 8 * K * N));
+    if (!vdev) BRPA_TRY(to_device(ctx, b.V, V, 8 * K * nt));
+    if (!VX) BRPA_TRY(copy_sync(ctx, b.B, hB, 8 * nt, hipMemcpyHostToDevice));
     struct SplitLend {
         brpa_ctx *c;
         ~SplitLend() {
@@ -780,14 +799,14 @@ int sosex_explicit(brpa_ctx *ctx, double *ec, double alpha, const double *V, con
             c->split_ws_cap = 0;
         }
     } lend{ctx};
-    ctx->split_ws = splitws;
-    ctx->split_ws_cap = (size_t)nsplit;
+    ctx->split_ws = b.splitws;
+    ctx->split_ws_cap = (size_t)b.nsplit;
     kstat_drop(ctx);
     BRPA_HIP(ctx, hipEventRecord(ctx->ev0, ctx->stream));
     BRPA_TRY(stage_begin(ctx, BRPA_STAGE_SOSEX));
     // R and V are column-major N x K and NT2 x K here: every product is TN, both
     // operands contiguous in k
-    if (!VX) BRPA_TRY(launch_row_scale(ctx, VB, dV, dB, nt, K));
+    if (!VX) BRPA_TRY(launch_row_scale(ctx, VB, dV, b.B, nt, K));
     int64_t np = 0;
     for (int64_t i0 = 0; i0 < o; i0 += ob) {
         const int64_t ni = std::min(ob, o - i0), mi = ni * v;
@@ -1047,31 +1066,47 @@ int brpa_sosex(brpa_ctx *ctx, int precision, double *ec_exchange, double alpha, 
     // B = A, or A/(1-4A^2) for the cumulant route (rpa_CC_Exchange.f90:62-68)
     std::vector<double> hB(nt);
     for (int64_t k = 0; k < nt; ++k) hB[k] = s2_operator ? hA[k] / (1.0 - 4.0 * hA[k] * hA[k]) : hA[k];
-    if (sosex_prefers_explicit(precision, o, v, N, nt))
-        return sosex_explicit(ctx, ec_exchange, alpha, V, hB.data(), nullptr, R, o, v, N, nt);
-    const bool rdev = is_device_ptr(R), vdev = is_device_ptr(V);
-    if (precision == BRPA_SPLIT_I8) {
-        // fused split-int8 pair kernel: 5 int8 slices per value, 15 products,
-        // exact int32 level sums, W_ij and W_ji never stored
-        const int64_t nparts = sosex_i8_nparts(o, N, nt);
-        double *dR, *dV, *dB, *scR, *scV, *part, *out2;
-        int8_t *SR, *SV;
-        auto layout = [&](Arena &ar) {
-            dR = rdev ? const_cast<double *>(R) : ar.take<double>(K * N);
-            dV = vdev ? const_cast<double *>(V) : ar.take<double>(K * nt);
-            dB = ar.take<double>(nt);
+    const bool rdev = is_device_ptr(R), vdev = is_device_ptr(V), i8 = precision == BRPA_SPLIT_I8;
+    // the pair forms' buffers; in FP64 pairs (i, j >= i) are processed per i in batches of
+    // jb occupied indices
+    const size_t wbytes_per_j = 2 * 8 * (size_t)N * nt;
+    int64_t jb = std::max<int64_t>(1, std::min<int64_t>(o, (int64_t)((8ull << 30) / wbytes_per_j)));
+    const int nchunk = sosex_nchunk(N, nt);
+    double *dR, *dV, *dB, *part, *scR, *scV, *out2, *W1, *W2;
+    int8_t *SR, *SV;
+    auto layout = [&](Arena &ar) {
+        dR = rdev ? const_cast<double *>(R) : ar.take<double>(K * N);
+        dV = vdev ? const_cast<double *>(V) : ar.take<double>(K * nt);
+        dB = ar.take<double>(nt);
+        if (i8) {
             scR = ar.take<double>(o * N);
             scV = ar.take<double>(o * nt);
             SR = ar.take<int8_t>(sosex_i8_slice_bytes(o, N, v));
             SV = ar.take<int8_t>(sosex_i8_slice_bytes(o, nt, v));
-            part = ar.take<double>(2 * nparts);
+            part = ar.take<double>(2 * sosex_i8_nparts(o, N, nt));
             out2 = ar.take<double>(2);
-        };
-        Arena count;
-        layout(count);
-        Arena ar;
-        BRPA_TRY(ws_reserve(ctx, count.off, &ar));
-        layout(ar);
+        } else {
+            W1 = ar.take<double>(jb * N * nt);
+            W2 = ar.take<double>(jb * N * nt);
+            part = ar.take<double>(2 * o * o * nchunk);   // (i, j) pair partials
+        }
+    };
+    Arena count;
+    layout(count);
+    if (sosex_prefers_explicit(precision, o, v, N, nt)) {
+        // where its buffers are no larger than these, or affordable
+        const size_t xb = sosex_explicit_bytes(rdev, vdev, false, o, v, N, nt);
+        if (xb <= count.off || ws_affords(ctx, xb)) {
+            const int rc = sosex_explicit(ctx, ec_exchange, alpha, V, hB.data(), nullptr, R, o, v, N, nt);
+            if (rc != BRPA_ERR_OOM) return rc;
+        }
+    }
+    Arena ar;
+    BRPA_TRY(ws_reserve(ctx, count.off, &ar));
+    layout(ar);
+    if (i8) {
+        // fused split-int8 pair kernel: 5 int8 slices per value, 15 products,
+        // exact int32 level sums, W_ij and W_ji never stored
         if (!rdev) BRPA_TRY(to_device(ctx, dR, R, 8 * K * N));
         if (!vdev) BRPA_TRY(to_device(ctx, dV, V, 8 * K * nt));
         BRPA_TRY(copy_sync(ctx, dB, hB.data(), 8 * nt, hipMemcpyHostToDevice));
@@ -1092,24 +1127,6 @@ int brpa_sosex(brpa_ctx *ctx, int precision, double *ec_exchange, double alpha, 
         *ec_exchange = (double)(-(long double)alpha * ((long double)h2[0] + (long double)h2[1]));
         return BRPA_OK;
     }
-    // pairs (i, j >= i) are processed per i in batches of jb occupied indices
-    const size_t wbytes_per_j = 2 * 8 * (size_t)N * nt;
-    int64_t jb = std::max<int64_t>(1, std::min<int64_t>(o, (int64_t)((8ull << 30) / wbytes_per_j)));
-    const int nchunk = sosex_nchunk(N, nt);
-    double *dR, *dV, *dB, *W1, *W2, *part;
-    auto layout = [&](Arena &ar) {
-        dR = rdev ? const_cast<double *>(R) : ar.take<double>(K * N);
-        dV = vdev ? const_cast<double *>(V) : ar.take<double>(K * nt);
-        dB = ar.take<double>(nt);
-        W1 = ar.take<double>(jb * N * nt);
-        W2 = ar.take<double>(jb * N * nt);
-        part = ar.take<double>(2 * o * o * nchunk);   // (i, j) pair partials
-    };
-    Arena count;
-    layout(count);
-    Arena ar;
-    BRPA_TRY(ws_reserve(ctx, count.off, &ar));
-    layout(ar);
     if (!rdev) BRPA_TRY(to_device(ctx, dR, R, 8 * K * N));
     if (!vdev) BRPA_TRY(to_device(ctx, dV, V, 8 * K * nt));
     BRPA_TRY(copy_sync(ctx, dB, hB.data(), 8 * nt, hipMemcpyHostToDevice));

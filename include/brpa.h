@@ -68,7 +68,12 @@ const char *brpa_last_error(const brpa_ctx *ctx);
 /* Use an external HIP stream (e.g. torch's current stream); NULL restores the
  * context's own stream.  The caller keeps ownership of the stream. */
 int brpa_ctx_set_stream(brpa_ctx *ctx, void *hip_stream);
-/* Release the device workspace (it grows on demand and is kept otherwise). */
+/* Release the device workspace (it grows on demand and is kept otherwise).
+ * Calls with a faster form that takes more scratch choose it only where the
+ * workspace holds that much already or may grow to it within the budget:
+ * the environment variable BRPA_WS_BUDGET_GB, else 3/4 of the device memory
+ * that is free at the call plus what the context holds.  The other form runs
+ * otherwise; the two agree to rounding (or to the bound of `precision`). */
 int brpa_ctx_trim(brpa_ctx *ctx);
 /* hipGraph replay of the batched E_RPA launch sequence (no counterpart in the
  * reference, which has no GPU path).  When enabled and every fragment's R is
@@ -455,8 +460,9 @@ int brpa_t2_copyout_ov(brpa_ctx *ctx, double *A, double *V);
 /* EcExchange = -alpha sum_{aibj} (aj|bi) T(ai,bj), T = V^T diag(B) V with
  * B = A (or A/(1-4A^2) when s2_operator).  Where it takes less time (all but few
  * amplitude vectors) (ai|bj) and T are formed as ov x ov blocks on the library's
- * FP64 GEMM in both precisions (up to 4.3 GB of device scratch beside a copy of V);
- * otherwise pair by pair, W_ij = R_i V_j^T, in `precision`.  Replaces rpa_CC_Exchange_SOSEX
+ * FP64 GEMM in both precisions (up to 5.4 GB of device scratch beside a copy of V:
+ * two blocks of 16384 x 16384 and 1.1 GB of split-k partials) if the workspace may
+ * grow to that (brpa_ctx_trim); otherwise pair by pair, W_ij = R_i V_j^T, in `precision`.  Replaces rpa_CC_Exchange_SOSEX
  * (rpa/rpa_CC_Exchange.f90:36-97).  V: C V[ai][mu] (Fortran Vkai(NVecsT2, v, o)),
  * R: C R[ai][P] (Fortran Rkai(NVecsPiU, v, o)).  precision: BRPA_FP64 (the
  * drop-in: rocBLAS FP64 GEMMs per pair block, double-double pair sums) or
@@ -476,9 +482,9 @@ int brpa_sosex(brpa_ctx *ctx, int precision, double *ec_exchange, double alpha, 
  *   EcExchange = -sum_{aibj} (aj|bi) (V X V^T)(ai, bj).
  * V: C V[ai][mu] (Fortran Vkai(NVecsT2, v, o)), R: C R[ai][P]; host or device.
  * The Lyapunov equation is solved by a scaled matrix-sign iteration (no
- * Schur form); X is factored (-X = U'^T U', or its eigenpairs) and the trace
- * is the SOSEX contraction of brpa_sosex in `precision` (BRPA_FP64 or
- * BRPA_SPLIT_I8).  OccEnergies/VirtEnergies: the orbital energies the
+ * Schur form).  The trace is the SOSEX contraction of brpa_sosex: its explicit
+ * form takes X itself, the pair forms in `precision` (BRPA_FP64 or BRPA_SPLIT_I8)
+ * a factor of X (-X = U'^T U', or its eigenpairs).  OccEnergies/VirtEnergies: the orbital energies the
  * caller's route uses (canonical or semicanonical, rpa_CC.f90:977-987). */
 int brpa_mbpt3_1(brpa_ctx *ctx, int precision, double *ec_exchange, const double *V,
                  const double *A, int64_t nvecs_t2, const double *R, int64_t naux,

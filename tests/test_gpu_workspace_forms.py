@@ -1,0 +1,100 @@
+"""Calls with a faster form that takes more device scratch run in the other form where the
+workspace may not grow that far (BRPA_WS_BUDGET_GB, else 3/4 of the free memory): same
+results, and the form that ran as the kernel times tell it.  A context of its own per
+case, since a workspace once held is used."""
+import math
+
+import numpy as np
+import pytest
+
+import brpa
+from brpa import _lib, synth
+from oracle import mbpt3
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+
+U = 2.0 ** -53
+
+
+@pytest.fixture
+def small(monkeypatch):
+    """Runs a call on a new context whose workspace may not grow beyond what the call
+    cannot do without; returns its result and the launches of one measured kernel."""
+    def run(call, kernel):
+        monkeypatch.setenv("BRPA_WS_BUDGET_GB", "0")
+        c = brpa.Context(0)
+        try:
+            return call(c), _launches(c, kernel)
+        finally:
+            c.close()
+            monkeypatch.delenv("BRPA_WS_BUDGET_GB")
+    return run
+
+
+def _launches(c, kernel):
+    import ctypes as C
+    n = C.c_int64()
+    assert c._lib.brpa_last_kernel_stats(c._h, kernel, None, None, C.byref(n)) == 0
+    return n.value
+
+
+def _amplitudes(o, v, n, nt, seed, s2=False):
+    rng = np.random.default_rng(seed)
+    R = 0.3 * rng.standard_normal((o * v, n)) * np.exp(-4.0 * np.arange(n) / n)
+    V = rng.standard_normal((o * v, nt)) / math.sqrt(o * v)
+    return R, V, -0.45 * np.exp(-7.0 * np.arange(nt) / nt)
+
+
+def _sosex(R, V, B, o, v):
+    """-sum (aj|bi) T(ai, bj) and (N + NT2) u times its absolute sum, doubled."""
+    G = (R @ R.T).reshape(o, v, o, v)
+    T = ((V * B) @ V.T).reshape(o, v, o, v)
+    p = np.einsum("iajb,jaib->iajb", G, T)
+    return -p.sum(), 2.0 * (R.shape[1] + V.shape[1]) * U * np.abs(p).sum()
+
+
+# shapes that take the explicit form where there is memory for it
+@pytest.mark.parametrize("o,v,n,nt", [(2, 16, 20, 24), (3, 12, 40, 36), (5, 26, 64, 90),
+                                      (6, 33, 97, 190), (9, 65, 150, 300)])
+@pytest.mark.parametrize("precision", ["fp64", "split_i8"])
+@pytest.mark.parametrize("dev", [False, True])
+def test_sosex_pairs(ctx, small, o, v, n, nt, precision, dev):
+    R, V, A = _amplitudes(o, v, n, nt, 10 * o + v)
+    conv = (lambda x: torch.from_numpy(x).cuda()) if dev else (lambda x: x)
+    # the split pair kernel truncates at 2^-35 of the column maxima
+    slack = 1e-7 if precision == "split_i8" else 0.0
+    for s2, b in ((False, A), (True, A / (1.0 - 4.0 * A * A))):
+        ref, tol = _sosex(R, V, b, o, v)
+        call = lambda c: c.sosex(conv(V), conv(A), conv(R), o, v, s2_operator=s2,  # noqa: E731
+                                 precision=precision)
+        e, dots = small(call, _lib.KERNEL_SOSEX_DOT)
+        assert dots == 0 and abs(e - ref) <= tol + slack, (dots, e, ref)
+        e = call(ctx)
+        assert _launches(ctx, _lib.KERNEL_SOSEX_DOT) > 0 and abs(e - ref) <= tol, (e, ref)
+
+
+@pytest.mark.parametrize("precision", ["fp64", "split_i8"])
+@pytest.mark.parametrize("signs", ["negative", "both"])
+@pytest.mark.parametrize("o,v,n,nt", [(4, 60, 30, 12), (10, 200, 500, 480)])
+def test_mbpt3_1_pairs(ctx, small, o, v, n, nt, precision, signs):
+    """MBPT3-1 by a factor of X and the pair products, its Cholesky factor, or with
+    amplitudes of both signs (X indefinite) the eigenpairs: few vectors, which take it
+    anyway, and many where the explicit form's blocks are not affordable."""
+    f = synth.make_fragment(o, v, n, 12)
+    rng = np.random.default_rng(5)
+    V = np.ascontiguousarray(np.linalg.qr(rng.standard_normal((o * v, nt)))[0])
+    A = rng.uniform(-0.3, 0.3 if signs == "both" else -0.01, nt)
+    Am, Bm = mbpt3.mbpt3_1_matrices(f.R, V, A, f.eocc, f.evir)
+    X = mbpt3.lyapunov(Bm, Am)
+    ev = np.linalg.eigvalsh(0.5 * (X + X.T))
+    assert ev.min() < 0.0 and (ev.max() > 0.0) == (signs == "both")
+    ref = -mbpt3.trxk(f.R, V, X, o, v)
+    e, dots = small(lambda c: c.mbpt3_1(V, A, f.R, f.eocc, f.evir, precision=precision),
+                    _lib.KERNEL_SOSEX_DOT)
+    assert dots == 0
+    assert abs(e - ref) <= (1e-10 * abs(ref) if precision == "fp64" else 1e-7)
+    e = ctx.mbpt3_1(V, A, f.R, f.eocc, f.evir, precision=precision)
+    assert (_launches(ctx, _lib.KERNEL_SOSEX_DOT) > 0) == (nt > v / 2)
+    assert abs(e - ref) <= (1e-10 * abs(ref) if precision == "fp64" else 1e-7)
