@@ -70,9 +70,11 @@ int brpa_thc_1b2g(brpa_ctx *ctx, const double *Zgh, const double *Xgi, const dou
     else
         std::memcpy(a.data(), Am, 8 * nt);
     const int npairs = thc_1b2g_npairs(G);
-    const bool ex = explicit_pays(G, o, v, nt);
+    bool ex = explicit_pays(G, o, v, nt);
     const int64_t K = o * v;
-    // even leading dimensions: the GEMM then loads its panels straight into LDS
+    // leading dimensions of the explicit form's own matrices: a multiple of 16 bytes, for loads
+    // on that boundary (TN 4096^3: 1945 us with an odd one, 1893 with an even one; a
+    // padded copy of an operand that the caller gave would cost as much)
     const int64_t gp = G + (G & 1), kp = K + (K & 1), L = o * (o + 1) / 2;
     // amplitude vectors per chunk: YU (G x o per vector) below ~1 GB, at most 65535
     const int64_t nmu = std::max<int64_t>(
@@ -81,7 +83,7 @@ int brpa_thc_1b2g(brpa_ctx *ctx, const double *Zgh, const double *Xgi, const dou
                udev = is_device_ptr(Uaim), ddev = yxu_diag && is_device_ptr(yxu_diag);
     const double *dZ = Zgh, *dX = Xgi, *dY = Yga, *dU = Uaim;
     double *YU, *part, *S, *dD = yxu_diag;
-    double *Zp = nullptr, *P, *ZP, *Q, *W, *D, *Up = nullptr, *DU, *splitws = nullptr;
+    double *P, *ZP, *Q, *W, *D, *DU, *splitws = nullptr;
     const int64_t nsplit = (int64_t)1 << 24;   // the GEMM's split-k partials: 128 MB
     auto layout = [&](Arena &ar) {
         if (!zdev) dZ = ar.take<double>(G * G);
@@ -93,8 +95,6 @@ int brpa_thc_1b2g(brpa_ctx *ctx, const double *Zgh, const double *Xgi, const dou
         part = ar.take<double>(ex ? thc_s2_blocks(G) * nmu : (int64_t)npairs * nmu * 2);
         S = ar.take<double>(2 * nt);
         if (!ex) return;
-        if (gp != G) Zp = ar.take<double>(gp * G);
-        if (kp != K) Up = ar.take<double>(kp * nt);
         P = ar.take<double>(gp * std::max(K, L));
         ZP = ar.take<double>(gp * K);
         Q = ar.take<double>(gp * L);
@@ -103,8 +103,15 @@ int brpa_thc_1b2g(brpa_ctx *ctx, const double *Zgh, const double *Xgi, const dou
         DU = ar.take<double>(K * nt);
         splitws = ar.take<double>(nsplit);
     };
+    // the explicit form where its buffers are affordable
     Arena count, ar;
     layout(count);
+    if (ex && (!ws_affords(ctx, count.off) ||
+               ws_reserve(ctx, count.off, &ar) == BRPA_ERR_OOM)) {
+        ex = false;
+        count = Arena{};
+        layout(count);
+    }
     BRPA_TRY(ws_reserve(ctx, count.off, &ar));
     dZ = Zgh;
     dX = Xgi;
@@ -133,25 +140,15 @@ int brpa_thc_1b2g(brpa_ctx *ctx, const double *Zgh, const double *Xgi, const dou
     if (ex) {
         ctx->split_ws = splitws;
         ctx->split_ws_cap = (size_t)nsplit;
-        const double *Zs = dZ;
-        if (Zp) {
-            BRPA_HIP(ctx, hipMemcpy2DAsync(Zp, 8 * gp, dZ, 8 * G, 8 * G, G, hipMemcpyDeviceToDevice,
-                                           ctx->stream));
-            Zs = Zp;
-        }
         // Q = Z XX, D from P^T (Z P); Z is symmetric, so every product is TN
         BRPA_TRY(launch_thc_xx(ctx, dX, G, o, P, gp));
-        BRPA_TRY(launch_gemm_f64(ctx, true, false, G, L, G, 1.0, Zs, gp, P, gp, 0.0, Q, gp, false));
+        BRPA_TRY(launch_gemm_f64(ctx, true, false, G, L, G, 1.0, dZ, G, P, gp, 0.0, Q, gp, false));
         BRPA_TRY(launch_thc_pairs(ctx, dY, dX, G, v, o, P, gp));
-        BRPA_TRY(launch_gemm_f64(ctx, true, false, G, K, G, 1.0, Zs, gp, P, gp, 0.0, ZP, gp, false));
+        BRPA_TRY(launch_gemm_f64(ctx, true, false, G, K, G, 1.0, dZ, G, P, gp, 0.0, ZP, gp, false));
         BRPA_TRY(launch_gemm_f64(ctx, true, false, K, K, G, 1.0, P, gp, ZP, gp, 0.0, W, K, true));
         BRPA_TRY(launch_swap_occ(ctx, W, v, o, D, kp));
         // D U of every vector in one product (its grid is too small chunk by chunk)
-        if (Up)
-            BRPA_HIP(ctx, hipMemcpy2DAsync(Up, 8 * kp, dU, 8 * K, 8 * K, nt,
-                                           hipMemcpyDeviceToDevice, ctx->stream));
-        BRPA_TRY(launch_gemm_f64(ctx, true, false, K, nt, K, 1.0, D, kp, Up ? Up : dU, kp, 0.0, DU,
-                                 K, false));
+        BRPA_TRY(launch_gemm_f64(ctx, true, false, K, nt, K, 1.0, D, kp, dU, K, 0.0, DU, K, false));
     }
     for (int64_t mu0 = 0; mu0 < nt; mu0 += nmu) {
         const int64_t m = std::min(nmu, nt - mu0);

@@ -368,8 +368,9 @@ int brpa_thc_piu(brpa_ctx *ctx, double *PiU, double *Rkai, const double *Xga, co
  * Few vectors: one fused FP64 MFMA kernel per chunk of vectors, M built and
  * contracted in registers, never stored.  Many: (aj|bi) (ov x ov) and Z (X_i o X_j)
  * are formed once and every vector's two terms follow from products with them
- * (device scratch 2 (ov)^2 + 2 ov ngrid + ov NVecsT2 doubles, at most 64 GB for the
- * first two). */
+ * (device scratch 2 (ov)^2 + 2 ov ngrid + ngrid o (o + 1) / 2 + ov NVecsT2
+ * doubles, 128 MB and up to 1 GB of Yga U; the first two at most 64 GB, and only
+ * where the workspace may grow to it all: brpa_ctx_trim). */
 int brpa_thc_1b2g(brpa_ctx *ctx, const double *Zgh, const double *Xgi, const double *Yga,
                   const double *Uaim, const double *Am, int64_t ngrid, int64_t nocc, int64_t nvir,
                   int64_t nvecs_t2, double *ec1b, double *ec2g, double *eig_sosex, double *eig_2g,

@@ -15,7 +15,7 @@ pytestmark = pytest.mark.gpu
 
 torch = pytest.importorskip("torch")
 
-U = 2.0 ** -53
+U_ = 2.0 ** -53
 
 
 @pytest.fixture
@@ -52,7 +52,7 @@ def _sosex(R, V, B, o, v):
     G = (R @ R.T).reshape(o, v, o, v)
     T = ((V * B) @ V.T).reshape(o, v, o, v)
     p = np.einsum("iajb,jaib->iajb", G, T)
-    return -p.sum(), 2.0 * (R.shape[1] + V.shape[1]) * U * np.abs(p).sum()
+    return -p.sum(), 2.0 * (R.shape[1] + V.shape[1]) * U_ * np.abs(p).sum()
 
 
 # shapes that take the explicit form where there is memory for it
@@ -98,3 +98,42 @@ def test_mbpt3_1_pairs(ctx, small, o, v, n, nt, precision, signs):
     e = ctx.mbpt3_1(V, A, f.R, f.eocc, f.evir, precision=precision)
     assert (_launches(ctx, _lib.KERNEL_SOSEX_DOT) > 0) == (nt > v / 2)
     assert abs(e - ref) <= (1e-10 * abs(ref) if precision == "fp64" else 1e-7)
+
+
+def _thc_inputs(o, v, g, nt, seed):
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(seed)
+    rnd = lambda *s: torch.randn(s, generator=gen, dtype=torch.float64, device="cuda")  # noqa: E731
+    X, Y, Zk = rnd(o, g), rnd(v, g), rnd(max(2, g // 3), g) * 0.1
+    Z, U = Zk.T @ Zk, rnd(nt, o, v) / np.sqrt(o * v)
+    return 0.5 * (Z + Z.T), X, Y, U, -0.4 * torch.rand(nt, generator=gen, dtype=torch.float64,
+                                                       device="cuda")
+
+
+@pytest.mark.parametrize("o,v,g,nt", [(12, 45, 700, 540), (11, 49, 701, 539)])
+def test_thc_1b2g_fused(small, o, v, g, nt):
+    """The workspace tells the form: the explicit one takes 128 MB for split k."""
+    ins = _thc_inputs(o, v, g, nt, o + g)
+    Z, X, Y, U, A = ins
+    bound = (2 * g + 2 * o * v + v + o) * U_
+    held = {}
+
+    def call(c):
+        free0 = torch.cuda.mem_get_info()[0]
+        out = c.thc_1b2g(*ins, want_diag=True)
+        held[len(held)] = free0 - torch.cuda.mem_get_info()[0]
+        return out
+
+    fused, _ = small(call, _lib.KERNEL_GEMM_F64)
+    c = brpa.Context(0)
+    explicit = call(c)
+    c.close()
+    assert held[0] < 200 << 20 < held[1], held
+    for m in range(nt):
+        M, B = Y.T @ (U[m].T @ X), Y.abs().T @ (U[m].abs().T @ X.abs())
+        a = float(A[m])
+        s1, c1 = float((Z * M * M.T).sum()), bound * float((Z.abs() * B * B.T).sum())
+        s2, c2 = float((Z * M * M).sum()), bound * float((Z.abs() * B * B).sum())
+        for es, eg in (fused[2:4], explicit[2:4]):
+            assert abs(es[m] + s1 * a) <= c1 * abs(a)
+            assert abs(eg[m] + 4 * s2 * a * a) <= 4 * c2 * a * a
