@@ -97,8 +97,9 @@ int brpa_thc_piu(brpa_ctx *ctx, double *PiU, double *Rkai, const double *Xga, co
     double *dR = nullptr, *dP = nullptr, *dOut = nullptr, *H = nullptr, *splitws = nullptr;
     // occupied orbitals per product, leading dimension of H, split-k partials (up to 4 of R)
     const int64_t gp = G + (G & 1);
-    const int64_t ni = std::max<int64_t>(1, std::min(nocc, ((int64_t)1 << 26) / (gp * nvir)));
-    const int64_t nsplit = std::min<int64_t>(4 * ni * nvir * N, (int64_t)1 << 26);
+    int64_t ni = std::max<int64_t>(1, std::min(nocc, ((int64_t)1 << 26) / (gp * nvir)));
+    int64_t na = nvir;   // and virtual orbitals (all, unless scratch is short)
+    int64_t nsplit = std::min<int64_t>(4 * ni * nvir * N, (int64_t)1 << 26);
     auto layout = [&](Arena &ar) {
         dfd = ar.take<FragDev>(1);
         dpre = ar.take<int64_t>(2);
@@ -109,11 +110,19 @@ int brpa_thc_piu(brpa_ctx *ctx, double *PiU, double *Rkai, const double *Xga, co
         dR = rdev ? Rkai : ar.take<double>(K * N);
         dP = direct ? PiU : ar.take<double>(F * N * N);
         dOut = (accumulate && !pdev) ? ar.take<double>(F * N * N) : nullptr;
-        H = ar.take<double>(gp * ni * nvir);
+        H = ar.take<double>(gp * ni * na);
         splitws = ar.take<double>(nsplit);
     };
     Arena count;
     layout(count);
+    if (!ws_affords(ctx, count.off)) {
+        // products of one occupied and as many virtual orbitals as 32 MB hold, no split k
+        ni = 1;
+        na = std::max<int64_t>(1, std::min(nvir, ((int64_t)1 << 22) / gp));
+        nsplit = 0;
+        count = Arena{};
+        layout(count);
+    }
     Arena ar;
     BRPA_TRY(ws_reserve(ctx, count.off, &ar));
     dXa = Xga;
@@ -146,11 +155,13 @@ int brpa_thc_piu(brpa_ctx *ctx, double *PiU, double *Rkai, const double *Xga, co
         ctx->split_ws = splitws;
         ctx->split_ws_cap = (size_t)nsplit;
         kstat_drop(ctx);
-        for (int64_t i = 0; i < nocc; i += ni) {
-            const int64_t m = std::min(ni, nocc - i) * nvir;
-            BRPA_TRY(launch_thc_pairs(ctx, dXa, dXi + i * G, G, nvir, m / nvir, H, gp));
-            BRPA_TRY(dense_gemm(ctx, true, false, N, m, G, 1.0, dZ, G, H, gp, 0.0, dR + i * nvir * N, N));
-        }
+        for (int64_t i = 0; i < nocc; i += ni)
+            for (int64_t a = 0; a < nvir; a += na) {
+                const int64_t mi = std::min(ni, nocc - i), ma = std::min(na, nvir - a);
+                BRPA_TRY(launch_thc_pairs(ctx, dXa + a * G, dXi + i * G, G, ma, mi, H, gp));
+                BRPA_TRY(dense_gemm(ctx, true, false, N, mi * ma, G, 1.0, dZ, G, H, gp, 0.0,
+                                    dR + (i * nvir + a) * N, N));
+            }
     }
     BRPA_TRY(stage_end(ctx, BRPA_STAGE_THC_R));
     BRPA_TRY(stage_begin(ctx, BRPA_STAGE_THC_PI));

@@ -137,3 +137,28 @@ def test_thc_1b2g_fused(small, o, v, g, nt):
         for es, eg in (fused[2:4], explicit[2:4]):
             assert abs(es[m] + s1 * a) <= c1 * abs(a)
             assert abs(eg[m] + 4 * s2 * a * a) <= 4 * c2 * a * a
+
+
+@pytest.mark.parametrize("o,v,n,g,launches", [(1, 1, 1, 1, 1), (3, 21, 70, 37, 3),
+                                              (5, 60, 200, 333, 5), (2, 45, 30, 131073, 4)])
+def test_thc_piu_chunks(ctx, small, o, v, n, g, launches):
+    """Products of one occupied orbital, and of as many virtual ones as 32 MB hold."""
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(g)
+    Xi, Xa, Z = (torch.randn(s, g, generator=gen, dtype=torch.float64, device="cuda")
+                 for s in (o, v, n))
+    eo, ev, x = -np.arange(o, 0.0, -1.0), np.arange(1.0, v + 1.0), np.array([0.3, 2.0])
+    call = lambda c: c.thc_piu(Xa, Xi, Z, eo, ev, x, want_R=True)  # noqa: E731
+    (Pi, R), ran = small(call, _lib.KERNEL_GEMM_F64)
+    assert ran == launches
+    Pi0, R0 = call(ctx)
+    assert _launches(ctx, _lib.KERNEL_GEMM_F64) == 1
+    H = (Xi[:, None, :] * Xa[None, :, :]).reshape(o * v, g)
+    ref, tol = H @ Z.T, 2.0 * (g + 2) * U_ * (H.abs() @ Z.abs().T)
+    assert bool(((R - ref).abs() <= tol).all()) and bool(((R0 - ref).abs() <= tol).all())
+    d = torch.from_numpy(ev[None, :] - eo[:, None]).reshape(-1, 1).cuda()
+    for w, u in enumerate(x):
+        c = 4.0 * d / (d * d + u * u)
+        for P, r in ((Pi, R), (Pi0, R0)):
+            bound = 2.0 * (o * v + 4) * U_ * (r.abs().T @ (c * r.abs()))
+            assert bool(((P[w] - r.T @ (c * r)).abs() <= bound).all())
