@@ -49,9 +49,6 @@ int brpa_thc_piu(brpa_ctx *ctx, double *PiU, double *Rkai, const double *Xga, co
     const int64_t K = nocc * nvir, N = naux, F = nfreqs, G = ngrid;
     if (K > INT32_MAX || N > 65536 || F > 4096)
         return brpa_fail(ctx, BRPA_ERR_ARG, "brpa_thc_piu: sizes beyond the supported range");
-    if (G * std::max(std::max(nocc, nvir), N) + 64 > INT32_MAX)
-        return brpa_fail(ctx, BRPA_ERR_ARG,
-                         "THC R: ngrid x max(nocc, nvir, naux) must stay below 2^31 elements");
     BRPA_HIP(ctx, hipSetDevice(ctx->device));
     std::vector<double> eo, ev, fx;
     BRPA_TRY(host_copy(ctx, eo, eocc, nocc));
@@ -76,6 +73,9 @@ int brpa_thc_piu(brpa_ctx *ctx, double *PiU, double *Rkai, const double *Xga, co
         }
         return BRPA_OK;
     }
+    if (G * std::max(std::max(nocc, nvir), N) + 64 > INT32_MAX)
+        return brpa_fail(ctx, BRPA_ERR_ARG,
+                         "THC R: ngrid x max(nocc, nvir, naux) must stay below 2^31 elements");
     // c_w(ai) = prefactor d/(d^2 + u_w^2) (rpa_THC_ChiRkai 342-370 with Alpha folded in)
     std::vector<double> c(F * K);
     for (int64_t w = 0; w < F; ++w)
