@@ -24,6 +24,8 @@
 //   k_swap_occ             D from the upper triangle of P^T Z P
 //   k_thc_s2               S2g partials and the diagonal M_mu(g, g)
 //   k_thc_terms            both sums of each vector
+#include <algorithm>
+
 #include "device_common.h"
 #include "internal.h"
 
@@ -171,14 +173,19 @@ __global__ __launch_bounds__(256) void k_thc_1b2g_reduce(const double *__restric
     }
 }
 
-// P(g, a + v j) = Y(g, a) X(g, j), leading dimension ldp; y: column a + v j
+// P(g, a + v j) = Y(g, a) X(g, j) for the ncol columns a + v j, leading dimension ldp.  The
+// grid covers the columns (x) and groups of 256 points (y) within a launch's limits and
+// walks on from there.
+constexpr int64_t PAIRS_X = 1 << 22, PAIRS_Y = 65535;   // below 2^32 threads, 2^16 groups
 __global__ __launch_bounds__(256) void k_thc_pairs(const double *__restrict__ Y,
-                                                   const double *__restrict__ X, int G, int v,
-                                                   double *__restrict__ P, int64_t ldp) {
-    const int g = blockIdx.y * 256 + threadIdx.x, c = blockIdx.x;
-    if (g >= G) return;
-    const int j = c / v, a = c - j * v;
-    P[g + ldp * c] = Y[g + (int64_t)G * a] * X[g + (int64_t)G * j];
+                                                   const double *__restrict__ X, int64_t G, int v,
+                                                   int64_t ncol, double *__restrict__ P, int64_t ldp) {
+    for (int64_t c = blockIdx.x; c < ncol; c += gridDim.x) {
+        const int j = (int)c / v, a = (int)c - j * v;
+        const double *__restrict__ y = Y + G * a, *__restrict__ x = X + G * j;
+        for (int64_t g = blockIdx.y * 256 + threadIdx.x; g < G; g += 256 * (int64_t)gridDim.y)
+            P[g + ldp * c] = y[g] * x[g];
+    }
 }
 
 // XX(g, i (i + 1) / 2 + j) = X(g, i) X(g, j), i >= j
@@ -331,8 +338,8 @@ __global__ __launch_bounds__(256) void k_thc_terms(const double *__restrict__ pa
 
 int launch_thc_pairs(brpa_ctx *ctx, const double *Y, const double *X, int64_t G, int64_t v,
                      int64_t o, double *P, int64_t ldp) {
-    hipLaunchKernelGGL(k_thc_pairs, dim3((unsigned)(v * o), (unsigned)((G + 255) / 256)), dim3(256),
-                       0, ctx->stream, Y, X, (int)G, (int)v, P, ldp);
+    const dim3 grid((unsigned)std::min(v * o, PAIRS_X), (unsigned)std::min((G + 255) / 256, PAIRS_Y));
+    hipLaunchKernelGGL(k_thc_pairs, grid, dim3(256), 0, ctx->stream, Y, X, G, (int)v, v * o, P, ldp);
     LAUNCH_CHECK(ctx);
     return BRPA_OK;
 }

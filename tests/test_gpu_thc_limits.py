@@ -28,3 +28,20 @@ def test_empty_block(ctx, o, v, g, n):
 
 def test_refused(ctx):
     assert _piu(ctx, np.zeros((1, 8, 8)), np.zeros(1), 1 << 29, 2, 3, 8, 1, 0) == _lib.ERR_ARG
+
+
+@pytest.mark.parametrize("o,v,g", [(64, (1 << 18) + 3, 1), (1, 1, (1 << 24) + 77)])
+def test_long_launches(ctx, o, v, g):
+    """More columns, and more points, of orbital products than one launch's grid covers.
+    R is an exact integer here: products of -1, 0 and 1."""
+    torch = pytest.importorskip("torch")
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(1)
+    Xi, Xa, Z = (torch.randint(-1, 2, (s, g), generator=gen, device="cuda").double()
+                 for s in (o, v, 1))
+    eo, ev, x = -np.arange(o, 0.0, -1.0), np.arange(1.0, v + 1.0), np.array([1.0])
+    _, R = ctx.thc_piu(Xa, Xi, Z, eo, ev, x, want_R=True)
+    ref = torch.zeros(o, v, dtype=torch.float64, device="cuda")
+    for i in range(o):
+        ref[i] = (Xa * (Xi[i] * Z[0])).sum(1)
+    assert torch.equal(R.view(o, v), ref)
