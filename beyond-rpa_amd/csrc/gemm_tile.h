@@ -1,6 +1,8 @@
 // One output tile of an FP64 product on v_mfma_f64_16x16x4_f64 by a work-group of four
 // waves (2 x 2): the loop of k_gemm_f64 and of the Cholesky's trailing update.
 #pragma once
+#include <type_traits>
+
 #include "device_common.h"
 
 constexpr int GKB = 16;    // k per LDS stage
@@ -16,34 +18,36 @@ typedef double d2_t __attribute__((ext_vector_type(2)));
 // vector load, so odd leading dimensions take them too): KC the 8-row blocks ROWS / 4 w +
 // 8 c, lane L the k pair (L % 8) ^ swizzle of row L / 8 of its block; rows-contiguous (128
 // rows only) the k rows 4 w + c, lane L the rows 2 L, 2 L + 1.  The byte offsets from the
-// tile's base at k = 0 (dma_base) are 32-bit; leading dimensions of 2^21 or more take
-// the register path of the last stage for all of them.
+// tile's base at k = 0 (dma_base) are 32-bit (off_t), with leading dimensions of 2^21 or
+// more (FAR) 64-bit, at the cost of their registers.
 constexpr int DMA_KPR = 132;
 template <bool KC>
 constexpr int gemm_lds(int rows) {   // doubles of one stage
     return KC ? rows * GKB : GKB * DMA_KPR;
 }
-template <bool KC, int ROWS>
+template <bool KC, int ROWS, bool FAR>
 struct DmaSrc {
     static_assert(KC || ROWS == 128, "rows-contiguous operands have 128-row tiles");
     static constexpr int NLOAD = ROWS / 32;   // loads per wave and stage
-    uint32_t off[NLOAD];
+    typedef std::conditional_t<FAR, uint64_t, uint32_t> off_t;
+    off_t off[NLOAD];
 };
-template <bool KC, int ROWS>
-__device__ __forceinline__ DmaSrc<KC, ROWS> dma_offsets(int64_t ldx, int r0, int rows, int wave,
-                                                       int lane) {
-    DmaSrc<KC, ROWS> s;
+template <bool KC, int ROWS, bool FAR>
+__device__ __forceinline__ DmaSrc<KC, ROWS, FAR> dma_offsets(int64_t ldx, int r0, int rows, int wave,
+                                                            int lane) {
+    DmaSrc<KC, ROWS, FAR> s;
+    typedef typename DmaSrc<KC, ROWS, FAR>::off_t off_t;
 #pragma unroll
-    for (int c = 0; c < DmaSrc<KC, ROWS>::NLOAD; ++c) {
+    for (int c = 0; c < s.NLOAD; ++c) {
         if (KC) {
             const int row = ROWS / 4 * wave + 8 * c + (lane >> 3);
             const int dk = 2 * ((lane & 7) ^ ((row >> 1) & 7));
-            s.off[c] = 8u * ((uint32_t)ldx * (uint32_t)(min(r0 + row, rows - 1) - r0) + (uint32_t)dk);
+            s.off[c] = 8u * ((off_t)ldx * (uint32_t)(min(r0 + row, rows - 1) - r0) + (uint32_t)dk);
         } else {
             // the pair of the last row of an odd count ends in the next k's first row
             // (dma_over)
             s.off[c] = 8u * ((uint32_t)(min(r0 + 2 * lane, (rows - 1) & ~1) - r0) +
-                             (uint32_t)ldx * (uint32_t)(4 * wave + c));
+                             (off_t)ldx * (uint32_t)(4 * wave + c));
         }
     }
     return s;
@@ -72,8 +76,8 @@ __host__ __device__ __forceinline__ d2_t dma_frag(const double *L, int row, int 
 }
 
 // one operand's full stage at k0 into the LDS buffer L, straight from global memory
-template <bool KC, int ROWS>
-__device__ __forceinline__ void dma_stage(const char *base, const DmaSrc<KC, ROWS> &src, int64_t ldx,
+template <bool KC, int ROWS, bool FAR>
+__device__ __forceinline__ void dma_stage(const char *base, const DmaSrc<KC, ROWS, FAR> &src, int64_t ldx,
                                           double *L, int wave, int k0) {
     // the builtin exists for the device pass only; the host pass never runs this
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -82,7 +86,7 @@ __device__ __forceinline__ void dma_stage(const char *base, const DmaSrc<KC, ROW
     typedef __attribute__((address_space(3))) void lvoid_t;
     gchar_t *b = (gchar_t *)(base + 8 * (KC ? (int64_t)k0 : ldx * k0));
 #pragma unroll
-    for (int c = 0; c < DmaSrc<KC, ROWS>::NLOAD; ++c)
+    for (int c = 0; c < src.NLOAD; ++c)
         __builtin_amdgcn_global_load_lds(
             (gvoid_t *)(b + src.off[c]),
             (lvoid_t *)(L + (KC ? (ROWS / 4 * wave + 8 * c) * GKB : (4 * wave + c) * DMA_KPR)), 16, 0, 0);
@@ -106,8 +110,7 @@ __device__ __forceinline__ void dma_stage_tail(const double *__restrict__ X, int
 // acc += rows m0 .. of op(A) times columns n0 .. of op(B) over k in [kbeg, kend) of [0, k): wave
 // (wm, wn) = (wave / 2, wave % 2) holds the ROWS/2 x ROWS/2 block (wm, wn), acc[i][j][r]
 // = element (16 i + lane % 16, 16 j + lane / 16 + 4 r) of it.  m, n: rows of the whole
-// operands (past them the last row repeats).  far: leading dimensions beyond 32-bit
-// offsets.  Waves with active false only stage.  sA0/1, sB0/1: the two stages of each operand
+// operands (past them the last row repeats).  FAR: 64-bit offsets.  Waves with active false only stage.  sA0/1, sB0/1: the two stages of each operand
 // (gemm_lds doubles per stage).
 //
 // The fragments of either half of a stage are read while the other half is
@@ -119,25 +122,25 @@ __device__ __forceinline__ void dma_stage_tail(const double *__restrict__ X, int
 // leading dimensions), 3072^2 x 4096 (whose last 64 of 576 tiles run one
 // per CU) 52 (68.5, 64.0 and 38-46 with all reads, then all loads, ahead of the stage's
 // MFMAs).
-template <bool KCA, bool KCB, int ROWS>
+template <bool KCA, bool KCB, int ROWS, bool FAR = false>
 __device__ __forceinline__ void gemm_tile(d4_t (&acc)[ROWS / 32][ROWS / 32],
                                           const double *__restrict__ A, int64_t lda, int m0, int m,
                                           const double *__restrict__ B, int64_t ldb, int n0, int n,
-                                          int kbeg, int kend, int k, bool far, bool active, double *sA0,
+                                          int kbeg, int kend, int k, bool active, double *sA0,
                                           double *sA1, double *sB0, double *sB1) {
     constexpr int NB = ROWS / 32;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave >> 1, wn = wave & 1;
     const int rl = lane & 15, g4 = lane >> 4;
-    const auto oa = dma_offsets<KCA, ROWS>(lda, m0, m, wave, lane);
-    const auto ob = dma_offsets<KCB, ROWS>(ldb, n0, n, wave, lane);
+    const auto oa = dma_offsets<KCA, ROWS, FAR>(lda, m0, m, wave, lane);
+    const auto ob = dma_offsets<KCB, ROWS, FAR>(ldb, n0, n, wave, lane);
     const char *ba = dma_base<KCA>(A, lda, m0), *bb = dma_base<KCB>(B, ldb, n0);
     const bool over = kend == k && (dma_over<KCA, ROWS>(m0, m) || dma_over<KCB, ROWS>(n0, n));
-    const int nfull = far ? 0 : (kend - kbeg - (over ? 1 : 0)) / GKB, ns = (kend - kbeg + GKB - 1) / GKB;
+    const int nfull = (kend - kbeg - (over ? 1 : 0)) / GKB, ns = (kend - kbeg + GKB - 1) / GKB;
     auto stage = [&](int buf, int k0) {
-        dma_stage<KCA, ROWS>(ba, oa, lda, buf ? sA1 : sA0, wave, k0);
-        dma_stage<KCB, ROWS>(bb, ob, ldb, buf ? sB1 : sB0, wave, k0);
+        dma_stage(ba, oa, lda, buf ? sA1 : sA0, wave, k0);
+        dma_stage(bb, ob, ldb, buf ? sB1 : sB0, wave, k0);
     };
     auto put = [&](int buf, int q) {
         if (q < nfull) {

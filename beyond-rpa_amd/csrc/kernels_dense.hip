@@ -4,7 +4,7 @@
 // at r + ld c), the layout of the reference's Fortran arrays and of the
 // explicit-space exchange.
 //
-//   k_gemm_f64<TA, TB>  batched C = alpha op(A) op(B) diag(cs) + beta C on
+//   k_gemm_f64          batched C = alpha op(A) op(B) diag(cs) + beta C on
 //                       128 x 128 tiles; upper mode (SYRK) and triangular
 //                       operands whose zero triangle is skipped; 16-k stages
 //                       loaded straight into LDS where alignment allows
@@ -73,7 +73,6 @@ struct GemmArgs {
     int upper, tri, nb1;
     int nsplit, kchunk;
     int tail0, tsplit;   // tiles from tail0 on in tsplit chunks of k each (1: none)
-    int far;   // a leading dimension too large for 32-bit offsets: every stage through registers
     double alpha, beta;
     const double *A;
     int64_t lda, sA1, sA2;
@@ -103,10 +102,12 @@ __device__ __forceinline__ void gemm_tile_of(const GemmArgs &g, int t, int &ti, 
     }
 }
 
-// TAIL: with the last tiles' k split (tsplit > 1, one item)
-template <bool TA, bool TB, bool TAIL>
+// G_TAIL: with the last tiles' k split (tsplit > 1, one item); G_FAR: 64-bit offsets
+enum { G_PLAIN, G_TAIL, G_FAR };
+template <bool TA, bool TB, int FORM>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_gemm_f64(const GemmArgs g) {
     constexpr bool KCA = TA, KCB = !TB;   // operand contiguous in k
+    constexpr bool TAIL = FORM == G_TAIL;
     __shared__ __attribute__((aligned(16))) double sA0[gemm_lds<KCA>(GT)], sA1[gemm_lds<KCA>(GT)];
     __shared__ __attribute__((aligned(16))) double sB0[gemm_lds<KCB>(GT)], sB1[gemm_lds<KCB>(GT)];
     const bool tail = TAIL && (int)blockIdx.x >= g.tail0;
@@ -147,8 +148,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         for (int j = 0; j < 4; ++j) acc[i][j] = (d4_t){0.0, 0.0, 0.0, 0.0};
 
     if (kbeg < kend)
-        gemm_tile<KCA, KCB, GT>(acc, A, lda, m0, m, B, ldb, n0, n, kbeg, kend, g.k, g.far != 0, true,
-                                   sA0, sA1, sB0, sB1);
+        gemm_tile<KCA, KCB, GT, FORM == G_FAR>(acc, A, lda, m0, m, B, ldb, n0, n, kbeg, kend, g.k, true,
+                                               sA0, sA1, sB0, sB1);
 
     if (g.nsplit > 1) {
         // partial tile, reduced by k_gemm_reduce
@@ -276,8 +277,10 @@ int launch_gemm_f64_batched(brpa_ctx *ctx, bool ta, bool tb, int64_t m, int64_t 
     g.scs1 = scs1;
     g.scs2 = scs2;
     g.P = nullptr;
-    // 32-bit byte offsets within a tile
-    g.far = lda >= (1 << 21) || ldb >= (1 << 21);
+    // 32-bit byte offsets within a tile (127 rows), beyond them 64-bit ones: TN 256 x 256 x
+    // (2^21 + 64) 230 ms, as long as at 2^21 - 64 (1186 with every stage through
+    // registers); NN (2^21 + 64) x 128 x 128 1.42 ms (2.91)
+    const bool far = lda >= (1 << 21) || ldb >= (1 << 21);
     // split k when the last wave of tiles would leave much of the chip idle:
     // the split count s (<= 8, chunks of >= 256 k) minimises the modelled time
     // 1/eff(s) + (reduction traffic), eff(s) = tiles s / (slots ceil(tiles s /
@@ -315,7 +318,7 @@ int launch_gemm_f64_batched(brpa_ctx *ctx, bool ta, bool tb, int64_t m, int64_t 
             }
         }
         const int64_t full = wgs / (int64_t)slots * (int64_t)slots, L = wgs - full;
-        const int64_t ts = L > 0 && full > 0 && tri == TRI_NONE
+        const int64_t ts = L > 0 && full > 0 && tri == TRI_NONE && !far
                                ? std::min<int64_t>({8, (int64_t)slots / L, g.k / 256,
                                                     (int64_t)(ctx->split_ws_cap / (size_t)(L * GT * GT))})
                                : 1;
@@ -338,14 +341,18 @@ int launch_gemm_f64_batched(brpa_ctx *ctx, bool ta, bool tb, int64_t m, int64_t 
     size_t slot = 0;
     BRPA_TRY(kstat_begin(ctx, &slot));
     auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, block, 0, ctx->stream, g); };
-    if (!ta && !tb)
-        g.tsplit > 1 ? launch(k_gemm_f64<false, false, true>) : launch(k_gemm_f64<false, false, false>);
-    else if (!ta && tb)
-        g.tsplit > 1 ? launch(k_gemm_f64<false, true, true>) : launch(k_gemm_f64<false, true, false>);
-    else if (ta && !tb)
-        g.tsplit > 1 ? launch(k_gemm_f64<true, false, true>) : launch(k_gemm_f64<true, false, false>);
-    else
-        g.tsplit > 1 ? launch(k_gemm_f64<true, true, true>) : launch(k_gemm_f64<true, true, false>);
+    auto form = [&](auto a, auto b) {
+        constexpr bool TA = decltype(a)::value, TB = decltype(b)::value;
+        if (far)
+            launch(k_gemm_f64<TA, TB, G_FAR>);
+        else if (g.tsplit > 1)
+            launch(k_gemm_f64<TA, TB, G_TAIL>);
+        else
+            launch(k_gemm_f64<TA, TB, G_PLAIN>);
+    };
+    const std::true_type yes;
+    const std::false_type no;
+    ta ? (tb ? form(yes, yes) : form(yes, no)) : (tb ? form(no, yes) : form(no, no));
     LAUNCH_CHECK(ctx);
     if (g.nsplit > 1) {
         hipLaunchKernelGGL(k_gemm_reduce, dim3((unsigned)((m * n + 255) / 256)), dim3(256), 0,

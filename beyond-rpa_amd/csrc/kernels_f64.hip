@@ -1099,7 +1099,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
     for (int r = 0; r < 16; ++r) sL[4 * r + wave][lane] = linv[(4 * r + wave) * CHOL_NB + lane];
     if (s_in > 0)
-        gemm_tile<true, true, T>(acc, A, N, j0, N, A, N, R0, N, kbase, j0, j0, false, true, sA0, sA1, sB0,
+        gemm_tile<true, true, T>(acc, A, N, j0, N, A, N, R0, N, kbase, j0, j0, true, sA0, sA1, sB0,
                                  sB1);
     __syncthreads();   // the stage buffers are read
     // row q of B's block row c, columns XOR-swizzled by 4 q
@@ -1200,7 +1200,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
     for (int i = 0; i < NB; ++i)
 #pragma unroll
         for (int j = 0; j < NB; ++j) acc[i][j] = (d4_t){0.0, 0.0, 0.0, 0.0};
-    gemm_tile<true, true, T>(acc, A, N, Rj, N, A, N, Ri, N, kbase, t0, t0, false, active, sA0, sA1, sB0,
+    gemm_tile<true, true, T>(acc, A, N, Rj, N, A, N, Ri, N, kbase, t0, t0, active, sA0, sA1, sB0,
                              sB1);
     if (!active) return;
     gdouble_mut_t *C = (gdouble_mut_t *)A;
