@@ -65,12 +65,15 @@ def test_sosex_pairs(ctx, small, o, v, n, nt, precision, dev):
     conv = (lambda x: torch.from_numpy(x).cuda()) if dev else (lambda x: x)
     # the split pair kernel truncates at 2^-35 of the column maxima
     slack = 1e-7 if precision == "split_i8" else 0.0
+    # its slices are padded to tiles: the smallest take more than the explicit blocks, which
+    # then run all the same
+    pairs = precision == "fp64" or n > 40
     for s2, b in ((False, A), (True, A / (1.0 - 4.0 * A * A))):
         ref, tol = _sosex(R, V, b, o, v)
         call = lambda c: c.sosex(conv(V), conv(A), conv(R), o, v, s2_operator=s2,  # noqa: E731
                                  precision=precision)
         e, dots = small(call, _lib.KERNEL_SOSEX_DOT)
-        assert dots == 0 and abs(e - ref) <= tol + slack, (dots, e, ref)
+        assert (dots == 0) == pairs and abs(e - ref) <= tol + slack, (dots, e, ref)
         e = call(ctx)
         assert _launches(ctx, _lib.KERNEL_SOSEX_DOT) > 0 and abs(e - ref) <= tol, (e, ref)
 
@@ -112,7 +115,8 @@ def _thc_inputs(o, v, g, nt, seed):
 
 @pytest.mark.parametrize("o,v,g,nt", [(12, 45, 700, 540), (11, 49, 701, 539)])
 def test_thc_1b2g_fused(small, o, v, g, nt):
-    """The workspace tells the form: the explicit one takes 128 MB for split k."""
+    """The device memory that a context takes tells the form: 128 MB for split k and
+    more in the explicit one, beside what both take (rocBLAS's own among it)."""
     ins = _thc_inputs(o, v, g, nt, o + g)
     Z, X, Y, U, A = ins
     bound = (2 * g + 2 * o * v + v + o) * U_
@@ -128,7 +132,7 @@ def test_thc_1b2g_fused(small, o, v, g, nt):
     c = brpa.Context(0)
     explicit = call(c)
     c.close()
-    assert held[0] < 200 << 20 < held[1], held
+    assert held[1] - held[0] >= 128 << 20, held
     for m in range(nt):
         M, B = Y.T @ (U[m].T @ X), Y.abs().T @ (U[m].abs().T @ X.abs())
         a = float(A[m])
