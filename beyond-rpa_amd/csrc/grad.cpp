@@ -79,7 +79,6 @@ extern "C" int brpa_ecrpa_grad(brpa_ctx *ctx, const double *R, int64_t naux, con
     double *dRd, *ddR, *dc, *ddc, *X, *dd;
     double *Uinv;
     int64_t *dchol;
-    // matrices per batch of the triangular inverse: its scratch is X
     // frequencies per product M_k R^T: the number with the fewest rounds of tiles (two
     // work-groups per CU) over all F, within 2 GB of X.  N = 2400, K = 19200, F = 16: 2850
     // tiles each, 6 rounds of 512 (0.93 full); five together 28 (0.99): the gradient 122.6
@@ -94,7 +93,11 @@ extern "C" int brpa_ecrpa_grad(brpa_ctx *ctx, const double *R, int64_t naux, con
             kb = b;
         }
     }
-    const int64_t nbi = std::max<int64_t>(1, std::min<int64_t>({F, kb * K * N / trinv_scratch(N), 65535}));
+    // matrices per batch of the triangular inverse: its scratch is X
+    auto nbi_of = [&](int64_t k) {
+        return std::max<int64_t>(1, std::min<int64_t>({F, k * K * N / trinv_scratch(N), 65535}));
+    };
+    int64_t nbi = nbi_of(kb);
     auto layout = [&](Arena &ar) {
         dfd = ar.take<FragDev>(1);
         dpre = ar.take<int64_t>(pre.size());
@@ -119,6 +122,12 @@ extern "C" int brpa_ecrpa_grad(brpa_ctx *ctx, const double *R, int64_t naux, con
     };
     Arena count;
     layout(count);
+    if (kb > 1 && !ws_affords(ctx, count.off)) {
+        kb = 1;
+        nbi = nbi_of(kb);
+        count = Arena{};
+        layout(count);
+    }
     Arena ar;
     BRPA_TRY(ws_reserve(ctx, count.off, &ar));
     layout(ar);

@@ -162,8 +162,8 @@ int brpa_mbpt3_1(brpa_ctx *ctx, int precision, double *ec_exchange, const double
     const double *dV = V, *dA = A, *dR = R;
     double *dd, *W, *U, *Dm, *Vd, *Am, *Bm, *Bi, *T1, *ev_x, *work;
     int *ipiv, *info;
-    double *Fi, *tw, *splitws;
-    const int64_t nsplit = 16 << 20;   // split-k partials of k_gemm_f64
+    double *splitws;
+    int64_t nsplit = 16 << 20;   // split-k partials of k_gemm_f64, where affordable
     DenseChol ch;
     auto layout = [&](Arena &ar) {
         if (!vdev) dV = ar.take<double>(K * n);
@@ -182,13 +182,16 @@ int brpa_mbpt3_1(brpa_ctx *ctx, int precision, double *ec_exchange, const double
         work = ar.take<double>(n);
         ipiv = ar.take<int>(n);
         info = ar.take<int>(2);
-        Fi = ar.take<double>(n * n);
-        tw = ar.take<double>(trinv_scratch(n));
         splitws = ar.take<double>(nsplit);
         ch.layout(ar, n);
     };
     Arena count, ar;
     layout(count);
+    if (!ws_affords(ctx, count.off)) {
+        nsplit = 0;
+        count = Arena{};
+        layout(count);
+    }
     BRPA_TRY(ws_reserve(ctx, count.off, &ar));
     dV = V;
     dA = A;
@@ -226,7 +229,9 @@ int brpa_mbpt3_1(brpa_ctx *ctx, int precision, double *ec_exchange, const double
     // inverted (then LU decides): a breakdown, or r not down there after three steps.
     // Matrix products instead of rocSOLVER's column by column getrf / getri: 6.1 ms less per
     // inverse at n = 1200 (four inverses: MBPT3-1 of 36 to 11.5 ms).
+    // D and U are not needed any more: they hold F^{-1} and the inverse's scratch.
     auto inverse = [&](bool *done) -> int {
+        double *Fi = Dm, *tw = U;
         *done = false;
         BRPA_TRY(dense_syrk(ctx, true, n, n, 1.0, Bm, n, 0.0, T1, n));
         bool okc = false;

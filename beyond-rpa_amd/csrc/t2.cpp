@@ -256,14 +256,14 @@ int t2_build(brpa_ctx *ctx, int precision, const double *R, int64_t naux, const 
     const int64_t nsteps = cdiv(N, CHOL_NB);
     FragDev fd{};
     double *dR = nullptr, *dchi, *omega, *tmp, *iom, *Y, *Sm, *sev, *sE, *Uinv, *Rt;
-    double *DG = nullptr, *dcoef = nullptr, *tinv = nullptr, *splitws = nullptr;
+    double *DG = nullptr, *dcoef = nullptr, *splitws = nullptr;
     // FP64, NG < o*v: chi_k is folded into Rt_k and the F matrices are stacked to one
     // (F N) x K matrix, so that I Omega and T^T I T are two products each over kf
     // frequencies at a time (all of them, unless N kf NG passes 16 M elements)
     // instead of two per frequency.
     const bool stack = !split && !over;
-    const int64_t kf = std::max<int64_t>(1, std::min<int64_t>(F, (16 << 20) / (N * NG)));
-    const int64_t nsplit = over ? 0 : 16 << 20;   // split-k partials of k_gemm_f64
+    int64_t kf = std::max<int64_t>(1, std::min<int64_t>(F, (16 << 20) / (N * NG)));
+    int64_t nsplit = over ? 0 : 16 << 20;   // split-k partials of k_gemm_f64
     int *dinfo;
     int64_t *dchol = nullptr, *dchol2 = nullptr;
     FragDev fm{};                  // one dense matrix for the library's Cholesky
@@ -302,13 +302,10 @@ int t2_build(brpa_ctx *ctx, int precision, const double *R, int64_t naux, const 
         iom = ar.take<double>(K * NG);
         Y = over ? nullptr : ar.take<double>((stack ? kf : 1) * N * NG);
         if (stack) {
-            DG = ar.take<double>(kf * N * NG);
+            DG = kf > 1 ? ar.take<double>(kf * N * NG) : nullptr;
             dcoef = ar.take<double>(F * N);
         }
-        if (!over) {
-            tinv = ar.take<double>(trinv_scratch(NG));
-            splitws = ar.take<double>(nsplit);
-        }
+        splitws = nsplit > 0 ? ar.take<double>(nsplit) : nullptr;
         Sm = ar.take<double>(nd * nd);
         sev = ar.take<double>(nd);
         sE = ar.take<double>(nd);
@@ -337,6 +334,12 @@ int t2_build(brpa_ctx *ctx, int precision, const double *R, int64_t naux, const 
     };
     Arena count;
     layout(count);
+    if (!over && !ws_affords(ctx, count.off)) {
+        kf = 1;
+        nsplit = 0;
+        count = Arena{};
+        layout(count);
+    }
     Arena ar;
     BRPA_TRY(ws_reserve(ctx, count.off, &ar));
     layout(ar);
@@ -577,8 +580,9 @@ int t2_build(brpa_ctx *ctx, int precision, const double *R, int64_t naux, const 
                         return brpa_fail(ctx, BRPA_ERR_SOLVER,
                                          "Cholesky-QR pass %d of the T2 basis broke down", pass);
                 }
-                // X <- X U^{-1}, so that X^T X = 1, by the inverse and one triangular product
-                BRPA_TRY(dense_trinv(ctx, NG, Sm, NG, 0, omega, NG, 0, 1, tinv));
+                // X <- X U^{-1}, so that X^T X = 1, by the inverse (scratch: tmp, NG < K) and
+                // one triangular product
+                BRPA_TRY(dense_trinv(ctx, NG, Sm, NG, 0, omega, NG, 0, 1, tmp));
                 BRPA_TRY(launch_gemm_f64_batched(ctx, false, false, K, NG, NG, 1.0, iom, K, 0, 0,
                                                  omega, NG, 0, 0, 0.0, tmp, K, 0, 0, 1, 1, false,
                                                  TRI_B_UPPER, nullptr, 0, 0));
@@ -625,10 +629,15 @@ int t2_build(brpa_ctx *ctx, int precision, const double *R, int64_t naux, const 
                 const int64_t nr = std::min(kf, F - k) * N;
                 BRPA_TRY(dense_gemm(ctx, true, true, nt, nr, K, 1.0, Tkeep, K, Rt + k * N, FN, 0.0,
                                     G, nt));
-                BRPA_TRY(launch_col_scale(ctx, DG, G, dcoef + k * N, nt, nr));
-                BRPA_TRY(launch_gemm_f64_batched(ctx, false, true, nt, nt, nr, 1.0, G, nt, 0, 0, DG,
-                                                 nt, 0, 0, k == 0 ? 0.0 : 1.0, TIT, nt, 0, 0, 1, 1,
-                                                 true, TRI_NONE, nullptr, 0, 0));
+                const double *Gc = G;   // of one frequency the factor is a number
+                if (kf > 1) {
+                    BRPA_TRY(launch_col_scale(ctx, DG, G, dcoef + k * N, nt, nr));
+                    Gc = DG;
+                }
+                BRPA_TRY(launch_gemm_f64_batched(
+                    ctx, false, true, nt, nt, nr, kf > 1 ? 1.0 : -fw[k] * lambda / (4.0 * kPi), G, nt, 0,
+                    0, Gc, nt, 0, 0, k == 0 ? 0.0 : 1.0, TIT, nt, 0, 0, 1, 1, true, TRI_NONE, nullptr,
+                    0, 0));
             }
             if (stack) BRPA_TRY(dense_symm_fill(ctx, TIT, nt));
             BRPA_TRY(stage_end(ctx, BRPA_STAGE_T2_TIT));

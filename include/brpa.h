@@ -410,10 +410,9 @@ int brpa_ao_mo(brpa_ctx *ctx, double *CRG, const double *RG, int64_t nvecs, int6
  * a Cholesky factor of 1 + l Pi(u) built from R.  Guess vectors: uniform
  * (-1/2, 1/2) from a SplitMix64 counter hash of (seed, column, row), columns
  * normalised (the reference draws them from gfortran's RNG, 571-588).
- * precision: BRPA_FP64 (the drop-in: FP64 GEMMs; beside the operands 128 MB of
- * device scratch, an nguess x nguess block, and two more of 128 MB or
- * naux x nguess) or BRPA_SPLIT_I8: the
- * amplitude contractions R^T chi_k Omega, R Y_k and R^T chi_k T run as
+ * precision: BRPA_FP64 (the drop-in: FP64 GEMMs; beside the operands up to
+ * 384 MB of scratch for split k and products of several frequencies, where the
+ * workspace may grow to it: brpa_ctx_trim) or BRPA_SPLIT_I8: the amplitude contractions R^T chi_k Omega, R Y_k and R^T chi_k T run as
  * split-int8 GEMMs (5 int8 slices per value, 15 products, exact int32 level
  * sums, FP64 combination; nocc*nvir <= 65536); Pi(u), the Cholesky factors,
  * the solves, the Gram matrices and the amplitude core stay FP64. */
@@ -570,8 +569,9 @@ int brpa_dtrtri(brpa_ctx *ctx, int64_t n, int64_t nmat, const double *U, int64_t
 /* dE_RPA/dR (C R[ai][P], same shape as R) and dE_RPA/d(eps_occ), dE_RPA/d(eps_vir)
  * of the FP64 energy of brpa_ecrpa, with the frequency grid held fixed.  Pi(u)
  * of every frequency is recomputed in this call, never kept from the forward
- * pass; the call's device workspace holds 2 F N^2 + N K + O(F K) doubles,
- * plus N K for each of R and dR given as a host buffer (F = nfreqs,
+ * pass; the call's device workspace holds 2 F N^2 + N K + O(F K) doubles (N K
+ * for each of several frequencies, at most 2 GB, where the workspace may grow to
+ * it: brpa_ctx_trim), plus N K for each of R and dR given as a host buffer (F = nfreqs,
  * N = naux, K = nocc*nvir).  No reference counterpart: the
  * reference computes no RPA gradients.  deocc/devir may be NULL. */
 int brpa_ecrpa_grad(brpa_ctx *ctx, const double *R, int64_t naux, const double *eocc,

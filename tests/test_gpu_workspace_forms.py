@@ -2,6 +2,7 @@
 workspace may not grow that far (BRPA_WS_BUDGET_GB, else 3/4 of the free memory): same
 results, and the form that ran as the kernel times tell it.  A context of its own per
 case, since a workspace once held is used."""
+import ctypes as C
 import math
 
 import numpy as np
@@ -9,7 +10,7 @@ import pytest
 
 import brpa
 from brpa import _lib, synth
-from oracle import mbpt3
+from oracle import adjoint, erpa, grid, mbpt3, t2
 
 pytestmark = pytest.mark.gpu
 
@@ -34,10 +35,23 @@ def small(monkeypatch):
 
 
 def _launches(c, kernel):
-    import ctypes as C
     n = C.c_int64()
     assert c._lib.brpa_last_kernel_stats(c._h, kernel, None, None, C.byref(n)) == 0
     return n.value
+
+
+def _workspace(c, monkeypatch):
+    """Bytes of the context's workspace: the largest size that it affords without growing
+    (the library's own ws_affords)."""
+    affords = getattr(c._lib, "_Z10ws_affordsPK8brpa_ctxm")
+    affords.argtypes, affords.restype = [C.c_void_p, C.c_size_t], C.c_bool
+    with monkeypatch.context() as m:
+        m.setenv("BRPA_WS_BUDGET_GB", "0")
+        lo, hi = 0, 1 << 40
+        while hi - lo > 1:
+            mid = (lo + hi) // 2
+            lo, hi = (mid, hi) if affords(c._h, mid) else (lo, mid)
+    return lo
 
 
 def _amplitudes(o, v, n, nt, seed, s2=False):
@@ -114,25 +128,13 @@ def _thc_inputs(o, v, g, nt, seed):
 
 
 @pytest.mark.parametrize("o,v,g,nt", [(12, 45, 700, 540), (11, 49, 701, 539)])
-def test_thc_1b2g_fused(small, o, v, g, nt):
-    """The device memory that a context takes tells the form: 128 MB for split k and
-    more in the explicit one, beside what both take (rocBLAS's own among it)."""
+def test_thc_1b2g_fused(small, monkeypatch, o, v, g, nt):
+    """The workspace tells the form: 128 MB for split k and more in the explicit one."""
     ins = _thc_inputs(o, v, g, nt, o + g)
     Z, X, Y, U, A = ins
     bound = (2 * g + 2 * o * v + v + o) * U_
-    held = {}
-
-    def call(c):
-        free0 = torch.cuda.mem_get_info()[0]
-        out = c.thc_1b2g(*ins, want_diag=True)
-        held[len(held)] = free0 - torch.cuda.mem_get_info()[0]
-        return out
-
-    fused, _ = small(call, _lib.KERNEL_GEMM_F64)
-    c = brpa.Context(0)
-    explicit = call(c)
-    c.close()
-    assert held[1] - held[0] >= 128 << 20, held
+    fused, explicit, kept = _both(small, monkeypatch, lambda c: c.thc_1b2g(*ins, want_diag=True))
+    assert kept[1] - kept[0] >= 128 << 20, kept
     for m in range(nt):
         M, B = Y.T @ (U[m].T @ X), Y.abs().T @ (U[m].abs().T @ X.abs())
         a = float(A[m])
@@ -166,3 +168,68 @@ def test_thc_piu_chunks(ctx, small, o, v, n, g, launches):
         for P, r in ((Pi, R), (Pi0, R0)):
             bound = 2.0 * (o * v + 4) * U_ * (r.abs().T @ (c * r.abs()))
             assert bool(((P[w] - r.T @ (c * r)).abs() <= bound).all())
+
+
+def _both(small, monkeypatch, call):
+    """The call on a context without room and on one with it, and the bytes of workspace
+    that each holds afterwards."""
+    kept = []
+
+    def run(c):
+        out = call(c)
+        kept.append(_workspace(c, monkeypatch))
+        return out
+
+    lean, _ = small(run, _lib.KERNEL_GEMM_F64)
+    c = brpa.Context(0)
+    full = run(c)
+    c.close()
+    return lean, full, kept
+
+
+def test_grad_one_frequency_at_a_time(small, monkeypatch):
+    """Two frequencies per product take one K x N matrix (33 MB) more."""
+    o, v, n, nf = 10, 409, 1000, 5
+    f = synth.make_fragment(o, v, n, seed=23)
+    x, w, _ = grid.freq_grid(f.eocc, f.evir, 12)
+    x, w = x[:nf], w[:nf]
+    lean, full, kept = _both(small, monkeypatch,
+                             lambda c: c.ecrpa_grad(f.R, f.eocc, f.evir, x, w))
+    assert kept[1] - kept[0] >= 30 << 20, kept
+    for a, b, r in zip(lean, full, adjoint.ecrpa_grad(f.R, f.eocc, f.evir, x, w)):
+        assert max(np.max(np.abs(a - r)), np.max(np.abs(b - r))) <= 1e-10 * np.max(np.abs(r))
+
+
+def test_mbpt3_1_without_split(small, monkeypatch):
+    o, v, n, nt = 6, 40, 90, 70
+    f = synth.make_fragment(o, v, n, 12)
+    V = np.ascontiguousarray(np.linalg.qr(
+        np.random.default_rng(5).standard_normal((o * v, nt)))[0])
+    A = -np.linspace(0.3, 0.01, nt)
+    ref = mbpt3.mbpt3_1(f.R, V, A, o, v, f.eocc, f.evir)
+    lean, full, kept = _both(small, monkeypatch,
+                             lambda c: c.mbpt3_1(V, A, f.R, f.eocc, f.evir))
+    assert kept[1] - kept[0] >= 128 << 20, kept
+    assert max(abs(lean - ref), abs(full - ref)) <= 1e-10 * abs(ref)
+
+
+@pytest.mark.parametrize("o,v,n,nf,ng,neg", [(8, 40, 80, 12, 0, False), (5, 31, 33, 10, 65, True)])
+@pytest.mark.parametrize("precision", ["fp64", "split_i8"])
+def test_t2_without_stacks(small, monkeypatch, o, v, n, nf, ng, neg, precision):
+    """One frequency per product and no split k; the bounds of the oracle tests."""
+    f = synth.make_fragment(o, v, n, 103)
+    x, w, _ = grid.freq_grid(f.eocc, f.evir, nf)
+    if neg:
+        w[0] = -0.25 * w[0]
+    Pis = [erpa.gpiug_mo(f.R, f.gaps(), u) for u in x]
+    A_ref, V_ref = t2.t2_v5(f.R, f.gaps(), x, w, Pis, nguess=ng or None, seed=5)
+    T_ref = (V_ref * A_ref) @ V_ref.T
+    lean, full, kept = _both(small, monkeypatch, lambda c: c.t2(
+        f.R, f.eocc, f.evir, x, w, nguess=ng, seed=5, precision=precision))
+    assert kept[1] - kept[0] >= 128 << 20, kept
+    if precision == "split_i8":   # against its own result with the room
+        A_ref, T_ref = full[0], (full[1] * full[0]) @ full[1].T
+    for A, V in (lean, full):
+        assert len(A) == len(A_ref)
+        assert np.max(np.abs(A - A_ref)) <= 1e-9 * np.max(np.abs(A_ref))
+        assert np.max(np.abs((V * A) @ V.T - T_ref)) <= 1e-9 * np.max(np.abs(T_ref))
