@@ -1,6 +1,8 @@
 // Elementwise / reduction kernels of the amplitude (T2) and SOSEX paths.
 // Matrices here are column-major (the reference's Fortran layout): element
 // (r, c) of an m-row matrix is at r + m*c.
+#include <algorithm>
+
 #include "device_common.h"
 #include "internal.h"
 
@@ -59,18 +61,18 @@ int launch_normalize_columns(brpa_ctx *ctx, double *X, int64_t m, int64_t n) {
     return BRPA_OK;
 }
 
-// out(r, c) = s[r] * in(r, c)   (out may alias in)
+// out(r, c) = s[r] * in(r, c)   (out may alias in).  A grid holds fewer than 2^32 threads
+// (one of more is dropped without an error): from 2^30 elements on it walks on.
 __global__ void k_row_scale(double *out, const double *in, const double *__restrict__ s, int64_t m,
                             int64_t n) {
-    int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (e >= m * n) return;
-    out[e] = s[e % m] * in[e];
+    for (int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x; e < m * n; e += 256 * (int64_t)gridDim.x)
+        out[e] = s[e % m] * in[e];
 }
 
 int launch_row_scale(brpa_ctx *ctx, double *out, const double *in, const double *s, int64_t m,
                      int64_t n) {
     if (m * n <= 0) return BRPA_OK;
-    hipLaunchKernelGGL(k_row_scale, dim3(nblocks(m * n)), dim3(256), 0, ctx->stream, out, in, s, m, n);
+    hipLaunchKernelGGL(k_row_scale, dim3(nblocks(std::min(m * n, (int64_t)1 << 30))), dim3(256), 0, ctx->stream, out, in, s, m, n);
     LAUNCH_CHECK(ctx);
     return BRPA_OK;
 }
