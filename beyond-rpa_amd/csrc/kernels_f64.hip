@@ -454,50 +454,6 @@ int launch_set_diag(brpa_ctx *ctx, const FragDev *fr, const int64_t *pre, int nf
 // and after every outer panel of four steps k_chol_rest, the rest of A22 (launch_cholesky).
 // Work-groups per fragment: chol_items.
 
-template <int ROWS, int THREADS, int NP>
-__device__ __forceinline__ void load_panels64(double (*const *s)[CHOL_NB + 1],
-                                              const double *__restrict__ A, int64_t ld,
-                                              const int *row0, int rowmax, int col0, int colmax,
-                                              int tid) {
-    constexpr int PER = ROWS * CHOL_NB / THREADS;
-    constexpr int RSTEP = THREADS / CHOL_NB;
-    const int c = tid & (CHOL_NB - 1), r0 = tid / CHOL_NB;
-    const gdouble_t *G = (const gdouble_t *)A;
-    double v[NP][PER];
-#pragma unroll
-    for (int p = 0; p < NP; ++p)
-#pragma unroll
-        for (int u = 0; u < PER; ++u) {
-            const int r = r0 + RSTEP * u;
-            const bool ok = row0[p] + r < rowmax && col0 + c < colmax;
-            const int64_t idx = ok ? (int64_t)(row0[p] + r) * ld + col0 + c : 0;
-            v[p][u] = G[idx];
-            v[p][u] = ok ? v[p][u] : 0.0;
-        }
-#pragma unroll
-    for (int p = 0; p < NP; ++p)
-#pragma unroll
-        for (int u = 0; u < PER; ++u) s[p][r0 + RSTEP * u][c] = v[p][u];
-}
-
-template <int ROWS, int THREADS>
-__device__ __forceinline__ void load_panel64(double (*s)[CHOL_NB + 1], const double *__restrict__ A,
-                                             int64_t ld, int row0, int rowmax, int col0, int colmax,
-                                             int tid) {
-    double(*sp[1])[CHOL_NB + 1] = {s};
-    const int r[1] = {row0};
-    load_panels64<ROWS, THREADS, 1>(sp, A, ld, r, rowmax, col0, colmax, tid);
-}
-
-// ---------------------------------------------------------------------------
-// Panel body of the blocked Cholesky.  NT is the work-group size; every thread
-// calls the body (the barriers are uniform) and the work is guarded by the
-// thread index.
-
-// Number of L21 chunks of step j.
-// ---------------------------------------------------------------------------
-// Per-step kernels (flat work lists over fragments and frequencies)
-
 // 1 / p for p within 2^-1000 .. 2^1000: the hardware estimate and two Newton
 // steps (5 dependent instructions instead of the ~12 of a division)
 __device__ __forceinline__ double rcp_newton(double p) {
