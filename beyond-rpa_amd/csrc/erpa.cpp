@@ -555,11 +555,12 @@ int brpa_gpiug_mo(brpa_ctx *ctx, double *gpiug, const double *crg, int64_t naux,
     // GPiUG += CRG diag(W) CRG^T, half of it on the SYRK of the E_RPA pipeline.  One
     // frequency alone has few tiles, so the rows of R are cut into nk chunks, each a work
     // list entry with a partial product of its own, and k_syrk_acc adds them to both
-    // triangles: enough chunks for three work-groups per CU (N = 905, K = 3620, twelve calls and
-    // the rest of the MO route: 2693 us with one per CU, 2492 two, 2486 three, 2480 six), of
-    // 256 rows or more, and partial products of no more than R's own size.  Fewer rows than N: the reference's own
-    // shape (rpa_core_MO.f90:398-402), DCRG = CRG diag(W) and one plain dgemm.
-    // N = 905, K = 3620: 143 us by way of DCRG, 96 us.
+    // triangles: enough chunks for three work-groups per CU, but no more than K / 256 + 1, and
+    // partial products of no more than R's own size (K / N chunks).  N = 905, K = 3620,
+    // twelve calls and the rest of the MO route, without the last bound: 2693 us with one
+    // work-group per CU, 2492 two, 2486 three, 2480 six; it leaves four chunks, 480 work-groups,
+    // 78 us and 11 us for the sum (143 us by way of DCRG).  Fewer rows than N: the
+    // reference's own shape (rpa_core_MO.f90:398-402), DCRG = CRG diag(W) and one plain dgemm.
     const int64_t ncu = ctx->ncu > 0 ? ctx->ncu : 256, tiles = syrk_items(N, 1, true);
     const int64_t nk = std::min({cdiv(3 * ncu, tiles), K / 256 + 1, K / N});
     const int64_t kc = nk > 0 ? cdiv(cdiv(K, nk), 16) * 16 : 0;

@@ -173,9 +173,10 @@ int launch_split(brpa_ctx *ctx, const FragDev *fr, const int64_t *pre, int nfrag
 // rows are made under the MFMAs of the next one.  A wave above the diagonal of a
 // diagonal tile only stages.
 //
-// Bound by the bf16 matrix rate of ten products: 913 us at K = 4853, N = 1053, 16
-// frequencies, 1250 TFLOP/s bf16 (1408 us with the operands read behind the barrier and
-// every wave waiting for its loads there).
+// 913 us at K = 4853, N = 1053, 16 frequencies (1408 us with the operands read behind the
+// barrier and every wave waiting for its loads there): 1250 TFLOP/s of the 2000 to 2300
+// that MFMAs alone reach on random data, counting whole tiles.  Their area is 1.33 times
+// N (N + 1) / 2 there (waves past N multiply like the others): 940 TFLOP/s on the triangle.
 constexpr int T16 = 128;
 constexpr int KS = 32;          // rows per stage (one MFMA k-depth)
 

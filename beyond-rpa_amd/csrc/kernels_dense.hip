@@ -7,7 +7,7 @@
 //   k_gemm_f64          batched C = alpha op(A) op(B) diag(cs) + beta C on
 //                       128 x 128 tiles; upper mode (SYRK) and triangular
 //                       operands whose zero triangle is skipped; 16-k stages
-//                       loaded straight into LDS where alignment allows
+//                       loaded straight into LDS at any alignment of the doubles
 //   k_trinv_diag        inverses of the 64 x 64 diagonal blocks of upper
 //                       triangular matrices; with GEMM levels on top, the
 //                       batched triangular inverse (launch_trinv_f64)

@@ -224,8 +224,8 @@ __device__ __forceinline__ void syrk_f64_tile(const FragDev &F, int w0, int tp, 
     frags(a0, b0, 0, 0);
     // buf constant, arrays of their own: as in gemm_tile.h.  d: c_w of this stage, replaced by
     // that of the stage after the next as soon as it is used; loaded one stage ahead, just before
-    // the barrier that waits for it, it held up the quad form at every stage (K = 3620, N =
-    // 905 in seven chunks: 97 us instead of 86).
+    // the barrier that waits for it, it held up the quad form at every stage (840 work-groups
+    // of 517 rows: 97 us instead of 86).
     auto step = [&](int buf, int q, double (&d)[4]) {
         frags(a1, b1, buf, 1);
         mma(a0, b0, d[0], d[1]);
@@ -352,8 +352,8 @@ int launch_syrk_f64(brpa_ctx *ctx, const FragDev *fr, const int64_t *pre, int nf
 
 // 16 rows of a 64 x 64 tile pair per work-group: the sum of the partial tiles is added
 // to P as it is and, off the diagonal, transposed through LDS.  Bound by memory:
-// (nq / 2 + 2) N^2 doubles: 11 us at N = 905, nq = 7 (30 us with a whole tile pair per
-// work-group).
+// (nq / 2 + 2) N^2 doubles: 11 us at N = 905, nq = 4 and 7 (30 us with a whole tile pair
+// per work-group at 7).
 __global__ __launch_bounds__(256) void k_syrk_acc(double *__restrict__ P,
                                                  const double *__restrict__ S, int N, int nq) {
     __shared__ double sT[16][65];

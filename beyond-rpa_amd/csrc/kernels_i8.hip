@@ -454,13 +454,13 @@ __global__ __launch_bounds__(128) void k_syrk_i8_64(
 // over fragments of different K (one contiguous range of the grid per XCD did not: 1.4
 // times slower on the batch).
 //
-// Bound by the int8 matrix rate at the clock that it runs at (1.8 GHz under this load),
-// then the LDS reads (24 KB per wave and stage).  Measured at K = 10800, N = 1800, 24
-// frequencies: 3.80 ms (221 TFLOP/s FP64-equivalent; 4.19 ms with both stages in one
-// array, where the compiler made the first read after the loads wait for them, 4.43
-// without xcd, 5.97 with one LDS read or wait ahead of each group of MFMAs); 32
-// fragments of the batch shapes: 14.7 ms (16.5, 17.5, 23.8).  Loads of later stages into L2
-// ahead of their use made it no faster.
+// At K = 10800, N = 1800, 24 frequencies 3.80 ms (221 TFLOP/s FP64-equivalent): 2.7 POP/s
+// counting whole tiles, whose area is 1.21 times N (N + 1) / 2 there, of the 3.8 that the
+// MFMAs allow at the clock of this load (1.8 GHz); the LDS reads (24 KB per wave and stage)
+// come next.  Before: 4.19 ms with both stages in one array, where the compiler made the
+// first read after the loads wait for them, 4.43 without xcd, 5.97 with one LDS read or
+// wait ahead of each group of MFMAs.  32 fragments of the batch shapes: 14.7 ms (16.5,
+// 17.5, 23.8).  Loads of later stages into L2 ahead of their use made it no faster.
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_syrk_i8_128(
     const FragDev *__restrict__ fr, const int64_t *__restrict__ pre, int nfrag, int xcd) {
     constexpr int T = 128;

@@ -342,10 +342,12 @@ int brpa_ecrpa_packed(brpa_ctx *ctx, double *ecrpa, const double *piu_packed, co
  * closed shell, 2 per spin block of an open shell (rpa_THC.f90:254-266).
  * Rkai (may be NULL): receives R as Fortran Rkai(naux, nvir*nocc) == C
  * R[ai][P], the FullRkai = .true. output that the amplitudes read; NULL keeps R
- * inside the library (FullRkai = .false.).  R is built once in HBM by one FP64
- * MFMA kernel that forms Xga(g, a) Xgi(g, i) while loading its operand (no
- * ngrid x ov intermediate); the block size MaxBlockDim of the reference only
- * bounded its memory and has no counterpart.  Device times: stages
+ * inside the library (FullRkai = .false.).  R is built once in HBM: the products
+ * Xga(g, a) Xgi(g, i) of as many occupied i as 512 MB hold (of one at least), then
+ * R by the library's FP64 GEMM with up to 512 MB of split-k partials; 32 MB (or one
+ * column) of products and no partials where the workspace may not grow to that
+ * (brpa_ctx_trim).  The block size MaxBlockDim of the reference only bounded its
+ * memory and has no counterpart.  Device times: stages
  * BRPA_STAGE_THC_R and BRPA_STAGE_THC_PI. */
 int brpa_thc_piu(brpa_ctx *ctx, double *PiU, double *Rkai, const double *Xga, const double *Xgi,
                  const double *Zgk, int64_t ngrid, int64_t nocc, int64_t nvir, int64_t naux,
