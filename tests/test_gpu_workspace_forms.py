@@ -233,3 +233,19 @@ def test_t2_without_stacks(small, monkeypatch, o, v, n, nf, ng, neg, precision):
         assert len(A) == len(A_ref)
         assert np.max(np.abs(A - A_ref)) <= 1e-9 * np.max(np.abs(A_ref))
         assert np.max(np.abs((V * A) @ V.T - T_ref)) <= 1e-9 * np.max(np.abs(T_ref))
+
+
+def test_sosex_split_i8_pairs_large(ctx, small):
+    """The split-int8 pair kernel on a large fragment's own amplitudes (o=64, v=600,
+    NAux=3200, 16 frequencies, NT2 = 3 NAux) within 1e-7 Ha of the FP64 explicit form."""
+    o, v, n = 64, 600, 3200
+    f = synth.make_fragment(o, v, n, synth.BASE_SEED)
+    x, w, _ = grid.freq_grid(f.eocc, f.evir, 16)
+    R = torch.from_numpy(f.R).cuda()
+    A, V = ctx.t2(R, f.eocc, f.evir, x, w, nguess=3 * n, seed=1, device=True)
+    e = ctx.sosex(V, A, R, o, v)
+    assert _launches(ctx, _lib.KERNEL_SOSEX_DOT) > 0
+    ctx._lib.brpa_ctx_trim(ctx._h)
+    e8, dots = small(lambda c: c.sosex(V, A, R, o, v, precision="split_i8"), _lib.KERNEL_SOSEX_DOT)
+    print("E_x explicit %.10f  split-int8 pairs - explicit %.3e" % (e, e8 - e))
+    assert dots == 0 and abs(e8 - e) <= 1e-7
