@@ -101,19 +101,20 @@ int launch_ritz_resid(brpa_ctx *ctx, const double *AZ, const double *Z, const do
 // the full sum; only the upper triangle of G is read.  Otherwise all rows with
 // w = 2 (the block J, I adds the same).  One work-group per column c, so the
 // reads of G (column c) and of M (column c' = i v + b, rows j v + a) are contiguous
-// in a.  Fixed-order reduction (per-thread sums, wave butterfly, the waves in order).
+// in a.  Sums in double-double, as in the pair form (k_pair_dot), in a fixed order
+// (per-thread sums, wave butterfly, the waves in order).
 __global__ __launch_bounds__(256) void k_sosex_contract(const double *__restrict__ G, int64_t ldg,
                                                         int v, int ni,
                                                         const double *__restrict__ M, int64_t ldm,
                                                         double gamma, double delta,
                                                         double *__restrict__ part) {
-    __shared__ double sred[4];
+    __shared__ dd_t sred[4];
     const int64_t c = blockIdx.x;
     const int j = (int)(c / v), b = (int)(c - (int64_t)j * v);
     const double *__restrict__ Gc = G + ldg * c;
     const bool tri = ni == 0;
     const int iend = tri ? j + 1 : ni;
-    double s = 0.0;
+    dd_t s = {0.0, 0.0};
     for (int i = 0; i < iend; ++i) {
         const int amax = tri && i == j ? b + 1 : v;   // rows r = i v + a <= c
         const double *__restrict__ Mc = M + ldm * ((int64_t)i * v + b) + (int64_t)j * v;
@@ -122,14 +123,18 @@ __global__ __launch_bounds__(256) void k_sosex_contract(const double *__restrict
             const bool dg = tri && i == j && a == b;
             double t = gamma * Mc[a];
             if (dg) t += delta;
-            s = fma(dg ? Gr[a] : 2.0 * Gr[a], t, s);
+            s = dd_add(s, (dg ? Gr[a] : 2.0 * Gr[a]) * t);
         }
     }
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+    for (int off = 32; off > 0; off >>= 1)
+        s = dd_add(s, (dd_t){__shfl_xor(s.hi, off, 64), __shfl_xor(s.lo, off, 64)});
     if ((threadIdx.x & 63) == 0) sred[threadIdx.x >> 6] = s;
     __syncthreads();
-    if (threadIdx.x == 0) part[c] = (sred[0] + sred[1]) + (sred[2] + sred[3]);
+    if (threadIdx.x == 0) {
+        s = dd_add(dd_add(sred[0], sred[1]), dd_add(sred[2], sred[3]));
+        part[c] = s.hi + s.lo;
+    }
 }
 
 int launch_sosex_contract(brpa_ctx *ctx, const double *G, int64_t ldg, int64_t v, int64_t ni,
