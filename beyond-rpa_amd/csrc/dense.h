@@ -28,13 +28,14 @@ int dense_trsm_left_t(brpa_ctx *ctx, int64_t m, int64_t n, const double *U, int6
 // z1 < nb1, z2 < nb2 and X_z = X + z1 sX1 + z2 sX2 for every operand; upper:
 // only the tiles on or above the diagonal of C (m = n); tri: TRI_* (the zero
 // triangle of a triangular operand is skipped and must be stored as zeros);
-// cs may be null.
+// cs may be null.  chunk > 0: a sum takes at most that many k (rounded up to 16), as far as
+// the context's split scratch holds the partial sums.
 int launch_gemm_f64_batched(brpa_ctx *ctx, bool ta, bool tb, int64_t m, int64_t n, int64_t k,
                             double alpha, const double *A, int64_t lda, int64_t sA1, int64_t sA2,
                             const double *B, int64_t ldb, int64_t sB1, int64_t sB2, double beta,
                             double *C, int64_t ldc, int64_t sC1, int64_t sC2, int64_t nb1,
                             int64_t nb2, bool upper, int tri, const double *cs, int64_t scs1,
-                            int64_t scs2);
+                            int64_t scs2, int64_t chunk = 0);
 // W_z = U_z^{-1} for nmat upper triangular n x n matrices (U_z = U + z su, read
 // in its upper triangle only; W_z = W + z sw, written whole: upper triangle and
 // zeros below).  T: scratch of nmat * trinv_scratch(n) doubles.

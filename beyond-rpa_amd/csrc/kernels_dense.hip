@@ -241,7 +241,7 @@ int launch_gemm_f64_batched(brpa_ctx *ctx, bool ta, bool tb, int64_t m, int64_t 
                             const double *B, int64_t ldb, int64_t sB1, int64_t sB2, double beta,
                             double *C, int64_t ldc, int64_t sC1, int64_t sC2, int64_t nb1,
                             int64_t nb2, bool upper, int tri, const double *cs, int64_t scs1,
-                            int64_t scs2) {
+                            int64_t scs2, int64_t chunk) {
     if (m <= 0 || n <= 0 || nb1 <= 0 || nb2 <= 0) return BRPA_OK;
     if (m > INT32_MAX / 2 || n > INT32_MAX / 2 || k > INT32_MAX / 2 || (upper && m != n) ||
         nb2 > 65535 || tri < 0 || tri > TRI_B_LOWER)
@@ -294,7 +294,7 @@ int launch_gemm_f64_batched(brpa_ctx *ctx, bool ta, bool tb, int64_t m, int64_t 
     g.tail0 = (int)ntiles;
     g.kchunk = g.k;
     const int64_t wgs = ntiles * nb1 * nb2;
-    if (nb1 == 1 && nb2 == 1 && ctx->split_ws && g.k >= 512) {
+    if (nb1 == 1 && nb2 == 1 && ctx->split_ws && (g.k >= 512 || (chunk > 0 && g.k > chunk))) {
         // CUs of the context's stream (its share of the chip, or all of them)
         int ncu = ctx->ncu;
         if (ncu <= 0 &&
@@ -308,7 +308,13 @@ int launch_gemm_f64_batched(brpa_ctx *ctx, bool ta, bool tb, int64_t m, int64_t 
         int64_t bs = 1;
         const int64_t smax = std::min<int64_t>({8, g.k / 256,
                                                 (int64_t)(ctx->split_ws_cap / (size_t)(m * n))});
-        for (int64_t sp = 1; sp <= std::max<int64_t>(smax, 1); ++sp) {
+        int64_t smin = 1;
+        if (chunk > 0) {
+            const int64_t ck = (chunk + GKB - 1) / GKB * GKB;
+            smin = std::max<int64_t>(
+                1, std::min((g.k + ck - 1) / ck, (int64_t)(ctx->split_ws_cap / (size_t)(m * n))));
+        }
+        for (int64_t sp = smin; sp <= std::max(smax, smin); ++sp) {
             const double w = (double)(wgs * sp);
             const double eff = w / (slots * std::ceil(w / slots));
             const double cost = 1.0 / eff + (sp > 1 ? 48.0 * (double)(sp + 1) / (double)g.k : 0.0);
@@ -318,7 +324,7 @@ int launch_gemm_f64_batched(brpa_ctx *ctx, bool ta, bool tb, int64_t m, int64_t 
             }
         }
         const int64_t full = wgs / (int64_t)slots * (int64_t)slots, L = wgs - full;
-        const int64_t ts = L > 0 && full > 0 && tri == TRI_NONE && !far
+        const int64_t ts = smin == 1 && L > 0 && full > 0 && tri == TRI_NONE && !far
                                ? std::min<int64_t>({8, (int64_t)slots / L, g.k / 256,
                                                     (int64_t)(ctx->split_ws_cap / (size_t)(L * GT * GT))})
                                : 1;
@@ -376,7 +382,7 @@ int launch_gemm_f64(brpa_ctx *ctx, bool ta, bool tb, int64_t m, int64_t n, int64
                     double alpha, const double *A, int64_t lda, const double *B, int64_t ldb,
                     double beta, double *C, int64_t ldc, bool upper) {
     return launch_gemm_f64_batched(ctx, ta, tb, m, n, k, alpha, A, lda, 0, 0, B, ldb, 0, 0, beta,
-                                   C, ldc, 0, 0, 1, 1, upper, TRI_NONE, nullptr, 0, 0);
+                                   C, ldc, 0, 0, 1, 1, upper, TRI_NONE, nullptr, 0, 0, 0);
 }
 
 // ---------------------------------------------------------------------------
@@ -476,12 +482,12 @@ int launch_trinv_f64(brpa_ctx *ctx, int64_t n, const double *U, int64_t ldu, int
             BRPA_TRY(launch_gemm_f64_batched(
                 ctx, false, false, b, bb, bb, 1.0, U + r0 + ldu * (r0 + b), ldu, 2 * b * (1 + ldu),
                 su, W + (r0 + b) * (1 + ldw), ldw, 2 * b * (1 + ldw), sw, 0.0, Tp, b, b * b, sT2,
-                pt.cnt, nmat, false, TRI_B_UPPER, nullptr, 0, 0));
+                pt.cnt, nmat, false, TRI_B_UPPER, nullptr, 0, 0, 0));
             // W12 = -W11 T: W11 (b x b) upper
             BRPA_TRY(launch_gemm_f64_batched(
                 ctx, false, false, b, bb, b, -1.0, W + r0 * (1 + ldw), ldw, 2 * b * (1 + ldw), sw, Tp,
                 b, b * b, sT2, 0.0, W + r0 + ldw * (r0 + b), ldw, 2 * b * (1 + ldw), sw, pt.cnt,
-                nmat, false, TRI_A_UPPER, nullptr, 0, 0));
+                nmat, false, TRI_A_UPPER, nullptr, 0, 0, 0));
         }
     }
     return BRPA_OK;
