@@ -477,10 +477,14 @@ __device__ __forceinline__ double rcp_newton(double p) {
 //   L(p, p)^{-1}  from panel p itself, whose lanes 0 .. 15 would idle: rows of the
 //               identity below the block become those of L(p, p)^{-T}.  Panel 0 has no
 //               idle lanes; wave 2 inverts its block during panel 2.
+// The block's own diagonal, 1 + Pi, stays apart (T.diag) and S starts with zeros there:
+// the updates, small beside the 1, are summed by themselves and added to it once, when
+// the pivot is due.  Added to it one by one they leave an error of 26 x 2^-53 in E(u) at
+// N = 64, so 11; the addition costs 0.17 us a block (k_chol_step 28.2 us, 28.4 so).
 // chol_panels returns whether a pivot was not positive.
 //
 // Bound by latency: 64 pivots in a chain of broadcast, reciprocal, multiply and
-// multiply-add.  Measured on MI355X: 21300 cycles for the four panels (26600 by
+// multiply-add.  Measured on MI355X: 21700 cycles for the four panels (26600 by
 // readlane); a k_potrf_diag launch of 160 matrices 15 us (17.7; 61.3 for one left-looking
 // wave per matrix with rows of L from LDS, the square root and division in the chain
 // and the whole inverse by substitution).
@@ -491,6 +495,7 @@ struct CholLds {
     double S[CHOL_NB][CH_LP];
     double Xd[4][16][CH_XP];   // L(p, p)^{-1}
     double rdiag[CHOL_NB];
+    double diag[CHOL_NB];      // of the given block
 };
 
 // the block at (j0, j0): lower triangle only; rows and columns past nbj are those of
@@ -506,7 +511,11 @@ __device__ __forceinline__ void chol_load64(CholLds &T, const gdouble_t *G, int 
         v[u] = in ? v[u] : ((r >= nbj && lane == r) ? 1.0 : 0.0);
     }
 #pragma unroll
-    for (int u = 0; u < 16; ++u) T.S[wave + 4 * u][lane] = v[u];
+    for (int u = 0; u < 16; ++u) {
+        const int r = wave + 4 * u;
+        T.S[r][lane] = lane == r ? 0.0 : v[u];
+        if (lane == r) T.diag[r] = v[u];
+    }
 }
 
 // L(p, p)^{-1} by substitution (lane n: column n): x_i = (delta_in - sum_{k<i} L_ik x_k) / L_ii
@@ -592,15 +601,15 @@ __device__ __forceinline__ double row_bcast(double v) {
 // Pivot C: its reciprocal rp is given; that of pivot C + 1 (rcp_newton, in steps) is made
 // between the eliminations, five columns at a time.
 template <int C>
-__device__ __forceinline__ void chol_pivots(double (&d)[16], double (&a)[16], double piv, double rp,
-                                            double &mypiv, bool &inrange, int l16) {
+__device__ __forceinline__ void chol_pivots(double (&d)[16], double (&a)[16], double dg, double piv,
+                                            double rp, double &mypiv, bool &inrange, int l16) {
     inrange = inrange && piv >= 0x1p-1000 && piv <= 0x1p+1000;
     mypiv = l16 == C ? piv : mypiv;
     if constexpr (C < 15) {
         constexpr int R = 15 - C, N1 = R < 5 ? R : 5, N2 = R - N1 < 5 ? R - N1 : 5, N3 = R - N1 - N2;
         const double ma = -(a[C] * rp), md = -(d[C] * rp);
         chol_eliminate<C + 1, N1>(d, a, d[C], md, ma);
-        const double p1 = row_bcast<C + 1>(d[C + 1]);
+        const double p1 = row_bcast<C + 1>(dg + d[C + 1]);
         double r1 = __builtin_amdgcn_rcp(p1);
         __builtin_amdgcn_sched_barrier(0);
         chol_eliminate<C + 1 + N1, N2>(d, a, d[C], md, ma);
@@ -608,7 +617,7 @@ __device__ __forceinline__ void chol_pivots(double (&d)[16], double (&a)[16], do
         __builtin_amdgcn_sched_barrier(0);
         chol_eliminate<C + 1 + N1 + N2, N3>(d, a, d[C], md, ma);
         r1 = fma(fma(-p1, r1, 1.0), r1, r1);
-        chol_pivots<C + 1>(d, a, p1, r1, mypiv, inrange, l16);
+        chol_pivots<C + 1>(d, a, dg, p1, r1, mypiv, inrange, l16);
     }
 }
 template <int C>
@@ -643,15 +652,15 @@ __device__ __forceinline__ bool chol_panels(CholLds &T, int lane) {
         double mypiv = 1.0;
         bool inrange = true;
         // lanes above row j update entries that are never read
-        const double p0 = row_bcast<0>(d[0]);
-        chol_pivots<0>(d, a, p0, rcp_newton(p0), mypiv, inrange, l16);
+        const double dg = T.diag[16 * p + l16], p0 = row_bcast<0>(dg + d[0]);
+        chol_pivots<0>(d, a, dg, p0, rcp_newton(p0), mypiv, inrange, l16);
         if (!inrange) {
             // a pivot that is not positive, or outside the range of rcp_newton: the
             // panel again, on its columns in LDS, with divisions
 #pragma unroll 1
             for (int c = 0; c < 16; ++c) {
                 const int pc = 16 * p + c;
-                double piv = S[pc][pc];
+                double piv = T.diag[pc] + S[pc][pc];
                 if (!(piv > 0.0) || !isfinite(piv)) {
                     bad = true;
                     piv = 1.0;
